@@ -586,6 +586,7 @@ struct akx_batch {
   bool lists_dirty = true, inst_dirty = true;
   // launch shape
   int block = 256, tile = 2048, blocks_per_cu = 0, cus = 256;
+  bool launch_chosen = false; // set by set_launch or the autotuner
   bool use_graph = true;
   hipGraphExec_t graph = nullptr;
   // timing
@@ -646,12 +647,37 @@ void upload_inst(akx_batch *b) {
   b->inst_dirty = false;
 }
 
+// Elements per tile of a group of n elements whose workgroups walk their tile
+// (groups without block tables).  A shape the caller or the autotuner chose
+// is used as it is.  Otherwise Tet4 takes one element per lane, and Hex8 up
+// to four groups of 32 elements (they run one after another; a workgroup
+// fills the dN/dxi table once), fewer while the CUs would get less than five
+// workgroups each.  Steps of FP64 batches, us, by tile:
+//   Hex8 neo-Hookean     64    128    256    512   2048 (the former tile)
+//     5,700 elements   20.4   30.2   50.2   89.9    331
+//     170,000           110    103    105    145    364
+//     2.1 M            1016   1020   1024   1044   1262
+//   Tet4 plastic, 1.06 M  207  199    187    209    243
+//                 4.5 M   840  793    728    811    868
+int64_t group_tile(const akx_batch *b, int etype, int64_t n) {
+  if (b->launch_chosen)
+    return b->tile;
+  if (etype == AKX_TET4)
+    return std::min(b->block, b->tile);
+  const int64_t t = n / (5 * (int64_t)b->cus) / 32 * 32;
+  return std::max<int64_t>(32, std::min<int64_t>(t, 128));
+}
+
 // work lists of the live instances: element tiles per group, node slices
 void rebuild_lists(akx_batch *b) {
   std::vector<std::vector<BTile>> groups(NGROUP);
   std::vector<std::vector<BBlk>> gblks(NGROUP);
   std::vector<BSlice> slices;
   b->bmaxu_live = 0;
+  int64_t group_n[NGROUP] = {0};
+  for (const HostInst &I : b->inst)
+    if (I.live)
+      group_n[I.etype * 4 + I.law] += I.nel; // elements of each group
   for (size_t id = 0; id < b->inst.size(); ++id) {
     const HostInst &I = b->inst[id];
     if (!I.live)
@@ -670,8 +696,9 @@ void rebuild_lists(akx_batch *b) {
           b->bmaxu_live = std::max(b->bmaxu_live, I.blk_cnt[k]);
       }
     } else {
-      for (int64_t f = 0; f < I.nel; f += b->tile) {
-        G.push_back({I.elem0 + f, (int32_t)std::min<int64_t>(b->tile, I.nel - f), (int32_t)id});
+      const int64_t tile = group_tile(b, I.etype, group_n[I.etype * 4 + I.law]);
+      for (int64_t f = 0; f < I.nel; f += tile) {
+        G.push_back({I.elem0 + f, (int32_t)std::min<int64_t>(tile, I.nel - f), (int32_t)id});
         GB.push_back({0, 0, 0});
       }
     }
@@ -1538,6 +1565,7 @@ int akx_batch_set_launch(akx_batch *b, int block, int tile, int blocks_per_cu,
     b->tile = tile;
     b->blocks_per_cu = blocks_per_cu;
     b->use_graph = use_graph != 0;
+    b->launch_chosen = true;
     b->lists_dirty = true;
   });
 }
@@ -1573,6 +1601,7 @@ int akx_batch_autotune(akx_batch *b, int repeats, int *block, int *tile,
     const int blocks[3] = {64, 128, 256};
     const int tiles[5] = {256, 512, 1024, 2048, 4096};
     const int bpcs[1] = {0}; // one tile per workgroup: no persistent blocks
+    b->launch_chosen = true;
     double best = 1e300;
     int bb = b->block, bt = b->tile, bc = b->blocks_per_cu;
     hipEvent_t e0, e1;

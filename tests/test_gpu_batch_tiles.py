@@ -1,0 +1,38 @@
+"""FP64 batches under the default launch shape: the tile of a group follows
+its element count (32, 64, 96 or 128 Hex8 per workgroup), one tile per
+workgroup, instances whose last tile is ragged.  The arithmetic of an element
+does not depend on its tile, so every instance keeps the bits it has under a
+chosen shape (setLaunch), whose results the other batch tests compare with
+the oracle."""
+import numpy as np
+import pytest
+
+from akantu2_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+# cells of the Hex8 instances: few elements (tile 32), then totals about
+# 5 x 256 x 64 and 5 x 256 x 128 elements, with ragged last tiles
+SETS = [[(2, 1, 1)], [(33, 1, 1), (5, 3, 2)], [(43, 43, 45), (7, 3, 2)],
+        [(55, 54, 56), (31, 3, 3)]]
+
+
+@pytest.mark.parametrize("cells", SETS, ids=lambda s: "x".join(map(str, s[0])))
+def test_default_tiles_keep_the_bits(cells):
+    from akantu2_amd.batch import Batch
+
+    def steps(launch):
+        meshes = [M.box_mesh("_hexahedron_8", *c, jitter=0.1, seed=3) for c in cells]
+        meshes.append(M.box_mesh("_tetrahedron_4", 7, 2, 3, jitter=0.1, seed=4))
+        b = Batch("fp64", nodes=sum(m.nb_nodes + 255 for m in meshes),
+                  tets=meshes[-1].nb_elements, hexes=sum(m.nb_elements for m in meshes[:-1]))
+        if launch:
+            b.setLaunch(**launch)
+        ids = [b.add(m, "neohookean", E=1.3, nu=0.31, blocked=M.clamped_face_x0(m),
+                     velocity=M.initial_velocity(m, 1e-3, 5)) for m in meshes]
+        b.solveStep(4)
+        return [b.get(i, f) for i in ids for f in ("displacement", "velocity",
+                                                   "internal_force")]
+
+    for got, want in zip(steps(None), steps(dict(block=64, tile=64))):
+        assert np.array_equal(got, want)
