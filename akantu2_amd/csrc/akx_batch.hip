@@ -37,6 +37,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <type_traits>
 #include <vector>
 
 namespace akx {
@@ -117,96 +118,101 @@ struct BatchGatherArgs {
 
 // One 256-node slice per workgroup (a persistent loop over slices measured
 // 8% slower: each wave walked its slices' dependent loads one after another).
-template <class FT, bool PREDICT, bool COMP>
+// FEW: the nodal state ahead of the entries, eight entries at a time
+// (sum_entries), for up to GATHER_FEW_NODES nodes.
+template <class FT, bool PREDICT, bool COMP, bool FEW>
 __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs G) {
-  {
-    const int64_t s = blockIdx.x;
-    if (s >= G.nslices)
-      return;
-    const BSlice SL = G.slices[s];
-    if ((int)threadIdx.x >= SL.count)
-      return;
-    const double dt = G.inst[SL.inst].dt;
-    const bool urec = G.inst[SL.inst].urec != 0;
-    const int64_t n = SL.node0 + threadIdx.x;
-    const FT *p = reinterpret_cast<const FT *>(G.fe) + (G.ell_off[n >> 8] + (n & 255)) * FE_W;
-    double f[3] = {0., 0., 0.};
-    const int deg = G.deg[n];
-    for (int d = 0; d < deg; ++d, p += 256 * FE_W) {
-      double e0, e1, e2;
-      if constexpr (FE_W == 3) { // read once per step: non-temporal
-        e0 = __builtin_nontemporal_load(p);
-        e1 = __builtin_nontemporal_load(p + 1);
-        e2 = __builtin_nontemporal_load(p + 2);
-      } else if constexpr (sizeof(FT) == 4) {
-        const float4 v = *reinterpret_cast<const float4 *>(p);
-        e0 = v.x;
-        e1 = v.y;
-        e2 = v.z;
-      } else {
-        const double2 v0 = reinterpret_cast<const double2 *>(p)[0];
-        const double2 v1 = reinterpret_cast<const double2 *>(p)[1];
-        e0 = v0.x;
-        e1 = v0.y;
-        e2 = v1.x;
-      }
-      f[0] = f[0] + -1. * e0;
-      f[1] = f[1] + -1. * e1;
-      f[2] = f[2] + -1. * e2;
+  static_assert(FE_W == 3, "sum_entries reads three values per entry");
+  const int64_t s = blockIdx.x;
+  if (s >= G.nslices)
+    return;
+  const BSlice SL = G.slices[s];
+  if ((int)threadIdx.x >= SL.count)
+    return;
+  const double dt = G.inst[SL.inst].dt;
+  const bool urec = G.inst[SL.inst].urec != 0;
+  const int64_t n = SL.node0 + threadIdx.x;
+  const FT *p = reinterpret_cast<const FT *>(G.fe) + (G.ell_off[n >> 8] + (n & 255)) * FE_W;
+  const int deg = G.deg[n];
+  double M = 0., v0[3], a0[3];
+  float cv0[3], cu0[3];
+  uint8_t blk = 0;
+  // u of the node's record (u0 at 48 n + 24 bytes, then an aligned pair)
+  // or of the [3][ncap] array, read and written whole; blocked components
+  // keep their value
+  double us[3] = {0., 0., 0.};
+  auto load_u = [&] {
+    if (urec) {
+      const double2 u12 = *reinterpret_cast<const double2 *>(G.xu + 6 * n + 4);
+      us[0] = G.xu[6 * n + 3];
+      us[1] = u12.x;
+      us[2] = u12.y;
+    } else {
+      us[0] = G.u[n];
+      us[1] = G.u[G.ncap + n];
+      us[2] = G.u[2 * G.ncap + n];
     }
-    const double M = G.mass[n];
-    const uint8_t blk = G.blocked[n];
-    // u of the node's record (u0 at 48 n + 24 bytes, then an aligned pair)
-    // or of the [3][ncap] array, read and written whole; blocked components
-    // keep their value
-    double us[3] = {0., 0., 0.};
-    if constexpr (PREDICT) {
-      if (urec) {
-        const double2 u12 = *reinterpret_cast<const double2 *>(G.xu + 6 * n + 4);
-        us[0] = G.xu[6 * n + 3];
-        us[1] = u12.x;
-        us[2] = u12.y;
-      } else {
-        us[0] = G.u[n];
-        us[1] = G.u[G.ncap + n];
-        us[2] = G.u[2 * G.ncap + n];
-      }
-    }
+  };
+  if constexpr (FEW) {
+    M = G.mass[n];
+    blk = G.blocked[n];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       const int64_t o = (int64_t)c * G.ncap + n;
-      if (G.fint) // null while more steps follow in the same call
-        G.fint[o] = f[c];
-      if ((blk >> c) & 1)
-        continue;
-      if constexpr (COMP) { // FP32 form: half-step velocity (akx_math.hpp)
-        double w = G.v[o], a;
-        float cw = G.cv[o], cu = 0.f;
+      v0[c] = G.v[o];
+      if constexpr (COMP) {
+        cv0[c] = G.cv[o];
         if constexpr (PREDICT)
-          cu = G.cu[o];
-        half_step_gather<PREDICT>(f[c], M, dt, w, cw, us[c], cu, a);
-        if constexpr (PREDICT)
-          G.cu[o] = cu;
-        else
-          G.a[o] = a;
-        G.v[o] = w;
-        G.cv[o] = cw;
-      } else { // reference order, zero external force (akx_math.hpp)
-        double a = G.a[o], v = G.v[o];
-        reference_gather<PREDICT>(0., f[c], M, dt, a, v, us[c]);
-        G.a[o] = a;
-        G.v[o] = v;
+          cu0[c] = G.cu[o];
+      } else {
+        a0[c] = G.a[o];
       }
     }
-    if constexpr (PREDICT) {
-      if (urec) {
-        G.xu[6 * n + 3] = us[0];
-        *reinterpret_cast<double2 *>(G.xu + 6 * n + 4) = make_double2(us[1], us[2]);
-      } else {
-        G.u[n] = us[0];
-        G.u[G.ncap + n] = us[1];
-        G.u[2 * G.ncap + n] = us[2];
-      }
+    if constexpr (PREDICT)
+      load_u();
+  }
+  double f[3];
+  sum_entries<FEW, FE_W>(p, deg, f);
+  if constexpr (!FEW) {
+    M = G.mass[n];
+    blk = G.blocked[n];
+    if constexpr (PREDICT)
+      load_u();
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const int64_t o = (int64_t)c * G.ncap + n;
+    if (G.fint) // null while more steps follow in the same call
+      G.fint[o] = f[c];
+    if ((blk >> c) & 1)
+      continue;
+    if constexpr (COMP) { // FP32 form: half-step velocity (akx_math.hpp)
+      double w = FEW ? v0[c] : G.v[o], a;
+      float cw = FEW ? cv0[c] : G.cv[o], cu = 0.f;
+      if constexpr (PREDICT)
+        cu = FEW ? cu0[c] : G.cu[o];
+      half_step_gather<PREDICT>(f[c], M, dt, w, cw, us[c], cu, a);
+      if constexpr (PREDICT)
+        G.cu[o] = cu;
+      else
+        G.a[o] = a;
+      G.v[o] = w;
+      G.cv[o] = cw;
+    } else { // reference order, zero external force (akx_math.hpp)
+      double a = FEW ? a0[c] : G.a[o], v = FEW ? v0[c] : G.v[o];
+      reference_gather<PREDICT>(0., f[c], M, dt, a, v, us[c]);
+      G.a[o] = a;
+      G.v[o] = v;
+    }
+  }
+  if constexpr (PREDICT) {
+    if (urec) {
+      G.xu[6 * n + 3] = us[0];
+      *reinterpret_cast<double2 *>(G.xu + 6 * n + 4) = make_double2(us[1], us[2]);
+    } else {
+      G.u[n] = us[0];
+      G.u[G.ncap + n] = us[1];
+      G.u[2 * G.ncap + n] = us[2];
     }
   }
 }
@@ -847,17 +853,23 @@ void gather_pass(akx_batch *b, bool predict) {
   if (predict)
     G.fint = nullptr;
   dim3 grid((unsigned)G.nblocks), block(256);
-  if (b->fp32()) {
-    if (predict)
-      hipLaunchKernelGGL((k_batch_gather<float, true, true>), grid, block, 0, b->stream, G);
+  auto launch = [&](auto few) {
+    constexpr bool FEW = decltype(few)::value;
+    if (b->fp32() && predict)
+      hipLaunchKernelGGL((k_batch_gather<float, true, true, FEW>), grid, block, 0, b->stream, G);
+    else if (b->fp32())
+      hipLaunchKernelGGL((k_batch_gather<float, false, true, FEW>), grid, block, 0, b->stream, G);
+    else if (predict)
+      hipLaunchKernelGGL((k_batch_gather<double, true, false, FEW>), grid, block, 0, b->stream,
+                         G);
     else
-      hipLaunchKernelGGL((k_batch_gather<float, false, true>), grid, block, 0, b->stream, G);
-  } else {
-    if (predict)
-      hipLaunchKernelGGL((k_batch_gather<double, true, false>), grid, block, 0, b->stream, G);
-    else
-      hipLaunchKernelGGL((k_batch_gather<double, false, false>), grid, block, 0, b->stream, G);
-  }
+      hipLaunchKernelGGL((k_batch_gather<double, false, false, FEW>), grid, block, 0, b->stream,
+                         G);
+  };
+  if (256 * G.nslices <= GATHER_FEW_NODES)
+    launch(std::true_type{});
+  else
+    launch(std::false_type{});
   HIPCHECK(hipGetLastError());
 }
 

@@ -953,32 +953,93 @@ struct GatherArgs {
   int64_t nblocks_padded;
 };
 
-template <class FT, bool UPDATE, bool PREDICT, bool COMP>
+// Sum of the entries d = 0 .. deg - 1 of a node, f = (0 + -1 e_0) + -1 e_1 ...
+// The table is read once per step: non-temporal loads keep it from displacing
+// the nodal state in the caches.  FEW: eight entries are loaded before the
+// first is added (the loads past the last entry repeat it and are not added),
+// so a node waits for one or two round trips instead of one per entry.
+template <bool FEW, int W, class FT>
+__device__ __forceinline__ void sum_entries(const FT *p, int deg, double (&f)[3]) {
+  f[0] = f[1] = f[2] = 0.;
+  if constexpr (FEW) {
+    constexpr int CH = 8;
+    for (int d0 = 0; d0 < deg; d0 += CH) {
+      FT e[CH][3];
+#pragma unroll
+      for (int j = 0; j < CH; ++j) {
+        const FT *q = p + (int64_t)(d0 + j < deg ? d0 + j : deg - 1) * (256 * W);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          e[j][c] = __builtin_nontemporal_load(q + c);
+      }
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+        if (d0 + j < deg)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            f[c] = f[c] + -1. * double(e[j][c]);
+    }
+  } else {
+    for (int d = 0; d < deg; ++d, p += 256 * W)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        f[c] = f[c] + -1. * double(__builtin_nontemporal_load(p + c));
+  }
+}
+
+// Up to this many nodes a gather reads its nodal state ahead of the entries
+// and the entries eight at a time (FEW).  With one wave per SIMD or less
+// (1,024 SIMDs x 64 nodes) its time is one node's chain of dependent loads;
+// above, the plain loop's other waves hide that chain, and the repeated loads
+// of the short chunks cost.  Step before -> with FEW, us: 525 nodes (1,920
+// Tet4) 14.1 -> 11.6, 1,331 (Hex8, FP64) 11.4 -> 10.3, 6,975 (plastic Tet4)
+// 19.9 -> 17.0; 158,661 nodes (FP64 Tet4) 46.0 -> 49.0.
+constexpr int64_t GATHER_FEW_NODES = 1024 * 64;
+
+template <class FT, bool UPDATE, bool PREDICT, bool COMP, bool FEW = false>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
   const int64_t n = A.node0 + xcd_block(A.nblocks_padded) * blockDim.x + threadIdx.x;
   if (n >= A.node_end)
     return;
   const FT *fe = reinterpret_cast<const FT *>(A.fe);
-  double f0 = 0., f1 = 0., f2 = 0.;
   const int deg = A.deg[n];
   const FT *p = fe + (A.ell_off[n >> 8] + (n & 255)) * 3;
-  // the table is read once per step: non-temporal loads keep it from
-  // displacing the nodal state in the caches
-  for (int d = 0; d < deg; ++d, p += 256 * 3) {
-    f0 = f0 + -1. * double(__builtin_nontemporal_load(p));
-    f1 = f1 + -1. * double(__builtin_nontemporal_load(p + 1));
-    f2 = f2 + -1. * double(__builtin_nontemporal_load(p + 2));
+  // FEW: the nodal state ahead of the entries
+  double M = 0., v0[3], a0[3], u0[3], x0[3];
+  float cv0[3], cu0[3];
+  uint8_t blk = 0;
+  if constexpr (UPDATE && FEW) {
+    M = A.mass[n];
+    blk = A.blocked[n];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int64_t o = (int64_t)c * A.nn + n;
+      v0[c] = A.v[o];
+      if constexpr (PREDICT)
+        u0[c] = A.u[o];
+      if constexpr (COMP) {
+        cv0[c] = A.cv[o];
+        if constexpr (PREDICT)
+          cu0[c] = A.cu[o];
+      } else {
+        a0[c] = A.a[o];
+      }
+      x0[c] = A.fext ? A.fext[o] : 0.;
+    }
   }
+  double f[3];
+  sum_entries<FEW, 3>(p, deg, f);
   if (A.fint) { // null while more steps follow in the same batch
-    A.fint[n] = f0;
-    A.fint[A.nn + n] = f1;
-    A.fint[2 * A.nn + n] = f2;
+    A.fint[n] = f[0];
+    A.fint[A.nn + n] = f[1];
+    A.fint[2 * A.nn + n] = f[2];
   }
   if constexpr (!UPDATE)
     return;
-  const double M = A.mass[n];
-  const uint8_t blk = A.blocked[n];
-  double f[3] = {f0, f1, f2};
+  if constexpr (!FEW) {
+    M = A.mass[n];
+    blk = A.blocked[n];
+  }
   // u after the predictor (blocked components keep theirs), for the record
   double un[3] = {0., 0., 0.};
   if constexpr (PREDICT) {
@@ -993,13 +1054,13 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
     if ((blk >> c) & 1)
       continue;
     const int64_t o = (int64_t)c * A.nn + n;
-    const double fx = A.fext ? A.fext[o] : 0.;
+    const double fx = FEW ? x0[c] : A.fext ? A.fext[o] : 0.;
     if constexpr (COMP) { // FP32 form: half-step velocity (akx_math.hpp)
-      double w = A.v[o], a, u = 0.;
-      float cw = A.cv[o], cu = 0.f;
+      double w = FEW ? v0[c] : A.v[o], a, u = 0.;
+      float cw = FEW ? cv0[c] : A.cv[o], cu = 0.f;
       if constexpr (PREDICT) {
-        u = A.u[o];
-        cu = A.cu[o];
+        u = FEW ? u0[c] : A.u[o];
+        cu = FEW ? cu0[c] : A.cu[o];
       }
       half_step_gather<PREDICT>(fx + f[c], M, A.dt, w, cw, u, cu, a);
       if constexpr (PREDICT) {
@@ -1012,9 +1073,9 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
       A.v[o] = w;
       A.cv[o] = cw;
     } else { // reference order (akx_math.hpp)
-      double a = A.a[o], v = A.v[o], u = 0.;
+      double a = FEW ? a0[c] : A.a[o], v = FEW ? v0[c] : A.v[o], u = 0.;
       if constexpr (PREDICT)
-        u = A.u[o];
+        u = FEW ? u0[c] : A.u[o];
       reference_gather<PREDICT>(fx, f[c], M, A.dt, a, v, u);
       if constexpr (PREDICT) {
         A.u[o] = u;

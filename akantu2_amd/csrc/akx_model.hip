@@ -1509,6 +1509,30 @@ GatherArgs gather_args(akx_model *m, bool per_corner = false) {
   return G;
 }
 
+template <class FT, bool COMP, bool FEW>
+void launch_gather_form(const GatherArgs &G, bool update, bool predict, hipStream_t s) {
+  const dim3 grid((unsigned)G.nblocks_padded), block(TPB);
+  if (!update)
+    hipLaunchKernelGGL((k_gather_update<FT, false, false, false, FEW>), grid, block, 0, s, G);
+  else if (predict)
+    hipLaunchKernelGGL((k_gather_update<FT, true, true, COMP, FEW>), grid, block, 0, s, G);
+  else
+    hipLaunchKernelGGL((k_gather_update<FT, true, false, COMP, FEW>), grid, block, 0, s, G);
+}
+
+void launch_gather_kernel(const GatherArgs &G, bool f64, bool update, bool predict,
+                          hipStream_t s) {
+  const bool few = G.node_end - G.node0 <= GATHER_FEW_NODES;
+  if (f64 && few)
+    launch_gather_form<double, false, true>(G, update, predict, s);
+  else if (f64)
+    launch_gather_form<double, false, false>(G, update, predict, s);
+  else if (few)
+    launch_gather_form<float, true, true>(G, update, predict, s);
+  else
+    launch_gather_form<float, true, false>(G, update, predict, s);
+}
+
 // f_int is stored by the last step of a solve_step call (and by the gathers
 // without update): the steps in between use it only inside the gather, and
 // nothing reads the stored array before the call returns.
@@ -1516,33 +1540,9 @@ void launch_gather(akx_model *m, bool update, bool predict) {
   GatherArgs G = gather_args(m);
   if (update && predict)
     G.fint = nullptr;
-  dim3 grid((unsigned)G.nblocks_padded), block(TPB);
   const bool f64 = m->precision != AKX_PRECISION_FP32;
   check_gather_args(G, update, update && !f64);
-  m->timed(1, [&] {
-    if (!update) {
-      if (f64)
-        hipLaunchKernelGGL((k_gather_update<double, false, false, false>), grid,
-                           block, 0, m->stream, G);
-      else
-        hipLaunchKernelGGL((k_gather_update<float, false, false, false>), grid,
-                           block, 0, m->stream, G);
-    } else if (f64) {
-      if (predict)
-        hipLaunchKernelGGL((k_gather_update<double, true, true, false>), grid,
-                           block, 0, m->stream, G);
-      else
-        hipLaunchKernelGGL((k_gather_update<double, true, false, false>), grid,
-                           block, 0, m->stream, G);
-    } else {
-      if (predict)
-        hipLaunchKernelGGL((k_gather_update<float, true, true, true>), grid,
-                           block, 0, m->stream, G);
-      else
-        hipLaunchKernelGGL((k_gather_update<float, true, false, true>), grid,
-                           block, 0, m->stream, G);
-    }
-  });
+  m->timed(1, [&] { launch_gather_kernel(G, f64, update, predict, m->stream); });
   HIPCHECK(hipGetLastError());
 }
 
@@ -1697,22 +1697,7 @@ void launch_gather_group(akx_model *m, int p, bool predict) {
   G.nblocks_padded = padded_blocks(G.node_end - G.node0);
   const bool f64 = m->precision != AKX_PRECISION_FP32;
   check_gather_args(G, true, !f64);
-  dim3 grid((unsigned)G.nblocks_padded), block(TPB);
-  if (f64) {
-    if (predict)
-      hipLaunchKernelGGL((k_gather_update<double, true, true, false>), grid, block, 0,
-                         m->stream2, G);
-    else
-      hipLaunchKernelGGL((k_gather_update<double, true, false, false>), grid, block, 0,
-                         m->stream2, G);
-  } else {
-    if (predict)
-      hipLaunchKernelGGL((k_gather_update<float, true, true, true>), grid, block, 0,
-                         m->stream2, G);
-    else
-      hipLaunchKernelGGL((k_gather_update<float, true, false, true>), grid, block, 0,
-                         m->stream2, G);
-  }
+  launch_gather_kernel(G, f64, true, predict, m->stream2);
   HIPCHECK(hipGetLastError());
 }
 
