@@ -571,17 +571,17 @@ struct akx_batch {
   DevBuf<long long> bad;
   DevBuf<double> staging;
   FreeList fl_nodes, fl_tet, fl_hex, fl_ell;
-  // FP32 Tet4 block-partial assembly: per element its local corners and LDS
+  // FP32 block-partial assembly: per element its local corners and LDS
   // slots, per (block, distinct node) the arena node id, the end of its slot
   // range and its table entry
   bool bpa = false;
   int64_t bcap = 0;
-  DevBuf<uint16_t> lc_t, ls_t, ls_h; // local corners (Tet4), slots (Tet4, Hex8)
+  DevBuf<uint16_t> lc_t, ls_t, lc_h, ls_h; // local corners, slots
   DevBuf<int32_t> bnode, bpos;
   DevBuf<uint16_t> bsend;
   FreeList fl_bent;
   DevBuf<BBlk> d_blks; // parallel to d_tiles
-  int32_t bmaxu_live = 0; // most distinct nodes of a live Tet4 block (staged)
+  int32_t bmaxu_live[2] = {0, 0}; // most distinct nodes of a live Tet4 / Hex8 block
   std::vector<HostInst> inst;
   // device tables
   DevBuf<BInst> d_inst; // MAX_INSTANCES entries, address fixed
@@ -679,7 +679,7 @@ void rebuild_lists(akx_batch *b) {
   std::vector<std::vector<BTile>> groups(NGROUP);
   std::vector<std::vector<BBlk>> gblks(NGROUP);
   std::vector<BSlice> slices;
-  b->bmaxu_live = 0;
+  b->bmaxu_live[0] = b->bmaxu_live[1] = 0;
   int64_t group_n[NGROUP] = {0};
   for (const HostInst &I : b->inst)
     if (I.live)
@@ -698,8 +698,8 @@ void rebuild_lists(akx_batch *b) {
         G.push_back({I.elem0 + f, (int32_t)std::min<int64_t>(bs, I.nel - f), (int32_t)id});
         GB.push_back({off, I.blk_cnt[k], 0});
         off += I.blk_cnt[k];
-        if (I.etype == AKX_TET4)
-          b->bmaxu_live = std::max(b->bmaxu_live, I.blk_cnt[k]);
+        int32_t &most = b->bmaxu_live[I.etype == AKX_HEX8];
+        most = std::max(most, I.blk_cnt[k]);
       }
     } else {
       const int64_t tile = group_tile(b, I.etype, group_n[I.etype * 4 + I.law]);
@@ -756,23 +756,16 @@ BatchElemArgs elem_args(akx_batch *b, int etype, int64_t t0, int64_t t1, int par
   A.hoff = etype == AKX_TET4 ? 0 : b->tcap;
   A.hex_tab = b->hex_tab.p;
   A.parity = parity;
-  if (b->bpa && etype == AKX_TET4) {
+  if (b->bpa) {
     A.blks = b->d_blks.p + t0;
     A.bnode = b->bnode.p;
     A.bsend = b->bsend.p;
     A.bpos = b->bpos.p;
-    A.lc = b->lc_t.p;
-    A.ls = b->ls_t.p;
-    A.bmaxu = b->bmaxu_live;
+    A.lc = etype == AKX_TET4 ? b->lc_t.p : b->lc_h.p;
+    A.ls = etype == AKX_TET4 ? b->ls_t.p : b->ls_h.p;
+    A.bmaxu = b->bmaxu_live[etype == AKX_HEX8];
     require(A.blks && A.bnode && A.bsend && A.bpos && A.lc && A.ls && A.bmaxu > 0 &&
-                A.bmaxu <= 1024,
-            "block-partial pass launched without its block tables");
-  } else if (b->bpa) { // Hex8: corner slots only (no staged records)
-    A.blks = b->d_blks.p + t0;
-    A.bsend = b->bsend.p;
-    A.bpos = b->bpos.p;
-    A.ls = b->ls_h.p;
-    require(A.blks && A.bsend && A.bpos && A.ls,
+                A.bmaxu <= (etype == AKX_TET4 ? 4 * BPA_TET4 : 8 * BPA_HEX8),
             "block-partial pass launched without its block tables");
   }
   return A;
@@ -798,7 +791,7 @@ void element_pass(akx_batch *b, int parity) {
       continue;
     const int etype = g / 4, law = g % 4;
     BatchElemArgs A = elem_args(b, etype, t0, t1, parity);
-    require(A.conn && A.pos && A.xu && A.fe && A.inst && A.tiles && A.hex_tab,
+    require(A.conn && (A.pos || A.blks) && A.xu && A.fe && A.inst && A.tiles && A.hex_tab,
             "batch element arena not allocated");
     if (law == AKX_LAW_PLASTIC_LIH)
       for (int s = 0; s < 2; ++s)
@@ -1053,25 +1046,28 @@ int akx_batch_create(int device, int precision, int64_t node_capacity,
       b->cu.alloc(3 * b->ncap);
       b->cv.alloc(3 * b->ncap);
     }
+    // FP32 instances assemble by block partials (no table position per
+    // corner).  A block of BPA_TET4 Tet4 of a box has about 0.7 distinct nodes
+    // per element, so twice the Tet4 capacity holds the entries of any box
+    // mesh; a Hex8 element adds at most its eight nodes
+    b->bpa = b->fp32() && (b->tcap > 0 || b->hexcap > 0);
     if (b->tcap) {
       b->conn_t.alloc(4 * b->tcap);
-      b->pos_t.alloc(4 * b->tcap);
+      if (!b->bpa)
+        b->pos_t.alloc(4 * b->tcap);
     }
-    // FP32 instances assemble by block partials; a block of BPA_TET4 / BPA_HEX8 box
-    // elements has about 0.7 (Tet4) and at most 4.03 (Hex8: part of one row
-    // of cells) distinct nodes per element, so twice the Tet4 and five times
-    // the Hex8 capacity hold the distinct-node entries of any box mesh
-    b->bpa = b->fp32() && (b->tcap > 0 || b->hexcap > 0);
     if (b->bpa) {
-      b->bcap = 2 * b->tcap + 5 * b->hexcap + 2048;
+      b->bcap = 2 * b->tcap + 8 * b->hexcap + 2048;
       if (b->tcap) {
         b->lc_t.alloc(4 * b->tcap);
         b->ls_t.alloc(4 * b->tcap);
       }
       b->bx.alloc(3 * b->ncap);
       b->bu.alloc(3 * b->ncap);
-      if (b->hexcap)
+      if (b->hexcap) {
+        b->lc_h.alloc(8 * b->hexcap);
         b->ls_h.alloc(8 * b->hexcap);
+      }
       b->bnode.alloc(b->bcap);
       b->bpos.alloc(b->bcap);
       b->bsend.alloc(b->bcap);
@@ -1079,7 +1075,8 @@ int akx_batch_create(int device, int precision, int64_t node_capacity,
     }
     if (b->hexcap) {
       b->conn_h.alloc(8 * b->hexcap);
-      b->pos_h.alloc(8 * b->hexcap);
+      if (!b->bpa)
+        b->pos_h.alloc(8 * b->hexcap);
     }
     b->fe.alloc(b->ellcap * FE_W * b->fe_size());
     if (b->plastic)
@@ -1159,7 +1156,7 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
     for (int64_t i = 0; i < nb_elements * nnpe; ++i)
       require(conn[i] >= 0 && conn[i] < nb_nodes, "connectivity refers to a missing node");
     // block-partial assembly (FP32): per block of bs elements its distinct
-    // nodes in order of first use, each corner's index among them and its
+    // nodes in ascending order (the staging loads coalesce), each corner's index among them and its
     // LDS slot (the corners of one distinct node take consecutive slots in
     // ascending element order); the table then holds one entry per (block,
     // distinct node) and a node's degree is the number of blocks touching it
@@ -1173,22 +1170,18 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       ls.resize(nb_elements * nnpe);
       bl_nodes.reserve(nb_elements);
       I.blk_cnt.resize(nblk);
-      std::vector<int64_t> stamp(nb_nodes, -1);
       std::vector<int32_t> local(nb_nodes, 0);
+      DistinctNodes distinct(nb_nodes);
       std::vector<uint16_t> cnt(bs * nnpe + 1);
       for (int64_t bk = 0; bk < nblk; ++bk) {
         const int64_t e0 = bk * bs, e1 = std::min<int64_t>(nb_elements, e0 + bs);
         const int64_t start = (int64_t)bl_nodes.size();
-        for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i) {
-          const int32_t nd = conn[i];
-          if (stamp[nd] != bk) {
-            stamp[nd] = bk;
-            local[nd] = (int32_t)((int64_t)bl_nodes.size() - start);
-            bl_nodes.push_back(nd);
-          }
-          lc[i] = (uint16_t)local[nd];
-        }
+        distinct.append(conn + e0 * nnpe, (e1 - e0) * nnpe, bl_nodes);
         const int32_t nloc = (int32_t)((int64_t)bl_nodes.size() - start);
+        for (int32_t k = 0; k < nloc; ++k)
+          local[bl_nodes[start + k]] = k;
+        for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i)
+          lc[i] = (uint16_t)local[conn[i]];
         I.blk_cnt[bk] = nloc;
         std::fill(cnt.begin(), cnt.begin() + nloc + 1, 0);
         for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i)
@@ -1294,16 +1287,13 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       if (!bpa)
         HIPCHECK(hipMemcpy(dpos + I.elem0 * nnpe, gpos.data(), gpos.size() * 4,
                            hipMemcpyHostToDevice));
-      if (bpa && element_type == AKX_TET4) {
-        HIPCHECK(hipMemcpy(b->lc_t.p + I.elem0 * 4, lc.data(), lc.size() * 2,
-                           hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(b->ls_t.p + I.elem0 * 4, ls.data(), ls.size() * 2,
-                           hipMemcpyHostToDevice));
-      } else if (bpa) {
-        HIPCHECK(hipMemcpy(b->ls_h.p + I.elem0 * 8, ls.data(), ls.size() * 2,
-                           hipMemcpyHostToDevice));
-      }
       if (bpa) {
+        uint16_t *dlc = element_type == AKX_TET4 ? b->lc_t.p : b->lc_h.p;
+        uint16_t *dls = element_type == AKX_TET4 ? b->ls_t.p : b->ls_h.p;
+        HIPCHECK(hipMemcpy(dlc + I.elem0 * nnpe, lc.data(), lc.size() * 2,
+                           hipMemcpyHostToDevice));
+        HIPCHECK(hipMemcpy(dls + I.elem0 * nnpe, ls.data(), ls.size() * 2,
+                           hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(b->bnode.p + I.bent0, gbnode.data(), gbnode.size() * 4,
                            hipMemcpyHostToDevice));
         HIPCHECK(hipMemcpy(b->bpos.p + I.bent0, gbpos.data(), gbpos.size() * 4,
@@ -1725,11 +1715,10 @@ int akx_batch_get_kernel_bytes(akx_batch *b, int kernel_class, double *bytes) {
       const bool bpa = !I.blk_cnt.empty();
       const double entries = bpa ? (double)I.nbent : corners;
       if (kernel_class == 0) {
-        if (bpa) // per corner the local corner (Tet4, 2 B) or the node id
-                 // (Hex8, 4 B) and the slot (2 B); per entry the node id
-                 // (Tet4), slot end and table position, the partial written
-          total += corners * (I.etype == AKX_TET4 ? 4 : 6) +
-                   entries * ((I.etype == AKX_TET4 ? 4 : 0) + 2 + 4 + 3 * fs) + nn * 2 * 3 * 8;
+        if (bpa) // per corner the local corner (2 B) and the slot (2 B); per
+                 // entry the node id, slot end and table position, the
+                 // partial written
+          total += corners * 4 + entries * (4 + 2 + 4 + 3 * fs) + nn * 2 * 3 * 8;
         else
           total += corners * (4 + 4 + 3 * fs) + nn * 2 * 3 * 8;
         if (I.law == AKX_LAW_PLASTIC_LIH) // history read and written

@@ -43,8 +43,8 @@ struct BSlice {
   int32_t inst;
 };
 
-// FP32 Tet4 block-partial assembly: the distinct nodes of one 256-element
-// block of an instance (its tile) are entries off .. off + count - 1 of the
+// FP32 block-partial assembly: the distinct nodes of one block of BPA_TET4 /
+// BPA_HEX8 elements of an instance (its tile) are entries off .. off + count - 1 of the
 // block arenas (node ids, slot ends, table positions)
 struct BBlk {
   int64_t off;
@@ -55,9 +55,9 @@ struct BBlk {
 struct BatchElemArgs {
   const BTile *tiles;
   int64_t ntiles;
-  // block-partial assembly (FP32 Tet4 groups; null otherwise): per tile (one
-  // 256-element block) its distinct-node range, the block arenas, and each
-  // element's local corners and LDS slots ([elem][4] uint16)
+  // block-partial assembly (FP32 groups; null otherwise): per tile (one
+  // block) its distinct-node range, the block arenas, and each element's
+  // local corners and LDS slots ([elem][nnpe] uint16)
   const BBlk *blks;
   const int32_t *bnode;   // arena node id of each distinct node
   const uint16_t *bsend;  // end of each distinct node's slot range
@@ -84,10 +84,9 @@ struct BatchElemArgs {
 
 constexpr int HEX_TAB_N = 192, HEX_TAB_W = 256, HEX_TAB_SIZE = 264;
 
-// elements per block of the block-partial assembly: 256 Tet4; 192 Hex8, whose
-// 1,536 corner slots (18 KB of LDS) leave room for eight 256-lane
-// workgroups per CU (256 elements' 24 KB allowed six)
-constexpr int BPA_TET4 = 256, BPA_HEX8 = 192;
+// elements per block of the block-partial assembly: 256 Tet4, one per lane; 63
+// Hex8, four lanes each (k_hex8_bpa)
+constexpr int BPA_TET4 = 256, BPA_HEX8 = 63;
 
 // values per elemental-force entry in a batch's table.  3: a zero-padded
 // 4-wide entry (one vector store per corner) measured slower, its extra

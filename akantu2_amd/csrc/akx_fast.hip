@@ -387,28 +387,23 @@ __device__ __forceinline__ float hex_sf_force(float R, float qx, float qy, float
   return (E + lane_x4(E) * R) + (Cz - lane_x4(Cz));     // axis 2: I, D^T
 }
 
+// corner of the lane with bits b
+__device__ __forceinline__ int hex_node_of_lane(int b) {
+  const int node = b ^ ((b >> 1) & 1);
+  return node;
+}
+
 // All 64 lanes of the wave call it (cross-lane steps); lanes 8 e .. 8 e + 7
 // are element e, lane bits b = l % 8.  Lanes of elements beyond the range
-// pass active = false and compute on zeros.  SLOT: the node's force goes to
-// LDS slot ls_e[node] of `slots` (block-partial assembly) instead of table
-// entry pos_e[node] of fe.
-template <int LAW, class FT, class VT, class NA, int W = 3, bool SLOT = false>
-__device__ __forceinline__ void hex8_group_sf(int b, bool active, const int32_t *conn_e,
-                                              const NA &nodes_of, float lambda, float mu,
-                                              float sy, float hh, const VT &V, int64_t iq,
-                                              const int32_t *pos_e, FT *fe,
-                                              float *slots = nullptr,
-                                              const uint16_t *ls_e = nullptr) {
-  const int node = b ^ ((b >> 1) & 1);
+// pass active = false and compute on zeros.  nd: the node of the lane's
+// corner (hex_node_of_lane) in nodes_of; F: the force on it.
+template <int LAW, class VT, class NA>
+__device__ __forceinline__ void hex8_group_sf(int b, bool active, int32_t nd, const NA &nodes_of,
+                                              float lambda, float mu, float sy, float hh,
+                                              const VT &V, int64_t iq, float (&F)[3]) {
   double x[3] = {0., 0., 0.}, d[3] = {0., 0., 0.};
-  int32_t pq = 0;
-  if (active) {
-    nodes_of.load(conn_e[node], x, d);
-    if constexpr (SLOT)
-      pq = ls_e[node];
-    else
-      pq = pos_e[node];
-  }
+  if (active)
+    nodes_of.load(nd, x, d);
   const float R = hex_r_vgpr();
   // relative to node 0 (lane bits 0): exact FP64 difference, rounded once
   float J[3][3], H[3][3];
@@ -438,7 +433,6 @@ __device__ __forceinline__ void hex8_group_sf(int b, bool active, const int32_t 
   // sigma = s_0 s_1 s_2 = +1 when an even number of bits are clear
   const float sig = ((3 - __builtin_popcount(b)) & 1) ? -1.f : 1.f;
   const float w = dJ * (sig / HEX_C3);
-  float F[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     float q[3];
@@ -451,16 +445,6 @@ __device__ __forceinline__ void hex8_group_sf(int b, bool active, const int32_t 
       q[m] = w * s;
     }
     F[k] = hex_sf_force(R, q[0], q[1], q[2]);
-  }
-  if (active) {
-    if constexpr (SLOT) {
-      float *o = slots + 3 * pq;
-      o[0] = F[0];
-      o[1] = F[1];
-      o[2] = F[2];
-    } else {
-      akx::put_entry<W>(fe, (int64_t)pq, FT(F[0]), FT(F[1]), FT(F[2]));
-    }
   }
 }
 
@@ -475,53 +459,374 @@ __global__ void __launch_bounds__(256) k_hex8_sf(ElemArgs A) {
     e = A.filter ? (int64_t)A.filter[i] : A.first + i;
     element_params(A, i, lambda, mu, sy, hh);
   }
-  hex8_group_sf<LAW, FT, QpViewT<double>>(
-      b, active, A.conn + e * 8, NodesSoA{A.X, A.u, A.nn}, lambda, mu, sy, hh, qp_view(A, 8),
-      i * 8 + b, A.pos + (A.pos_offset + (active ? i : 0)) * 8, reinterpret_cast<FT *>(A.fe));
+  int32_t nd = 0, pos = 0;
+  if (active) {
+    nd = A.conn[e * 8 + hex_node_of_lane(b)];
+    pos = A.pos[(A.pos_offset + i) * 8 + hex_node_of_lane(b)];
+  }
+  float F[3];
+  hex8_group_sf<LAW>(b, active, nd, NodesSoA{A.X, A.u, A.nn}, lambda, mu, sy, hh, qp_view(A, 8),
+                     i * 8 + b, F);
+  if (active)
+    akx::put_entry<3>(reinterpret_cast<FT *>(A.fe), (int64_t)pos, FT(F[0]), FT(F[1]), FT(F[2]));
 }
 
-// FP32 Hex8 with block-partial assembly: each workgroup (256 lanes, 32
-// elements at a time through the sum-factorised body) does one block of
-// BPA_HEX8 consecutive elements; the lanes put their nodes' forces in LDS
-// slots (the corners of one distinct node of the block take consecutive
-// slots in ascending element order), then one thread per distinct node adds
-// its slots in that order (FP64, rounded once) and writes one table entry
-// per (block, node).  The gather adds a node's partials in block order.
-template <int LAW>
+// ---------------------------------------------------------------------------
+// Hex8, FP32 form, four lanes per element (the block-partial passes).  Lane
+// bits (y, z) own the two nodes and the two Gauss points of one x edge: the x
+// axis is worked in the lane, y and z as the butterflies above with the lanes
+// 1 and 2 away, all within a quad:
+//   D: v_own - v_partner,   I: v_own + r v_partner
+// With d = v+ - v- and s = v+ + v- along x, the rows of J' and H' at
+// xi = +-G are
+//   d/dxi = I_y I_z d,  d/deta = D_y I_z (KS s +- KD d),  d/dzeta = I_y D_z (KS s +- KD d)
+// KD = G KS: the two Gauss points share every step but one addition per row.
+// The rows are c_m s_m times the true ones (c_0 = 2 (1 + r)^2, c_1 = c_2 =
+// 4 KS (1 + r), s_0 = 1), which g = H' J'^-1 does not see, and the transposed
+// steps (D and I are symmetric) applied to Q' = W s_y s_z P adj(J'),
+// W = 1 / (c_0 c_1 c_2), give the nodal forces.  tests/test_hex8_quad_cpu.py
+// restates the steps lane by lane.
+//
+// A constant's rounding shifts the stiffness of every element and step alike:
+// 1e-8 of it is 1e-6 of the displacement after 300 steps.  So the constants
+// are ones that FP32 holds well: r to 5e-9, KS exactly, KD to 1e-10 (KS is
+// free; 1 / 2 with KD = G / 2 would be off by 1.8e-8), and W goes into the Lame
+// constants in FP64 (LameF).  Stiffness bias -1e-9, against -3.6e-8 of
+// hex8_group_sf (numpy emulation of both).
+//
+// Bound by FP32 vector issue on large meshes: 700 VALU instructions per wave
+// of 16 elements against 2 x 408 with one lane per Gauss point
+// (hex8_group_sf), 93% of the cycles busy (SQ_ACTIVE_INST_VALU against
+// GRBM_GUI_ACTIVE).  Block pass, neo-Hookean, 2 M elements 163-173 -> 155 us,
+// 255,000 33.9 -> 27.6 us, 19,740 16.7 -> 8.8 us and 1,000 16.1 -> 6.9 us (the
+// former blocks of 192 elements ran six groups of 32 one after another, on
+// 104 workgroups for the 19,740).  Also measured on 2 M elements: one lane
+// per element 259 us (181 VGPRs, two waves per SIMD); four lanes with the
+// corners read from the X and u arrays 169 us (lanes of a quad lie in four
+// rows, so every lane is an L1 access of its own: 110 M per pass against 23 M
+// with the records staged in LDS).
+// ---------------------------------------------------------------------------
+constexpr float HEX_KS = 0.63818359375f;      // 1307 / 2048
+constexpr float HEX_KD = 0.36845546964396530f; // HEX_KS / sqrt(3)
+constexpr double HEX_W = 1. / (2. * (1. + (double)HEX_R) * (1. + (double)HEX_R) * 16. *
+                               (double)HEX_KS * (double)HEX_KS * (1. + (double)HEX_R) *
+                               (1. + (double)HEX_R));
+
+// the value of the lane 1 / 2 away, of the quad's first lane
+__device__ __forceinline__ float quad_x1(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float quad_x2(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double quad_first(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x00, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x00, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// One component's node values (v0 at x-, v1 at x+ of the lane's edge) ->
+// d/dxi and the parts of d/deta = e0 +- e1 and d/dzeta = z0 +- z1.
+__device__ __forceinline__ void quad_grad(float v0, float v1, float &dxi, float &e0, float &e1,
+                                          float &z0, float &z1) {
+  const float d = v1 - v0, s = HEX_KS * (v0 + v1);
+  const float dp = quad_x2(d), sp = quad_x2(s);
+  const float dzd = d - dp, izd = d + HEX_R * dp;
+  const float dzs = s - sp, izs = s + HEX_R * sp;
+  const float ip = quad_x1(izd);
+  dxi = izd + HEX_R * ip;
+  e0 = izs - quad_x1(izs);
+  e1 = HEX_KD * (izd - ip);
+  z0 = dzs + HEX_R * quad_x1(dzs);
+  z1 = HEX_KD * (dzd + HEX_R * quad_x1(dzd));
+}
+
+// The transposed steps: one force component of the lane's nodes from the
+// rows of Q' at xi = -G (m) and xi = +G (p).
+__device__ __forceinline__ void quad_force(const float (&m)[3], const float (&p)[3], float &f0,
+                                           float &f1) {
+  const float X = p[0] + m[0];
+  const float Se = p[1] + m[1], E = HEX_KD * (p[1] - m[1]);
+  const float Sz = p[2] + m[2], Z = HEX_KD * (p[2] - m[2]);
+  // I a + D b = (a + b) + partner's (r a - b)
+  const float da = (X + E) + quad_x1(HEX_R * X - E); // I_y X + D_y E
+  const float db = Z + HEX_R * quad_x1(Z);
+  const float d = (da + db) + quad_x2(HEX_R * da - db);
+  const float sa = Se - quad_x1(Se);
+  const float sb = Sz + HEX_R * quad_x1(Sz);
+  const float s = (sa + sb) + quad_x2(HEX_R * sa - sb);
+  f0 = HEX_KS * s - d;
+  f1 = HEX_KS * s + d;
+}
+
+// adjugate: K = det(m) m^-1
+__device__ __forceinline__ void adjugate(const float (&m)[3][3], float (&K)[3][3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const int i1 = (i + 1) % 3, i2 = (i + 2) % 3, j1 = (j + 1) % 3, j2 = (j + 2) % 3;
+      K[j][i] = m[i1][j1] * m[i2][j2] - m[i1][j2] * m[i2][j1];
+    }
+}
+
+// Lame constants times HEX_W and the lane's sign as hi + lo floats: rounded to
+// FP32 alone, a material's constants are off by up to 3e-8 in every element
+// and step (per-element constants come rounded, theirs scatter).
+struct LameF {
+  float l, m, l_lo, m_lo;
+  __device__ __forceinline__ float times_l(float x) const { return fmaf(l, x, l_lo * x); }
+  __device__ __forceinline__ float times_m(float x) const { return fmaf(m, x, m_lo * x); }
+};
+
+// b: the quad lane, s_y s_z = -1 on lanes 1 and 2
+__device__ __forceinline__ LameF lame_quad(double lambda, double mu, int b) {
+  const double w = (b == 1 || b == 2) ? -HEX_W : HEX_W;
+  const double lw = lambda * w, mw = mu * w;
+  const float l = float(lw), m = float(mw);
+  return LameF{l, m, float(lw - double(l)), float(mw - double(m))};
+}
+
+// Q'[k][m] = W s_y s_z (P adj(J'))[k][m] of one Gauss point from the rows
+// J'[m][c] = c_m s_m dX_c/dxi_m and H'[m][c] (elastic laws and neo-Hookean);
+// lambda, mu: the material's constants, for the stress that is stored.
+template <int LAW, class VT>
+__device__ __forceinline__ void hex8_point(const float (&J)[3][3], const float (&H)[3][3],
+                                           const LameF &L, float lambda, float mu,
+                                           const VT &V, int64_t iq, float (&Q)[3][3]) {
+  float K[3][3], g[3][3];
+  adjugate(J, K);
+  const float id = akx_rcp(J[0][0] * K[0][0] + J[0][1] * K[1][0] + J[0][2] * K[2][0]);
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+#pragma unroll
+    for (int b = 0; b < 3; ++b)
+      g[a][b] = (H[0][a] * K[b][0] + H[1][a] * K[b][1] + H[2][a] * K[b][2]) * id;
+  constexpr int I6[6] = {0, 1, 2, 0, 0, 1}, J6[6] = {0, 1, 2, 1, 2, 2};
+  float T[3][3], P[3][3];
+  if (V.grad_u) { // materialise grad u and the stress
+    law_at<LAW, float>(V, iq, lambda, mu, 0.f, 0.f, g, T, P);
+  }
+  if constexpr (LAW == LAW_NEOHOOKEAN) {
+    // on the current configuration: tau = F S F^T = mu (b - I) + lambda ln J I
+    // with b - I = g + g^T + g g^T, and det J P J^-1 = (1 / det F) tau
+    // adj(J + H): no inverse of C and no product F S, and like the form with
+    // S free of cancellation (neohookean_pk2_stable)
+    const float tr = g[0][0] + g[1][1] + g[2][2];
+    // J - 1 = tr g + (sum of the principal 2 x 2 minors) + det g
+    float Kg[3][3];
+    adjugate(g, Kg);
+    const float dg = g[0][0] * Kg[0][0] + g[0][1] * Kg[1][0] + g[0][2] * Kg[2][0];
+    const float jm1 = tr + (Kg[0][0] + Kg[1][1] + Kg[2][2] + dg);
+    const float w = akx_rcp(1.f + jm1);
+    const float wm = L.times_m(w), wl = w * L.times_l(akx_log1p(jm1));
+#pragma unroll
+    for (int v = 0; v < 6; ++v) {
+      const int i = I6[v], j = J6[v];
+      float p = g[i][j] + g[j][i];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        p += g[i][k] * g[j][k];
+      T[i][j] = T[j][i] = i == j ? wm * p + wl : wm * p;
+    }
+    float jc[3][3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        jc[m][c] = J[m][c] + H[m][c];
+    adjugate(jc, K);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int m = 0; m < 3; ++m)
+        P[k][m] = T[k][m];
+  } else {
+    // S = lambda tr(e) I + 2 mu e, e the strain (2 e = g + g^T (+ g^T g))
+    float e2[6];
+#pragma unroll
+    for (int v = 0; v < 6; ++v) {
+      const int i = I6[v], j = J6[v];
+      e2[v] = g[i][j] + g[j][i];
+      if constexpr (LAW == LAW_ELASTIC_FD)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          e2[v] += g[k][i] * g[k][j];
+    }
+    const float sd = 0.5f * L.times_l(e2[0] + e2[1] + e2[2]);
+#pragma unroll
+    for (int v = 0; v < 6; ++v)
+      T[I6[v]][J6[v]] = T[J6[v]][I6[v]] = v < 3 ? L.times_m(e2[v]) + sd : L.times_m(e2[v]);
+    // P = sigma, or F S
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        P[k][m] = T[k][m];
+        if constexpr (LAW == LAW_ELASTIC_FD)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            P[k][m] += g[k][c] * T[c][m];
+      }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      Q[k][m] = P[k][0] * K[0][m] + P[k][1] * K[1][m] + P[k][2] * K[2][m];
+}
+
+// Quad lane b (bit 0 y, bit 1 z) of one element; lc, ls: its two corners'
+// indices in the block's node records and their LDS slots.  All four lanes of
+// an active element call it.
+template <int LAW, class VT, class NA>
+__device__ __forceinline__ void hex8_quad(int b, uint32_t lc, uint32_t ls, const NA &nodes_of,
+                                          const LameF &L, float lambda, float mu,
+                                          const VT &V, int64_t iq0, float *s_f) {
+  // nodes of a face run counter-clockwise: (x-, x+) at y-, (x+, x-) at y+
+  const int yp = (b & 1) * 16;
+  lc = __funnelshift_r(lc, lc, yp);
+  ls = __funnelshift_r(ls, ls, yp);
+  double x0[3], d0[3], x1[3], d1[3];
+  nodes_of.load((int32_t)(lc & 0xffffu), x0, d0);
+  nodes_of.load((int32_t)(lc >> 16), x1, d1);
+  // relative to node 0 (lane 0, x-): exact FP64 difference, rounded once
+  float Jx[3], Hx[3], xe0[3], xe1[3], xz0[3], xz1[3], ue0[3], ue1[3], uz0[3], uz1[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const double xr = quad_first(x0[c]), ur = quad_first(d0[c]);
+    quad_grad(float(x0[c] - xr), float(x1[c] - xr), Jx[c], xe0[c], xe1[c], xz0[c], xz1[c]);
+    quad_grad(float(d0[c] - ur), float(d1[c] - ur), Hx[c], ue0[c], ue1[c], uz0[c], uz1[c]);
+  }
+  float Qm[3][3], Qp[3][3];
+#pragma unroll
+  for (int ix = 0; ix < 2; ++ix) {
+    float J[3][3], H[3][3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      J[0][c] = Jx[c];
+      H[0][c] = Hx[c];
+      J[1][c] = ix ? xe0[c] + xe1[c] : xe0[c] - xe1[c];
+      H[1][c] = ix ? ue0[c] + ue1[c] : ue0[c] - ue1[c];
+      J[2][c] = ix ? xz0[c] + xz1[c] : xz0[c] - xz1[c];
+      H[2][c] = ix ? uz0[c] + uz1[c] : uz0[c] - uz1[c];
+    }
+    hex8_point<LAW>(J, H, L, lambda, mu, V, iq0 + (ix + 2 * b), ix ? Qp : Qm);
+  }
+  float *o0 = s_f + 3 * (ls & 0xffffu), *o1 = s_f + 3 * (ls >> 16);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    quad_force(Qm[k], Qp[k], o0[k], o1[k]);
+}
+
+// The plastic law of a block of n elements goes eight lanes per element, 32
+// elements at a time: consecutive lanes then read consecutive Gauss points of
+// its history (four lanes per element, two points each, read every second
+// value per load: block pass of 150,000 elements 143 -> 233 us).  lconn,
+// lslot, iq0: the block's first element and Gauss point; params(i, lambda, mu,
+// sy, hh) gives the constants of its i-th element.
+template <class VT, class PF>
+__device__ __forceinline__ void hex8_plastic_block(int n, const uint16_t *lconn,
+                                                   const uint16_t *lslot,
+                                                   const akx::NodesLDS &rec, const VT &V,
+                                                   int64_t iq0, const PF &params, float *s_f) {
+  for (int base = 0; base < n; base += 32) {
+    const int el = base + (threadIdx.x >> 3), b = threadIdx.x & 7;
+    const bool active = el < n;
+    const int ec = active ? el : 0, c = ec * 8 + hex_node_of_lane(b);
+    float lambda, mu, sy, hh, F[3];
+    params(ec, lambda, mu, sy, hh);
+    hex8_group_sf<LAW_PLASTIC>(b, active, lconn[c], rec, lambda, mu, sy, hh, V, iq0 + ec * 8 + b,
+                               F);
+    if (active) {
+      float *o = s_f + 3 * lslot[c];
+      o[0] = F[0];
+      o[1] = F[1];
+      o[2] = F[2];
+    }
+  }
+}
+
+// the slots s0 .. s1 - 1 of one (block, node) in order, FP64, rounded once
+__device__ __forceinline__ void sum_slots(const float *s_f, int s0, int s1, float *fe,
+                                          int64_t entry) {
+  double fx = 0., fy = 0., fz = 0.;
+  for (int sl = s0; sl < s1; ++sl) {
+    fx += (double)s_f[3 * sl];
+    fy += (double)s_f[3 * sl + 1];
+    fz += (double)s_f[3 * sl + 2];
+  }
+  akx::put_entry<3>(fe, entry, float(fx), float(fy), float(fz));
+}
+
+// FP32 Hex8 with block-partial assembly: each workgroup does one block of
+// BPA_HEX8 consecutive elements, four lanes each.  The {X, u} records of the
+// block's distinct nodes (ascending ids) are staged in LDS; the lanes put
+// their nodes' forces in LDS slots (the corners of one distinct node of the
+// block take consecutive slots in ascending element order), then one thread
+// per distinct node adds its slots in that order (FP64, rounded once) and
+// writes one table entry per (block, node).  The gather adds a node's
+// partials in block order.  63 elements: 252 of the 256 lanes, and a block
+// inside one row of cells has 4 x 64 distinct nodes, one per lane in the
+// staging and summing phases.
+// MAT: grad u and the stress are stored (computeAllStresses); a variant of its
+// own, whose code kept 60 registers more alive in every step's pass.
+template <int LAW, bool MAT>
 __global__ void __launch_bounds__(256) k_hex8_bpa(ElemArgs A) {
-  __shared__ float s_f[akx::BPA_HEX8 * 8 * 3];
-  const int t = threadIdx.x, el = t >> 3, b = t & 7;
+  extern __shared__ double2 s_xu[]; // [bl_maxu][3] records, then [63 * 8][3] floats
+  float *s_f = reinterpret_cast<float *>(s_xu + 3 * A.bl_maxu);
+  QpViewT<double> V = qp_view(A, 8);
+  if constexpr (!MAT)
+    V.grad_u = V.stress = nullptr;
+  const int t = threadIdx.x;
   const int64_t blk = xcd_block(A.nblocks_padded);
-  const int64_t i0 = blk * akx::BPA_HEX8;
+  const int64_t i0 = blk * akx::BPA_HEX8, i = i0 + (t >> 2);
   if (i0 >= A.n) // padding block: no elements, no node list
     return;
-  for (int base = 0; base < akx::BPA_HEX8; base += HEX_EPB) {
-    const int64_t i = i0 + base + el;
-    const bool active = base + el < akx::BPA_HEX8 && i < A.n;
-    const int64_t ic = active ? i : i0;
-    float lambda = 0.f, mu = 0.f, sy = 0.f, hh = 0.f;
-    if (active)
-      element_params(A, i, lambda, mu, sy, hh);
-    hex8_group_sf<LAW, float, QpViewT<double>, NodesSoA, 3, true>(
-        b, active, A.conn + (A.first + ic) * 8, NodesSoA{A.X, A.u, A.nn}, lambda, mu, sy,
-        hh, qp_view(A, 8), ic * 8 + b, nullptr, nullptr, s_f, A.lslot + ic * 8);
+  const bool active = (t >> 2) < akx::BPA_HEX8 && i < A.n;
+  // the lane's own streams and its first node of the summing phase first, so
+  // that their loads overlap the staging
+  uint32_t lc = 0, ls = 0;
+  double lambda = A.lambda, mu = A.mu;
+  if (LAW != LAW_PLASTIC && active) {
+    lc = reinterpret_cast<const uint32_t *>(A.lconn + i * 8)[t & 3];
+    ls = reinterpret_cast<const uint32_t *>(A.lslot + i * 8)[t & 3];
+    if (A.lm_f) {
+      lambda = A.lm_f[i].x;
+      mu = A.lm_f[i].y;
+    }
   }
-  __syncthreads();
   const uint16_t *soff = A.bl_soff + blk * (A.bl_maxu + 1);
   const int32_t *dst = A.bl_pos + blk * A.bl_maxu;
+  int32_t d_first = -1;
+  int s0_first = 0, s1_first = 0;
+  if (t < A.bl_maxu) {
+    d_first = dst[t];
+    s0_first = soff[t];
+    s1_first = soff[t + 1];
+  }
+  akx::stage_block_records(A, blk, s_xu);
+  __syncthreads();
+  const akx::NodesLDS rec{reinterpret_cast<const double *>(s_xu)};
+  if constexpr (LAW == LAW_PLASTIC)
+    hex8_plastic_block((int)min((int64_t)akx::BPA_HEX8, A.n - i0), A.lconn + i0 * 8,
+                       A.lslot + i0 * 8, rec, V, i0 * 8,
+                       [&](int el, float &l, float &m, float &y, float &h) {
+                         element_params(A, i0 + el, l, m, y, h);
+                       },
+                       s_f);
+  else if (active)
+    hex8_quad<LAW>(t & 3, lc, ls, rec, lame_quad(lambda, mu, t & 3), float(lambda), float(mu), V,
+                   i * 8, s_f);
+  __syncthreads();
   float *fe = reinterpret_cast<float *>(A.fe);
-  for (int k = t; k < A.bl_maxu; k += blockDim.x) {
-    const int32_t d = dst[k];
+  for (int k = t; k < A.bl_maxu; k += 256) {
+    const bool first = k == t;
+    const int32_t d = first ? d_first : dst[k];
     if (d < 0)
       continue;
-    const int s0 = soff[k], s1 = soff[k + 1];
-    double fx = 0., fy = 0., fz = 0.;
-    for (int sl = s0; sl < s1; ++sl) {
-      fx += (double)s_f[3 * sl];
-      fy += (double)s_f[3 * sl + 1];
-      fz += (double)s_f[3 * sl + 2];
-    }
-    akx::put_entry<3>(fe, (int64_t)d, float(fx), float(fy), float(fz));
+    const int s0 = first ? s0_first : soff[k], s1 = first ? s1_first : soff[k + 1];
+    sum_slots(s_f, s0, s1, fe, (int64_t)d);
   }
 }
 
@@ -733,13 +1038,7 @@ __global__ void __launch_bounds__(256) k_tet4_bpa(ElemArgs A) {
     if (d < 0)
       continue;
     const int s0 = first ? s0_first : soff[k], s1 = first ? s1_first : soff[k + 1];
-    double fx = 0., fy = 0., fz = 0.;
-    for (int sl = s0; sl < s1; ++sl) {
-      fx += (double)s_f[3 * sl];
-      fy += (double)s_f[3 * sl + 1];
-      fz += (double)s_f[3 * sl + 2];
-    }
-    akx::put_entry<3>(fe, (int64_t)d, float(fx), float(fy), float(fz));
+    sum_slots(s_f, s0, s1, fe, (int64_t)d);
   }
 }
 
@@ -768,6 +1067,18 @@ __global__ void __launch_bounds__(256) k_batch_tet4_f32(BatchElemArgs A) {
                                          float(P.h), V, A.hoff + e, A.pos + e * 4,
                                          reinterpret_cast<float *>(A.fe));
     }
+  }
+}
+
+// the {X, u} records of a tile's distinct nodes, built in LDS from the X and
+// u arrays (FP32 instances keep u in the [3][ncap] array, BInst::urec = 0)
+__device__ __forceinline__ void stage_tile_records(const BatchElemArgs &A, const BBlk &B,
+                                                   double2 *s) {
+  for (int k = threadIdx.x; k < B.count; k += blockDim.x) {
+    const int64_t nd = A.bnode[B.off + k];
+    s[3 * k] = make_double2(A.X[nd], A.X[A.ncap + nd]);
+    s[3 * k + 1] = make_double2(A.X[2 * A.ncap + nd], A.u[nd]);
+    s[3 * k + 2] = make_double2(A.u[A.ncap + nd], A.u[2 * A.ncap + nd]);
   }
 }
 
@@ -803,14 +1114,7 @@ __global__ void __launch_bounds__(256) k_batch_tet4_bpa(BatchElemArgs A) {
       s1_first = A.bsend[B.off + t];
       pos_first = A.bpos[B.off + t];
     }
-    // the records of the block's distinct nodes, built from X and u (FP32
-    // instances keep u in the [3][ncap] array, BInst::urec = 0)
-    for (int k = threadIdx.x; k < B.count; k += blockDim.x) {
-      const int64_t nd = A.bnode[B.off + k];
-      s_xu[3 * k] = make_double2(A.X[nd], A.X[A.ncap + nd]);
-      s_xu[3 * k + 1] = make_double2(A.X[2 * A.ncap + nd], A.u[nd]);
-      s_xu[3 * k + 2] = make_double2(A.u[A.ncap + nd], A.u[2 * A.ncap + nd]);
-    }
+    stage_tile_records(A, B, s_xu);
     __syncthreads();
     for (int j = threadIdx.x; j < T.count; j += blockDim.x) {
       const int64_t e = T.first + j;
@@ -835,13 +1139,7 @@ __global__ void __launch_bounds__(256) k_batch_tet4_bpa(BatchElemArgs A) {
       const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
       const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
       const int pos = first ? pos_first : A.bpos[B.off + k];
-      double fx = 0., fy = 0., fz = 0.;
-      for (int sl = s0; sl < s1; ++sl) {
-        fx += (double)s_f[3 * sl];
-        fy += (double)s_f[3 * sl + 1];
-        fz += (double)s_f[3 * sl + 2];
-      }
-      akx::put_entry<FE_W>(fe, (int64_t)pos, float(fx), float(fy), float(fz));
+      sum_slots(s_f, s0, s1, fe, (int64_t)pos);
     }
   }
 }
@@ -859,25 +1157,25 @@ __global__ void __launch_bounds__(EPB * 8) k_batch_hex8_f32(BatchElemArgs A) {
     for (int base = 0; base < T.count; base += EPB) {
       const bool active = base + el < T.count;
       const int64_t e = T.first + (active ? base + el : 0);
-      hex8_group_sf<LAW, float, QpCompact, NodesSoA, FE_W>(
-          q, active, A.conn + e * 8, NodesSoA{A.X, A.u, A.ncap}, float(P.lambda),
-          float(P.mu), float(P.sigma_y), float(P.h), V, A.hoff + e * 8 + q,
-          A.pos + e * 8, reinterpret_cast<float *>(A.fe));
+      const int32_t nd = A.conn[e * 8 + hex_node_of_lane(q)];
+      float F[3];
+      hex8_group_sf<LAW>(q, active, nd, NodesSoA{A.X, A.u, A.ncap}, float(P.lambda),
+                         float(P.mu), float(P.sigma_y), float(P.h), V, A.hoff + e * 8 + q, F);
+      if (active)
+        akx::put_entry<FE_W>(reinterpret_cast<float *>(A.fe),
+                             (int64_t)A.pos[e * 8 + hex_node_of_lane(q)], F[0], F[1], F[2]);
     }
   }
 }
 
 // Batched FP32 Hex8 with block-partial assembly: each tile is one block of at
-// most BPA_HEX8 consecutive elements of one instance and each workgroup (256
-// lanes, 32 elements at a time) does one tile.  The lanes put their nodes'
-// forces in LDS slots (the corners of one distinct node of the block take
-// consecutive slots in ascending element order), then one thread per
-// distinct node adds its slots in that order (FP64, rounded once) and
-// writes one table entry per (block, node).
+// most BPA_HEX8 consecutive elements of one instance and each workgroup does
+// one tile, as k_hex8_bpa.
 template <int LAW>
 __global__ void __launch_bounds__(256) k_batch_hex8_bpa(BatchElemArgs A) {
-  __shared__ float s_f[akx::BPA_HEX8 * 8 * 3]; // one slot per element corner of the block
-  const int t = threadIdx.x, el = t >> 3, q = t & 7;
+  extern __shared__ double2 s_xu[]; // [bmaxu][3] records, then [63 * 8][3] floats
+  float *s_f = reinterpret_cast<float *>(s_xu + 3 * A.bmaxu);
+  const int t = threadIdx.x;
   const int64_t tt = blockIdx.x;
   if (tt >= A.ntiles)
     return;
@@ -885,25 +1183,39 @@ __global__ void __launch_bounds__(256) k_batch_hex8_bpa(BatchElemArgs A) {
   const BBlk B = A.blks[tt];
   const BInst P = A.inst[T.inst];
   const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
-  for (int base = 0; base < T.count; base += 32) {
-    const bool active = base + el < T.count;
-    const int64_t e = T.first + (active ? base + el : 0);
-    hex8_group_sf<LAW, float, QpCompact, NodesSoA, FE_W, true>(
-        q, active, A.conn + e * 8, NodesSoA{A.X, A.u, A.ncap}, float(P.lambda), float(P.mu),
-        float(P.sigma_y), float(P.h), V, A.hoff + e * 8 + q, nullptr, nullptr, s_f,
-        A.ls + e * 8);
+  const bool active = (t >> 2) < T.count;
+  const int64_t e = T.first + (t >> 2);
+  uint32_t lc = 0, ls = 0;
+  if (LAW != LAW_PLASTIC && active) {
+    lc = reinterpret_cast<const uint32_t *>(A.lc + e * 8)[t & 3];
+    ls = reinterpret_cast<const uint32_t *>(A.ls + e * 8)[t & 3];
   }
+  int s0_first = 0, s1_first = 0, pos_first = 0;
+  if (t < B.count) {
+    s0_first = t > 0 ? (int)A.bsend[B.off + t - 1] : 0;
+    s1_first = A.bsend[B.off + t];
+    pos_first = A.bpos[B.off + t];
+  }
+  stage_tile_records(A, B, s_xu);
+  __syncthreads();
+  const akx::NodesLDS rec{reinterpret_cast<const double *>(s_xu)};
+  if constexpr (LAW == LAW_PLASTIC)
+    hex8_plastic_block(T.count, A.lc + T.first * 8, A.ls + T.first * 8, rec, V,
+                       A.hoff + T.first * 8,
+                       [&](int, float &l, float &m, float &y, float &h) {
+                         l = float(P.lambda), m = float(P.mu), y = float(P.sigma_y), h = float(P.h);
+                       },
+                       s_f);
+  else if (active)
+    hex8_quad<LAW>(t & 3, lc, ls, rec, lame_quad(P.lambda, P.mu, t & 3), float(P.lambda),
+                   float(P.mu), V, A.hoff + e * 8, s_f);
   __syncthreads();
   float *fe = reinterpret_cast<float *>(A.fe);
-  for (int k = t; k < B.count; k += blockDim.x) {
-    const int s0 = k > 0 ? (int)A.bsend[B.off + k - 1] : 0, s1 = A.bsend[B.off + k];
-    double fx = 0., fy = 0., fz = 0.;
-    for (int sl = s0; sl < s1; ++sl) {
-      fx += (double)s_f[3 * sl];
-      fy += (double)s_f[3 * sl + 1];
-      fz += (double)s_f[3 * sl + 2];
-    }
-    akx::put_entry<3>(fe, (int64_t)A.bpos[B.off + k], float(fx), float(fy), float(fz));
+  for (int k = t; k < B.count; k += 256) {
+    const bool first = k == t;
+    const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
+    const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
+    sum_slots(s_f, s0, s1, fe, (int64_t)(first ? pos_first : A.bpos[B.off + k]));
   }
 }
 
@@ -935,7 +1247,8 @@ static void launch_one(int etype, const ElemArgs &A, hipStream_t s) {
   }
   else if constexpr (sizeof(CT) == 4) { // FP32: sum-factorised Hex8
     if (A.lslot) // block-partial assembly
-      hipLaunchKernelGGL((k_hex8_bpa<L>), grid, block, 0, s, A);
+      hipLaunchKernelGGL((A.grad_u ? k_hex8_bpa<L, true> : k_hex8_bpa<L, false>), grid, block,
+                         (size_t)A.bl_maxu * 48 + akx::BPA_HEX8 * 8 * 12, s, A);
     else
       hipLaunchKernelGGL((k_hex8_sf<L, FT>), grid, block, 0, s, A);
   }
@@ -973,8 +1286,9 @@ static void launch_batch_law(int etype, int block, const BatchElemArgs &A,
                          (size_t)A.bmaxu * 48 + 1024 * 12, s, A);
     else
       hipLaunchKernelGGL(k_batch_tet4_f32<LAW>, grid, dim3(block), 0, s, A);
-  } else if (A.blks) { // block-partial assembly: 256 lanes, LDS corner slots
-    hipLaunchKernelGGL(k_batch_hex8_bpa<LAW>, grid, dim3(256), 0, s, A);
+  } else if (A.blks) { // block-partial assembly: records, then the corner slots
+    hipLaunchKernelGGL(k_batch_hex8_bpa<LAW>, grid, dim3(256),
+                       (size_t)A.bmaxu * 48 + akx::BPA_HEX8 * 8 * 12, s, A);
   } else if (block == 64) {
     hipLaunchKernelGGL((k_batch_hex8_f32<LAW, 8>), grid, dim3(64), 0, s, A);
   } else if (block == 128) {

@@ -5,9 +5,12 @@
 #include "../../include/akantu_mi355x.h"
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cstdint>
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <vector>
 
 namespace akx {
 
@@ -67,6 +70,35 @@ template <class T> struct DevBuf {
   size_t bytes() const { return n * sizeof(T); }
 };
 
+
+// The distinct values of a block's node ids in ascending order: a bit per
+// node, read back over the words the block spans; ids scattered over far more
+// words than there are ids are sorted instead.
+class DistinctNodes {
+  std::vector<uint64_t> bits;
+
+public:
+  explicit DistinctNodes(int64_t nb_nodes) : bits((nb_nodes + 63) / 64, 0) {}
+  // appends the distinct values of ids[0 .. n), n > 0, to out
+  void append(const int32_t *ids, int64_t n, std::vector<int32_t> &out) {
+    const auto mm = std::minmax_element(ids, ids + n);
+    const int64_t w0 = *mm.first >> 6, w1 = *mm.second >> 6;
+    if (w1 - w0 > 4 * n) {
+      const size_t start = out.size();
+      out.insert(out.end(), ids, ids + n);
+      std::sort(out.begin() + start, out.end());
+      out.erase(std::unique(out.begin() + start, out.end()), out.end());
+      return;
+    }
+    for (int64_t i = 0; i < n; ++i)
+      bits[ids[i] >> 6] |= uint64_t(1) << (ids[i] & 63);
+    for (int64_t w = w0; w <= w1; ++w) {
+      for (uint64_t b = bits[w]; b; b &= b - 1)
+        out.push_back((int32_t)(w * 64 + __builtin_ctzll(b)));
+      bits[w] = 0;
+    }
+  }
+};
 
 // Run f and turn any exception into a status code (nothing throws across
 // the C ABI).

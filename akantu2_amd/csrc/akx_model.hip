@@ -753,8 +753,8 @@ void refresh_xu(akx_model *m, bool with_x) {
 }
 
 // Element passes with block lists: for each block of bs consecutive
-// elements of a contiguous material, its distinct nodes in order of first
-// use (every block's list padded with -1 to the longest) and each element's
+// elements of a contiguous material, its distinct nodes in ascending order
+// (the staging loads coalesce; every block's list padded with -1 to the longest) and each element's
 // corners as indices into them (the Tet4 passes stage these nodes' records
 // in LDS).  In FP32 also, for block-partial assembly, the LDS slot of every
 // corner: the corners of distinct node k of a block take consecutive slots
@@ -764,22 +764,19 @@ void build_block_nodes(akx_model *m, Material &mat, int64_t bs = 256) {
   const int64_t n = mat.n, nb = (n + bs - 1) / bs;
   std::vector<int32_t> off(nb + 1, 0), nodes;
   std::vector<uint16_t> lc(n * nnpe);
-  std::vector<int64_t> stamp(m->nn, -1);
   std::vector<int32_t> local(m->nn, 0);
+  DistinctNodes distinct(m->nn);
+  const int32_t *conn = m->conn_host.data() + mat.first * nnpe;
   nodes.reserve(n);
   int32_t maxu = 0;
   for (int64_t b = 0; b < nb; ++b) {
     const int64_t start = (int64_t)nodes.size();
-    for (int64_t i = b * bs; i < std::min<int64_t>(n, b * bs + bs); ++i)
-      for (int a = 0; a < nnpe; ++a) {
-        const int32_t node = m->conn_host[(mat.first + i) * nnpe + a];
-        if (stamp[node] != b) {
-          stamp[node] = b;
-          local[node] = (int32_t)((int64_t)nodes.size() - start);
-          nodes.push_back(node);
-        }
-        lc[i * nnpe + a] = (uint16_t)local[node];
-      }
+    const int64_t c0 = b * bs * nnpe, c1 = std::min<int64_t>(n, b * bs + bs) * nnpe;
+    distinct.append(conn + c0, c1 - c0, nodes);
+    for (int64_t k = start; k < (int64_t)nodes.size(); ++k)
+      local[nodes[k]] = (int32_t)(k - start);
+    for (int64_t i = c0; i < c1; ++i)
+      lc[i] = (uint16_t)local[conn[i]];
     require((int64_t)nodes.size() < (int64_t)INT32_MAX, "block node lists too large");
     off[b + 1] = (int32_t)nodes.size();
     maxu = std::max<int32_t>(maxu, off[b + 1] - off[b]);
@@ -3345,7 +3342,7 @@ int akx_model_get_kernel_bytes(akx_model *m, int kernel_class, double *bytes) {
       nel_all += mp->n;
       if (mp->per_element) // lambda, mu per element: FP64, or the FP32 pair
         extra += mp->n * (mp->lm_f.p ? 2.0 * 4.0 : 2.0 * 8.0);
-      if (mp->lconn.p && m->etype == AKX_TET4) // staged records: 2-byte local
+      if (mp->lconn.p) // staged records: 2-byte local
         // corners instead of 4-byte node ids, plus the blocks' node lists
         extra += -2.0 * m->nnpe * mp->n + 4.0 * (double)mp->bl_nodes.n;
       if (mp->law == AKX_LAW_PLASTIC_LIH)
