@@ -80,6 +80,9 @@ def _declare(lib):
         "akx_model_assemble_internal_forces": (C.c_int, [_vp]),
         "akx_model_get_nb_nodes": (C.c_int, [_vp, C.POINTER(_i64)]),
         "akx_model_get_field": (C.c_int, [_vp, C.c_int, _vp]),
+        "akx_model_get_fields": (C.c_int, [_vp, C.c_int, C.POINTER(C.c_int),
+                                           C.POINTER(_vp), C.POINTER(_vp)]),
+        "akx_host_differs": (C.c_int, [_vp, _vp, _i64, C.POINTER(C.c_int)]),
         "akx_model_set_field": (C.c_int, [_vp, C.c_int, _vp]),
         "akx_model_compute_all_stresses": (C.c_int, [_vp]),
         "akx_model_get_internal": (C.c_int, [_vp, C.c_int, C.c_int, _vp]),

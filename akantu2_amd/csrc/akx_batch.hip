@@ -26,6 +26,7 @@
 // the mix.
 #include "../../include/akantu_mi355x.h"
 #include "akx_batch.hpp"
+#include "akx_download.hpp"
 #include "akx_fast.hpp"
 #include "akx_host.hpp"
 #include "akx_kernels.hpp"
@@ -570,6 +571,7 @@ struct akx_batch {
   DevBuf<unsigned long long> dt_bits;
   DevBuf<long long> bad;
   DevBuf<double> staging;
+  Downloader download;
   FreeList fl_nodes, fl_tet, fl_hex, fl_ell;
   // FP32 block-partial assembly: per element its local corners and LDS
   // slots, per (block, distinct node) the arena node id, the end of its slot
@@ -1542,14 +1544,15 @@ int akx_batch_get_field(akx_batch *b, int id, int field, double *host) {
       break;
     default: throw Error(AKX_ERR_INVALID, "field not available for batch instances");
     }
-    sync(b);
-    b->staging.reserve(3 * I.nn);
-    hipLaunchKernelGGL(k_batch_get3, dim3(gridn(3 * I.nn)), dim3(TPB), 0, b->stream, src,
-                       b->staging.p, comp_stride, node_stride, I.node0, I.nn);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(host, b->staging.p, 3 * I.nn * sizeof(double),
-                            hipMemcpyDeviceToHost, b->stream));
-    sync(b);
+    hipStream_t st = b->stream;
+    const int64_t node0 = I.node0;
+    std::vector<Downloader::Field> f{
+        {I.nn, 24, host, nullptr, [=](void *p, int64_t first, int64_t n) {
+           hipLaunchKernelGGL(k_batch_get3, dim3(gridn(3 * n)), dim3(TPB), 0, st, src,
+                              (double *)p, comp_stride, node_stride, node0 + first, n);
+           HIPCHECK(hipGetLastError());
+         }}};
+    b->download.get(b->device, st, f);
   });
 }
 

@@ -1,0 +1,257 @@
+// akx_download.hpp -- device fields to host arrays.
+//
+// A field is packed by a kernel that writes the caller's layout straight into
+// pinned host memory, and copied from there.  What a plain device-to-host
+// copy into the caller's (pageable, often untouched) array spent its time on
+// was the host: the runtime's own staging at 10 GB/s or less, the page faults
+// of a new array, one synchronisation and one copy command per field.  Here
+// several fields share one synchronisation, and large ones go in chunks of
+// 1 MB that one to eight threads claim in turn: each launches the next chunk's
+// kernel into one of its two pinned slots while it copies the one before out
+// (to the array and, where asked, to a second one), so the link, the copies
+// and the page faults overlap.  Times: Downloader::get.
+#pragma once
+
+#include "akx_host.hpp"
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <exception>
+#include <functional>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace akx {
+
+// Chunks 0 .. n - 1 claimed by the calling thread and up to threads - 1
+// others.  The caller waits for every claimed chunk, not for the threads: on a
+// host whose CPUs are busy (an OpenMP runtime spinning after its last loop)
+// one that has not been scheduled yet is not waited for, and finds nothing to
+// claim when it is.
+struct ChunkJob {
+  std::atomic<int64_t> next{0}, done{0}, skipped{0};
+  int64_t n = 0;
+  std::mutex mutex;
+  std::exception_ptr error;
+
+  int64_t claim() {
+    const int64_t c = next.fetch_add(1);
+    return c < n ? c : -1;
+  }
+  void finish() { done.fetch_add(1); }
+  void fail(std::exception_ptr e) { // no further chunk is claimed
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      if (!error)
+        error = e;
+    }
+    const int64_t c = next.exchange(n);
+    if (c < n) // the caller may return once these are counted
+      skipped.fetch_add(n - c);
+  }
+};
+
+// work(job) claims and finishes chunks until none is left; it finishes what it
+// claimed also when it throws
+template <class F> void run_chunks(int threads, int64_t n, const F &work) {
+  auto job = std::make_shared<ChunkJob>();
+  job->n = n;
+  // the threads hold the job alive and copies of what work refers to only
+  // through it: work itself is run by a thread that has claimed a chunk
+  std::shared_ptr<const F *> body = std::make_shared<const F *>(&work);
+  auto loop = [job, body] {
+    const int64_t c = job->claim();
+    if (c < 0)
+      return; // the caller may have returned: work is not touched
+    try {
+      (**body)(*job, c);
+    } catch (...) {
+      job->fail(std::current_exception());
+    }
+  };
+  try {
+    for (int t = 1; t < threads; ++t)
+      std::thread(loop).detach();
+  } catch (...) { // no thread to be had: their share is done here
+  }
+  loop();
+  while (job->done.load() + job->skipped.load() < n)
+    std::this_thread::yield();
+  std::lock_guard<std::mutex> lock(job->mutex);
+  if (job->error)
+    std::rethrow_exception(job->error);
+}
+
+constexpr size_t COPY_CHUNK = 1u << 20;
+
+// Threads for a copy: one per 8 MB, at most eight.  More did not pay for what
+// a thread costs where the CPUs are busy: an 8 MB field by four threads 0.4 ms
+// on idle CPUs, but 3.5 ms (a scheduler's slice) beside 16 spinning ones; by
+// one thread 0.6 to 0.8 ms.
+inline int copy_threads(size_t bytes) {
+  const size_t hw = std::max(1u, std::thread::hardware_concurrency());
+  return (int)std::max<size_t>(1, std::min<size_t>({8, hw, bytes >> 23}));
+}
+
+// whether two host arrays differ
+inline bool host_differs(const void *a, const void *b, size_t bytes) {
+  const int T = copy_threads(bytes);
+  if (T == 1)
+    return std::memcmp(a, b, bytes) != 0;
+  std::atomic<bool> differ{false};
+  run_chunks(T, (int64_t)((bytes + COPY_CHUNK - 1) / COPY_CHUNK),
+             [&](ChunkJob &job, int64_t c) {
+               for (; c >= 0; c = job.claim()) {
+                 const size_t o = (size_t)c * COPY_CHUNK;
+                 if (!differ.load(std::memory_order_relaxed) &&
+                     std::memcmp((const char *)a + o, (const char *)b + o,
+                                 std::min(COPY_CHUNK, bytes - o)) != 0)
+                   differ = true;
+                 job.finish();
+               }
+             });
+  return differ;
+}
+
+class Downloader {
+  unsigned char *pin = nullptr;
+  size_t cap = 0;
+  std::vector<hipEvent_t> events; // two per thread
+
+  void reserve(size_t bytes) {
+    if (bytes <= cap)
+      return;
+    size_t want = 64u << 10;
+    while (want < bytes)
+      want *= 2;
+    if (pin)
+      (void)hipHostFree(pin);
+    pin = nullptr;
+    cap = 0;
+    HIPCHECK(hipHostMalloc((void **)&pin, want, hipHostMallocCoherent));
+    cap = want;
+  }
+
+public:
+  // n items of `item` bytes; pack(p, first, count) launches, on the stream,
+  // the kernel that writes items first .. first + count - 1 to p (16-byte
+  // aligned); copy: a second destination, or null
+  struct Field {
+    int64_t n;
+    size_t item;
+    void *host, *copy;
+    std::function<void(void *, int64_t, int64_t)> pack;
+    size_t bytes() const { return (size_t)n * item; }
+  };
+
+  Downloader() = default;
+  Downloader(const Downloader &) = delete;
+  Downloader &operator=(const Downloader &) = delete;
+  ~Downloader() {
+    for (hipEvent_t e : events)
+      (void)hipEventDestroy(e);
+    if (pin)
+      (void)hipHostFree(pin);
+  }
+
+  // Waits for the stream's work and delivers the fields.  (device is current.)
+  // Per field: 525 nodes 50-100 -> 19 us; 2 M nodes (49 MB) 5.2 -> 1.2 ms, with
+  // the second copy 9.1 -> 1.6 ms (arrays used before; the comparison of two
+  // such pairs at the next call 4.4 -> 1.7 ms).
+  void get(int device, hipStream_t stream, std::vector<Field> &fields) {
+    size_t total = 0;
+    for (auto &f : fields)
+      total += (f.bytes() + 63) / 64 * 64;
+    if (total <= COPY_CHUNK) {
+      reserve(std::max<size_t>(total, 64));
+      size_t o = 0;
+      for (auto &f : fields) {
+        if (f.n > 0)
+          f.pack(pin + o, 0, f.n);
+        o += (f.bytes() + 63) / 64 * 64;
+      }
+      HIPCHECK(hipStreamSynchronize(stream));
+      o = 0;
+      for (auto &f : fields) {
+        if (f.n > 0) {
+          std::memcpy(f.host, pin + o, f.bytes());
+          if (f.copy)
+            std::memcpy(f.copy, pin + o, f.bytes());
+        }
+        o += (f.bytes() + 63) / 64 * 64;
+      }
+      return;
+    }
+    struct Chunk {
+      const Field *f;
+      int64_t first, count;
+    };
+    std::vector<Chunk> chunks;
+    for (auto &f : fields) {
+      const int64_t per = std::max<int64_t>(1, (int64_t)(COPY_CHUNK / f.item));
+      for (int64_t i = 0; i < f.n; i += per)
+        chunks.push_back({&f, i, std::min(per, f.n - i)});
+    }
+    const int T = copy_threads(total);
+    reserve((size_t)T * 2 * COPY_CHUNK);
+    while ((int)events.size() < 2 * T) {
+      hipEvent_t e;
+      HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      events.push_back(e);
+    }
+    std::atomic<int> workers{0};
+    run_chunks(T, (int64_t)chunks.size(), [&](ChunkJob &job, int64_t c) {
+      // the thread's chunks in flight: claimed, the kernel launched.  After
+      // its last finish() it touches nothing of the caller's.
+      const int w = workers.fetch_add(1);
+      struct Flight {
+        hipEvent_t ev;
+        int64_t c;
+      } fl[2] = {{events[2 * w], -1}, {events[2 * w + 1], -1}};
+      unsigned char *slots = pin + (size_t)w * 2 * COPY_CHUNK;
+      struct Finish { // on every way out: what was claimed is finished
+        ChunkJob &job;
+        Flight (&fl)[2];
+        int64_t &c;
+        ~Finish() {
+          for (Flight &f : fl)
+            if (f.c >= 0) {
+              (void)hipEventSynchronize(f.ev); // its kernel writes the slot
+              job.finish();
+            }
+          if (c >= 0)
+            job.finish();
+        }
+      } finish{job, fl, c};
+      HIPCHECK(hipSetDevice(device));
+      for (int k = 0;; k ^= 1) {
+        if (c >= 0) {
+          chunks[c].f->pack(slots + k * COPY_CHUNK, chunks[c].first, chunks[c].count);
+          HIPCHECK(hipEventRecord(fl[k].ev, stream));
+          fl[k].c = c;
+          c = -1;
+        }
+        Flight &o = fl[k ^ 1]; // the one before
+        if (o.c >= 0) {
+          HIPCHECK(hipEventSynchronize(o.ev));
+          const Chunk &h = chunks[o.c];
+          const size_t at = (size_t)h.first * h.f->item, b = (size_t)h.count * h.f->item;
+          const unsigned char *slot = slots + (k ^ 1) * COPY_CHUNK;
+          std::memcpy((char *)h.f->host + at, slot, b);
+          if (h.f->copy)
+            std::memcpy((char *)h.f->copy + at, slot, b);
+          o.c = -1;
+          job.finish();
+        }
+        c = job.claim();
+        if (c < 0 && fl[0].c < 0 && fl[1].c < 0)
+          break;
+      }
+    });
+  }
+};
+
+} // namespace akx

@@ -7,6 +7,7 @@
 // with the predictor of step k+1 fused into the gather of step k when
 // several steps are queued together.
 #include "../../include/akantu_mi355x.h"
+#include "akx_download.hpp"
 #include "akx_fast.hpp"
 #include "akx_host.hpp"
 #include "akx_kernels.hpp"
@@ -43,13 +44,15 @@ __global__ void k_aos_to_soa(const T *aos, T *soa, int64_t n, int comps) {
   soa[c * n + r] = aos[i];
 }
 
+// rows first .. first + count - 1 of the n
 template <class T>
-__global__ void k_soa_to_aos(const T *soa, T *aos, int64_t n, int comps) {
+__global__ void k_soa_to_aos(const T *soa, T *aos, int64_t n, int comps, int64_t first,
+                             int64_t count) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n * comps)
+  if (i >= count * comps)
     return;
   int64_t r = i / comps, c = i % comps;
-  aos[i] = soa[c * n + r];
+  aos[i] = soa[c * n + first + r];
 }
 
 __global__ void k_bits_from_bool3(const uint8_t *b3, uint8_t *bits, int64_t n) {
@@ -59,23 +62,25 @@ __global__ void k_bits_from_bool3(const uint8_t *b3, uint8_t *bits, int64_t n) {
   bits[i] = (b3[3 * i] ? 1 : 0) | (b3[3 * i + 1] ? 2 : 0) | (b3[3 * i + 2] ? 4 : 0);
 }
 
-__global__ void k_bool3_from_bits(const uint8_t *bits, uint8_t *b3, int64_t n) {
+__global__ void k_bool3_from_bits(const uint8_t *bits, uint8_t *b3, int64_t first,
+                                  int64_t count) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n)
+  if (i >= count)
     return;
-  uint8_t b = bits[i];
+  uint8_t b = bits[first + i];
   b3[3 * i] = b & 1;
   b3[3 * i + 1] = (b >> 1) & 1;
   b3[3 * i + 2] = (b >> 2) & 1;
 }
 
-__global__ void k_mass_to3(const double *m, double *m3, int64_t n) {
+__global__ void k_mass_to3(const double *m, double *m3, int64_t first, int64_t count) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n)
+  if (i >= count)
     return;
-  m3[3 * i] = m[i];
-  m3[3 * i + 1] = m[i];
-  m3[3 * i + 2] = m[i];
+  const double v = m[first + i];
+  m3[3 * i] = v;
+  m3[3 * i + 1] = v;
+  m3[3 * i + 2] = v;
 }
 
 // streaming copy used to calibrate the HBM byte counters and to report the
@@ -598,6 +603,7 @@ struct akx_model {
   int64_t pp_total = 0;
   int64_t pp_entries = 0, pp_runs = 0; // table entries, summed runs
   DevBuf<unsigned char> staging;
+  Downloader download;
   DevBuf<unsigned long long> scratch_u64;
   DevBuf<long long> scratch_i64;
   std::vector<std::unique_ptr<Material>> mats;
@@ -732,15 +738,19 @@ void upload_soa(akx_model *m, const T *host_aos, T *dev_soa, int64_t n, int comp
 }
 
 template <class T>
+Downloader::Field soa_field(akx_model *m, const T *dev_soa, T *host_aos, T *copy, int64_t n,
+                            int comps) {
+  return {n, comps * sizeof(T), host_aos, copy, [=](void *p, int64_t first, int64_t count) {
+            hipLaunchKernelGGL(k_soa_to_aos<T>, dim3(grid_for(count * comps)), dim3(TPB), 0,
+                               m->stream, dev_soa, (T *)p, n, comps, first, count);
+            HIPCHECK(hipGetLastError());
+          }};
+}
+
+template <class T>
 void download_soa(akx_model *m, const T *dev_soa, T *host_aos, int64_t n, int comps) {
-  size_t bytes = (size_t)n * comps * sizeof(T);
-  m->staging.alloc(std::max(m->staging.n, bytes));
-  hipLaunchKernelGGL(k_soa_to_aos<T>, dim3(grid_for(n * comps)), dim3(TPB), 0,
-                     m->stream, dev_soa, (T *)m->staging.p, n, comps);
-  HIPCHECK(hipGetLastError());
-  HIPCHECK(hipMemcpyAsync(host_aos, m->staging.p, bytes, hipMemcpyDeviceToHost,
-                          m->stream));
-  HIPCHECK(hipStreamSynchronize(m->stream));
+  std::vector<Downloader::Field> f{soa_field<T>(m, dev_soa, host_aos, nullptr, n, comps)};
+  m->download.get(m->device, m->stream, f);
 }
 
 // Tet4 node records: X and u (init) or u alone (after an upload of u)
@@ -2379,53 +2389,69 @@ int akx_model_get_nb_nodes(akx_model *m, int64_t *nb_nodes) {
 }
 
 int akx_model_get_field(akx_model *m, int field, void *host) {
+  return akx_model_get_fields(m, 1, &field, &host, nullptr);
+}
+
+int akx_model_get_fields(akx_model *m, int count, const int *fields, void *const *host,
+                         void *const *copy) {
   return guard([&] {
     require(m != nullptr && m->etype >= 0, "set the mesh first");
-    require(host != nullptr, "null host array");
+    require(count >= 0 && (count == 0 || (fields && host)), "null argument");
     m->set_device();
-    HIPCHECK(hipStreamSynchronize(m->stream));
-    double *src = nullptr;
-    switch (field) {
-    case AKX_FIELD_DISPLACEMENT: src = m->u.p; break;
-    case AKX_FIELD_VELOCITY: src = m->v.p; break;
-    case AKX_FIELD_ACCELERATION: src = m->a.p; break;
-    case AKX_FIELD_INTERNAL_FORCE: src = m->fint.p; break;
-    case AKX_FIELD_NODES: src = m->X.p; break;
-    case AKX_FIELD_EXTERNAL_FORCE:
-      if (!m->has_fext) {
-        std::memset(host, 0, sizeof(double) * 3 * m->nn);
-        return;
+    std::vector<Downloader::Field> list;
+    const int64_t nn = m->nn;
+    hipStream_t st = m->stream;
+    for (int k = 0; k < count; ++k) {
+      require(host[k] != nullptr, "null host array");
+      void *dst = host[k], *dup = copy ? copy[k] : nullptr;
+      const double *src = nullptr;
+      switch (fields[k]) {
+      case AKX_FIELD_DISPLACEMENT: src = m->u.p; break;
+      case AKX_FIELD_VELOCITY: src = m->v.p; break;
+      case AKX_FIELD_ACCELERATION: src = m->a.p; break;
+      case AKX_FIELD_INTERNAL_FORCE: src = m->fint.p; break;
+      case AKX_FIELD_NODES: src = m->X.p; break;
+      case AKX_FIELD_EXTERNAL_FORCE:
+        if (!m->has_fext) {
+          std::memset(dst, 0, sizeof(double) * 3 * nn);
+          if (dup)
+            std::memset(dup, 0, sizeof(double) * 3 * nn);
+          continue;
+        }
+        src = m->fext.p;
+        break;
+      case AKX_FIELD_MASS: {
+        const double *mass = m->mass.p;
+        list.push_back({nn, 24, dst, dup, [=](void *p, int64_t first, int64_t n) {
+                          hipLaunchKernelGGL(k_mass_to3, dim3(grid_for(n)), dim3(TPB), 0, st,
+                                             mass, (double *)p, first, n);
+                          HIPCHECK(hipGetLastError());
+                        }});
+        continue;
       }
-      src = m->fext.p;
-      break;
-    case AKX_FIELD_MASS: {
-      size_t bytes = sizeof(double) * 3 * m->nn;
-      m->staging.alloc(std::max(m->staging.n, bytes));
-      hipLaunchKernelGGL(k_mass_to3, dim3(grid_for(m->nn)), dim3(TPB), 0,
-                         m->stream, (const double *)m->mass.p,
-                         (double *)m->staging.p, m->nn);
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipMemcpyAsync(host, m->staging.p, bytes, hipMemcpyDeviceToHost,
-                              m->stream));
-      HIPCHECK(hipStreamSynchronize(m->stream));
-      return;
+      case AKX_FIELD_BLOCKED_DOFS: {
+        const uint8_t *bits = m->blocked.p;
+        list.push_back({nn, 3, dst, dup, [=](void *p, int64_t first, int64_t n) {
+                          hipLaunchKernelGGL(k_bool3_from_bits, dim3(grid_for(n)), dim3(TPB), 0,
+                                             st, bits, (uint8_t *)p, first, n);
+                          HIPCHECK(hipGetLastError());
+                        }});
+        continue;
+      }
+      default:
+        throw Error(AKX_ERR_INVALID, "unknown field");
+      }
+      list.push_back(soa_field<double>(m, src, (double *)dst, (double *)dup, nn, 3));
     }
-    case AKX_FIELD_BLOCKED_DOFS: {
-      size_t bytes = 3 * m->nn;
-      m->staging.alloc(std::max(m->staging.n, bytes));
-      hipLaunchKernelGGL(k_bool3_from_bits, dim3(grid_for(m->nn)), dim3(TPB), 0,
-                         m->stream, (const uint8_t *)m->blocked.p,
-                         (uint8_t *)m->staging.p, m->nn);
-      HIPCHECK(hipGetLastError());
-      HIPCHECK(hipMemcpyAsync(host, m->staging.p, bytes, hipMemcpyDeviceToHost,
-                              m->stream));
-      HIPCHECK(hipStreamSynchronize(m->stream));
-      return;
-    }
-    default:
-      throw Error(AKX_ERR_INVALID, "unknown field");
-    }
-    download_soa(m, (const double *)src, (double *)host, m->nn, 3);
+    if (!list.empty())
+      m->download.get(m->device, m->stream, list);
+  });
+}
+
+int akx_host_differs(const void *a, const void *b, int64_t bytes, int *differs) {
+  return guard([&] {
+    require(a && b && differs && bytes >= 0, "bad arguments");
+    *differs = host_differs(a, b, (size_t)bytes);
   });
 }
 

@@ -57,6 +57,7 @@ def _p(a):
 _libc = C.CDLL(None)
 _libc.memcmp.restype = C.c_int
 _libc.memcmp.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t]
+_LARGE = 4 << 20  # bytes from which the library's threads compare host arrays
 _SOLVER_IDS = ("", "explicit_lumped")
 
 
@@ -80,10 +81,11 @@ class _Mirror:
 
     __slots__ = ("base", "snap", "view", "writable")
 
-    def __init__(self, base, writable):
+    def __init__(self, base, writable, snap=None):
         self.base = base
         self.writable = writable
-        self.snap = base.copy() if writable else None
+        # what base held when it was last filled (by then snap holds it too)
+        self.snap = (base.copy() if snap is None else snap) if writable else None
         self.view = None  # weak reference to the last view handed out
 
     def held(self):
@@ -91,8 +93,14 @@ class _Mirror:
         return sys.getrefcount(self.base) > 2
 
     def edited(self):
-        return self.writable and _libc.memcmp(self.base.ctypes.data, self.snap.ctypes.data,
-                                              self.base.nbytes) != 0
+        if not self.writable:
+            return False
+        n = self.base.nbytes
+        if n < _LARGE:
+            return _libc.memcmp(self.base.ctypes.data, self.snap.ctypes.data, n) != 0
+        differs = C.c_int(0)
+        N.check(N.lib().akx_host_differs(_p(self.base), _p(self.snap), n, C.byref(differs)))
+        return bool(differs.value)
 
 
 class MaterialFactory:
@@ -371,6 +379,7 @@ class SolidMechanicsModel:
         self.nb_nodes = nodes.shape[0]
         self.materials = []
         self._mirrors = {}
+        self._spare = {}  # field -> arrays of its last dropped copy
         self._initialized = False
         self._stresses_fresh = False
         self.time_step = 0.0
@@ -572,30 +581,53 @@ class SolidMechanicsModel:
                 np.copyto(mir.snap, mir.base)
                 self._stresses_fresh = False
             if not mir.held():
-                del self._mirrors[name]
+                self._drop(name)
+
+    def _drop(self, name):
+        """Forget a copy nothing refers to.  Its memory (the copy's and the
+        snapshot's) is kept for the field's next copy, one per field: a new
+        array's page faults cost more than the download."""
+        mir = self._mirrors.pop(name)
+        self._spare[name] = (mir.base, mir.snap)
+
+    def _download(self, mirs):
+        """Fill the copies (name, mirror), all with one wait for the device."""
+        n = len(mirs)
+        if n == 0:
+            return
+        fields = (C.c_int * n)(*[_FIELDS[name] for name, _ in mirs])
+        host = (C.c_void_p * n)(*[m.base.ctypes.data for _, m in mirs])
+        copy = (C.c_void_p * n)(*[m.snap.ctypes.data if m.writable else None for _, m in mirs])
+        N.check(N.lib().akx_model_get_fields(self._h, n, fields, host, copy))
 
     def _refresh(self, names=None):
         """After a call that changed device fields: bring the held copies up
         to date in place (all of them, or those in ``names``)."""
         self._stresses_fresh = False
+        if not self._mirrors:
+            return
+        fill = []
         for name in list(self._mirrors):
             if names is not None and name not in names:
                 continue
             mir = self._mirrors[name]
-            if not mir.held():
-                del self._mirrors[name]
-                continue
-            N.check(N.lib().akx_model_get_field(self._h, _FIELDS[name], _p(mir.base)))
-            if mir.writable:
-                np.copyto(mir.snap, mir.base)
+            if mir.held():
+                fill.append((name, mir))
+            else:
+                self._drop(name)
+        self._download(fill)
 
     def _get(self, name):
         mir = self._mirrors.get(name)
         if mir is None:
-            dtype = np.uint8 if name == "blocked_dofs" else np.float64
-            base = np.empty((self.nb_nodes, 3), dtype)
-            N.check(N.lib().akx_model_get_field(self._h, _FIELDS[name], _p(base)))
-            mir = _Mirror(base, name in _WRITABLE)
+            base, snap = self._spare.pop(name, (None, None))
+            if base is None:
+                dtype = np.uint8 if name == "blocked_dofs" else np.float64
+                base = np.empty((self.nb_nodes, 3), dtype)
+                snap = np.empty_like(base) if name in _WRITABLE else None
+            mir = _Mirror(base, name in _WRITABLE, snap)
+            del base
+            self._download([(name, mir)])
             self._mirrors[name] = mir
         view = mir.view() if mir.view is not None else None
         if view is None:

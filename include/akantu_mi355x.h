@@ -253,6 +253,12 @@ int akx_model_assemble_internal_forces(akx_model *m);
 /* Fields --------------------------------------------------------------------*/
 int akx_model_get_nb_nodes(akx_model *m, int64_t *nb_nodes);
 int akx_model_get_field(akx_model *m, int field, void *host);
+/* Several fields with one wait; copy (or copy[k]) may be null, otherwise
+ * field k is written to copy[k] too. */
+int akx_model_get_fields(akx_model *m, int count, const int *fields, void *const *host,
+                         void *const *copy);
+/* Whether two host arrays differ (compared by several threads when large). */
+int akx_host_differs(const void *a, const void *b, int64_t bytes, int *differs);
 int akx_model_set_field(akx_model *m, int field, const void *host);
 /* BC::Neumann::FromTraction applied on a group of boundary facets
  * (boundary_condition_tmpl.hh:100-160, boundary_condition_functor_inline_impl
