@@ -16,7 +16,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
+#include <condition_variable>
 #include <cstring>
+#include <deque>
 #include <exception>
 #include <functional>
 #include <memory>
@@ -26,10 +29,58 @@
 
 namespace akx {
 
+// Threads that help with copies, for the whole process: at most seven, started
+// when work is there and none is idle, gone after two idle seconds.  Waiting
+// threads are scheduled at once when they are woken; a new thread waits a
+// scheduler's slice (3 ms) where the CPUs are busy, as they are for a while
+// after an OpenMP loop.  Never destroyed: a thread may wait in it at exit.
+class CopyThreads {
+  static constexpr int MOST = 7;
+  std::mutex mutex;
+  std::condition_variable wake;
+  std::deque<std::function<void()>> queue;
+  int threads = 0, idle = 0;
+
+  void loop() {
+    std::unique_lock<std::mutex> lock(mutex);
+    for (;;) {
+      ++idle;
+      const bool work = wake.wait_for(lock, std::chrono::seconds(2),
+                                      [&] { return !queue.empty(); });
+      --idle;
+      if (!work) {
+        --threads;
+        return;
+      }
+      std::function<void()> f = std::move(queue.front());
+      queue.pop_front();
+      lock.unlock();
+      f(); // does not throw
+      f = nullptr;
+      lock.lock();
+    }
+  }
+
+public:
+  static CopyThreads &get() {
+    static CopyThreads *p = new CopyThreads;
+    return *p;
+  }
+  void submit(const std::function<void()> &f, int copies) {
+    std::lock_guard<std::mutex> lock(mutex);
+    for (int k = 0; k < copies; ++k)
+      queue.push_back(f);
+    while (threads < MOST && (int)queue.size() > threads) {
+      std::thread([this] { loop(); }).detach();
+      ++threads;
+    }
+    wake.notify_all();
+  }
+};
+
 // Chunks 0 .. n - 1 claimed by the calling thread and up to threads - 1
-// others.  The caller waits for every claimed chunk, not for the threads: on a
-// host whose CPUs are busy (an OpenMP runtime spinning after its last loop)
-// one that has not been scheduled yet is not waited for, and finds nothing to
+// others.  The caller waits for every claimed chunk, not for the threads: one
+// that has not been scheduled yet is not waited for, and finds nothing to
 // claim when it is.
 struct ChunkJob {
   std::atomic<int64_t> next{0}, done{0}, skipped{0};
@@ -72,11 +123,11 @@ template <class F> void run_chunks(int threads, int64_t n, const F &work) {
       job->fail(std::current_exception());
     }
   };
-  try {
-    for (int t = 1; t < threads; ++t)
-      std::thread(loop).detach();
-  } catch (...) { // no thread to be had: their share is done here
-  }
+  if (threads > 1)
+    try {
+      CopyThreads::get().submit(loop, threads - 1);
+    } catch (...) { // no thread to be had: their share is done here
+    }
   loop();
   while (job->done.load() + job->skipped.load() < n)
     std::this_thread::yield();
