@@ -79,6 +79,40 @@ struct ElemArgs {
 };
 
 // ---------------------------------------------------------------------------
+// One step of a small model in one launch (akx_step.hpp).  Workgroup b owns
+// the nodes b * own ..; its lists, padded to the longest of any workgroup,
+// hold every node of the elements around them (padded with -1) and those
+// elements (the padding repeats the first).  The corners of
+// one owned node take consecutive LDS slots in assembly order; all other
+// corners take the slot after the last, which nothing reads.
+// ---------------------------------------------------------------------------
+struct StepArgs {
+  const int32_t *lnode, *lelem; // [blocks][max_nodes], [blocks][max_elems]
+  const uint16_t *lc, *ls;      // [blocks][max_elems][nnpe] local node, slot
+  const uint16_t *send;         // [blocks][own] end of each node's slots
+  const uint8_t *run;           // [blocks][max_slots] last corner of a partial sum
+  int32_t own, max_nodes, max_elems, max_slots;
+  int32_t nblocks, nblocks_padded;
+  int64_t nn, nel;
+  int32_t first, last; // first / last step of the call
+  // [3][nn] before the step (when first, before its predictor) ...
+  const double *X, *u, *v, *a;
+  const float *cu, *cv; // FP32 form: compensation terms
+  // ... and after it.  u2 never is u (null: u stays as it is); the others are
+  // the same arrays unless first, when other workgroups read them
+  double *u2, *v2, *a2;
+  float *cu2, *cv2;
+  const double *mass, *fext; // fext: null for none
+  const uint8_t *blocked;
+  double *fint; // null while steps follow in the call
+  double dt;
+  double lambda, mu;
+  const double *lam_el, *mu_el; // per element, or null
+  const float2 *lm_f;           // FP32 form: the pair per element, or null
+  const double2 *jw;            // Hex8: the jacobian table
+};
+
+// ---------------------------------------------------------------------------
 // Where the Gauss-point state of one launch lives: previous (read) and
 // current (written) plastic history, [9][nq_all] column-major 3x3 and
 // [nq_all] for the hardening, stored in HT; and the optional grad u /
@@ -186,6 +220,13 @@ struct NodesLDS {
     x[0] = a.x;
     x[1] = a.y;
     x[2] = b.x;
+    d[0] = b.y;
+    d[1] = c.x;
+    d[2] = c.y;
+  }
+  __device__ __forceinline__ void load_u(int32_t n, double (&d)[3]) const {
+    const double2 *p = reinterpret_cast<const double2 *>(s + 6 * n);
+    const double2 b = p[1], c = p[2];
     d[0] = b.y;
     d[1] = c.x;
     d[2] = c.y;

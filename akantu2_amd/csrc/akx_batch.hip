@@ -86,11 +86,10 @@ __global__ void __launch_bounds__(EPB * 8) k_batch_hex8(BatchElemArgs A) {
     for (int base = 0; base < T.count; base += EPB) {
       const bool active = base + el < T.count;
       const int64_t e = T.first + (active ? base + el : 0);
-      hex8_strict_group<LAW, EPB, double, NodesXU, FE_W>(sN, sD, wq, el, q, active,
-                                                         A.conn + e * 8,
-                                          NodesXU{A.xu}, P.lambda, P.mu, P.sigma_y, P.h,
-                                          V, A.hoff + e * 8 + q, A.pos + e * 8,
-                                          reinterpret_cast<double *>(A.fe));
+      hex8_strict_group<LAW, EPB, double, NodesXU>(
+          sN, sD, wq, el, q, active, A.conn[e * 8 + q], NodesXU{A.xu}, P.lambda, P.mu,
+          P.sigma_y, P.h, V, A.hoff + e * 8 + q,
+          PutEntries{A.pos + e * 8, reinterpret_cast<double *>(A.fe)});
     }
   }
 }

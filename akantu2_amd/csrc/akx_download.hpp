@@ -170,6 +170,11 @@ inline bool host_differs(const void *a, const void *b, size_t bytes) {
 class Downloader {
   unsigned char *pin = nullptr;
   size_t cap = 0;
+  // A model's first few small copies go through device memory: they cost 40 us
+  // more each, but pinning and unpinning a buffer costs a model 0.3 ms.
+  static constexpr int UNPINNED = 4;
+  int small_copies = 0;
+  DevBuf<unsigned char> dev;
   std::vector<hipEvent_t> events; // two per thread
 
   void reserve(size_t bytes) {
@@ -216,6 +221,22 @@ public:
     size_t total = 0;
     for (auto &f : fields)
       total += (f.bytes() + 63) / 64 * 64;
+    if (total <= COPY_CHUNK && total > cap && ++small_copies <= UNPINNED) {
+      dev.reserve(total);
+      size_t o = 0;
+      for (auto &f : fields) {
+        if (f.n > 0) {
+          f.pack(dev.p + o, 0, f.n);
+          HIPCHECK(hipMemcpyAsync(f.host, dev.p + o, f.bytes(), hipMemcpyDeviceToHost, stream));
+        }
+        o += (f.bytes() + 63) / 64 * 64;
+      }
+      HIPCHECK(hipStreamSynchronize(stream));
+      for (auto &f : fields)
+        if (f.copy)
+          std::memcpy(f.copy, f.host, f.bytes());
+      return;
+    }
     if (total <= COPY_CHUNK) {
       reserve(std::max<size_t>(total, 64));
       size_t o = 0;

@@ -24,6 +24,7 @@
 #include "akx_args.hpp"
 #include "akx_math.hpp"
 #include "akx_fast.hpp"
+#include "akx_step.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -1042,6 +1043,51 @@ __global__ void __launch_bounds__(256) k_tet4_bpa(ElemArgs A) {
   }
 }
 
+// One step of a small FP32 Tet4 model (akx_step.hpp): one lane per element of
+// the workgroup's list, the corners of its own nodes to LDS slots.
+template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepArgs S) {
+  extern __shared__ double2 s_rec[]; // records, then slots, then the runs' ends
+  const int64_t b = xcd_block(S.nblocks_padded);
+  if (b >= S.nblocks) // padding block
+    return;
+  const int t = threadIdx.x;
+  float *s_slot = reinterpret_cast<float *>(s_rec + 3 * S.max_nodes);
+  uint8_t *s_run = reinterpret_cast<uint8_t *>(s_slot + 3 * (S.max_slots + 1));
+  // lanes past the list do its last element again, to the slot nothing reads
+  const bool active = t < S.max_elems;
+  const int64_t i = b * S.max_elems + (active ? t : S.max_elems - 1);
+  const ushort4 lc = *reinterpret_cast<const ushort4 *>(S.lc + i * 4);
+  const ushort4 ls = *reinterpret_cast<const ushort4 *>(S.ls + i * 4);
+  float lambda = (float)S.lambda, mu = (float)S.mu;
+  if (S.lm_f) {
+    const float2 lm = S.lm_f[S.lelem[i]];
+    lambda = lm.x;
+    mu = lm.y;
+  }
+  StepDof<true> dof;
+  dof.load(S, b);
+  for (int k = t; k < S.max_slots; k += blockDim.x)
+    s_run[k] = S.run[b * S.max_slots + k];
+  step_stage<true>(S, b, s_rec);
+  __syncthreads();
+  if (active) {
+    float Q[3][3];
+    tet4_Q<LAW, float, QpViewT<double>, akx::NodesLDS, false>(
+        make_int4(lc.x, lc.y, lc.z, lc.w),
+        akx::NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, 0.f, 0.f,
+        QpViewT<double>{}, 0, Q);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      s_slot[3 * ls.x + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
+      s_slot[3 * ls.y + c] = Q[c][1];
+      s_slot[3 * ls.z + c] = Q[c][2];
+      s_slot[3 * ls.w + c] = Q[c][0];
+    }
+  }
+  __syncthreads();
+  dof.update<true>(S, s_slot, s_run);
+}
+
 // ---------------------------------------------------------------------------
 // Batched FP32 form, one tile of one (element type, law) group per
 // workgroup; per-instance parameters, compact FP32 plastic state (ping-pong
@@ -1273,6 +1319,24 @@ hipError_t launch_elements(int etype, int law, bool fp32, const ElemArgs &A,
                            hipStream_t stream) {
   return fp32 ? launch_t<float, float>(etype, law, A, stream)
               : launch_t<double, double>(etype, law, A, stream);
+}
+
+hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream) {
+  const dim3 grid((unsigned)S.nblocks_padded), block(256);
+  switch (law) {
+  case LAW_ELASTIC:
+    hipLaunchKernelGGL(k_tet4_step_f32<LAW_ELASTIC>, grid, block, lds, stream, S);
+    break;
+  case LAW_ELASTIC_FD:
+    hipLaunchKernelGGL(k_tet4_step_f32<LAW_ELASTIC_FD>, grid, block, lds, stream, S);
+    break;
+  case LAW_NEOHOOKEAN:
+    hipLaunchKernelGGL(k_tet4_step_f32<LAW_NEOHOOKEAN>, grid, block, lds, stream, S);
+    break;
+  default:
+    return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 template <int LAW>

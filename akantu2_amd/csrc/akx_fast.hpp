@@ -14,6 +14,8 @@ int64_t elements_per_block(int etype, bool bpa = false);
 // launch the element pass of one material (etype 0 = Tet4, 1 = Hex8)
 hipError_t launch_elements(int etype, int law, bool fp32, const akx::ElemArgs &A,
                            hipStream_t stream);
+// launch one step of a small FP32 Tet4 model (akx_step.hpp)
+hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream);
 // launch the FP32-form batched element pass of one (element type, law) group;
 // block = threads per block (64, 128 or 256; Hex8: 8 lanes per element)
 hipError_t launch_batch_elements_f32(int etype, int law, int block,

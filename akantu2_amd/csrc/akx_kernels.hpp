@@ -728,17 +728,42 @@ __global__ void __launch_bounds__(PPA_TB) k_tet4_ppa(ElemArgs A) {
 // hex8_strict_group handles one group of EPB elements; every lane of the
 // block calls it (it holds barriers), inactive lanes with active = false.
 // sD holds dN_n/dxi_m at the Gauss points, [q][m][n]; wq is the Gauss weight;
-// with PRE, jw points at the lane's Gauss point in the [5][jw_stride] table.
+// nd: node q of the element; put(n, c, s): component c of the force on node n;
+// with PRE, pre holds the lane's Gauss point's J^-1 and w det J.
 // ---------------------------------------------------------------------------
 constexpr int HEX_STRICT_EPB = 8;
 
-template <int LAW, int EPB, class HT, class NA, int W = 3, bool PRE = false, bool EXT = false>
+// J^-1 and w det J of one Gauss point, from the table that init fills (jw: the
+// Gauss point's column 0 of [5][stride]).  Streamed once per step:
+// non-temporal loads leave the caches to the nodal data.
+struct HexJac {
+  double Ji[3][3], wJ;
+  __device__ __forceinline__ void load(const double2 *jw, int64_t stride) {
+    typedef double dv2 __attribute__((ext_vector_type(2)));
+    const dv2 *jv = reinterpret_cast<const dv2 *>(jw);
+    const dv2 j0 = __builtin_nontemporal_load(jv), j1 = __builtin_nontemporal_load(jv + stride),
+              j2 = __builtin_nontemporal_load(jv + 2 * stride),
+              j3 = __builtin_nontemporal_load(jv + 3 * stride),
+              j4 = __builtin_nontemporal_load(jv + 4 * stride);
+    Ji[0][0] = j0.x;
+    Ji[0][1] = j0.y;
+    Ji[0][2] = j1.x;
+    Ji[1][0] = j1.y;
+    Ji[1][1] = j2.x;
+    Ji[1][2] = j2.y;
+    Ji[2][0] = j3.x;
+    Ji[2][1] = j3.y;
+    Ji[2][2] = j4.x;
+    wJ = j4.y;
+  }
+};
+
+template <int LAW, int EPB, class HT, class NA, bool PRE = false, bool EXT = false, class PUT>
 __device__ __forceinline__ void hex8_strict_group(
     double (&sN)[EPB][8][6], const double (&sD)[8][3][8],
-    double wq, int el, int q, bool active, const int32_t *conn_e, const NA &nodes_of,
+    double wq, int el, int q, bool active, int32_t nd, const NA &nodes_of,
     double lambda, double mu, double sy, double hh,
-    const QpViewT<HT> &V, int64_t iq, const int32_t *pos_e, double *fe,
-    const double2 *jw = nullptr, int64_t jw_stride = 0) {
+    const QpViewT<HT> &V, int64_t iq, const PUT &put, const HexJac &pre = HexJac{}) {
   // The dN/dX columns of the gradient are kept for the force terms (24
   // registers instead of J^-1's 9 and 120 operations); the plastic law keeps
   // recomputing them, its history already holds registers.
@@ -747,34 +772,20 @@ __device__ __forceinline__ void hex8_strict_group(
   double Bk[KEEP_B ? 8 : 1][3];
   if (active) {
     if constexpr (PRE) {
-      // J^-1 and w det J from the table (jw: this Gauss point's column 0),
-      // streamed once per step: non-temporal loads leave the caches to the
-      // nodal data
       double d[3];
-      nodes_of.load_u(conn_e[q], d);
+      nodes_of.load_u(nd, d);
 #pragma unroll
       for (int c = 0; c < 3; ++c)
         sN[el][q][3 + c] = d[c];
-      typedef double dv2 __attribute__((ext_vector_type(2)));
-      const dv2 *jv = reinterpret_cast<const dv2 *>(jw);
-      const dv2 j0 = __builtin_nontemporal_load(jv),
-                j1 = __builtin_nontemporal_load(jv + jw_stride),
-                j2 = __builtin_nontemporal_load(jv + 2 * jw_stride),
-                j3 = __builtin_nontemporal_load(jv + 3 * jw_stride),
-                j4 = __builtin_nontemporal_load(jv + 4 * jw_stride);
-      Ji[0][0] = j0.x;
-      Ji[0][1] = j0.y;
-      Ji[0][2] = j1.x;
-      Ji[1][0] = j1.y;
-      Ji[1][1] = j2.x;
-      Ji[1][2] = j2.y;
-      Ji[2][0] = j3.x;
-      Ji[2][1] = j3.y;
-      Ji[2][2] = j4.x;
-      wJ = j4.y;
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+          Ji[r][c] = pre.Ji[r][c];
+      wJ = pre.wJ;
     } else {
       double x[3], d[3];
-      nodes_of.load(conn_e[q], x, d);
+      nodes_of.load(nd, x, d);
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         sN[el][q][c] = x[c];
@@ -862,32 +873,27 @@ __device__ __forceinline__ void hex8_strict_group(
       }
     }
     __syncthreads();
-    if constexpr (W == 3) {
-      // lane q < 6 sums component q % 3 of node 2 hh2 + q / 3
-      if (active && q < 6) {
-        const int c = q >= 3 ? 1 : 0;
-        double s = sR[el][0][q];
+    // lane q < 6 sums component q % 3 of node 2 hh2 + q / 3
+    if (active && q < 6) {
+      const int c = q >= 3 ? 1 : 0;
+      double s = sR[el][0][q];
 #pragma unroll
-        for (int qq = 1; qq < 8; ++qq)
-          s += sR[el][qq][q];
-        fe[(int64_t)pos_e[2 * hh2 + c] * 3 + (q - 3 * c)] = s;
-      }
-    } else if (active && q < 2) {
-      const int n = 2 * hh2 + q;
-      double r[3];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        double s = sR[el][0][3 * q + k];
-#pragma unroll
-        for (int qq = 1; qq < 8; ++qq)
-          s += sR[el][qq][3 * q + k];
-        r[k] = s;
-      }
-      put_entry<W>(fe, (int64_t)pos_e[n], r[0], r[1], r[2]);
+      for (int qq = 1; qq < 8; ++qq)
+        s += sR[el][qq][q];
+      put(2 * hh2 + c, q - 3 * c, s);
     }
     __syncthreads();
   }
 }
+
+// hex8_strict_group's results to their entries of the force table
+struct PutEntries {
+  const int32_t *pos_e;
+  double *fe;
+  __device__ __forceinline__ void operator()(int n, int c, double s) const {
+    fe[(int64_t)pos_e[n] * 3 + c] = s;
+  }
+};
 
 // The single-model launch reads J^-1 and w det J from the table that init
 // fills (k_hex8_jacobian_table): they depend on the reference coordinates
@@ -915,10 +921,14 @@ __global__ void __launch_bounds__(64) k_hex8_strict(ElemArgs A) {
     if (A.h_el)
       hh = A.h_el[i];
   }
-  hex8_strict_group<LAW, HEX_STRICT_EPB, double, NodesSoA, 3, true, EXT>(
-      sN, sD, c_hex8.w[q], el, q, active, A.conn + e * 8, NodesSoA{A.X, A.u, A.nn},
-      lambda, mu, sy, hh, qp_view(A, 8), i * 8 + q, A.pos + (A.pos_offset + (active ? i : 0)) * 8,
-      reinterpret_cast<double *>(A.fe), A.jw + e * 8 + q, A.nel * 8);
+  HexJac pre{};
+  if (active)
+    pre.load(A.jw + e * 8 + q, A.nel * 8);
+  hex8_strict_group<LAW, HEX_STRICT_EPB, double, NodesSoA, true, EXT>(
+      sN, sD, c_hex8.w[q], el, q, active, active ? A.conn[e * 8 + q] : 0,
+      NodesSoA{A.X, A.u, A.nn}, lambda, mu, sy, hh, qp_view(A, 8), i * 8 + q,
+      PutEntries{A.pos + (A.pos_offset + (active ? i : 0)) * 8, reinterpret_cast<double *>(A.fe)},
+      pre);
 }
 
 // ---------------------------------------------------------------------------

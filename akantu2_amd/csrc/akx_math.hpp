@@ -492,10 +492,19 @@ AKX_HD void reference_gather(double f_ext, double f_int, double M, double dt, do
     reference_predict(a, dt, v, u);
 }
 
+// a * b, rounded: not contracted with what follows in any translation unit
+AKX_HD double rounded_product(double a, double b) {
+  double p = a * b;
+#ifdef __HIP_DEVICE_COMPILE__
+  asm("" : "+v"(p));
+#endif
+  return p;
+}
+
 AKX_HD void half_step_predict(double a, double dt, double &v, float &cv, double &u,
                               float &cu) {
-  kahan_add(v, cv, (.5 * dt) * a);
-  kahan_add(u, cu, dt * v);
+  kahan_add(v, cv, rounded_product(.5 * dt, a));
+  kahan_add(u, cu, rounded_product(dt, v));
 }
 
 // w, cw: the half-step velocity on entry; the velocity (PREDICT = false)
@@ -504,10 +513,11 @@ template <bool PREDICT>
 AKX_HD void half_step_gather(double f, double M, double dt, double &w, float &cw, double &u,
                              float &cu, double &a) {
   a = f / M;
-  kahan_add(w, cw, (.5 * dt) * a);
+  const double half = rounded_product(.5 * dt, a);
+  kahan_add(w, cw, half);
   if constexpr (PREDICT) {
-    kahan_add(w, cw, (.5 * dt) * a);
-    kahan_add(u, cu, dt * w);
+    kahan_add(w, cw, half);
+    kahan_add(u, cu, rounded_product(dt, w));
   }
 }
 

@@ -5,12 +5,14 @@
 // (default priority).  The per-step work is two launches:
 //   element pass (one kernel per material)  ->  nodal gather + update
 // with the predictor of step k+1 fused into the gather of step k when
-// several steps are queued together.
+// several steps are queued together; small models take one launch per step
+// (plan_small_steps).
 #include "../../include/akantu_mi355x.h"
 #include "akx_download.hpp"
 #include "akx_fast.hpp"
 #include "akx_host.hpp"
 #include "akx_kernels.hpp"
+#include "akx_step.hpp"
 
 #include <hip/hip_runtime.h>
 #include <hip/hiprtc.h>
@@ -30,6 +32,94 @@ namespace akx {
 __constant__ Hex8Tables c_hex8;
 
 thread_local std::string g_last_error;
+
+// ---------------------------------------------------------------------------
+// One step of a small FP64 model (akx_step.hpp).
+// ---------------------------------------------------------------------------
+
+// Tet4: one lane per element of the workgroup's list
+template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step(StepArgs S) {
+  extern __shared__ double2 s_rec[]; // records, then slots
+  const int64_t b = xcd_block(S.nblocks_padded);
+  if (b >= S.nblocks) // padding block
+    return;
+  const int t = threadIdx.x;
+  double *s_slot = reinterpret_cast<double *>(s_rec + 3 * S.max_nodes);
+  const bool active = t < S.max_elems;
+  const int64_t i = b * S.max_elems + (active ? t : S.max_elems - 1);
+  const ushort4 lc = *reinterpret_cast<const ushort4 *>(S.lc + i * 4);
+  const ushort4 ls = *reinterpret_cast<const ushort4 *>(S.ls + i * 4);
+  double lambda = S.lambda, mu = S.mu;
+  if (S.lam_el) {
+    const int32_t e = S.lelem[i];
+    lambda = S.lam_el[e];
+    mu = S.mu_el[e];
+  }
+  StepDof<false> dof;
+  dof.load(S, b);
+  step_stage<false>(S, b, s_rec);
+  __syncthreads();
+  if (active) {
+    const int4 nd = make_int4(lc.x, lc.y, lc.z, lc.w);
+    const int4 slots = make_int4(-1 - ls.x, -1 - ls.y, -1 - ls.z, -1 - ls.w);
+    element_forces_one<ET_TET4, LAW, double, double, double, NodesLDS, 3, false, true>(
+        reinterpret_cast<const int32_t *>(&nd),
+        NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, 0., 0., QpView{}, 0,
+        reinterpret_cast<const int32_t *>(&slots), s_slot, s_slot);
+  }
+  __syncthreads();
+  dof.update<false>(S, s_slot, nullptr);
+}
+
+// hex8_strict_group's results to the slots of the element's corners
+struct PutSlots {
+  const uint16_t *ls; // LDS, the element's 8 corners
+  double *s_slot;
+  __device__ __forceinline__ void operator()(int n, int c, double s) const {
+    s_slot[3 * ls[n] + c] = s;
+  }
+};
+
+// Hex8: eight lanes per element, STEP_HEX_EPB elements at a time
+constexpr int STEP_HEX_EPB = 32;
+template <int LAW> __global__ void __launch_bounds__(STEP_HEX_EPB * 8) k_hex8_step(StepArgs S) {
+  extern __shared__ double2 s_rec[]; // records, then slots
+  __shared__ double sN[STEP_HEX_EPB][8][6];
+  __shared__ double sD[8][3][8];
+  __shared__ uint16_t s_ls[STEP_HEX_EPB][8];
+  const int64_t b = xcd_block(S.nblocks_padded);
+  if (b >= S.nblocks) // padding block
+    return;
+  const int t = threadIdx.x, el = t >> 3, q = t & 7;
+  double *s_slot = reinterpret_cast<double *>(s_rec + 3 * S.max_nodes);
+  StepDof<false> dof;
+  dof.load(S, b);
+  for (int base = 0; base < S.max_elems; base += STEP_HEX_EPB) {
+    const bool active = base + el < S.max_elems;
+    const int64_t i = b * S.max_elems + (active ? base + el : S.max_elems - 1);
+    const int32_t e = S.lelem[i];
+    const int32_t nd = S.lc[i * 8 + q];
+    double lambda = S.lambda, mu = S.mu;
+    if (S.lam_el) {
+      lambda = S.lam_el[e];
+      mu = S.mu_el[e];
+    }
+    s_ls[el][q] = S.ls[i * 8 + q];
+    HexJac pre;
+    pre.load(S.jw + (int64_t)e * 8 + q, S.nel * 8);
+    if (base == 0) {
+      step_stage<false>(S, b, s_rec);
+      for (int k = t; k < 192; k += STEP_HEX_EPB * 8)
+        (&sD[0][0][0])[k] = (&c_hex8.dnds[0][0][0])[k];
+      __syncthreads();
+    }
+    hex8_strict_group<LAW, STEP_HEX_EPB, double, NodesLDS, true>(
+        sN, sD, c_hex8.w[q], el, q, active, nd,
+        NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, 0., 0., QpView{}, 0,
+        PutSlots{s_ls[el], s_slot}, pre);
+  }
+  dof.update<false>(S, s_slot, nullptr); // the group's last barrier is behind
+}
 
 // ---------------------------------------------------------------------------
 // Layout kernels (array-of-structures at the API, structure-of-arrays on the
@@ -561,6 +651,11 @@ struct Material {
   std::unique_ptr<DeviceLaw> dlaw;
 };
 
+// meshes of up to this many nodes hold u, v and a twice
+constexpr int64_t STEP_NODES_MAX = 10240;
+// doubles or floats from one [3][nn] array of the state to the next
+inline int64_t state_stride(int64_t nn) { return (3 * nn + 31) / 32 * 32; }
+
 struct akx_model {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -571,9 +666,17 @@ struct akx_model {
   bool has_fext = false;
   double dt = 0.;
   std::vector<int32_t> conn_host; // AoS copy for filters and the gather table
-  DevBuf<double> X, u, v, a, fint, fext, mass;
+  DevBuf<double> X, fint, fext, mass;
+  // u, v, a and the FP32 form's compensation terms, each [3][nn], with the
+  // second ones of meshes small enough for single-launch steps
+  template <class T> struct Part {
+    T *p = nullptr;
+  };
+  DevBuf<double> state;
+  DevBuf<float> comp;
+  Part<double> u, v, a, u2, v2, a2;
+  Part<float> cu, cv, cu2, cv2;
   DevBuf<uint8_t> blocked;
-  DevBuf<float> cu, cv;
   DevBuf<int32_t> conn, pos;
   DevBuf<double2> jw;      // Hex8 plain FP64: J^-1, w det J [5][nel * 8]
   DevBuf<double> xu;       // Tet4: [nn][6] {X, u} node records of the element pass
@@ -602,6 +705,11 @@ struct akx_model {
   DevBuf<uint8_t> pp_deg;
   int64_t pp_total = 0;
   int64_t pp_entries = 0, pp_runs = 0; // table entries, summed runs
+  // one launch per step (plan_small_steps; step.nblocks 0: not planned): the
+  // lists and the dynamic LDS
+  StepArgs step{};
+  DevBuf<unsigned char> step_lists;
+  size_t step_lds = 0;
   DevBuf<unsigned char> staging;
   Downloader download;
   DevBuf<unsigned long long> scratch_u64;
@@ -1567,6 +1675,247 @@ void launch_predictor(akx_model *m) {
 }
 
 // ---------------------------------------------------------------------------
+// One launch per step for small models (akx_step.hpp): one contiguous material
+// of a non-plastic built-in law over the whole mesh, FP64 or FP32 Tet4.
+//
+// A step of two launches takes 8 to 14 us however small the mesh; in one
+// launch it takes 5, what the host needs to queue it.  An element's arithmetic
+// is repeated in every workgroup that owns one of its nodes (on boxes 3.1
+// times for Tet4, 4.6 times for Hex8), so the gain ends where that fills the
+// chip.  us a step, two launches -> one (boxes):
+//   Tet4 FP64 elastic   525 nodes 12.0 -> 5.1, 4,032 12.5 -> 5.9, 10,416
+//                       13.6 -> 9.3, 26,691 16.8 -> 16.9
+//   Tet4 FP64 neo-H.    4,032 13.6 -> 7.5, 10,416 14.4 -> 12.7, 13,776
+//                       15.6 -> 14.8, 26,691 19.0 -> 25.1
+//   Tet4 FP32 elastic   1,152 7.9 -> 5.2, 10,416 8.4 -> 6.9, 13,776 9.0 ->
+//                       8.3, 26,691 9.5 -> 12.0
+//   Hex8 FP64 neo-H.    1,331 10.4 -> 7.8, 2,520 10.5 -> 10.0, 4,032 10.8 ->
+//                       12.5
+//   Hex8 FP64 elastic   1,536 9.1 -> 6.4, 2,520 9.2 -> 7.7, 4,032 9.3 -> 9.3
+// A Tet4 workgroup owns 8 nodes (a run along a row of a box has 150 elements,
+// one a lane), a Hex8 one 6 (28 elements of eight lanes; 8 nodes have 36 and
+// would take a second round).
+// ---------------------------------------------------------------------------
+constexpr int STEP_OWN_TET4 = 8, STEP_OWN_HEX8 = 6;
+constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_HEX8 = 2560;
+static_assert(STEP_NODES_TET4 <= STEP_NODES_MAX && STEP_NODES_HEX8 <= STEP_NODES_MAX,
+              "larger meshes have no second state arrays");
+constexpr size_t STEP_LDS = 48 * 1024;
+
+void plan_small_steps(akx_model *m) {
+  const bool hex = m->etype == AKX_HEX8;
+  if (m->mats.size() != 1 || m->nn == 0 ||
+      m->nn > (hex ? STEP_NODES_HEX8 : STEP_NODES_TET4) ||
+      m->precision == AKX_PRECISION_FP64_FAST || (hex && m->precision == AKX_PRECISION_FP32))
+    return;
+  const Material &mat = *m->mats[0];
+  const bool f32 = m->precision == AKX_PRECISION_FP32;
+  if (!mat.contiguous || mat.first != 0 || mat.n != m->nel || mat.n == 0 || mat.user() ||
+      mat.law == AKX_LAW_PLASTIC_LIH)
+    return;
+  if (!f32 && m->ppa && m->assembly == AKX_ASSEMBLY_BLOCK_PARTIALS)
+    return; // sums runs in FP64 without rounding them as the FP32 form does
+  const int nnpe = m->nnpe, own = hex ? STEP_OWN_HEX8 : STEP_OWN_TET4;
+  const int32_t *conn = m->conn_host.data();
+  const int64_t nn = m->nn, nel = m->nel, nb = (nn + own - 1) / own;
+  // elements around every node, in ascending order
+  std::vector<int32_t> first(nn + 1, 0), around(nel * nnpe);
+  for (int64_t i = 0; i < nel * nnpe; ++i)
+    first[conn[i] + 1]++;
+  for (int64_t n = 0; n < nn; ++n)
+    first[n + 1] += first[n];
+  {
+    std::vector<int32_t> at(first.begin(), first.end() - 1);
+    for (int32_t e = 0; e < (int32_t)nel; ++e)
+      for (int a = 0; a < nnpe; ++a)
+        around[at[conn[(int64_t)e * nnpe + a]]++] = e;
+  }
+  // every workgroup's elements and their nodes, numbered as they are met
+  std::vector<int32_t> elems, nodes, eoff(nb + 1, 0), noff(nb + 1, 0);
+  std::vector<uint16_t> lcs;
+  std::vector<int32_t> elem_in(nel, -1), node_in(nn, -1), node_no(nn);
+  elems.reserve(4 * nel);
+  lcs.reserve(4 * nel * nnpe);
+  nodes.reserve(8 * nn);
+  int32_t max_elems = 1, max_nodes = 1, max_slots = 1;
+  for (int32_t b = 0; b < (int32_t)nb; ++b) {
+    const int64_t n0 = (int64_t)b * own, n1 = std::min<int64_t>(nn, n0 + own);
+    for (int32_t d = first[n0]; d < first[n1]; ++d) {
+      const int32_t e = around[d];
+      if (elem_in[e] == b)
+        continue;
+      elem_in[e] = b;
+      elems.push_back(e);
+      for (int a = 0; a < nnpe; ++a) {
+        const int32_t n = conn[(int64_t)e * nnpe + a];
+        if (node_in[n] != b) {
+          node_in[n] = b;
+          node_no[n] = (int32_t)nodes.size() - noff[b];
+          nodes.push_back(n);
+        }
+        lcs.push_back((uint16_t)node_no[n]);
+      }
+    }
+    eoff[b + 1] = (int32_t)elems.size();
+    noff[b + 1] = (int32_t)nodes.size();
+    max_elems = std::max(max_elems, eoff[b + 1] - eoff[b]);
+    max_nodes = std::max(max_nodes, noff[b + 1] - noff[b]);
+    max_slots = std::max(max_slots, first[n1] - first[n0]);
+  }
+  const size_t lds = (size_t)max_nodes * 48 +
+                     (size_t)(max_slots + 1) * 3 * (f32 ? sizeof(float) : sizeof(double)) +
+                     (f32 ? max_slots : 0);
+  // one lane per Tet4; at most two rounds of Hex8 (a numbering without
+  // locality makes long lists)
+  if (max_elems > (hex ? 2 * STEP_HEX_EPB : 256) || lds > STEP_LDS)
+    return;
+  // one buffer: lnode, lelem, lc, ls, send, run
+  const size_t n32 = nb * (max_nodes + max_elems), n16 = nb * (2 * max_elems * nnpe + own),
+               n8 = f32 ? nb * max_slots : 0;
+  std::vector<unsigned char> lists(((4 * n32 + 7) / 8 * 8) + 2 * n16 + n8);
+  int32_t *lnode = reinterpret_cast<int32_t *>(lists.data()), *lelem = lnode + nb * max_nodes;
+  uint16_t *lc = reinterpret_cast<uint16_t *>(lists.data() + (4 * n32 + 7) / 8 * 8),
+           *ls = lc + nb * max_elems * nnpe, *send = ls + nb * max_elems * nnpe;
+  uint8_t *run = reinterpret_cast<uint8_t *>(send + nb * own);
+  std::fill(lnode, lelem, -1);
+  std::fill(ls, send, (uint16_t)max_slots);
+  std::fill(run, run + n8, 1);
+  std::vector<int32_t> elem_no(nel);
+  for (int64_t b = 0; b < nb; ++b) {
+    const int64_t n0 = b * own, n1 = std::min<int64_t>(nn, n0 + own);
+    std::copy(nodes.begin() + noff[b], nodes.begin() + noff[b + 1], lnode + b * max_nodes);
+    const int32_t ne = eoff[b + 1] - eoff[b];
+    int32_t *lelem_b = lelem + b * max_elems;
+    uint16_t *lc_b = lc + b * max_elems * nnpe, *ls_b = ls + b * max_elems * nnpe;
+    std::copy(elems.begin() + eoff[b], elems.begin() + eoff[b + 1], lelem_b);
+    std::copy(lcs.begin() + (int64_t)eoff[b] * nnpe, lcs.begin() + (int64_t)eoff[b + 1] * nnpe,
+              lc_b);
+    // padding: the list's first element again (an empty list: element 0 of the
+    // mesh on the records of no node), to the slot nothing reads
+    for (int32_t k = ne; k < max_elems && ne > 0; ++k) {
+      lelem_b[k] = lelem_b[0];
+      std::copy(lc_b, lc_b + nnpe, lc_b + k * nnpe);
+    }
+    for (int32_t k = 0; k < ne; ++k)
+      elem_no[lelem_b[k]] = k;
+    for (int64_t n = n0; n < n1; ++n) {
+      for (int32_t d = first[n]; d < first[n + 1]; ++d) {
+        const int32_t *c = conn + (int64_t)around[d] * nnpe;
+        int a = 0;
+        while (c[a] != n)
+          ++a;
+        // a corner that repeats its node takes the next one's place
+        while (d > first[n] && around[d] == around[d - 1] &&
+               ls_b[elem_no[around[d]] * nnpe + a] != max_slots) {
+          ++a;
+          while (c[a] != n)
+            ++a;
+        }
+        ls_b[elem_no[around[d]] * nnpe + a] = (uint16_t)(d - first[n0]);
+      }
+      send[b * own + n - n0] = (uint16_t)(first[n + 1] - first[n0]);
+    }
+    // FP32 partial sums end where the element pass's block of 256 elements
+    // does (every corner is one without block assembly)
+    if (f32 && m->bpa)
+      for (int64_t n = n0; n < std::min<int64_t>(nn, n0 + own); ++n)
+        for (int32_t k = first[n]; k + 1 < first[n + 1]; ++k)
+          run[b * max_slots + k - first[n0]] = around[k] / 256 != around[k + 1] / 256;
+  }
+  m->step_lists.alloc(lists.size());
+  HIPCHECK(hipMemcpy(m->step_lists.p, lists.data(), lists.size(), hipMemcpyHostToDevice));
+  StepArgs &S = m->step;
+  const auto on_device = [&](const void *host) {
+    return m->step_lists.p + (static_cast<const unsigned char *>(host) - lists.data());
+  };
+  S.lnode = reinterpret_cast<const int32_t *>(on_device(lnode));
+  S.lelem = reinterpret_cast<const int32_t *>(on_device(lelem));
+  S.lc = reinterpret_cast<const uint16_t *>(on_device(lc));
+  S.ls = reinterpret_cast<const uint16_t *>(on_device(ls));
+  S.send = reinterpret_cast<const uint16_t *>(on_device(send));
+  S.run = on_device(run);
+  S.own = own;
+  S.max_nodes = max_nodes;
+  S.max_elems = max_elems;
+  S.max_slots = max_slots;
+  S.nn = nn;
+  S.nel = nel;
+  S.nblocks_padded = (int32_t)((nb + 7) / 8 * 8);
+  S.nblocks = (int32_t)nb;
+  m->step_lds = lds;
+}
+
+// whether the next call's steps are single launches: what plan_small_steps
+// could not know
+bool small_steps(const akx_model *m) {
+  return m->step.nblocks > 0 && !m->timing && !m->mats[0]->ext() && !m->records_live();
+}
+
+template <int LAW> void launch_step_law(akx_model *m, const StepArgs &S) {
+  const dim3 grid((unsigned)S.nblocks_padded);
+  if (m->etype == AKX_TET4)
+    hipLaunchKernelGGL(k_tet4_step<LAW>, grid, dim3(256), m->step_lds, m->stream, S);
+  else
+    hipLaunchKernelGGL(k_hex8_step<LAW>, grid, dim3(STEP_HEX_EPB * 8), m->step_lds, m->stream,
+                       S);
+}
+
+void launch_small_step(akx_model *m, bool first, bool last) {
+  Material &mat = *m->mats[0];
+  const bool f32 = m->precision == AKX_PRECISION_FP32;
+  StepArgs S = m->step;
+  S.first = first;
+  S.last = last;
+  S.X = m->X.p;
+  S.u = m->u.p;
+  S.v = m->v.p;
+  S.a = m->a.p;
+  S.cu = m->cu.p;
+  S.cv = m->cv.p;
+  const bool new_u = first || !last; // the last step has no predictor to follow
+  S.u2 = new_u ? m->u2.p : nullptr;
+  S.v2 = first ? m->v2.p : m->v.p;
+  S.a2 = first ? m->a2.p : m->a.p;
+  S.cu2 = first ? m->cu2.p : m->cu.p;
+  S.cv2 = first ? m->cv2.p : m->cv.p;
+  S.mass = m->mass.p;
+  S.fext = m->has_fext ? m->fext.p : nullptr;
+  S.blocked = m->blocked.p;
+  S.fint = last ? m->fint.p : nullptr;
+  S.dt = m->dt;
+  S.lambda = mat.lambda;
+  S.mu = mat.mu;
+  S.lam_el = mat.per_element ? mat.lam_el.p : nullptr;
+  S.mu_el = mat.per_element ? mat.mu_el.p : nullptr;
+  S.lm_f = mat.per_element ? mat.lm_f.p : nullptr;
+  S.jw = m->jw.p;
+  require(S.lnode && S.lc && S.X && S.mass && S.blocked && S.u && m->u2.p && S.v2 && S.a2,
+          "small-model step launched without its lists or state");
+  require(!f32 || (S.run && S.cu && S.cv && m->cu2.p && m->cv2.p),
+          "small-model step launched without compensation terms");
+  require(!S.lam_el == !S.mu_el && (!f32 || !S.lam_el == !S.lm_f),
+          "per-element parameters incomplete");
+  require(m->etype != AKX_HEX8 || S.jw, "Hex8 step launched without its jacobian table");
+  if (f32)
+    HIPCHECK(akxf::launch_tet4_step(mat.law, S, m->step_lds, m->stream));
+  else if (mat.law == AKX_LAW_ELASTIC)
+    launch_step_law<LAW_ELASTIC>(m, S);
+  else if (mat.law == AKX_LAW_ELASTIC_FD)
+    launch_step_law<LAW_ELASTIC_FD>(m, S);
+  else
+    launch_step_law<LAW_NEOHOOKEAN>(m, S);
+  HIPCHECK(hipGetLastError());
+  if (new_u)
+    std::swap(m->u, m->u2);
+  if (first) {
+    std::swap(m->v, m->v2);
+    std::swap(m->a, m->a2);
+    std::swap(m->cu, m->cu2);
+    std::swap(m->cv, m->cv2);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Pipelined step (opt-in): the elements are cut in P consecutive parts and the
 // nodes in P groups, group q = the 256-node slices whose last element (in
 // assembly order) lies in part q.  Then
@@ -1907,9 +2256,14 @@ int akx_model_set_mesh(akx_model *m, int element_type, int64_t nb_nodes,
     for (int32_t c : m->conn_host)
       require(c >= 0 && c < nb_nodes, "connectivity refers to a missing node");
     m->X.alloc(3 * nb_nodes);
-    m->u.alloc(3 * nb_nodes);
-    m->v.alloc(3 * nb_nodes);
-    m->a.alloc(3 * nb_nodes);
+    const int64_t per = state_stride(nb_nodes);
+    const bool twice = nb_nodes <= STEP_NODES_MAX;
+    m->state.alloc((twice ? 6 : 3) * per);
+    double *part = m->state.p;
+    for (auto *f : {&m->u, &m->v, &m->a, &m->u2, &m->v2, &m->a2}) {
+      f->p = part < m->state.p + m->state.n ? part : nullptr;
+      part += per;
+    }
     m->fint.alloc(3 * nb_nodes);
     m->mass.alloc(nb_nodes);
     m->blocked.alloc(nb_nodes);
@@ -1918,9 +2272,7 @@ int akx_model_set_mesh(akx_model *m, int element_type, int64_t nb_nodes,
     HIPCHECK(hipMemcpy(m->conn.p, connectivity,
                        nb_elements * m->nnpe * sizeof(int32_t),
                        hipMemcpyHostToDevice));
-    zero_async(m, m->u.p, 3 * nb_nodes);
-    zero_async(m, m->v.p, 3 * nb_nodes);
-    zero_async(m, m->a.p, 3 * nb_nodes);
+    zero_async(m, m->state.p, (int64_t)m->state.n);
     zero_async(m, m->fint.p, 3 * nb_nodes);
     zero_async(m, m->mass.p, nb_nodes);
     HIPCHECK(hipMemsetAsync(m->blocked.p, 0, nb_nodes, m->stream));
@@ -2242,18 +2594,22 @@ int akx_model_init_full(akx_model *m) {
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipStreamSynchronize(m->stream));
     }
+    plan_small_steps(m);
     for (auto &mp : m->mats)
       alloc_internals(m, *mp);
     if (m->precision == AKX_PRECISION_FP32) {
       for (auto &mp : m->mats)
         if (mp->per_element && mp->n > 0)
           fill_lame_f32(m, *mp);
-      m->cu.alloc(3 * m->nn);
-      m->cv.alloc(3 * m->nn);
-      hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(3 * m->nn)), dim3(TPB), 0,
-                         m->stream, m->cu.p, 3 * m->nn, 0.f);
-      hipLaunchKernelGGL(k_fill_f32, dim3(grid_for(3 * m->nn)), dim3(TPB), 0,
-                         m->stream, m->cv.p, 3 * m->nn, 0.f);
+      const int64_t per = state_stride(m->nn);
+      m->comp.alloc((m->step.nblocks > 0 ? 4 : 2) * per);
+      float *part = m->comp.p;
+      for (auto *f : {&m->cu, &m->cv, &m->cu2, &m->cv2}) {
+        f->p = part < m->comp.p + m->comp.n ? part : nullptr;
+        part += per;
+      }
+      hipLaunchKernelGGL(k_fill_f32, dim3(grid_for((int64_t)m->comp.n)), dim3(TPB), 0,
+                         m->stream, m->comp.p, (int64_t)m->comp.n, 0.f);
       HIPCHECK(hipGetLastError());
     }
     HIPCHECK(hipStreamSynchronize(m->stream));
@@ -2323,6 +2679,11 @@ int akx_model_solve_steps(akx_model *m, int64_t nb_steps) {
       plan_pipeline(m);
     if (m->pipe_parts > 1 && m->pipe_ok && !m->timing) {
       solve_pipelined(m, nb_steps);
+      return;
+    }
+    if (small_steps(m)) {
+      for (int64_t s = 0; s < nb_steps; ++s)
+        launch_small_step(m, s == 0, s + 1 == nb_steps);
       return;
     }
     launch_predictor(m);

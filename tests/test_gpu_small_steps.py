@@ -1,0 +1,82 @@
+"""Small models step in one launch; with kernel timing on they keep the two
+passes (element pass, gather) that larger models run.  Both give the same
+values: FP64 bit for bit, the FP32 form up to the rounding of its element
+forces (the compiler contracts the two kernels' products on its own: a few
+units of 6e-8 of each force, 2e-5 of the assembled forces with their
+cancellation, and at most 1e-6 of u and v after these few steps)."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from akantu2_amd import SolidMechanicsModel
+from akantu2_amd import mesh as M
+
+pytestmark = pytest.mark.gpu
+
+TET, HEX = "_tetrahedron_4", "_hexahedron_8"
+# one cell; fewer nodes than a workgroup owns in all; a partly filled last
+# workgroup; the largest planned meshes (10,240 and 2,560 nodes) and ones just above
+CELLS = {TET: [(1, 1, 1), (3, 2, 2), (20, 4, 4), (39, 15, 15), (40, 15, 15)],
+         HEX: [(1, 1, 1), (4, 1, 2), (10, 10, 10), (19, 15, 7), (20, 15, 7)]}
+
+
+def shuffled(mesh, seed):
+    """The same mesh with its nodes and elements numbered at random."""
+    rng = np.random.default_rng(seed)
+    to = rng.permutation(mesh.nb_nodes)
+    nodes = np.empty_like(mesh.nodes)
+    nodes[to] = mesh.nodes
+    conn = to[mesh.conn][rng.permutation(mesh.nb_elements)]
+    return dataclasses.replace(mesh, nodes=nodes, conn=np.ascontiguousarray(conn, np.int32))
+
+
+def make(mesh, law, precision, per_element, timing):
+    rng = np.random.default_rng(5)
+    m = SolidMechanicsModel(mesh)
+    E_el = rng.uniform(0.6, 1.2, mesh.nb_elements) if per_element else None
+    m.addMaterial(law, E=1.2, nu=0.28, E_el=E_el)
+    m.setPrecision(precision)
+    m.initFull()
+    m.getBlockedDOFs()[:] = rng.random((mesh.nb_nodes, 3)) < 0.1
+    m.getDisplacement()[:] = 0.02 * rng.standard_normal((mesh.nb_nodes, 3))
+    m.getVelocity()[:] = 0.05 * rng.standard_normal((mesh.nb_nodes, 3))
+    m.getExternalForce()[:] = 1e-3 * rng.standard_normal((mesh.nb_nodes, 3))
+    m.setTimeStep(0.3 * m.getStableTimeStep())
+    m.enableKernelTiming(timing)
+    return m
+
+
+FORMS = [(TET, c, law, "fp64") for c in CELLS[TET] for law in ("elastic", "neohookean")]
+FORMS += [(TET, c, law, "fp32") for c in CELLS[TET] for law in ("elastic", "neohookean")]
+FORMS += [(HEX, c, law, "fp64") for c in CELLS[HEX] for law in ("elastic", "neohookean")]
+FORMS += [(TET, (5, 4, 4), "elastic_fd", "fp64"), (TET, (5, 4, 4), "elastic_fd", "fp32"),
+          (HEX, (5, 4, 4), "elastic_fd", "fp64")]
+
+
+@pytest.mark.parametrize("order", ["grid", "random"])
+@pytest.mark.parametrize("etype,cells,law,precision", FORMS)
+def test_one_launch_equals_two(etype, cells, law, precision, order):
+    mesh = M.box_mesh(etype, *cells, jitter=0.1, seed=2)
+    if order == "random":
+        mesh = shuffled(mesh, 7)
+    per_element = law != "neohookean"
+    one = make(mesh, law, precision, per_element, False)
+    two = make(mesh, law, precision, per_element, True)
+    for k, steps in enumerate((1, 2, 5, 1)):
+        for m in (one, two):
+            m.solveSteps(steps)
+            if k == 1:  # a changed input between the calls
+                m.getVelocity()[:] *= 0.5
+        if k == 2:  # the two forms continue each other's runs
+            one.enableKernelTiming(True)
+            two.enableKernelTiming(False)
+        for name, bound in (("Displacement", 1e-6), ("Velocity", 1e-6),
+                            ("Acceleration", 2e-5), ("InternalForce", 2e-5)):
+            a = np.array(getattr(one, "get" + name)())
+            b = np.array(getattr(two, "get" + name)())
+            assert np.isfinite(a).all()
+            if precision == "fp64":
+                assert np.array_equal(a, b), (name, k)
+            else:
+                assert np.linalg.norm(a - b) <= bound * np.linalg.norm(b), (name, k)
