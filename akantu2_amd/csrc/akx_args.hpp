@@ -79,15 +79,64 @@ struct ElemArgs {
 };
 
 // ---------------------------------------------------------------------------
-// One step of a small model in one launch (akx_step.hpp).  Workgroup b owns
-// the nodes b * own ..; its lists, padded to the longest of any workgroup,
-// hold every node of the elements around them (padded with -1) and those
-// elements (the padding repeats the first).  The corners of
-// one owned node take consecutive LDS slots in assembly order; all other
-// corners take the slot after the last, which nothing reads.
+// Where the Gauss-point state of one launch lives: previous (read) and
+// current (written) plastic history, [9][nq_all] column-major 3x3 and
+// [nq_all] for the hardening, stored in HT; and the optional grad u /
+// stress output (FP64, same indexing).
 // ---------------------------------------------------------------------------
+template <class HT> struct QpViewT {
+  const HT *p_grad, *p_sig, *p_eps, *p_iso;
+  HT *c_grad, *c_sig, *c_eps, *c_iso;
+  double *grad_u, *stress;
+  int64_t nq_all;
+  const HT *p_pe; // accumulated plastic energy, or null (not tracked)
+  HT *c_pe;
+  // eigen grad u [9][nq_all] and thermal stress [nq_all] (plastic: previous /
+  // current), read by the element passes instantiated with them
+  const double *eig = nullptr, *sth_now = nullptr, *sth_p = nullptr;
+  double *sth_c = nullptr;
+  bool keep = true; // the current history is written (by one lane per element)
+
+  // previous history of Gauss point iq: grad u, stress, plastic strain, hardening
+  template <class CT>
+  __device__ __forceinline__ void history(int64_t iq, CT (&pg)[3][3], CT (&ps)[3][3],
+                                          CT (&pe)[3][3], CT &iso) const {
+#pragma unroll
+    for (int jj = 0; jj < 3; ++jj)
+#pragma unroll
+      for (int ii = 0; ii < 3; ++ii) {
+        const int64_t o = (int64_t)(ii + 3 * jj) * nq_all + iq;
+        pg[ii][jj] = CT(p_grad[o]);
+        ps[ii][jj] = CT(p_sig[o]);
+        pe[ii][jj] = CT(p_eps[o]);
+      }
+    iso = CT(p_iso[iq]);
+  }
+  __device__ __forceinline__ HT energy(int64_t iq) const { return p_pe[iq]; }
+};
+using QpView = QpViewT<double>;
+
+__host__ __device__ inline QpView qp_view(const ElemArgs &A, int nqp) {
+  return QpView{A.p_grad, A.p_sig,  A.p_eps,  A.p_iso,  A.c_grad, A.c_sig,
+                A.c_eps,  A.c_iso,  A.grad_u, A.stress, A.n * nqp, A.p_pe,
+                A.c_pe,   A.eig,    A.sth_now, A.sth_p, A.sth_c};
+}
+
+// ---------------------------------------------------------------------------
+// One step of a small model in one launch (akx_step.hpp).  Workgroup b owns up
+// to `own` nodes; its lists, padded to the longest of any workgroup, hold these
+// (padded with -1), every node of the elements around them (padded with -1)
+// and those elements (the padding repeats the first).  The corners of one
+// owned node take consecutive LDS slots in assembly order; all other corners
+// take the slot after the last, which nothing reads.
+// ---------------------------------------------------------------------------
+constexpr int32_t STEP_GUEST = -2147483647 - 1; // the sign bit
+
 struct StepArgs {
-  const int32_t *lnode, *lelem; // [blocks][max_nodes], [blocks][max_elems]
+  // [blocks][max_nodes]; [blocks][max_elems], STEP_GUEST set where another
+  // workgroup writes the element's history
+  const int32_t *lnode, *lelem;
+  const int32_t *onode; // [blocks][own]
   const uint16_t *lc, *ls;      // [blocks][max_elems][nnpe] local node, slot
   const uint16_t *send;         // [blocks][own] end of each node's slots
   const uint8_t *run;           // [blocks][max_slots] last corner of a partial sum
@@ -106,37 +155,12 @@ struct StepArgs {
   const uint8_t *blocked;
   double *fint; // null while steps follow in the call
   double dt;
-  double lambda, mu;
-  const double *lam_el, *mu_el; // per element, or null
+  double lambda, mu, sigma_y, h;
+  const double *lam_el, *mu_el, *sy_el, *h_el; // per element, or null
+  QpView hist;                                 // plastic law
   const float2 *lm_f;           // FP32 form: the pair per element, or null
   const double2 *jw;            // Hex8: the jacobian table
 };
-
-// ---------------------------------------------------------------------------
-// Where the Gauss-point state of one launch lives: previous (read) and
-// current (written) plastic history, [9][nq_all] column-major 3x3 and
-// [nq_all] for the hardening, stored in HT; and the optional grad u /
-// stress output (FP64, same indexing).
-// ---------------------------------------------------------------------------
-template <class HT> struct QpViewT {
-  const HT *p_grad, *p_sig, *p_eps, *p_iso;
-  HT *c_grad, *c_sig, *c_eps, *c_iso;
-  double *grad_u, *stress;
-  int64_t nq_all;
-  const HT *p_pe; // accumulated plastic energy, or null (not tracked)
-  HT *c_pe;
-  // eigen grad u [9][nq_all] and thermal stress [nq_all] (plastic: previous /
-  // current), read by the element passes instantiated with them
-  const double *eig = nullptr, *sth_now = nullptr, *sth_p = nullptr;
-  double *sth_c = nullptr;
-};
-using QpView = QpViewT<double>;
-
-__host__ __device__ inline QpView qp_view(const ElemArgs &A, int nqp) {
-  return QpView{A.p_grad, A.p_sig,  A.p_eps,  A.p_iso,  A.c_grad, A.c_sig,
-                A.c_eps,  A.c_iso,  A.grad_u, A.stress, A.n * nqp, A.p_pe,
-                A.c_pe,   A.eig,    A.sth_now, A.sth_p, A.sth_c};
-}
 
 // ---------------------------------------------------------------------------
 // Where the element pass finds the coordinates X and displacement u of a

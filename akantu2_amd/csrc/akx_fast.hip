@@ -1060,7 +1060,7 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepAr
   const ushort4 ls = *reinterpret_cast<const ushort4 *>(S.ls + i * 4);
   float lambda = (float)S.lambda, mu = (float)S.mu;
   if (S.lm_f) {
-    const float2 lm = S.lm_f[S.lelem[i]];
+    const float2 lm = S.lm_f[S.lelem[i] & ~akx::STEP_GUEST];
     lambda = lm.x;
     mu = lm.y;
   }
@@ -1322,7 +1322,7 @@ hipError_t launch_elements(int etype, int law, bool fp32, const ElemArgs &A,
 }
 
 hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream) {
-  const dim3 grid((unsigned)S.nblocks_padded), block(256);
+  const dim3 grid((unsigned)S.nblocks_padded), block((unsigned)(S.max_elems + 63) / 64 * 64);
   switch (law) {
   case LAW_ELASTIC:
     hipLaunchKernelGGL(k_tet4_step_f32<LAW_ELASTIC>, grid, block, lds, stream, S);

@@ -367,8 +367,8 @@ __device__ __forceinline__ void ext_terms(const QpViewT<HT> &V, int64_t iq, CT (
 // sth: MaterialThermal's sigma_th (-0 with the default alpha = 0,
 // material_thermal.hh:91-95), added by the elastic laws; dsth = previous -
 // current sigma_th, added to the plastic trial stress.
-template <int LAW, class CT, class HT>
-__device__ __forceinline__ void strict_law(const QpViewT<HT> &V, int64_t iq, CT lambda,
+template <int LAW, class CT, class HT, class VT>
+__device__ __forceinline__ void strict_law(const VT &V, int64_t iq, CT lambda,
                                            CT mu, CT sy, CT hh, const CT (&g)[3][3],
                                            CT (&S)[3][3], CT sth = CT(-0.0),
                                            CT dsth = CT(0)) {
@@ -417,29 +417,23 @@ __device__ __forceinline__ void strict_law(const QpViewT<HT> &V, int64_t iq, CT 
         S[ii][jj] = CT(sc[ii + 3 * jj]);
 #endif
   } else {
-    CT pg[3][3], ps[3][3], pe[3][3], eps[3][3], iso;
+    CT pg[3][3], ps[3][3], pe[3][3], eps[3][3], piso, iso;
+    V.history(iq, pg, ps, pe, piso);
+    plastic_lih(lambda, mu, sy, hh, g, pg, ps, piso, pe, S, iso, eps, dsth);
+    if (V.keep) {
 #pragma unroll
-    for (int jj = 0; jj < 3; ++jj)
+      for (int jj = 0; jj < 3; ++jj)
 #pragma unroll
-      for (int ii = 0; ii < 3; ++ii) {
-        const int64_t o = (int64_t)(ii + 3 * jj) * V.nq_all + iq;
-        pg[ii][jj] = CT(V.p_grad[o]);
-        ps[ii][jj] = CT(V.p_sig[o]);
-        pe[ii][jj] = CT(V.p_eps[o]);
-      }
-    plastic_lih(lambda, mu, sy, hh, g, pg, ps, CT(V.p_iso[iq]), pe, S, iso, eps, dsth);
-#pragma unroll
-    for (int jj = 0; jj < 3; ++jj)
-#pragma unroll
-      for (int ii = 0; ii < 3; ++ii) {
-        const int64_t o = (int64_t)(ii + 3 * jj) * V.nq_all + iq;
-        V.c_grad[o] = HT(g[ii][jj]);
-        V.c_sig[o] = HT(S[ii][jj]);
-        V.c_eps[o] = HT(eps[ii][jj]);
-      }
-    V.c_iso[iq] = HT(iso);
-    if (V.c_pe)
-      V.c_pe[iq] = HT(plastic_energy_update(CT(V.p_pe[iq]), S, ps, eps, pe));
+        for (int ii = 0; ii < 3; ++ii) {
+          const int64_t o = (int64_t)(ii + 3 * jj) * V.nq_all + iq;
+          V.c_grad[o] = HT(g[ii][jj]);
+          V.c_sig[o] = HT(S[ii][jj]);
+          V.c_eps[o] = HT(eps[ii][jj]);
+        }
+      V.c_iso[iq] = HT(iso);
+      if (V.c_pe)
+        V.c_pe[iq] = HT(plastic_energy_update(CT(V.energy(iq)), S, ps, eps, pe));
+    }
   }
   if (V.grad_u) {
 #pragma unroll
@@ -460,10 +454,10 @@ __device__ __forceinline__ void strict_law(const QpViewT<HT> &V, int64_t iq, CT 
 // launch (one material) and the batched persistent launch.
 // ---------------------------------------------------------------------------
 template <int ET, int LAW, class CT, class FT, class HT, class NA, int W = 3, bool EXT = false,
-          bool SLOTS = false>
+          bool SLOTS = false, class VT = QpViewT<HT>>
 __device__ __forceinline__ void element_forces_one(
     const int32_t *conn_e, const NA &nodes_of,
-    CT lambda, CT mu, CT sy, CT hh, const QpViewT<HT> &V, int64_t iq0,
+    CT lambda, CT mu, CT sy, CT hh, const VT &V, int64_t iq0,
     const int32_t *pos_e, void *fe_out, double *slots = nullptr) {
   constexpr int NN = Elem<ET>::nnpe, NQ = Elem<ET>::nqp;
   int32_t nodes[NN];

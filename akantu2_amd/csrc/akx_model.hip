@@ -37,8 +37,40 @@ thread_local std::string g_last_error;
 // One step of a small FP64 model (akx_step.hpp).
 // ---------------------------------------------------------------------------
 
+// A view whose previous history of one Gauss point is in registers, read ahead
+// of the staging (step of 4,032 nodes 10.6 -> 10.3 us; the two-launch pass keeps
+// reading it inside the law: its 330,000-element pass went from 34.7 to 37.7)
+struct QpHeld : QpView {
+  double pg[3][3], ps[3][3], pe[3][3], iso, work;
+  __device__ __forceinline__ void read(int64_t iq) {
+    QpView::history(iq, pg, ps, pe, iso);
+    work = p_pe ? p_pe[iq] : 0.;
+  }
+  __device__ __forceinline__ double energy(int64_t) const { return work; }
+  __device__ __forceinline__ void history(int64_t, double (&g)[3][3], double (&s)[3][3],
+                                          double (&e)[3][3], double &k) const {
+#pragma unroll
+    for (int ii = 0; ii < 3; ++ii)
+#pragma unroll
+      for (int jj = 0; jj < 3; ++jj) {
+        g[ii][jj] = pg[ii][jj];
+        s[ii][jj] = ps[ii][jj];
+        e[ii][jj] = pe[ii][jj];
+      }
+    k = iso;
+  }
+};
+
+template <int LAW> struct QpAhead {
+  using type = QpView;
+};
+template <> struct QpAhead<LAW_PLASTIC> {
+  using type = QpHeld;
+};
+
 // Tet4: one lane per element of the workgroup's list
-template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step(StepArgs S) {
+template <int LAW>
+__global__ void __launch_bounds__(256) k_tet4_step(StepArgs S) {
   extern __shared__ double2 s_rec[]; // records, then slots
   const int64_t b = xcd_block(S.nblocks_padded);
   if (b >= S.nblocks) // padding block
@@ -49,11 +81,21 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step(StepArgs S
   const int64_t i = b * S.max_elems + (active ? t : S.max_elems - 1);
   const ushort4 lc = *reinterpret_cast<const ushort4 *>(S.lc + i * 4);
   const ushort4 ls = *reinterpret_cast<const ushort4 *>(S.ls + i * 4);
-  double lambda = S.lambda, mu = S.mu;
+  const int32_t le = S.lelem[i], e = le & ~STEP_GUEST;
+  double lambda = S.lambda, mu = S.mu, sy = S.sigma_y, hh = S.h;
   if (S.lam_el) {
-    const int32_t e = S.lelem[i];
     lambda = S.lam_el[e];
     mu = S.mu_el[e];
+  }
+  typename QpAhead<LAW>::type V{};
+  if constexpr (LAW == LAW_PLASTIC) {
+    static_cast<QpView &>(V) = S.hist;
+    V.keep = le >= 0;
+    V.read(e);
+    if (S.sy_el)
+      sy = S.sy_el[e];
+    if (S.h_el)
+      hh = S.h_el[e];
   }
   StepDof<false> dof;
   dof.load(S, b);
@@ -64,7 +106,7 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step(StepArgs S
     const int4 slots = make_int4(-1 - ls.x, -1 - ls.y, -1 - ls.z, -1 - ls.w);
     element_forces_one<ET_TET4, LAW, double, double, double, NodesLDS, 3, false, true>(
         reinterpret_cast<const int32_t *>(&nd),
-        NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, 0., 0., QpView{}, 0,
+        NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, sy, hh, V, e,
         reinterpret_cast<const int32_t *>(&slots), s_slot, s_slot);
   }
   __syncthreads();
@@ -97,7 +139,7 @@ template <int LAW> __global__ void __launch_bounds__(STEP_HEX_EPB * 8) k_hex8_st
   for (int base = 0; base < S.max_elems; base += STEP_HEX_EPB) {
     const bool active = base + el < S.max_elems;
     const int64_t i = b * S.max_elems + (active ? base + el : S.max_elems - 1);
-    const int32_t e = S.lelem[i];
+    const int32_t e = S.lelem[i] & ~STEP_GUEST;
     const int32_t nd = S.lc[i * 8 + q];
     double lambda = S.lambda, mu = S.mu;
     if (S.lam_el) {
@@ -119,6 +161,56 @@ template <int LAW> __global__ void __launch_bounds__(STEP_HEX_EPB * 8) k_hex8_st
         PutSlots{s_ls[el], s_slot}, pre);
   }
   dof.update<false>(S, s_slot, nullptr); // the group's last barrier is behind
+}
+
+// The lists of StepArgs, one workgroup per workgroup of the step, from what
+// group_nodes found: owner, slot0 and rank give a node's workgroup, its first
+// slot and a corner's place among its node's; ends the partial sums' ends in
+// the order of `first`.
+struct StepListArgs {
+  int32_t *lnode, *onode, *lelem;
+  uint16_t *lc, *ls, *send;
+  uint8_t *run; // FP32 form, else null
+  const int32_t *ooff, *onodes, *eoff, *elems, *noff, *nodes, *owner, *slot0, *first;
+  const uint16_t *lcs;
+  const uint8_t *rank, *ends;
+  const int32_t *conn;
+  int32_t nnpe;
+};
+
+__global__ void __launch_bounds__(256) k_step_lists(StepArgs S, StepListArgs L) {
+  const int64_t b = blockIdx.x;
+  const int e0 = L.eoff[b], ne = L.eoff[b + 1] - e0;
+  for (int k = threadIdx.x; k < S.max_elems; k += blockDim.x) {
+    // padding: the list's first element again (an empty list: element 0 of the
+    // mesh on the records of no node), to the slot nothing reads
+    const int src = e0 + (k < ne ? k : 0);
+    const int32_t e = ne > 0 ? L.elems[src] : 0;
+    const int32_t *c = L.conn + (int64_t)e * L.nnpe;
+    const int64_t at = b * S.max_elems + k;
+    // an element's history is written where its first node is owned
+    L.lelem[at] = k < ne && L.owner[c[0]] == b ? e : e | STEP_GUEST;
+    for (int a = 0; a < L.nnpe; ++a) {
+      L.lc[at * L.nnpe + a] = ne > 0 ? L.lcs[(int64_t)src * L.nnpe + a] : 0;
+      L.ls[at * L.nnpe + a] =
+          (uint16_t)(k < ne && L.owner[c[a]] == b
+                         ? L.slot0[c[a]] + L.rank[(int64_t)e * L.nnpe + a]
+                         : S.max_slots);
+    }
+  }
+  const int n0 = L.noff[b], nb_nodes = L.noff[b + 1] - n0;
+  for (int k = threadIdx.x; k < S.max_nodes; k += blockDim.x)
+    L.lnode[b * S.max_nodes + k] = k < nb_nodes ? L.nodes[n0 + k] : -1;
+  const int o0 = L.ooff[b], nb_own = L.ooff[b + 1] - o0;
+  for (int k = threadIdx.x; k < S.own; k += blockDim.x) {
+    const int32_t n = k < nb_own ? L.onodes[o0 + k] : -1;
+    L.onode[b * S.own + k] = n;
+    const int deg = n < 0 ? 0 : L.first[n + 1] - L.first[n];
+    L.send[b * S.own + k] = (uint16_t)(n < 0 ? 0 : L.slot0[n] + deg);
+    if (L.run)
+      for (int d = 0; d < deg; ++d)
+        L.run[b * S.max_slots + L.slot0[n] + d] = L.ends[L.first[n] + d];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1676,164 +1768,191 @@ void launch_predictor(akx_model *m) {
 
 // ---------------------------------------------------------------------------
 // One launch per step for small models (akx_step.hpp): one contiguous material
-// of a non-plastic built-in law over the whole mesh, FP64 or FP32 Tet4.
+// of a built-in law over the whole mesh; Tet4 in FP64 (with plasticity) and
+// FP32, Hex8 in FP64.
 //
-// A step of two launches takes 8 to 14 us however small the mesh; in one
-// launch it takes 5, what the host needs to queue it.  An element's arithmetic
-// is repeated in every workgroup that owns one of its nodes (on boxes 3.1
-// times for Tet4, 4.6 times for Hex8), so the gain ends where that fills the
-// chip.  us a step, two launches -> one (boxes):
-//   Tet4 FP64 elastic   525 nodes 12.0 -> 5.1, 4,032 12.5 -> 5.9, 10,416
-//                       13.6 -> 9.3, 26,691 16.8 -> 16.9
-//   Tet4 FP64 neo-H.    4,032 13.6 -> 7.5, 10,416 14.4 -> 12.7, 13,776
-//                       15.6 -> 14.8, 26,691 19.0 -> 25.1
-//   Tet4 FP32 elastic   1,152 7.9 -> 5.2, 10,416 8.4 -> 6.9, 13,776 9.0 ->
-//                       8.3, 26,691 9.5 -> 12.0
-//   Hex8 FP64 neo-H.    1,331 10.4 -> 7.8, 2,520 10.5 -> 10.0, 4,032 10.8 ->
-//                       12.5
-//   Hex8 FP64 elastic   1,536 9.1 -> 6.4, 2,520 9.2 -> 7.7, 4,032 9.3 -> 9.3
-// A Tet4 workgroup owns 8 nodes (a run along a row of a box has 150 elements,
-// one a lane), a Hex8 one 6 (28 elements of eight lanes; 8 nodes have 36 and
-// would take a second round).
+// A step of two launches takes 8 to 16 us however small the mesh; in one
+// launch it takes 5 (plastic 7.5), what the host needs to queue it.  An
+// element's arithmetic is repeated in every workgroup that owns one of its
+// nodes, so the gain ends where that fills the chip.
+//
+// A workgroup owns a run of 8 nodes (Tet4; along a row of a box they have 150
+// elements, one a lane) or 6 (Hex8; 28 elements of eight lanes).  In runs a
+// Tet4 is computed 3.1 times, a Hex8 4.6 times.  Groups of up to 16
+// neighbouring nodes (group_nodes) take that to 2.3 for Tet4, with a longer sum
+// per lane: they pay in FP64 where the runs need more than two workgroups per
+// CU.  (Hex8 in groups of 8: 4.1; no faster up to 2,560 nodes.)  The lists cost
+// initFull 0.1 ms at 1,000 nodes, 1.5 ms at 7,000.  us a step of boxes, two
+// launches / runs / groups:
+//   Tet4 FP64 elastic   525 nodes 12.0/5.1/-, 4,032 12.5/5.9/6.7, 10,416
+//                       13.6/9.3/8.1
+//   Tet4 FP64 neo-H.    4,032 13.6/7.5/8.2, 6,630 14.1/9.4/8.5, 10,416
+//                       14.4/12.7/10.5
+//   Tet4 FP64 plastic   525 14.8/7.4/-, 4,032 16/10.3/13.2, 6,975
+//                       16.2/16.2/13.9, 10,416 18.3/-/21.6
+//   Tet4 FP32 elastic   1,152 7.9/5.2/-, 4,032 8.1/5.7/6.7, 10,416 8.4/6.9/7.9,
+//                       26,691 9.5/12.0/12.1
+//   Hex8 FP64 neo-H.    1,331 10.4/7.8/-, 2,520 10.5/10.0/10.4, 4,032
+//                       10.8/12.5/10.8
+//   Hex8 FP64 elastic   1,536 9.1/6.4/-, 2,520 9.2/7.7/8.0, 4,032 9.3/9.3/8.3
 // ---------------------------------------------------------------------------
-constexpr int STEP_OWN_TET4 = 8, STEP_OWN_HEX8 = 6;
-constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_HEX8 = 2560;
-static_assert(STEP_NODES_TET4 <= STEP_NODES_MAX && STEP_NODES_HEX8 <= STEP_NODES_MAX,
+constexpr int STEP_RUN_TET4 = 8, STEP_GROUP_TET4 = 16, STEP_RUN_HEX8 = 6;
+constexpr int64_t STEP_RUNS_TET4 = 4096; // most nodes in runs (FP64)
+constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_PLASTIC = 8192, STEP_NODES_HEX8 = 2560;
+static_assert(STEP_NODES_TET4 <= STEP_NODES_MAX && STEP_NODES_PLASTIC <= STEP_NODES_MAX &&
+                  STEP_NODES_HEX8 <= STEP_NODES_MAX,
               "larger meshes have no second state arrays");
 constexpr size_t STEP_LDS = 48 * 1024;
 
+// Who owns which nodes: workgroup b the nodes onodes[ooff[b]] .., around them
+// the elements elems[eoff[b]] .. whose corners lcs index its nodes noff[b] ..,
+// all numbered as they are met.
+struct StepGroups {
+  std::vector<int32_t> ooff{0}, onodes, eoff{0}, elems, noff{0}, nodes;
+  std::vector<uint16_t> lcs;
+};
+
+// grow: a group starts at the lowest node left and takes, up to `own` nodes and
+// max_elems elements, the node of its elements that adds the fewest elements;
+// else the groups are runs of `own` nodes.  first, around: the elements around
+// every node.
+void group_nodes(const akx_model *m, const std::vector<int32_t> &first,
+                 const std::vector<int32_t> &around, int own, int max_elems, bool grow,
+                 StepGroups &G) {
+  const int nnpe = m->nnpe;
+  const int32_t *conn = m->conn_host.data();
+  const int32_t nn = (int32_t)m->nn;
+  constexpr int16_t TAKEN = INT16_MAX / 2; // no node has that many elements
+  std::vector<int32_t> elem_in(m->nel, -1), node_in(nn, -1), node_no(nn);
+  std::vector<int16_t> more(256); // elements that each of the group's nodes would add
+  std::vector<uint8_t> taken(nn, 0);
+  G.onodes.reserve(nn);
+  G.elems.reserve(4 * m->nel);
+  G.lcs.reserve(4 * m->nel * nnpe);
+  G.nodes.reserve(8 * nn);
+  for (int32_t start = 0, b = 0; start < nn; ++start) {
+    if (taken[start])
+      continue;
+    const int32_t n0 = G.noff[b];
+    int32_t met = 0; // nodes of the group's elements
+    for (int32_t n = start;;) {
+      taken[n] = 1;
+      G.onodes.push_back(n);
+      if (node_in[n] == b)
+        more[node_no[n]] = TAKEN;
+      for (int32_t d = first[n]; d < first[n + 1]; ++d) {
+        const int32_t e = around[d];
+        if (elem_in[e] == b)
+          continue;
+        elem_in[e] = b;
+        G.elems.push_back(e);
+        const size_t at = G.lcs.size();
+        G.lcs.resize(at + nnpe);
+        for (int a = 0; a < nnpe; ++a) {
+          const int32_t c = conn[(int64_t)e * nnpe + a];
+          if (node_in[c] != b) {
+            node_in[c] = b;
+            node_no[c] = met;
+            G.nodes.push_back(c);
+            if ((size_t)met == more.size())
+              more.resize(2 * met);
+            more[met++] = taken[c] ? TAKEN : (int16_t)(first[c + 1] - first[c]);
+          }
+          more[node_no[c]]--;
+          G.lcs[at + a] = (uint16_t)node_no[c];
+        }
+      }
+      if ((int)G.onodes.size() - G.ooff[b] == own)
+        break;
+      if (!grow) {
+        if (++n == nn)
+          break;
+        continue;
+      }
+      int16_t fewest = TAKEN / 2;
+      for (int32_t k = 0; k < met; ++k)
+        fewest = std::min(fewest, more[k]);
+      if (fewest == TAKEN / 2 || fewest > max_elems - ((int32_t)G.elems.size() - G.eoff[b]))
+        break;
+      n = G.nodes[n0 + (std::find(more.begin(), more.end(), fewest) - more.begin())];
+    }
+    G.ooff.push_back((int32_t)G.onodes.size());
+    G.eoff.push_back((int32_t)G.elems.size());
+    G.noff.push_back((int32_t)G.nodes.size());
+    ++b;
+  }
+}
+
 void plan_small_steps(akx_model *m) {
   const bool hex = m->etype == AKX_HEX8;
-  if (m->mats.size() != 1 || m->nn == 0 ||
-      m->nn > (hex ? STEP_NODES_HEX8 : STEP_NODES_TET4) ||
-      m->precision == AKX_PRECISION_FP64_FAST || (hex && m->precision == AKX_PRECISION_FP32))
+  if (m->mats.size() != 1 || m->nn == 0 || m->precision == AKX_PRECISION_FP64_FAST)
     return;
   const Material &mat = *m->mats[0];
-  const bool f32 = m->precision == AKX_PRECISION_FP32;
+  const bool f32 = m->precision == AKX_PRECISION_FP32, plastic = mat.law == AKX_LAW_PLASTIC_LIH;
+  if (m->nn > (hex ? STEP_NODES_HEX8 : plastic ? STEP_NODES_PLASTIC : STEP_NODES_TET4))
+    return;
   if (!mat.contiguous || mat.first != 0 || mat.n != m->nel || mat.n == 0 || mat.user() ||
-      mat.law == AKX_LAW_PLASTIC_LIH)
+      (hex && (f32 || plastic)) || (plastic && f32))
     return;
   if (!f32 && m->ppa && m->assembly == AKX_ASSEMBLY_BLOCK_PARTIALS)
     return; // sums runs in FP64 without rounding them as the FP32 form does
-  const int nnpe = m->nnpe, own = hex ? STEP_OWN_HEX8 : STEP_OWN_TET4;
+  const int nnpe = m->nnpe;
   const int32_t *conn = m->conn_host.data();
-  const int64_t nn = m->nn, nel = m->nel, nb = (nn + own - 1) / own;
+  const int64_t nn = m->nn, nel = m->nel;
   // elements around every node, in ascending order
   std::vector<int32_t> first(nn + 1, 0), around(nel * nnpe);
   for (int64_t i = 0; i < nel * nnpe; ++i)
     first[conn[i] + 1]++;
   for (int64_t n = 0; n < nn; ++n)
     first[n + 1] += first[n];
+  std::vector<uint8_t> rank(nel * nnpe); // of a corner among its node's
   {
-    std::vector<int32_t> at(first.begin(), first.end() - 1);
+    std::vector<uint8_t> at(nn, 0);
     for (int32_t e = 0; e < (int32_t)nel; ++e)
-      for (int a = 0; a < nnpe; ++a)
-        around[at[conn[(int64_t)e * nnpe + a]]++] = e;
-  }
-  // every workgroup's elements and their nodes, numbered as they are met
-  std::vector<int32_t> elems, nodes, eoff(nb + 1, 0), noff(nb + 1, 0);
-  std::vector<uint16_t> lcs;
-  std::vector<int32_t> elem_in(nel, -1), node_in(nn, -1), node_no(nn);
-  elems.reserve(4 * nel);
-  lcs.reserve(4 * nel * nnpe);
-  nodes.reserve(8 * nn);
-  int32_t max_elems = 1, max_nodes = 1, max_slots = 1;
-  for (int32_t b = 0; b < (int32_t)nb; ++b) {
-    const int64_t n0 = (int64_t)b * own, n1 = std::min<int64_t>(nn, n0 + own);
-    for (int32_t d = first[n0]; d < first[n1]; ++d) {
-      const int32_t e = around[d];
-      if (elem_in[e] == b)
-        continue;
-      elem_in[e] = b;
-      elems.push_back(e);
       for (int a = 0; a < nnpe; ++a) {
         const int32_t n = conn[(int64_t)e * nnpe + a];
-        if (node_in[n] != b) {
-          node_in[n] = b;
-          node_no[n] = (int32_t)nodes.size() - noff[b];
-          nodes.push_back(n);
-        }
-        lcs.push_back((uint16_t)node_no[n]);
+        rank[(int64_t)e * nnpe + a] = at[n];
+        around[first[n] + at[n]++] = e;
       }
+  }
+  // who owns which nodes
+  const int lanes = hex ? STEP_HEX_EPB : 256; // elements at a time
+  const bool grouped = !hex && !f32 && nn > STEP_RUNS_TET4;
+  const int own = hex ? STEP_RUN_HEX8 : grouped ? STEP_GROUP_TET4 : STEP_RUN_TET4;
+  StepGroups G;
+  group_nodes(m, first, around, own, lanes, grouped, G);
+  const auto &[ooff, onodes, eoff, elems, noff, nodes, lcs] = G;
+  const int64_t nb = (int64_t)ooff.size() - 1;
+  std::vector<int32_t> owner(nn), slot0(nn);
+  int32_t max_elems = 1, max_nodes = 1, max_slots = 1;
+  for (int64_t b = 0; b < nb; ++b) {
+    int32_t slots = 0;
+    for (int32_t k = ooff[b]; k < ooff[b + 1]; ++k) {
+      owner[onodes[k]] = (int32_t)b;
+      slot0[onodes[k]] = slots;
+      slots += first[onodes[k] + 1] - first[onodes[k]];
     }
-    eoff[b + 1] = (int32_t)elems.size();
-    noff[b + 1] = (int32_t)nodes.size();
     max_elems = std::max(max_elems, eoff[b + 1] - eoff[b]);
     max_nodes = std::max(max_nodes, noff[b + 1] - noff[b]);
-    max_slots = std::max(max_slots, first[n1] - first[n0]);
+    max_slots = std::max(max_slots, slots);
   }
   const size_t lds = (size_t)max_nodes * 48 +
                      (size_t)(max_slots + 1) * 3 * (f32 ? sizeof(float) : sizeof(double)) +
                      (f32 ? max_slots : 0);
   // one lane per Tet4; at most two rounds of Hex8 (a numbering without
   // locality makes long lists)
-  if (max_elems > (hex ? 2 * STEP_HEX_EPB : 256) || lds > STEP_LDS)
+  if (max_elems > (hex ? 2 : 1) * lanes || lds > STEP_LDS)
     return;
-  // one buffer: lnode, lelem, lc, ls, send, run
-  const size_t n32 = nb * (max_nodes + max_elems), n16 = nb * (2 * max_elems * nnpe + own),
-               n8 = f32 ? nb * max_slots : 0;
-  std::vector<unsigned char> lists(((4 * n32 + 7) / 8 * 8) + 2 * n16 + n8);
-  int32_t *lnode = reinterpret_cast<int32_t *>(lists.data()), *lelem = lnode + nb * max_nodes;
-  uint16_t *lc = reinterpret_cast<uint16_t *>(lists.data() + (4 * n32 + 7) / 8 * 8),
-           *ls = lc + nb * max_elems * nnpe, *send = ls + nb * max_elems * nnpe;
-  uint8_t *run = reinterpret_cast<uint8_t *>(send + nb * own);
-  std::fill(lnode, lelem, -1);
-  std::fill(ls, send, (uint16_t)max_slots);
-  std::fill(run, run + n8, 1);
-  std::vector<int32_t> elem_no(nel);
-  for (int64_t b = 0; b < nb; ++b) {
-    const int64_t n0 = b * own, n1 = std::min<int64_t>(nn, n0 + own);
-    std::copy(nodes.begin() + noff[b], nodes.begin() + noff[b + 1], lnode + b * max_nodes);
-    const int32_t ne = eoff[b + 1] - eoff[b];
-    int32_t *lelem_b = lelem + b * max_elems;
-    uint16_t *lc_b = lc + b * max_elems * nnpe, *ls_b = ls + b * max_elems * nnpe;
-    std::copy(elems.begin() + eoff[b], elems.begin() + eoff[b + 1], lelem_b);
-    std::copy(lcs.begin() + (int64_t)eoff[b] * nnpe, lcs.begin() + (int64_t)eoff[b + 1] * nnpe,
-              lc_b);
-    // padding: the list's first element again (an empty list: element 0 of the
-    // mesh on the records of no node), to the slot nothing reads
-    for (int32_t k = ne; k < max_elems && ne > 0; ++k) {
-      lelem_b[k] = lelem_b[0];
-      std::copy(lc_b, lc_b + nnpe, lc_b + k * nnpe);
-    }
-    for (int32_t k = 0; k < ne; ++k)
-      elem_no[lelem_b[k]] = k;
-    for (int64_t n = n0; n < n1; ++n) {
-      for (int32_t d = first[n]; d < first[n + 1]; ++d) {
-        const int32_t *c = conn + (int64_t)around[d] * nnpe;
-        int a = 0;
-        while (c[a] != n)
-          ++a;
-        // a corner that repeats its node takes the next one's place
-        while (d > first[n] && around[d] == around[d - 1] &&
-               ls_b[elem_no[around[d]] * nnpe + a] != max_slots) {
-          ++a;
-          while (c[a] != n)
-            ++a;
-        }
-        ls_b[elem_no[around[d]] * nnpe + a] = (uint16_t)(d - first[n0]);
-      }
-      send[b * own + n - n0] = (uint16_t)(first[n + 1] - first[n0]);
-    }
-    // FP32 partial sums end where the element pass's block of 256 elements
-    // does (every corner is one without block assembly)
-    if (f32 && m->bpa)
-      for (int64_t n = n0; n < std::min<int64_t>(nn, n0 + own); ++n)
-        for (int32_t k = first[n]; k + 1 < first[n + 1]; ++k)
-          run[b * max_slots + k - first[n0]] = around[k] / 256 != around[k + 1] / 256;
-  }
-  m->step_lists.alloc(lists.size());
-  HIPCHECK(hipMemcpy(m->step_lists.p, lists.data(), lists.size(), hipMemcpyHostToDevice));
-  StepArgs &S = m->step;
-  const auto on_device = [&](const void *host) {
-    return m->step_lists.p + (static_cast<const unsigned char *>(host) - lists.data());
-  };
-  S.lnode = reinterpret_cast<const int32_t *>(on_device(lnode));
-  S.lelem = reinterpret_cast<const int32_t *>(on_device(lelem));
-  S.lc = reinterpret_cast<const uint16_t *>(on_device(lc));
-  S.ls = reinterpret_cast<const uint16_t *>(on_device(ls));
-  S.send = reinterpret_cast<const uint16_t *>(on_device(send));
-  S.run = on_device(run);
+  // FP32 partial sums end where the element pass's block of 256 elements does
+  // (every corner is one without block assembly)
+  std::vector<uint8_t> ends(f32 ? around.size() : 0, 1);
+  if (f32 && m->bpa)
+    for (int64_t n = 0; n < nn; ++n)
+      for (int32_t d = first[n]; d + 1 < first[n + 1]; ++d)
+        ends[d] = around[d] / 256 != around[d + 1] / 256;
+  // the lists, by k_step_lists from what was found here; the upload sits in the
+  // force table, which nothing uses yet
+  StepArgs S{};
   S.own = own;
   S.max_nodes = max_nodes;
   S.max_elems = max_elems;
@@ -1842,6 +1961,65 @@ void plan_small_steps(akx_model *m) {
   S.nel = nel;
   S.nblocks_padded = (int32_t)((nb + 7) / 8 * 8);
   S.nblocks = (int32_t)nb;
+  struct Part {
+    const void *host;
+    size_t bytes, at;
+  };
+  size_t total = 0;
+  auto part = [&](const auto &v) {
+    const Part p{v.data(), v.size() * sizeof(v[0]), total};
+    total += (p.bytes + 15) / 16 * 16;
+    return p;
+  };
+  const Part parts[] = {part(ooff), part(onodes), part(eoff),  part(elems), part(noff), part(nodes),
+                        part(lcs),  part(owner),  part(slot0), part(rank),  part(first), part(ends)};
+  std::unique_ptr<unsigned char[]> up(new unsigned char[total]);
+  for (const Part &p : parts)
+    std::memcpy(up.get() + p.at, p.host, p.bytes);
+  DevBuf<unsigned char> more;
+  unsigned char *dev = m->fe.p;
+  if (m->fe.n < total) {
+    more.alloc(total);
+    dev = more.p;
+  }
+  HIPCHECK(hipMemcpy(dev, up.get(), total, hipMemcpyHostToDevice));
+  const size_t n32 = nb * (max_nodes + own + max_elems), n16 = nb * (2 * max_elems * nnpe + own);
+  m->step_lists.alloc((4 * n32 + 7) / 8 * 8 + 2 * n16 + (f32 ? nb * max_slots : 0));
+  StepListArgs L{};
+  L.lnode = reinterpret_cast<int32_t *>(m->step_lists.p);
+  L.onode = L.lnode + nb * max_nodes;
+  L.lelem = L.onode + nb * own;
+  L.lc = reinterpret_cast<uint16_t *>(m->step_lists.p + (4 * n32 + 7) / 8 * 8);
+  L.ls = L.lc + nb * max_elems * nnpe;
+  L.send = L.ls + nb * max_elems * nnpe;
+  L.run = f32 ? reinterpret_cast<uint8_t *>(L.send + nb * own) : nullptr;
+  auto at = [&](int k) { return reinterpret_cast<const int32_t *>(dev + parts[k].at); };
+  L.ooff = at(0);
+  L.onodes = at(1);
+  L.eoff = at(2);
+  L.elems = at(3);
+  L.noff = at(4);
+  L.nodes = at(5);
+  L.lcs = reinterpret_cast<const uint16_t *>(at(6));
+  L.owner = at(7);
+  L.slot0 = at(8);
+  L.rank = reinterpret_cast<const uint8_t *>(at(9));
+  L.first = at(10);
+  L.ends = reinterpret_cast<const uint8_t *>(at(11));
+  L.conn = m->conn.p;
+  L.nnpe = nnpe;
+  hipLaunchKernelGGL(k_step_lists, dim3((unsigned)nb), dim3(TPB), 0, m->stream, S, L);
+  HIPCHECK(hipGetLastError());
+  if (more.p)
+    HIPCHECK(hipStreamSynchronize(m->stream));
+  S.lnode = L.lnode;
+  S.onode = L.onode;
+  S.lelem = L.lelem;
+  S.lc = L.lc;
+  S.ls = L.ls;
+  S.send = L.send;
+  S.run = L.run;
+  m->step = S;
   m->step_lds = lds;
 }
 
@@ -1854,7 +2032,8 @@ bool small_steps(const akx_model *m) {
 template <int LAW> void launch_step_law(akx_model *m, const StepArgs &S) {
   const dim3 grid((unsigned)S.nblocks_padded);
   if (m->etype == AKX_TET4)
-    hipLaunchKernelGGL(k_tet4_step<LAW>, grid, dim3(256), m->step_lds, m->stream, S);
+    hipLaunchKernelGGL(k_tet4_step<LAW>, grid, dim3((unsigned)(S.max_elems + 63) / 64 * 64),
+                       m->step_lds, m->stream, S);
   else
     hipLaunchKernelGGL(k_hex8_step<LAW>, grid, dim3(STEP_HEX_EPB * 8), m->step_lds, m->stream,
                        S);
@@ -1888,8 +2067,17 @@ void launch_small_step(akx_model *m, bool first, bool last) {
   S.lam_el = mat.per_element ? mat.lam_el.p : nullptr;
   S.mu_el = mat.per_element ? mat.mu_el.p : nullptr;
   S.lm_f = mat.per_element ? mat.lm_f.p : nullptr;
+  if (mat.law == AKX_LAW_PLASTIC_LIH) {
+    const ElemArgs A = elem_args(m, mat, false);
+    check_elem_args(A, mat.law);
+    S.sigma_y = A.sigma_y;
+    S.h = A.h;
+    S.sy_el = A.sy_el;
+    S.h_el = A.h_el;
+    S.hist = qp_view(A, 1);
+  }
   S.jw = m->jw.p;
-  require(S.lnode && S.lc && S.X && S.mass && S.blocked && S.u && m->u2.p && S.v2 && S.a2,
+  require(S.lnode && S.onode && S.lc && S.X && S.mass && S.blocked && S.u && m->u2.p && S.v2 && S.a2,
           "small-model step launched without its lists or state");
   require(!f32 || (S.run && S.cu && S.cv && m->cu2.p && m->cv2.p),
           "small-model step launched without compensation terms");
@@ -1902,9 +2090,15 @@ void launch_small_step(akx_model *m, bool first, bool last) {
     launch_step_law<LAW_ELASTIC>(m, S);
   else if (mat.law == AKX_LAW_ELASTIC_FD)
     launch_step_law<LAW_ELASTIC_FD>(m, S);
-  else
+  else if (mat.law == AKX_LAW_NEOHOOKEAN)
     launch_step_law<LAW_NEOHOOKEAN>(m, S);
+  else {
+    require(m->etype == AKX_TET4, "plastic Hex8 steps take two launches");
+    hipLaunchKernelGGL(k_tet4_step<LAW_PLASTIC>, dim3((unsigned)S.nblocks_padded),
+                       dim3((unsigned)(S.max_elems + 63) / 64 * 64), m->step_lds, m->stream, S);
+  }
   HIPCHECK(hipGetLastError());
+  flip_plastic_state(m);
   if (new_u)
     std::swap(m->u, m->u2);
   if (first) {

@@ -3,7 +3,7 @@
 //
 // A mesh of up to a few thousand nodes leaves most of the chip idle, so a step
 // costs its launches and the round trips of each kernel, not its work.  Here
-// every workgroup owns a few consecutive nodes, computes all elements around
+// every workgroup owns a few nodes, computes all elements around
 // them (each element in up to nnpe workgroups) and updates its nodes from
 // forces that never leave its LDS: no force table, no second launch, and the
 // predictor of a call's first step is applied to the nodes as they are read.
@@ -79,8 +79,8 @@ template <bool COMP> struct StepDof {
     const int t = threadIdx.x;
     c = t / S.own;
     const int k = t - c * S.own;
-    n = b * S.own + k;
-    on = c < 3 && n < S.nn;
+    n = c < 3 ? S.onode[b * S.own + k] : -1;
+    on = n >= 0;
     if (!on)
       return;
     o = c * S.nn + n;

@@ -16,9 +16,13 @@ pytestmark = pytest.mark.gpu
 
 TET, HEX = "_tetrahedron_4", "_hexahedron_8"
 # one cell; fewer nodes than a workgroup owns in all; a partly filled last
-# workgroup; the largest planned meshes (10,240 and 2,560 nodes) and ones just above
-CELLS = {TET: [(1, 1, 1), (3, 2, 2), (20, 4, 4), (39, 15, 15), (40, 15, 15)],
+# workgroup; Tet4: the largest mesh whose workgroups own runs of nodes (4,096)
+# and one above, with groups in FP64; the largest planned (Tet4 10,240 nodes,
+# plastic 8,192; Hex8 2,560) and ones above
+CELLS = {TET: [(1, 1, 1), (3, 2, 2), (20, 4, 4), (15, 15, 15), (16, 15, 15)],
          HEX: [(1, 1, 1), (4, 1, 2), (10, 10, 10), (19, 15, 7), (20, 15, 7)]}
+LARGEST = [(39, 15, 15), (40, 15, 15)]
+LARGEST_PLASTIC = [(31, 15, 15), (32, 15, 15)]
 
 
 def shuffled(mesh, seed):
@@ -35,7 +39,7 @@ def make(mesh, law, precision, per_element, timing):
     rng = np.random.default_rng(5)
     m = SolidMechanicsModel(mesh)
     E_el = rng.uniform(0.6, 1.2, mesh.nb_elements) if per_element else None
-    m.addMaterial(law, E=1.2, nu=0.28, E_el=E_el)
+    m.addMaterial(law, E=1.2, nu=0.28, E_el=E_el, sigma_y=2e-3, h=0.1)
     m.setPrecision(precision)
     m.initFull()
     m.getBlockedDOFs()[:] = rng.random((mesh.nb_nodes, 3)) < 0.1
@@ -47,9 +51,12 @@ def make(mesh, law, precision, per_element, timing):
     return m
 
 
-FORMS = [(TET, c, law, "fp64") for c in CELLS[TET] for law in ("elastic", "neohookean")]
-FORMS += [(TET, c, law, "fp32") for c in CELLS[TET] for law in ("elastic", "neohookean")]
-FORMS += [(HEX, c, law, "fp64") for c in CELLS[HEX] for law in ("elastic", "neohookean")]
+PLASTIC = "plastic_linear_isotropic_hardening"
+LAWS = ("elastic", "neohookean")
+FORMS = [(TET, c, law, p) for c in CELLS[TET] + LARGEST for law in LAWS
+         for p in ("fp64", "fp32")]
+FORMS += [(TET, c, PLASTIC, "fp64") for c in CELLS[TET] + LARGEST_PLASTIC]
+FORMS += [(HEX, c, law, "fp64") for c in CELLS[HEX] for law in LAWS]
 FORMS += [(TET, (5, 4, 4), "elastic_fd", "fp64"), (TET, (5, 4, 4), "elastic_fd", "fp32"),
           (HEX, (5, 4, 4), "elastic_fd", "fp64")]
 
@@ -80,3 +87,5 @@ def test_one_launch_equals_two(etype, cells, law, precision, order):
                 assert np.array_equal(a, b), (name, k)
             else:
                 assert np.linalg.norm(a - b) <= bound * np.linalg.norm(b), (name, k)
+    if law == PLASTIC:
+        assert one.getEnergy("plastic") == two.getEnergy("plastic") > 0
