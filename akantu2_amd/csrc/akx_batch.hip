@@ -25,6 +25,7 @@
 // single-model plain path, so an instance gives the same bits alone and in
 // the mix.
 #include "../../include/akantu_mi355x.h"
+#include "akx_admit.hpp"
 #include "akx_batch.hpp"
 #include "akx_download.hpp"
 #include "akx_fast.hpp"
@@ -444,18 +445,9 @@ __global__ void k_batch_gather_mass(int64_t node0, int64_t n, const int64_t *ell
   mass[nd] = m;
 }
 
-// host [n][3] <-> arena [3][ncap] (stride ncap, offset 0) or the node
-// records [ncap][6] (stride 1 per component, 6 per node, offset 0 for X and
-// 3 for u), at node0
-__global__ void k_batch_put3(const double *aos, double *dst, int64_t comp_stride,
-                             int64_t node_stride, int64_t node0, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 3 * n)
-    return;
-  const int64_t r = i / 3, c = i % 3;
-  dst[c * comp_stride + (node0 + r) * node_stride] = aos[i];
-}
-
+// arena [3][ncap] (stride ncap, offset 0) or the node records [ncap][6] (stride
+// 1 per component, 6 per node, offset 0 for X and 3 for u), at node0, to host
+// [n][3]
 __global__ void k_batch_get3(const double *src, double *aos, int64_t comp_stride,
                              int64_t node_stride, int64_t node0, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -569,7 +561,7 @@ struct akx_batch {
   DevBuf<double> hex_tab;
   DevBuf<unsigned long long> dt_bits;
   DevBuf<long long> bad;
-  DevBuf<double> staging;
+  DevBuf<unsigned char> admit; // upload and scratch of an instance that joins
   Downloader download;
   FreeList fl_nodes, fl_tet, fl_hex, fl_ell;
   // FP32 block-partial assembly: per element its local corners and LDS
@@ -1156,65 +1148,91 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
     I.nel = nb_elements;
     for (int64_t i = 0; i < nb_elements * nnpe; ++i)
       require(conn[i] >= 0 && conn[i] < nb_nodes, "connectivity refers to a missing node");
-    // block-partial assembly (FP32): per block of bs elements its distinct
-    // nodes in ascending order (the staging loads coalesce), each corner's index among them and its
-    // LDS slot (the corners of one distinct node take consecutive slots in
-    // ascending element order); the table then holds one entry per (block,
+    // block-partial assembly (FP32): the table holds one entry per (block,
     // distinct node) and a node's degree is the number of blocks touching it
     const bool bpa = b->bpa;
     const int64_t bs = element_type == AKX_TET4 ? BPA_TET4 : BPA_HEX8; // per block
     const int64_t nblk = bpa ? (nb_elements + bs - 1) / bs : 0;
-    std::vector<int32_t> bl_nodes; // instance-local node ids, blocks in order
-    std::vector<uint16_t> lc, ls, send;
-    if (bpa) {
-      lc.resize(nb_elements * nnpe);
-      ls.resize(nb_elements * nnpe);
-      bl_nodes.reserve(nb_elements);
-      I.blk_cnt.resize(nblk);
-      std::vector<int32_t> local(nb_nodes, 0);
-      DistinctNodes distinct(nb_nodes);
-      std::vector<uint16_t> cnt(bs * nnpe + 1);
-      for (int64_t bk = 0; bk < nblk; ++bk) {
-        const int64_t e0 = bk * bs, e1 = std::min<int64_t>(nb_elements, e0 + bs);
-        const int64_t start = (int64_t)bl_nodes.size();
-        distinct.append(conn + e0 * nnpe, (e1 - e0) * nnpe, bl_nodes);
-        const int32_t nloc = (int32_t)((int64_t)bl_nodes.size() - start);
-        for (int32_t k = 0; k < nloc; ++k)
-          local[bl_nodes[start + k]] = k;
-        for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i)
-          lc[i] = (uint16_t)local[conn[i]];
-        I.blk_cnt[bk] = nloc;
-        std::fill(cnt.begin(), cnt.begin() + nloc + 1, 0);
-        for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i)
-          cnt[lc[i] + 1]++;
-        for (int32_t k = 0; k < nloc; ++k) { // slot ends (inclusive prefix)
-          cnt[k + 1] = (uint16_t)(cnt[k + 1] + cnt[k]);
-          send.push_back(cnt[k + 1]);
-        }
-        for (int64_t i = e0 * nnpe; i < e1 * nnpe; ++i) // cnt[k]: start of k's slots
-          ls[i] = cnt[lc[i]]++;
-      }
-      I.nbent = (int64_t)bl_nodes.size();
+    const int64_t corners = nb_elements * nnpe, nsl = I.nn_pad / 256;
+    const int pad = element_type == AKX_TET4 ? 1024 : 512; // corners per block, 2^k
+    static_assert(BPA_TET4 * 4 <= 1024 && BPA_HEX8 * 8 <= 512, "a block's corners fit its sort");
+    const int64_t items = bpa ? nblk * pad : corners;
+    if (I.nn_pad > b->ncap) // no scratch for what never fits
+      throw Error(AKX_ERR_MEMORY, "node arena full");
+    if (I.nel > (element_type == AKX_TET4 ? b->tcap : b->hexcap))
+      throw Error(AKX_ERR_MEMORY, "element arena full");
+    // upload and scratch
+    size_t total = 0;
+    auto take = [&](int64_t n, size_t size) {
+      const size_t at = total;
+      total += ((size_t)n * size + 255) / 256 * 256;
+      return at;
+    };
+    const size_t o_nodes = take(3 * nb_nodes, 8), o_vel = take(velocity ? 3 * nb_nodes : 0, 8),
+                 o_blocked = take(blocked_dofs ? 3 * nb_nodes : 0, 1), o_conn = take(corners, 4),
+                 o_width = take(nsl + nblk, 4), o_deg = take(I.nn_pad, 4),
+                 o_item = take(bpa ? items : 0, 4), o_arrive = take(items, 1),
+                 o_send = take(bpa ? items : 0, 2), o_lc = take(bpa ? corners : 0, 2),
+                 o_ls = take(bpa ? corners : 0, 2), o_off = take(nsl + nblk, 8),
+                 o_blk = take(nblk, sizeof(BBlk));
+    if (b->admit.n < total) {
+      sync(b); // the buffer may still be read
+      b->admit.reserve(total);
     }
-    // node degrees and the sliced-ELL layout of this instance
-    std::vector<int32_t> deg(I.nn_pad, 0);
-    if (bpa) {
-      for (int32_t nd : bl_nodes)
-        deg[nd]++;
-    } else {
-      for (int64_t i = 0; i < nb_elements * nnpe; ++i)
-        deg[conn[i]]++;
-    }
-    const int64_t nsl = I.nn_pad / 256;
-    std::vector<int64_t> off(nsl + 1, 0);
+    unsigned char *scratch = b->admit.p;
+    auto up = [&](size_t at, const void *src, size_t bytes) {
+      HIPCHECK(hipMemcpyAsync(scratch + at, src, bytes, hipMemcpyHostToDevice, b->stream));
+      return scratch + at;
+    };
+    AdmitArgs T{};
+    T.nodes = (const double *)up(o_nodes, nodes, 24 * nb_nodes);
+    if (velocity)
+      T.velocity = (const double *)up(o_vel, velocity, 24 * nb_nodes);
+    if (blocked_dofs)
+      T.blocked3 = up(o_blocked, blocked_dofs, 3 * nb_nodes);
+    T.conn = (const int32_t *)up(o_conn, conn, corners * 4);
+    T.nn = nb_nodes;
+    T.nn_pad = I.nn_pad;
+    T.nel = nb_elements;
+    T.nnpe = nnpe;
+    T.bs = (int32_t)bs;
+    T.pad = pad;
+    T.nblk = nblk;
+    T.width = (int32_t *)(scratch + o_width);
+    T.count = T.width + nsl;
+    T.deg = (int32_t *)(scratch + o_deg);
+    T.item = (int32_t *)(scratch + o_item);
+    T.arrive = scratch + o_arrive;
+    T.send = (uint16_t *)(scratch + o_send);
+    T.lc = (uint16_t *)(scratch + o_lc);
+    T.ls = (uint16_t *)(scratch + o_ls);
+    T.blk = (BBlk *)(scratch + o_blk);
+    hipLaunchKernelGGL((k_batch_fill<int32_t>), dim3(gridn(I.nn_pad)), dim3(TPB), 0, b->stream,
+                       T.deg, I.nn_pad, 0);
+    if (!bpa)
+      hipLaunchKernelGGL(k_admit_corners, dim3(gridn(corners)), dim3(256), 0, b->stream, T);
+    else if (element_type == AKX_TET4)
+      hipLaunchKernelGGL(k_admit_blocks<1024>, dim3((unsigned)nblk), dim3(256), 0, b->stream, T);
+    else
+      hipLaunchKernelGGL(k_admit_blocks<512>, dim3((unsigned)nblk), dim3(256), 0, b->stream, T);
+    hipLaunchKernelGGL(k_admit_widths, dim3((unsigned)nsl), dim3(256), 0, b->stream, T);
+    HIPCHECK(hipGetLastError());
+    // the sliced-ELL layout of this instance
+    std::vector<int32_t> found(nsl + nblk);
+    HIPCHECK(hipMemcpyAsync(found.data(), T.width, found.size() * 4, hipMemcpyDeviceToHost,
+                            b->stream));
+    sync(b);
+    std::vector<int64_t> off(nsl + nblk); // of the slices, then of the blocks
     for (int64_t s = 0; s < nsl; ++s) {
-      int w = 0;
-      for (int64_t k = 0; k < 256; ++k)
-        w = std::max(w, deg[s * 256 + k]);
-      require(w <= 255, "a node belongs to more than 255 elements");
-      off[s + 1] = off[s] + (int64_t)w * 256;
+      require(found[s] <= 255, "a node belongs to more than 255 elements");
+      off[s] = I.nell;
+      I.nell += (int64_t)found[s] * 256;
     }
-    I.nell = off[nsl];
+    I.blk_cnt.assign(found.begin() + nsl, found.end());
+    for (int64_t k = 0; k < nblk; ++k) {
+      off[nsl + k] = I.nbent;
+      I.nbent += I.blk_cnt[k];
+    }
     // ranges in the arenas
     if (b->inst.size() >= (size_t)MAX_INSTANCES) {
       bool slot = false;
@@ -1248,121 +1266,63 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       }
     }
     try {
-      // arena connectivity, table entries, slice offsets, degrees, blocked bits
-      std::vector<int32_t> gconn(nb_elements * nnpe), gpos(bpa ? 0 : nb_elements * nnpe);
-      std::vector<int32_t> fill(I.nn_pad, 0);
-      for (int64_t e = 0; e < nb_elements; ++e)
-        for (int a = 0; a < nnpe; ++a) {
-          const int32_t nd = conn[e * nnpe + a];
-          gconn[e * nnpe + a] = (int32_t)(I.node0 + nd);
-          if (bpa)
-            continue;
-          const int32_t d = fill[nd]++; // elements in ascending order
-          gpos[e * nnpe + a] =
-              (int32_t)(I.ell0 + off[nd >> 8] + (int64_t)d * 256 + (nd & 255));
-        }
-      // block partials: entry of (block, distinct node) in ascending block order
-      std::vector<int32_t> gbnode(I.nbent), gbpos(I.nbent);
-      for (int64_t k = 0; k < I.nbent; ++k) {
-        const int32_t nd = bl_nodes[k];
-        gbnode[k] = (int32_t)(I.node0 + nd);
-        const int32_t d = fill[nd]++;
-        gbpos[k] = (int32_t)(I.ell0 + off[nd >> 8] + (int64_t)d * 256 + (nd & 255));
-      }
-      std::vector<int64_t> goff(nsl);
-      for (int64_t s = 0; s < nsl; ++s)
-        goff[s] = I.ell0 + off[s];
-      std::vector<uint8_t> deg8(I.nn_pad), bits(I.nn_pad, 7);
-      for (int64_t k = 0; k < I.nn_pad; ++k)
-        deg8[k] = (uint8_t)deg[k];
-      for (int64_t k = 0; k < nb_nodes; ++k)
-        bits[k] = blocked_dofs ? (uint8_t)((blocked_dofs[3 * k] ? 1 : 0) |
-                                           (blocked_dofs[3 * k + 1] ? 2 : 0) |
-                                           (blocked_dofs[3 * k + 2] ? 4 : 0))
-                               : 0;
-      sync(b);
+      // arena connectivity, table entries, slice offsets, degrees, blocked
+      // bits, nodal state.  The rows' scratch is the instance's own (not yet
+      // used) force-table range
       int32_t *dconn = element_type == AKX_TET4 ? b->conn_t.p : b->conn_h.p;
       int32_t *dpos = element_type == AKX_TET4 ? b->pos_t.p : b->pos_h.p;
-      HIPCHECK(hipMemcpy(dconn + I.elem0 * nnpe, gconn.data(), gconn.size() * 4,
-                         hipMemcpyHostToDevice));
-      if (!bpa)
-        HIPCHECK(hipMemcpy(dpos + I.elem0 * nnpe, gpos.data(), gpos.size() * 4,
-                           hipMemcpyHostToDevice));
-      if (bpa) {
-        uint16_t *dlc = element_type == AKX_TET4 ? b->lc_t.p : b->lc_h.p;
-        uint16_t *dls = element_type == AKX_TET4 ? b->ls_t.p : b->ls_h.p;
-        HIPCHECK(hipMemcpy(dlc + I.elem0 * nnpe, lc.data(), lc.size() * 2,
-                           hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(dls + I.elem0 * nnpe, ls.data(), ls.size() * 2,
-                           hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(b->bnode.p + I.bent0, gbnode.data(), gbnode.size() * 4,
-                           hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(b->bpos.p + I.bent0, gbpos.data(), gbpos.size() * 4,
-                           hipMemcpyHostToDevice));
-        HIPCHECK(hipMemcpy(b->bsend.p + I.bent0, send.data(), send.size() * 2,
-                           hipMemcpyHostToDevice));
-      }
-      HIPCHECK(hipMemcpy(b->ell_off.p + I.node0 / 256, goff.data(), nsl * 8,
-                         hipMemcpyHostToDevice));
-      HIPCHECK(hipMemcpy(b->deg.p + I.node0, deg8.data(), I.nn_pad, hipMemcpyHostToDevice));
-      HIPCHECK(hipMemcpy(b->blocked.p + I.node0, bits.data(), I.nn_pad,
-                         hipMemcpyHostToDevice));
-      // nodal state: X and v from the host, u = a = f_int = 0 (the records
-      // of the padding nodes are zeroed too)
-      hipLaunchKernelGGL((k_batch_fill<double>), dim3(gridn(6 * I.nn_pad)), dim3(TPB), 0,
-                         b->stream, b->xu.p + 6 * I.node0, 6 * I.nn_pad, 0.);
-      b->staging.reserve(3 * nb_nodes);
-      HIPCHECK(hipStreamSynchronize(b->stream));
-      HIPCHECK(hipMemcpy(b->staging.p, nodes, 3 * nb_nodes * sizeof(double),
-                         hipMemcpyHostToDevice));
-      hipLaunchKernelGGL(k_batch_put3, dim3(gridn(3 * nb_nodes)), dim3(TPB), 0, b->stream,
-                         (const double *)b->staging.p, b->xu.p, (int64_t)1, (int64_t)6,
-                         I.node0, nb_nodes);
+      T.off = (const int64_t *)up(o_off, off.data(), off.size() * 8);
+      T.boff = T.off + nsl;
+      T.row = reinterpret_cast<int32_t *>(b->fe.p + I.ell0 * FE_W * b->fe_size());
+      T.node0 = I.node0;
+      T.elem0 = I.elem0;
+      T.ell0 = I.ell0;
+      T.bent0 = I.bent0;
+      T.ncap = b->ncap;
+      T.a_conn = dconn;
+      T.a_pos = dpos;
+      T.a_bnode = b->bnode.p;
+      T.a_bpos = b->bpos.p;
+      T.a_bsend = b->bsend.p;
+      T.a_lc = element_type == AKX_TET4 ? b->lc_t.p : b->lc_h.p;
+      T.a_ls = element_type == AKX_TET4 ? b->ls_t.p : b->ls_h.p;
+      T.a_ell_off = b->ell_off.p;
+      T.a_deg = b->deg.p;
+      T.a_blocked = b->blocked.p;
+      T.a_xu = b->xu.p;
+      T.a_x = b->bx.p;
+      T.a_u = b->bu.p;
+      T.a_v = b->v.p;
+      T.a_a = b->a.p;
+      T.a_fint = b->fint.p;
+      T.a_cu = b->cu.p;
+      T.a_cv = b->cv.p;
+      T.first_bad = b->bad.p;
+      T.min_bits = b->dt_bits.p;
+      require(T.a_conn && (bpa ? T.a_lc && T.a_ls && T.a_bnode && T.a_bpos && T.a_bsend
+                               : T.a_pos != nullptr) &&
+                  T.a_xu && !T.a_x == !T.a_u && !T.a_cu == !T.a_cv,
+              "instance admitted without its arenas");
+      const dim3 item_grid(bpa ? (unsigned)nblk : gridn(corners));
+      hipLaunchKernelGGL(k_admit_rows, item_grid, dim3(256), 0, b->stream, T);
+      hipLaunchKernelGGL(k_admit_ranks, item_grid, dim3(256), 0, b->stream, T);
+      hipLaunchKernelGGL(k_admit_elements, dim3(gridn(corners)), dim3(256), 0, b->stream, T);
+      hipLaunchKernelGGL(k_admit_nodes, dim3((unsigned)nsl), dim3(256), 0, b->stream, T);
       HIPCHECK(hipGetLastError());
-      if (!I.urec) { // X and u = 0 in the [3][ncap] arrays
-        for (int c = 0; c < 3; ++c)
-          hipLaunchKernelGGL((k_batch_fill<double>), dim3(gridn(I.nn_pad)), dim3(TPB), 0,
-                             b->stream, b->bx.p + c * b->ncap + I.node0, I.nn_pad, 0.);
-        hipLaunchKernelGGL(k_batch_put3, dim3(gridn(3 * nb_nodes)), dim3(TPB), 0, b->stream,
-                           (const double *)b->staging.p, b->bx.p, b->ncap, (int64_t)1,
-                           I.node0, nb_nodes);
-        HIPCHECK(hipGetLastError());
-      }
-      for (auto *f : {&b->v, &b->a, &b->fint, &b->bu})
-        for (int c = 0; c < 3 && f->p; ++c)
-          hipLaunchKernelGGL((k_batch_fill<double>), dim3(gridn(I.nn_pad)), dim3(TPB), 0,
-                             b->stream, f->p + c * b->ncap + I.node0, I.nn_pad, 0.);
-      if (b->fp32())
-        for (auto *f : {&b->cu, &b->cv})
-          for (int c = 0; c < 3; ++c)
-            hipLaunchKernelGGL((k_batch_fill<float>), dim3(gridn(I.nn_pad)), dim3(TPB), 0,
-                               b->stream, f->p + c * b->ncap + I.node0, I.nn_pad, 0.f);
-      HIPCHECK(hipGetLastError());
-      sync(b);
-      if (velocity) {
-        HIPCHECK(hipMemcpy(b->staging.p, velocity, 3 * nb_nodes * sizeof(double),
-                           hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(k_batch_put3, dim3(gridn(3 * nb_nodes)), dim3(TPB), 0,
-                           b->stream, (const double *)b->staging.p, b->v.p, b->ncap,
-                           (int64_t)1, I.node0, nb_nodes);
-        HIPCHECK(hipGetLastError());
-      }
       if (law == AKX_LAW_PLASTIC_LIH) {
-        const int64_t stride = b->hist_stride();
-        const int64_t q0 = (element_type == AKX_TET4 ? 0 : b->tcap) + I.elem0 * nqp;
-        const int64_t nq = I.nel * nqp;
+        AdmitHist H{};
+        int comps = 0;
         for (int s = 0; s < 2; ++s)
-          for (int k = 0; k < 4; ++k)
-            for (int c = 0; c < b->hist_comps(k); ++c) {
-              if (b->fp32())
-                hipLaunchKernelGGL((k_batch_fill<float>), dim3(gridn(nq)), dim3(TPB), 0,
-                                   b->stream, (float *)b->hist[s][k].p + c * stride + q0,
-                                   nq, 0.f);
-              else
-                hipLaunchKernelGGL((k_batch_fill<double>), dim3(gridn(nq)), dim3(TPB), 0,
-                                   b->stream, (double *)b->hist[s][k].p + c * stride + q0,
-                                   nq, 0.);
-            }
+          for (int k = 0; k < 4; ++k) {
+            H.p[4 * s + k] = b->hist[s][k].p;
+            comps += H.comps[4 * s + k] = b->hist_comps(k);
+          }
+        H.stride = b->hist_stride();
+        H.q0 = (element_type == AKX_TET4 ? 0 : b->tcap) + I.elem0 * nqp;
+        H.n = I.nel * nqp;
+        H.bytes = (int32_t)b->hist_size();
+        hipLaunchKernelGGL(k_admit_history, dim3(gridn(H.n), (unsigned)comps), dim3(256), 0,
+                           b->stream, H);
         HIPCHECK(hipGetLastError());
       }
       // jacobians, lumped mass, stable time step; the mass contributions go
@@ -1382,31 +1342,18 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       // entry's force; ell0 is a multiple of 256, so the address is aligned
       A.me = reinterpret_cast<double *>(b->fe.p + I.ell0 * FE_W * b->fe_size());
       A.ell0 = I.ell0;
-      const long long big = INT64_MAX;
-      const unsigned long long dmax = 0x7FEFFFFFFFFFFFFFull;
-      HIPCHECK(hipMemcpy(b->bad.p, &big, 8, hipMemcpyHostToDevice));
-      HIPCHECK(hipMemcpy(b->dt_bits.p, &dmax, 8, hipMemcpyHostToDevice));
       A.first_bad = b->bad.p;
       A.min_bits = b->dt_bits.p;
-      DevBuf<BBlk> iblk; // this instance's blocks, for the mass kernel
       if (bpa) {
-        std::vector<BBlk> hb(nblk);
-        int64_t o = I.bent0;
-        for (int64_t k = 0; k < nblk; ++k) {
-          hb[k] = BBlk{o, I.blk_cnt[k], 0};
-          o += I.blk_cnt[k];
-        }
-        iblk.alloc(nblk);
-        HIPCHECK(hipMemcpy(iblk.p, hb.data(), hb.size() * sizeof(BBlk), hipMemcpyHostToDevice));
         if (element_type == AKX_TET4) {
           hipLaunchKernelGGL(k_batch_mass_bpa<ET_TET4>, dim3((unsigned)nblk), dim3(256), 0,
-                             b->stream, A, (const BBlk *)iblk.p, (const uint16_t *)b->ls_t.p,
+                             b->stream, A, (const BBlk *)T.blk, (const uint16_t *)b->ls_t.p,
                              (const uint16_t *)b->bsend.p, (const int32_t *)b->bpos.p);
           hipLaunchKernelGGL(k_batch_dt<ET_TET4>, dim3(gridn(I.nel)), dim3(TPB), 0,
                              b->stream, A);
         } else {
           hipLaunchKernelGGL(k_batch_mass_bpa<ET_HEX8>, dim3((unsigned)nblk), dim3(256), 0,
-                             b->stream, A, (const BBlk *)iblk.p, (const uint16_t *)b->ls_h.p,
+                             b->stream, A, (const BBlk *)T.blk, (const uint16_t *)b->ls_h.p,
                              (const uint16_t *)b->bsend.p, (const int32_t *)b->bpos.p);
           hipLaunchKernelGGL(k_batch_dt<ET_HEX8>, dim3(gridn(I.nel)), dim3(TPB), 0,
                              b->stream, A);

@@ -32,6 +32,12 @@ extern thread_local std::string g_last_error;
                   std::string(#x) + ": " + hipGetErrorString(err_));           \
   } while (0)
 
+// (a literal's string is built only when it is thrown: checks of every entry of
+// an array spent 10 ns each on it)
+inline void require(bool c, const char *msg) {
+  if (!c)
+    throw Error(AKX_ERR_INVALID, msg);
+}
 inline void require(bool c, const std::string &msg) {
   if (!c)
     throw Error(AKX_ERR_INVALID, msg);
