@@ -1,7 +1,7 @@
 // akx_batch.hip -- many independent meshes advanced together on one GPU: the
-// batching form (one persistent launch per substep over all instances,
-// captured in a hipGraph, launch shape chosen by a project-written
-// autotuner) and the substrate of the serving form (instances admitted and
+// batching form (one launch per substep over all instances, replayed from a
+// hipGraph once the instances have stayed the same for a while, launch shape
+// chosen by rule or by a project-written autotuner) and the substrate of the serving form (instances admitted and
 // retired between chunks of steps while the others stay resident).
 //
 // Memory: arenas sized at creation.
@@ -588,6 +588,7 @@ struct akx_batch {
   bool launch_chosen = false; // set by set_launch or the autotuner
   bool use_graph = true;
   hipGraphExec_t graph = nullptr;
+  int64_t plain_steps = 0; // launched one by one since the lists changed
   // timing
   bool timing = false;
   double t_ms[2] = {0, 0};
@@ -620,6 +621,7 @@ unsigned gridn(int64_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 void sync(akx_batch *b) { HIPCHECK(hipStreamSynchronize(b->stream)); }
 
 void drop_graph(akx_batch *b) {
+  b->plain_steps = 0;
   if (b->graph) {
     (void)hipGraphExecDestroy(b->graph);
     b->graph = nullptr;
@@ -891,16 +893,26 @@ template <class F> void timed(akx_batch *b, int cls, F &&f) {
   (void)hipEventDestroy(e1);
 }
 
-// Two steps (step parities 0 and 1, each element pass + gather with the next
-// predictor fused) captured once; the graph holds kernels only.
+// GRAPH_STEPS steps (step parities 0 and 1 in turn, each element pass + gather
+// with the next predictor fused) captured once; the graph holds kernels only.
+//
+// A replay starts 8 us after the one before has ended, however many kernels
+// it holds: graphs of two steps were slower than plain launches (a launch takes
+// the host 4.8 us, two per step with one group).  us a step, plain launches /
+// graphs of 2 / graphs of 16 steps: 10,000 plastic Tet4 (FP32) 9.1 / 10.7 / 8.2,
+// 1.1 M 34.2 / 36.4 / 34.3, four groups of 5,000 Tet4 or 1,000 Hex8 23.1 / 22.5
+// / 20.0.  Capturing takes 0.45 ms with one group, 1.5 ms with four: what 500
+// steps gain, so the lists have to last that long first.
+constexpr int GRAPH_STEPS = 16;
+constexpr int64_t GRAPH_AFTER = 512;
 void ensure_graph(akx_batch *b) {
   if (b->graph)
     return;
   hipGraph_t g = nullptr;
   HIPCHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   try {
-    for (int p = 0; p < 2; ++p) {
-      element_pass(b, p);
+    for (int k = 0; k < GRAPH_STEPS; ++k) {
+      element_pass(b, k & 1);
       gather_pass(b, true);
     }
   } catch (...) {
@@ -932,13 +944,13 @@ void do_steps(akx_batch *b, int64_t n) {
     return;
   predictor_pass(b);
   int64_t k = 0;
-  if (b->use_graph && !b->timing && n > 2) {
+  if (b->use_graph && !b->timing && n > GRAPH_STEPS &&
+      (b->graph || b->plain_steps >= GRAPH_AFTER)) {
     ensure_graph(b);
-    const int64_t pairs = (n - 1) / 2;
-    for (int64_t p = 0; p < pairs; ++p)
+    for (; k + GRAPH_STEPS < n; k += GRAPH_STEPS)
       HIPCHECK(hipGraphLaunch(b->graph, b->stream));
-    k = 2 * pairs;
   }
+  b->plain_steps += n - k;
   for (; k < n; ++k) {
     timed(b, 0, [&] { element_pass(b, (int)(k & 1)); });
     timed(b, 1, [&] { gather_pass(b, k + 1 < n); });
