@@ -28,6 +28,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace akxf {
 
 using akx::BatchElemArgs;
@@ -42,6 +44,7 @@ using akx::QpViewT;
 using akx::batch_compact_view;
 using akx::FE_W;
 using akx::qp_view;
+using akx::slot_pos;
 
 constexpr int LAW_ELASTIC = 0, LAW_ELASTIC_FD = 1, LAW_NEOHOOKEAN = 2,
               LAW_PLASTIC = 3;
@@ -748,14 +751,17 @@ __device__ __forceinline__ void hex8_plastic_block(int n, const uint16_t *lconn,
   }
 }
 
-// the slots s0 .. s1 - 1 of one (block, node) in order, FP64, rounded once
+// the slots s0 .. s1 - 1 of one (block, node) in order, FP64, rounded once.
+// SPREAD: they lie at slot_pos (Tet4)
+template <bool SPREAD>
 __device__ __forceinline__ void sum_slots(const float *s_f, int s0, int s1, float *fe,
                                           int64_t entry) {
   double fx = 0., fy = 0., fz = 0.;
   for (int sl = s0; sl < s1; ++sl) {
-    fx += (double)s_f[3 * sl];
-    fy += (double)s_f[3 * sl + 1];
-    fz += (double)s_f[3 * sl + 2];
+    const float *f = s_f + 3 * (SPREAD ? slot_pos(sl) : sl);
+    fx += (double)f[0];
+    fy += (double)f[1];
+    fz += (double)f[2];
   }
   akx::put_entry<3>(fe, entry, float(fx), float(fy), float(fz));
 }
@@ -827,7 +833,7 @@ __global__ void __launch_bounds__(256) k_hex8_bpa(ElemArgs A) {
     if (d < 0)
       continue;
     const int s0 = first ? s0_first : soff[k], s1 = first ? s1_first : soff[k + 1];
-    sum_slots(s_f, s0, s1, fe, (int64_t)d);
+    sum_slots<false>(s_f, s0, s1, fe, (int64_t)d);
   }
 }
 
@@ -862,13 +868,12 @@ __global__ void __launch_bounds__(256) k_hex8_fast(ElemArgs A) {
 // math, a third memory round trip per element).  Faster for the one-element-
 // per-thread FP32 pass; slower inside the persistent batch loop, and in FP64
 // it costs the pass a wave per SIMD.
-// Q = w detJ P J^-1 of one Tet4 element (its corner forces are the columns
-// of Q and minus their sum).  BARRIER: a scheduling barrier after the node
-// loads, so that a load issued before the call stays ahead of the math.
-template <int LAW, class CT, class VT, class NA, bool BARRIER>
-__device__ __forceinline__ void tet4_Q(const int4 nd, const NA &nodes_of, CT lambda, CT mu,
-                                       CT sy, CT hh, const VT &V, int64_t iq,
-                                       CT (&Q)[3][3]) {
+// J = dX/dxi and H = du/dxi of one Tet4 element, differences of its corners.
+// BARRIER: a scheduling barrier after the node loads, so that a load issued
+// before the call stays ahead of the math.
+template <class CT, class NA, bool BARRIER>
+__device__ __forceinline__ void tet4_JH(const int4 nd, const NA &nodes_of, CT (&J)[3][3],
+                                        CT (&H)[3][3]) {
   const int32_t nodes[4] = {nd.x, nd.y, nd.z, nd.w};
   double X[4][3], U[4][3];
 #pragma unroll
@@ -878,7 +883,6 @@ __device__ __forceinline__ void tet4_Q(const int4 nd, const NA &nodes_of, CT lam
     __builtin_amdgcn_sched_barrier(0);
   // natural directions: xi -> node 3, eta -> node 1, zeta -> node 2
   const int nm[3] = {3, 1, 2};
-  CT J[3][3], H[3][3];
 #pragma unroll
   for (int m = 0; m < 3; ++m)
 #pragma unroll
@@ -886,6 +890,14 @@ __device__ __forceinline__ void tet4_Q(const int4 nd, const NA &nodes_of, CT lam
       J[m][c] = CT(X[nm[m]][c] - X[0][c]);
       H[c][m] = CT(U[nm[m]][c] - U[0][c]);
     }
+}
+
+// Q = w detJ P J^-1 of one Tet4 element (its corner forces are the columns
+// of Q and minus their sum)
+template <int LAW, class CT, class VT>
+__device__ __forceinline__ void tet4_Q(const CT (&J)[3][3], const CT (&H)[3][3], CT lambda,
+                                       CT mu, CT sy, CT hh, const VT &V, int64_t iq,
+                                       CT (&Q)[3][3]) {
   CT Ji[3][3];
   const CT detJ = inv_det(J, Ji);
   const CT wJ = detJ * CT(1. / 6.);
@@ -921,8 +933,9 @@ __device__ __forceinline__ void tet4_one(const int4 nd, const NA &nodes_of,
   int4 pv;
   if constexpr (EARLY_POS)
     pv = *reinterpret_cast<const int4 *>(pos_e);
-  CT Q[3][3];
-  tet4_Q<LAW, CT, VT, NA, EARLY_POS>(nd, nodes_of, lambda, mu, sy, hh, V, iq, Q);
+  CT J[3][3], H[3][3], Q[3][3];
+  tet4_JH<CT, NA, EARLY_POS>(nd, nodes_of, J, H);
+  tet4_Q<LAW, CT, VT>(J, H, lambda, mu, sy, hh, V, iq, Q);
   if constexpr (!EARLY_POS)
     pv = *reinterpret_cast<const int4 *>(pos_e);
   akx::put_entry<W>(fe, (int64_t)pv.x, FT(-(Q[0][0] + Q[0][1] + Q[0][2])),
@@ -988,9 +1001,16 @@ __global__ void __launch_bounds__(256) k_tet4_lds(ElemArgs A) {
 // writes the partial.  The gather then adds a node's partials in ascending
 // block order.  The table traffic falls from four entries per element to
 // one per (block, node) pair: about 0.7 per element on the box meshes.
+//
+// Bound by a mix: VALU busy 44 % of the time, LDS 50 %, the rest the wait for
+// the element's streams, then the node list, then the nodes.  The slots lie
+// spread over the banks (slot_pos) and take the place of the records, whose
+// differences are in registers by then: 8 instead of 7 workgroups per CU.  1.9 M
+// elements 27.8 (dense slots, behind the records) -> 26.5 (spread) -> 25.6 us,
+// 4.4 M 52.5 -> 49.7 -> 48.
 template <int LAW>
 __global__ void __launch_bounds__(256) k_tet4_bpa(ElemArgs A) {
-  extern __shared__ double2 s_xu[]; // [bl_maxu][3] records, then [1024][3] floats
+  extern __shared__ double2 s_xu[]; // [bl_maxu][3] records, later the corner slots
   const int64_t blk = xcd_block(A.nblocks_padded);
   if (blk * 256 >= A.n) // padding block: no elements, no node list
     return;
@@ -1016,19 +1036,21 @@ __global__ void __launch_bounds__(256) k_tet4_bpa(ElemArgs A) {
   }
   akx::stage_block_records(A, blk, s_xu);
   __syncthreads();
-  float *s_f = reinterpret_cast<float *>(s_xu + 3 * A.bl_maxu);
+  float J[3][3], H[3][3];
+  tet4_JH<float, akx::NodesLDS, false>(
+      make_int4(lc.x, lc.y, lc.z, lc.w),
+      akx::NodesLDS{reinterpret_cast<const double *>(s_xu)}, J, H);
+  __syncthreads(); // the records are dead: the LDS now takes the slots
+  float *s_f = reinterpret_cast<float *>(s_xu);
   if (active) {
     float Q[3][3];
-    tet4_Q<LAW, float, QpViewT<double>, akx::NodesLDS, false>(
-        make_int4(lc.x, lc.y, lc.z, lc.w),
-        akx::NodesLDS{reinterpret_cast<const double *>(s_xu)}, lambda, mu, sy, hh,
-        qp_view(A, 1), i, Q);
+    tet4_Q<LAW, float>(J, H, lambda, mu, sy, hh, qp_view(A, 1), i, Q);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
-      s_f[3 * ls.x + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
-      s_f[3 * ls.y + c] = Q[c][1];
-      s_f[3 * ls.z + c] = Q[c][2];
-      s_f[3 * ls.w + c] = Q[c][0];
+      s_f[3 * slot_pos(ls.x) + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
+      s_f[3 * slot_pos(ls.y) + c] = Q[c][1];
+      s_f[3 * slot_pos(ls.z) + c] = Q[c][2];
+      s_f[3 * slot_pos(ls.w) + c] = Q[c][0];
     }
   }
   __syncthreads();
@@ -1039,7 +1061,7 @@ __global__ void __launch_bounds__(256) k_tet4_bpa(ElemArgs A) {
     if (d < 0)
       continue;
     const int s0 = first ? s0_first : soff[k], s1 = first ? s1_first : soff[k + 1];
-    sum_slots(s_f, s0, s1, fe, (int64_t)d);
+    sum_slots<true>(s_f, s0, s1, fe, (int64_t)d);
   }
 }
 
@@ -1071,11 +1093,11 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepAr
   step_stage<true>(S, b, s_rec);
   __syncthreads();
   if (active) {
-    float Q[3][3];
-    tet4_Q<LAW, float, QpViewT<double>, akx::NodesLDS, false>(
+    float J[3][3], H[3][3], Q[3][3];
+    tet4_JH<float, akx::NodesLDS, false>(
         make_int4(lc.x, lc.y, lc.z, lc.w),
-        akx::NodesLDS{reinterpret_cast<const double *>(s_rec)}, lambda, mu, 0.f, 0.f,
-        QpViewT<double>{}, 0, Q);
+        akx::NodesLDS{reinterpret_cast<const double *>(s_rec)}, J, H);
+    tet4_Q<LAW, float>(J, H, lambda, mu, 0.f, 0.f, QpViewT<double>{}, 0, Q);
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       s_slot[3 * ls.x + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
@@ -1140,53 +1162,56 @@ __device__ __forceinline__ void stage_tile_records(const BatchElemArgs &A, const
 // node).  The gather adds a node's partials in ascending block order.
 template <int LAW>
 __global__ void __launch_bounds__(256) k_batch_tet4_bpa(BatchElemArgs A) {
-  extern __shared__ double2 s_xu[]; // [bmaxu][3] records, then [1024][3] floats
-  float *s_f = reinterpret_cast<float *>(s_xu + 3 * A.bmaxu);
+  extern __shared__ double2 s_xu[]; // [bmaxu][3] records, later the corner slots
   float *fe = reinterpret_cast<float *>(A.fe);
-  {
-    const int64_t tt = blockIdx.x;
-    if (tt >= A.ntiles)
-      return;
-    const BTile T = A.tiles[tt];
-    const BBlk B = A.blks[tt];
-    const BInst P = A.inst[T.inst];
-    const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
-    // this lane's first distinct node of the summing phase, read ahead so
-    // that its loads overlap the staging instead of following the barriers
-    const int t = threadIdx.x;
-    int s0_first = 0, s1_first = 0, pos_first = 0;
-    if (t < B.count) {
-      s0_first = t > 0 ? (int)A.bsend[B.off + t - 1] : 0;
-      s1_first = A.bsend[B.off + t];
-      pos_first = A.bpos[B.off + t];
-    }
-    stage_tile_records(A, B, s_xu);
-    __syncthreads();
-    for (int j = threadIdx.x; j < T.count; j += blockDim.x) {
-      const int64_t e = T.first + j;
-      const ushort4 lc = *reinterpret_cast<const ushort4 *>(A.lc + e * 4);
-      const ushort4 ls = *reinterpret_cast<const ushort4 *>(A.ls + e * 4);
-      float Q[3][3];
-      tet4_Q<LAW, float, QpCompact, akx::NodesLDS, false>(
-          make_int4(lc.x, lc.y, lc.z, lc.w),
-          akx::NodesLDS{reinterpret_cast<const double *>(s_xu)}, float(P.lambda),
-          float(P.mu), float(P.sigma_y), float(P.h), V, A.hoff + e, Q);
+  const int64_t tt = blockIdx.x;
+  if (tt >= A.ntiles)
+    return;
+  const BTile T = A.tiles[tt];
+  const BBlk B = A.blks[tt];
+  const BInst P = A.inst[T.inst];
+  const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
+  // the element's own streams and this lane's first distinct node of the
+  // summing phase, read ahead so that their loads overlap the staging (lanes
+  // past the end read the last element's)
+  const int t = threadIdx.x;
+  const bool active = t < T.count;
+  const int64_t e = T.first + (active ? t : T.count - 1);
+  const ushort4 lc = *reinterpret_cast<const ushort4 *>(A.lc + e * 4);
+  const ushort4 ls = *reinterpret_cast<const ushort4 *>(A.ls + e * 4);
+  int s0_first = 0, s1_first = 0, pos_first = 0;
+  if (t < B.count) {
+    s0_first = t > 0 ? (int)A.bsend[B.off + t - 1] : 0;
+    s1_first = A.bsend[B.off + t];
+    pos_first = A.bpos[B.off + t];
+  }
+  stage_tile_records(A, B, s_xu);
+  __syncthreads();
+  float J[3][3], H[3][3];
+  tet4_JH<float, akx::NodesLDS, false>(
+      make_int4(lc.x, lc.y, lc.z, lc.w),
+      akx::NodesLDS{reinterpret_cast<const double *>(s_xu)}, J, H);
+  __syncthreads(); // the records are dead: the LDS now takes the slots
+  float *s_f = reinterpret_cast<float *>(s_xu);
+  if (active) {
+    float Q[3][3];
+    tet4_Q<LAW, float>(J, H, float(P.lambda), float(P.mu), float(P.sigma_y), float(P.h), V,
+                       A.hoff + e, Q);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        s_f[3 * ls.x + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
-        s_f[3 * ls.y + c] = Q[c][1];
-        s_f[3 * ls.z + c] = Q[c][2];
-        s_f[3 * ls.w + c] = Q[c][0];
-      }
+    for (int c = 0; c < 3; ++c) {
+      s_f[3 * slot_pos(ls.x) + c] = -(Q[c][0] + Q[c][1] + Q[c][2]);
+      s_f[3 * slot_pos(ls.y) + c] = Q[c][1];
+      s_f[3 * slot_pos(ls.z) + c] = Q[c][2];
+      s_f[3 * slot_pos(ls.w) + c] = Q[c][0];
     }
-    __syncthreads();
-    for (int k = threadIdx.x; k < B.count; k += blockDim.x) {
-      const bool first = k == t;
-      const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
-      const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
-      const int pos = first ? pos_first : A.bpos[B.off + k];
-      sum_slots(s_f, s0, s1, fe, (int64_t)pos);
-    }
+  }
+  __syncthreads();
+  for (int k = t; k < B.count; k += 256) {
+    const bool first = k == t;
+    const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
+    const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
+    const int pos = first ? pos_first : A.bpos[B.off + k];
+    sum_slots<true>(s_f, s0, s1, fe, (int64_t)pos);
   }
 }
 
@@ -1261,7 +1286,7 @@ __global__ void __launch_bounds__(256) k_batch_hex8_bpa(BatchElemArgs A) {
     const bool first = k == t;
     const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
     const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
-    sum_slots(s_f, s0, s1, fe, (int64_t)(first ? pos_first : A.bpos[B.off + k]));
+    sum_slots<false>(s_f, s0, s1, fe, (int64_t)(first ? pos_first : A.bpos[B.off + k]));
   }
 }
 
@@ -1276,15 +1301,20 @@ int64_t elements_per_block(int etype, bool bpa) {
   return etype == 1 ? (bpa ? akx::BPA_HEX8 : HEX_EPB) : 256;
 }
 
+// LDS of the FP32 Tet4 block passes: the records, later 1024 corner slots
+static size_t tet4_bpa_lds(int32_t maxu) {
+  return std::max((size_t)maxu * 48, (size_t)slot_pos(1024) * 12);
+}
+
 template <int L, class CT, class FT>
 static void launch_one(int etype, const ElemArgs &A, hipStream_t s) {
   dim3 grid((unsigned)A.nblocks_padded), block(256);
   if (etype != 1) {
     if constexpr (sizeof(CT) == 4)
       if (A.lconn) {
-        if (A.lslot) // block-partial assembly: records, then 1024 corner slots
+        if (A.lslot) // block-partial assembly
           hipLaunchKernelGGL((k_tet4_bpa<L>), grid, block,
-                             (size_t)A.bl_maxu * 48 + 1024 * 12, s, A);
+                             tet4_bpa_lds(A.bl_maxu), s, A);
         else
           hipLaunchKernelGGL((k_tet4_lds<L>), grid, block, (size_t)A.bl_maxu * 48, s, A);
         return;
@@ -1344,10 +1374,10 @@ static void launch_batch_law(int etype, int block, const BatchElemArgs &A,
                              hipStream_t s) {
   dim3 grid((unsigned)A.ntiles);
   if (etype == 0) {
-    if (A.blks) // block-partial assembly: one tile per workgroup; records,
-                // then 1024 corner slots
-      hipLaunchKernelGGL(k_batch_tet4_bpa<LAW>, dim3((unsigned)A.ntiles), dim3(block),
-                         (size_t)A.bmaxu * 48 + 1024 * 12, s, A);
+    if (A.blks) // block-partial assembly: one tile per workgroup, one element
+                // per lane whatever the chosen block
+      hipLaunchKernelGGL(k_batch_tet4_bpa<LAW>, dim3((unsigned)A.ntiles), dim3(256),
+                         tet4_bpa_lds(A.bmaxu), s, A);
     else
       hipLaunchKernelGGL(k_batch_tet4_f32<LAW>, grid, dim3(block), 0, s, A);
   } else if (A.blks) { // block-partial assembly: records, then the corner slots
