@@ -16,11 +16,11 @@
 //            plastic strain [2][6][qp_cap] and hardening, FP32
 // Free lists (first fit) hand out and take back ranges.
 //
-// Per step: element pass (one persistent launch per (element type, law)
-// group present, over tiles that never span an instance, so the material
-// parameters and the plastic parity are uniform per block) and the nodal
-// gather + update (one persistent launch over the 256-node slices of the
-// live instances, dt uniform per block).  The arithmetic of the FP64 form is
+// Per step: element pass (one launch per (element type, law) group present,
+// FP32 batches usually one for all, over tiles that never span an instance, so
+// the material parameters and the plastic parity are uniform per block) and the
+// nodal gather + update (one launch over the 256-node slices of the live
+// instances, dt uniform per block).  The arithmetic of the FP64 form is
 // the reference's operation order, element by element identical to the
 // single-model plain path, so an instance gives the same bits alone and in
 // the mix.
@@ -779,22 +779,55 @@ template <int LAW> void launch_strict(akx_batch *b, int etype, const BatchElemAr
   HIPCHECK(hipGetLastError());
 }
 
+// The groups of an FP32 batch share a launch (k_batch_bpa_all) when there are
+// several: one after another, each leaves the chip idle before it is full and
+// while its last workgroups end, and costs a launch.  Its 84 registers (one
+// group: 55 to 71) cost more than that above MERGE_TILES tiles.  us a step,
+// one launch per group -> one for all:
+//   4 groups of 5,000 Tet4 or 1,000 Hex8      22.9 ->   9.1
+//   4 of 54,000 Tet4 or 9,600 Hex8            24.8 ->  12.0
+//   2 of 270,000 Tet4 (neo-Hookean, elastic)  23.8 ->  20.5
+//   4 of 860,000 or 154,000, 11,600 tiles       92 ->    80
+//   4 of 2.7 M or 480,000, 36,000 tiles        242 ->   249
+constexpr int64_t MERGE_TILES = 20480;
+
+BatchElemArgs checked_elem_args(akx_batch *b, int etype, int64_t t0, int64_t t1, int parity,
+                                bool plastic) {
+  BatchElemArgs A = elem_args(b, etype, t0, t1, parity);
+  require(A.conn && (A.pos || A.blks) && A.xu && A.fe && A.inst && A.tiles && A.hex_tab,
+          "batch element arena not allocated");
+  require(!b->fp32() || A.blks, "FP32 batch without its block tables");
+  if (plastic)
+    for (int s = 0; s < 2; ++s)
+      for (int k = 0; k < 4; ++k)
+        require(b->hist_comps(k) == 0 || A.hist[s][k] != nullptr,
+                "plastic history not allocated");
+  return A;
+}
+
 void element_pass(akx_batch *b, int parity) {
+  const int64_t *first = b->group_first;
+  int groups = 0;
+  for (int g = 0; g < NGROUP; ++g)
+    groups += first[g + 1] > first[g];
+  if (b->fp32() && groups > 1 && first[NGROUP] <= MERGE_TILES) {
+    const bool plastic = first[4] > first[3] || first[8] > first[7];
+    BatchElemArgs T{}, H{};
+    if (first[4] > first[0])
+      T = checked_elem_args(b, AKX_TET4, first[0], first[4], parity, plastic);
+    if (first[8] > first[4])
+      H = checked_elem_args(b, AKX_HEX8, first[4], first[8], parity, plastic);
+    HIPCHECK(akxf::launch_batch_all_f32(T, H, b->stream));
+    return;
+  }
   for (int g = 0; g < NGROUP; ++g) {
-    const int64_t t0 = b->group_first[g], t1 = b->group_first[g + 1];
-    if (t1 == t0)
+    if (first[g + 1] == first[g])
       continue;
     const int etype = g / 4, law = g % 4;
-    BatchElemArgs A = elem_args(b, etype, t0, t1, parity);
-    require(A.conn && (A.pos || A.blks) && A.xu && A.fe && A.inst && A.tiles && A.hex_tab,
-            "batch element arena not allocated");
-    if (law == AKX_LAW_PLASTIC_LIH)
-      for (int s = 0; s < 2; ++s)
-        for (int k = 0; k < 4; ++k)
-          require(b->hist_comps(k) == 0 || A.hist[s][k] != nullptr,
-                  "plastic history not allocated");
+    const BatchElemArgs A = checked_elem_args(b, etype, first[g], first[g + 1], parity,
+                                              law == AKX_LAW_PLASTIC_LIH);
     if (b->fp32()) {
-      HIPCHECK(akxf::launch_batch_elements_f32(etype, law, b->block, A, b->stream));
+      HIPCHECK(akxf::launch_batch_elements_f32(etype, law, A, b->stream));
     } else {
       switch (law) {
       case AKX_LAW_ELASTIC: launch_strict<LAW_ELASTIC>(b, etype, A); break;

@@ -1111,33 +1111,10 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepAr
 }
 
 // ---------------------------------------------------------------------------
-// Batched FP32 form, one tile of one (element type, law) group per
-// workgroup; per-instance parameters, compact FP32 plastic state (ping-pong
-// by step parity), corners read from the X and u arrays.  The per-corner
-// kernels (k_batch_tet4_f32, k_batch_hex8_f32) serve groups without block
-// tables; FP32 batches build block tables for every group, so their tiles
-// run the block-partial kernels below.
+// Batched FP32 form (block-partial assembly): one tile, which is one block, of
+// one instance per workgroup; per-instance parameters, compact FP32 plastic
+// state (ping-pong by step parity).
 // ---------------------------------------------------------------------------
-template <int LAW>
-__global__ void __launch_bounds__(256) k_batch_tet4_f32(BatchElemArgs A) {
-  {
-    const int64_t tt = blockIdx.x; // one tile per workgroup
-    if (tt >= A.ntiles)
-      return;
-    const BTile T = A.tiles[tt];
-    const BInst P = A.inst[T.inst];
-    const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
-    for (int j = threadIdx.x; j < T.count; j += blockDim.x) {
-      const int64_t e = T.first + j;
-      tet4_one<LAW, float, float, QpCompact, NodesSoA, FE_W>(
-          *reinterpret_cast<const int4 *>(A.conn + e * 4), NodesSoA{A.X, A.u, A.ncap},
-                                         float(P.lambda), float(P.mu), float(P.sigma_y),
-                                         float(P.h), V, A.hoff + e, A.pos + e * 4,
-                                         reinterpret_cast<float *>(A.fe));
-    }
-  }
-}
-
 // the {X, u} records of a tile's distinct nodes, built in LDS from the X and
 // u arrays (FP32 instances keep u in the [3][ncap] array, BInst::urec = 0)
 __device__ __forceinline__ void stage_tile_records(const BatchElemArgs &A, const BBlk &B,
@@ -1161,15 +1138,11 @@ __device__ __forceinline__ void stage_tile_records(const BatchElemArgs &A, const
 // in that order (FP64, rounded once) and writes one table entry per (block,
 // node).  The gather adds a node's partials in ascending block order.
 template <int LAW>
-__global__ void __launch_bounds__(256) k_batch_tet4_bpa(BatchElemArgs A) {
-  extern __shared__ double2 s_xu[]; // [bmaxu][3] records, later the corner slots
+__device__ __forceinline__ void batch_tet4_block(const BatchElemArgs &A, const BTile &T,
+                                                 const BBlk &B, const BInst &P,
+                                                 double2 *s_xu) { // [bmaxu][3] records,
+                                                                  // later the corner slots
   float *fe = reinterpret_cast<float *>(A.fe);
-  const int64_t tt = blockIdx.x;
-  if (tt >= A.ntiles)
-    return;
-  const BTile T = A.tiles[tt];
-  const BBlk B = A.blks[tt];
-  const BInst P = A.inst[T.inst];
   const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
   // the element's own streams and this lane's first distinct node of the
   // summing phase, read ahead so that their loads overlap the staging (lanes
@@ -1215,44 +1188,16 @@ __global__ void __launch_bounds__(256) k_batch_tet4_bpa(BatchElemArgs A) {
   }
 }
 
-template <int LAW, int EPB>
-__global__ void __launch_bounds__(EPB * 8) k_batch_hex8_f32(BatchElemArgs A) {
-  const int t = threadIdx.x, el = t >> 3, q = t & 7;
-  {
-    const int64_t tt = blockIdx.x; // one tile per workgroup
-    if (tt >= A.ntiles)
-      return;
-    const BTile T = A.tiles[tt];
-    const BInst P = A.inst[T.inst];
-    const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
-    for (int base = 0; base < T.count; base += EPB) {
-      const bool active = base + el < T.count;
-      const int64_t e = T.first + (active ? base + el : 0);
-      const int32_t nd = A.conn[e * 8 + hex_node_of_lane(q)];
-      float F[3];
-      hex8_group_sf<LAW>(q, active, nd, NodesSoA{A.X, A.u, A.ncap}, float(P.lambda),
-                         float(P.mu), float(P.sigma_y), float(P.h), V, A.hoff + e * 8 + q, F);
-      if (active)
-        akx::put_entry<FE_W>(reinterpret_cast<float *>(A.fe),
-                             (int64_t)A.pos[e * 8 + hex_node_of_lane(q)], F[0], F[1], F[2]);
-    }
-  }
-}
-
 // Batched FP32 Hex8 with block-partial assembly: each tile is one block of at
 // most BPA_HEX8 consecutive elements of one instance and each workgroup does
 // one tile, as k_hex8_bpa.
 template <int LAW>
-__global__ void __launch_bounds__(256) k_batch_hex8_bpa(BatchElemArgs A) {
-  extern __shared__ double2 s_xu[]; // [bmaxu][3] records, then [63 * 8][3] floats
+__device__ __forceinline__ void batch_hex8_block(const BatchElemArgs &A, const BTile &T,
+                                                 const BBlk &B, const BInst &P,
+                                                 double2 *s_xu) { // [bmaxu][3] records, then
+                                                                  // [63 * 8][3] floats
   float *s_f = reinterpret_cast<float *>(s_xu + 3 * A.bmaxu);
   const int t = threadIdx.x;
-  const int64_t tt = blockIdx.x;
-  if (tt >= A.ntiles)
-    return;
-  const BTile T = A.tiles[tt];
-  const BBlk B = A.blks[tt];
-  const BInst P = A.inst[T.inst];
   const QpCompact V = batch_compact_view(A, (P.parity_base ^ A.parity) & 1);
   const bool active = (t >> 2) < T.count;
   const int64_t e = T.first + (t >> 2);
@@ -1287,6 +1232,51 @@ __global__ void __launch_bounds__(256) k_batch_hex8_bpa(BatchElemArgs A) {
     const int s0 = first ? s0_first : (int)A.bsend[B.off + k - 1];
     const int s1 = first ? s1_first : (int)A.bsend[B.off + k];
     sum_slots<false>(s_f, s0, s1, fe, (int64_t)(first ? pos_first : A.bpos[B.off + k]));
+  }
+}
+
+// one (element type, law) group
+template <int ET, int LAW>
+__global__ void __launch_bounds__(256) k_batch_bpa(BatchElemArgs A) {
+  extern __shared__ double2 s_xu[];
+  const int64_t tt = blockIdx.x;
+  if (tt >= A.ntiles)
+    return;
+  const BTile T = A.tiles[tt];
+  const BBlk B = A.blks[tt];
+  const BInst P = A.inst[T.inst];
+  if constexpr (ET == 0)
+    batch_tet4_block<LAW>(A, T, B, P, s_xu);
+  else
+    batch_hex8_block<LAW>(A, T, B, P, s_xu);
+}
+
+// all groups of a batch: the Hex8 tiles H, then the Tet4 tiles A
+__global__ void __launch_bounds__(256) k_batch_bpa_all(BatchElemArgs A, BatchElemArgs H) {
+  extern __shared__ double2 s_xu[];
+  const int64_t tt = blockIdx.x;
+  if (tt >= H.ntiles + A.ntiles)
+    return;
+  if (tt < H.ntiles) {
+    const BTile T = H.tiles[tt];
+    const BBlk B = H.blks[tt];
+    const BInst P = H.inst[T.inst];
+    switch (P.law) {
+    case LAW_ELASTIC: batch_hex8_block<LAW_ELASTIC>(H, T, B, P, s_xu); break;
+    case LAW_ELASTIC_FD: batch_hex8_block<LAW_ELASTIC_FD>(H, T, B, P, s_xu); break;
+    case LAW_NEOHOOKEAN: batch_hex8_block<LAW_NEOHOOKEAN>(H, T, B, P, s_xu); break;
+    default: batch_hex8_block<LAW_PLASTIC>(H, T, B, P, s_xu); break;
+    }
+  } else {
+    const BTile T = A.tiles[tt - H.ntiles];
+    const BBlk B = A.blks[tt - H.ntiles];
+    const BInst P = A.inst[T.inst];
+    switch (P.law) {
+    case LAW_ELASTIC: batch_tet4_block<LAW_ELASTIC>(A, T, B, P, s_xu); break;
+    case LAW_ELASTIC_FD: batch_tet4_block<LAW_ELASTIC_FD>(A, T, B, P, s_xu); break;
+    case LAW_NEOHOOKEAN: batch_tet4_block<LAW_NEOHOOKEAN>(A, T, B, P, s_xu); break;
+    default: batch_tet4_block<LAW_PLASTIC>(A, T, B, P, s_xu); break;
+    }
   }
 }
 
@@ -1369,40 +1359,36 @@ hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStre
   return hipGetLastError();
 }
 
-template <int LAW>
-static void launch_batch_law(int etype, int block, const BatchElemArgs &A,
-                             hipStream_t s) {
-  dim3 grid((unsigned)A.ntiles);
-  if (etype == 0) {
-    if (A.blks) // block-partial assembly: one tile per workgroup, one element
-                // per lane whatever the chosen block
-      hipLaunchKernelGGL(k_batch_tet4_bpa<LAW>, dim3((unsigned)A.ntiles), dim3(256),
-                         tet4_bpa_lds(A.bmaxu), s, A);
-    else
-      hipLaunchKernelGGL(k_batch_tet4_f32<LAW>, grid, dim3(block), 0, s, A);
-  } else if (A.blks) { // block-partial assembly: records, then the corner slots
-    hipLaunchKernelGGL(k_batch_hex8_bpa<LAW>, grid, dim3(256),
-                       (size_t)A.bmaxu * 48 + akx::BPA_HEX8 * 8 * 12, s, A);
-  } else if (block == 64) {
-    hipLaunchKernelGGL((k_batch_hex8_f32<LAW, 8>), grid, dim3(64), 0, s, A);
-  } else if (block == 128) {
-    hipLaunchKernelGGL((k_batch_hex8_f32<LAW, 16>), grid, dim3(128), 0, s, A);
-  } else {
-    hipLaunchKernelGGL((k_batch_hex8_f32<LAW, 32>), grid, dim3(256), 0, s, A);
-  }
+static size_t hex8_bpa_lds(int32_t maxu) {
+  return (size_t)maxu * 48 + akx::BPA_HEX8 * 8 * 12;
 }
 
-hipError_t launch_batch_elements_f32(int etype, int law, int block,
-                                     const BatchElemArgs &A, hipStream_t stream) {
-  if (block != 64 && block != 128 && block != 256)
-    return hipErrorInvalidValue;
+template <int LAW> static void launch_batch_law(int etype, const BatchElemArgs &A, hipStream_t s) {
+  const dim3 grid((unsigned)A.ntiles), block(256);
+  if (etype == 0)
+    hipLaunchKernelGGL((k_batch_bpa<0, LAW>), grid, block, tet4_bpa_lds(A.bmaxu), s, A);
+  else
+    hipLaunchKernelGGL((k_batch_bpa<1, LAW>), grid, block, hex8_bpa_lds(A.bmaxu), s, A);
+}
+
+hipError_t launch_batch_elements_f32(int etype, int law, const BatchElemArgs &A,
+                                     hipStream_t stream) {
   switch (law) {
-  case LAW_ELASTIC: launch_batch_law<LAW_ELASTIC>(etype, block, A, stream); break;
-  case LAW_ELASTIC_FD: launch_batch_law<LAW_ELASTIC_FD>(etype, block, A, stream); break;
-  case LAW_NEOHOOKEAN: launch_batch_law<LAW_NEOHOOKEAN>(etype, block, A, stream); break;
-  case LAW_PLASTIC: launch_batch_law<LAW_PLASTIC>(etype, block, A, stream); break;
+  case LAW_ELASTIC: launch_batch_law<LAW_ELASTIC>(etype, A, stream); break;
+  case LAW_ELASTIC_FD: launch_batch_law<LAW_ELASTIC_FD>(etype, A, stream); break;
+  case LAW_NEOHOOKEAN: launch_batch_law<LAW_NEOHOOKEAN>(etype, A, stream); break;
+  case LAW_PLASTIC: launch_batch_law<LAW_PLASTIC>(etype, A, stream); break;
   default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_batch_all_f32(const BatchElemArgs &tets, const BatchElemArgs &hexes,
+                                hipStream_t stream) {
+  const size_t lds = std::max(tets.ntiles > 0 ? tet4_bpa_lds(tets.bmaxu) : 0,
+                              hexes.ntiles > 0 ? hex8_bpa_lds(hexes.bmaxu) : 0);
+  hipLaunchKernelGGL(k_batch_bpa_all, dim3((unsigned)(tets.ntiles + hexes.ntiles)), dim3(256), lds,
+                     stream, tets, hexes);
   return hipGetLastError();
 }
 

@@ -16,8 +16,10 @@ hipError_t launch_elements(int etype, int law, bool fp32, const akx::ElemArgs &A
                            hipStream_t stream);
 // launch one step of a small FP32 Tet4 model (akx_step.hpp)
 hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream);
-// launch the FP32-form batched element pass of one (element type, law) group;
-// block = threads per block (64, 128 or 256; Hex8: 8 lanes per element)
-hipError_t launch_batch_elements_f32(int etype, int law, int block,
-                                     const akx::BatchElemArgs &A, hipStream_t stream);
+// launch the FP32-form batched element pass (block-partial assembly) of one
+// (element type, law) group, or of all groups: the Tet4 and the Hex8 tiles
+hipError_t launch_batch_elements_f32(int etype, int law, const akx::BatchElemArgs &A,
+                                     hipStream_t stream);
+hipError_t launch_batch_all_f32(const akx::BatchElemArgs &tets, const akx::BatchElemArgs &hexes,
+                                hipStream_t stream);
 } // namespace akxf
