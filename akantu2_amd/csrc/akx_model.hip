@@ -1429,34 +1429,29 @@ void launch_hex8_strict(akx_model *m, Material &mat, const ElemArgs &A) {
     launch_hex8_strict_x<false>(m, mat, A);
 }
 
-template <bool EXT>
-void launch_tet4_ppa_x(akx_model *m, Material &mat, const ElemArgs &A) {
-  dim3 grid((unsigned)A.nblocks_padded), block(PPA_TB);
+template <int LAW> void launch_tet4_ppa_law(akx_model *m, Material &mat, const ElemArgs &A) {
+  const dim3 grid((unsigned)A.nblocks_padded), block(PPA_TB);
   const size_t lds = std::max((size_t)A.bl_maxu * 48, (size_t)A.t_slots * 24);
+  if (mat.ext() && A.grad_u)
+    hipLaunchKernelGGL((k_tet4_ppa<LAW, true, true>), grid, block, lds, m->stream, A);
+  else if (mat.ext())
+    hipLaunchKernelGGL((k_tet4_ppa<LAW, true, false>), grid, block, lds, m->stream, A);
+  else if (A.grad_u)
+    hipLaunchKernelGGL((k_tet4_ppa<LAW, false, true>), grid, block, lds, m->stream, A);
+  else
+    hipLaunchKernelGGL((k_tet4_ppa<LAW, false, false>), grid, block, lds, m->stream, A);
+}
+
+void launch_tet4_ppa(akx_model *m, Material &mat, const ElemArgs &A) {
   switch (mat.law) {
-  case AKX_LAW_ELASTIC:
-    hipLaunchKernelGGL((k_tet4_ppa<LAW_ELASTIC, EXT>), grid, block, lds, m->stream, A);
-    break;
-  case AKX_LAW_ELASTIC_FD:
-    hipLaunchKernelGGL((k_tet4_ppa<LAW_ELASTIC_FD, EXT>), grid, block, lds, m->stream, A);
-    break;
-  case AKX_LAW_NEOHOOKEAN:
-    hipLaunchKernelGGL((k_tet4_ppa<LAW_NEOHOOKEAN, EXT>), grid, block, lds, m->stream, A);
-    break;
-  case AKX_LAW_PLASTIC_LIH:
-    hipLaunchKernelGGL((k_tet4_ppa<LAW_PLASTIC, EXT>), grid, block, lds, m->stream, A);
-    break;
+  case AKX_LAW_ELASTIC: launch_tet4_ppa_law<LAW_ELASTIC>(m, mat, A); break;
+  case AKX_LAW_ELASTIC_FD: launch_tet4_ppa_law<LAW_ELASTIC_FD>(m, mat, A); break;
+  case AKX_LAW_NEOHOOKEAN: launch_tet4_ppa_law<LAW_NEOHOOKEAN>(m, mat, A); break;
+  case AKX_LAW_PLASTIC_LIH: launch_tet4_ppa_law<LAW_PLASTIC>(m, mat, A); break;
   default: // user laws never take this path
     throw Error(AKX_ERR_UNSUPPORTED, "prefix-partial pass for a user law");
   }
   HIPCHECK(hipGetLastError());
-}
-
-void launch_tet4_ppa(akx_model *m, Material &mat, const ElemArgs &A) {
-  if (mat.ext())
-    launch_tet4_ppa_x<true>(m, mat, A);
-  else
-    launch_tet4_ppa_x<false>(m, mat, A);
 }
 
 void launch_device_law(akx_model *m, Material &mat, ElemArgs A, bool materialize);
