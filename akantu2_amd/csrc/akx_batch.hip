@@ -115,6 +115,7 @@ struct BatchGatherArgs {
   float *cu, *cv; // compensation terms (FP32 form) or null
   int64_t ncap;
   int64_t nblocks;
+  bool stream; // non-temporal reads of the table (STREAM_BYTES)
 };
 
 // One 256-node slice per workgroup (a persistent loop over slices measured
@@ -173,7 +174,7 @@ __global__ void __launch_bounds__(256) k_batch_gather(BatchGatherArgs G) {
       load_u();
   }
   double f[3];
-  sum_entries<FEW, FE_W>(p, deg, f);
+  sum_entries<FEW, FE_W>(p, deg, G.stream, f);
   if constexpr (!FEW) {
     M = G.mass[n];
     blk = G.blocked[n];
@@ -582,6 +583,7 @@ struct akx_batch {
   DevBuf<BSlice> d_slices;
   int64_t group_first[NGROUP + 1] = {0};
   int64_t nslices_live = 0;
+  bool stream_loads = true; // more than STREAM_BYTES a step
   bool lists_dirty = true, inst_dirty = true;
   // launch shape
   int block = 256, tile = 2048, blocks_per_cu = 0, cus = 256;
@@ -669,6 +671,40 @@ int64_t group_tile(const akx_batch *b, int etype, int64_t n) {
   return std::max<int64_t>(32, std::min<int64_t>(t, 128));
 }
 
+// Bytes the element passes (class 0) or the gather (1) of one step cannot do
+// without
+double kernel_bytes(const akx_batch *b, int kernel_class) {
+  const double fs = (double)b->fe_size(), hs = (double)b->hist_size();
+  double total = 0;
+  for (auto &I : b->inst) {
+    if (!I.live)
+      continue;
+    const double nnpe = I.etype == AKX_TET4 ? 4 : 8, nqp = I.etype == AKX_TET4 ? 1 : 8;
+    const double corners = (double)I.nel * nnpe, nn = (double)I.nn;
+    // table entries written and read: one per element corner, or one per
+    // (block, distinct node) under block-partial assembly
+    const bool bpa = !I.blk_cnt.empty();
+    const double entries = bpa ? (double)I.nbent : corners;
+    if (kernel_class == 0) {
+      if (bpa) // per corner the local corner (2 B) and the slot (2 B); per
+               // entry the node id, slot end and table position, the
+               // partial written
+        total += corners * 4 + entries * (4 + 2 + 4 + 3 * fs) + nn * 2 * 3 * 8;
+      else
+        total += corners * (4 + 4 + 3 * fs) + nn * 2 * 3 * 8;
+      if (I.law == AKX_LAW_PLASTIC_LIH) // history read and written
+        total += (double)I.nel * nqp * 2 * (b->fp32() ? 7 : 28) * hs;
+    } else {
+      // a step followed by another (f_int is written by the last one
+      // only): u, v and a read and written; FP32: u, the half-step
+      // velocity and their compensation terms
+      total += entries * 3 * fs + nn * (1 + 1 + 8 + (b->fp32() ? 2 * 3 * 2 * (8 + 4)
+                                                                : 3 * 3 * 2 * 8));
+    }
+  }
+  return total;
+}
+
 // work lists of the live instances: element tiles per group, node slices
 void rebuild_lists(akx_batch *b) {
   std::vector<std::vector<BTile>> groups(NGROUP);
@@ -729,6 +765,7 @@ void rebuild_lists(akx_batch *b) {
     HIPCHECK(hipMemcpy(b->d_slices.p, slices.data(), slices.size() * sizeof(BSlice),
                        hipMemcpyHostToDevice));
   b->nslices_live = (int64_t)slices.size();
+  b->stream_loads = kernel_bytes(b, 0) + kernel_bytes(b, 1) > STREAM_BYTES;
   b->lists_dirty = false;
 }
 
@@ -858,6 +895,7 @@ BatchGatherArgs gather_args(akx_batch *b) {
   G.cv = b->cv.p;
   G.ncap = b->ncap;
   G.nblocks = G.nslices; // one slice per workgroup
+  G.stream = b->stream_loads;
   require(G.slices && G.ell_off && G.deg && G.fe && G.fint && G.xu && G.v && G.a &&
               G.mass && G.blocked,
           "batch node arena not allocated");
@@ -1697,35 +1735,7 @@ int akx_batch_get_kernel_bytes(akx_batch *b, int kernel_class, double *bytes) {
   return guard([&] {
     require(b != nullptr && bytes != nullptr && kernel_class >= 0 && kernel_class < 2,
             "bad arguments");
-    const double fs = (double)b->fe_size(), hs = (double)b->hist_size();
-    double total = 0;
-    for (auto &I : b->inst) {
-      if (!I.live)
-        continue;
-      const double nnpe = I.etype == AKX_TET4 ? 4 : 8, nqp = I.etype == AKX_TET4 ? 1 : 8;
-      const double corners = (double)I.nel * nnpe, nn = (double)I.nn;
-      // table entries written and read: one per element corner, or one per
-      // (block, distinct node) under block-partial assembly
-      const bool bpa = !I.blk_cnt.empty();
-      const double entries = bpa ? (double)I.nbent : corners;
-      if (kernel_class == 0) {
-        if (bpa) // per corner the local corner (2 B) and the slot (2 B); per
-                 // entry the node id, slot end and table position, the
-                 // partial written
-          total += corners * 4 + entries * (4 + 2 + 4 + 3 * fs) + nn * 2 * 3 * 8;
-        else
-          total += corners * (4 + 4 + 3 * fs) + nn * 2 * 3 * 8;
-        if (I.law == AKX_LAW_PLASTIC_LIH) // history read and written
-          total += (double)I.nel * nqp * 2 * (b->fp32() ? 7 : 28) * hs;
-      } else {
-        // a step followed by another (f_int is written by the last one
-        // only): u, v and a read and written; FP32: u, the half-step
-        // velocity and their compensation terms
-        total += entries * 3 * fs + nn * (1 + 1 + 8 + (b->fp32() ? 2 * 3 * 2 * (8 + 4)
-                                                                  : 3 * 3 * 2 * 8));
-      }
-    }
-    *bytes = total;
+    *bytes = kernel_bytes(b, kernel_class);
   });
 }
 

@@ -735,17 +735,30 @@ __global__ void __launch_bounds__(PPA_TB) k_tet4_ppa(ElemArgs A) {
 constexpr int HEX_STRICT_EPB = 8;
 
 // J^-1 and w det J of one Gauss point, from the table that init fills (jw: the
-// Gauss point's column 0 of [5][stride]).  Streamed once per step:
-// non-temporal loads leave the caches to the nodal data.
+// Gauss point's column 0 of [5][stride]).  Read once per step: with STREAM,
+// non-temporal loads leave the caches to the nodal data (STREAM_BYTES; a
+// template parameter, as the compiler merges the two branches of a flag into
+// plain loads).
 struct HexJac {
   double Ji[3][3], wJ;
+  template <bool STREAM>
   __device__ __forceinline__ void load(const double2 *jw, int64_t stride) {
     typedef double dv2 __attribute__((ext_vector_type(2)));
     const dv2 *jv = reinterpret_cast<const dv2 *>(jw);
-    const dv2 j0 = __builtin_nontemporal_load(jv), j1 = __builtin_nontemporal_load(jv + stride),
-              j2 = __builtin_nontemporal_load(jv + 2 * stride),
-              j3 = __builtin_nontemporal_load(jv + 3 * stride),
-              j4 = __builtin_nontemporal_load(jv + 4 * stride);
+    dv2 j0, j1, j2, j3, j4;
+    if constexpr (STREAM) {
+      j0 = __builtin_nontemporal_load(jv);
+      j1 = __builtin_nontemporal_load(jv + stride);
+      j2 = __builtin_nontemporal_load(jv + 2 * stride);
+      j3 = __builtin_nontemporal_load(jv + 3 * stride);
+      j4 = __builtin_nontemporal_load(jv + 4 * stride);
+    } else {
+      j0 = jv[0];
+      j1 = jv[stride];
+      j2 = jv[2 * stride];
+      j3 = jv[3 * stride];
+      j4 = jv[4 * stride];
+    }
     Ji[0][0] = j0.x;
     Ji[0][1] = j0.y;
     Ji[0][2] = j1.x;
@@ -900,7 +913,7 @@ struct PutEntries {
 // fills (k_hex8_jacobian_table): they depend on the reference coordinates
 // only, as the reference's FEEngine precompute does (fe_engine_template_tmpl
 // .hh:98-120), so the pass loads u but not X.
-template <int LAW, bool EXT = false>
+template <int LAW, bool EXT = false, bool STREAM = true>
 __global__ void __launch_bounds__(64) k_hex8_strict(ElemArgs A) {
   __shared__ double sN[HEX_STRICT_EPB][8][6];
   __shared__ double sD[8][3][8];
@@ -924,7 +937,7 @@ __global__ void __launch_bounds__(64) k_hex8_strict(ElemArgs A) {
   }
   HexJac pre{};
   if (active)
-    pre.load(A.jw + e * 8 + q, A.nel * 8);
+    pre.load<STREAM>(A.jw + e * 8 + q, A.nel * 8);
   hex8_strict_group<LAW, HEX_STRICT_EPB, double, NodesSoA, true, EXT>(
       sN, sD, c_hex8.w[q], el, q, active, active ? A.conn[e * 8 + q] : 0,
       NodesSoA{A.X, A.u, A.nn}, lambda, mu, sy, hh, qp_view(A, 8), i * 8 + q,
@@ -962,15 +975,18 @@ struct GatherArgs {
   float *cu, *cv;        // compensation terms [3][nn] (FP32 form) or null
   double dt;
   int64_t nblocks_padded;
+  bool stream; // non-temporal reads of the table (STREAM_BYTES)
 };
 
 // Sum of the entries d = 0 .. deg - 1 of a node, f = (0 + -1 e_0) + -1 e_1 ...
-// The table is read once per step: non-temporal loads keep it from displacing
-// the nodal state in the caches.  FEW: eight entries are loaded before the
-// first is added (the loads past the last entry repeat it and are not added),
-// so a node waits for one or two round trips instead of one per entry.
+// The table is read once per step.  STREAM_BYTES: above it non-temporal loads
+// keep the table from displacing the nodal state in the caches (stream); below
+// it the table is still in the caches the element pass wrote it to, and plain
+// loads find it there.  FEW: eight entries are loaded before the first is added
+// (the loads past the last entry repeat it and are not added), so a node waits
+// for one or two round trips instead of one per entry.
 template <bool FEW, int W, class FT>
-__device__ __forceinline__ void sum_entries(const FT *p, int deg, double (&f)[3]) {
+__device__ __forceinline__ void sum_entries(const FT *p, int deg, bool stream, double (&f)[3]) {
   f[0] = f[1] = f[2] = 0.;
   if constexpr (FEW) {
     constexpr int CH = 8;
@@ -981,7 +997,7 @@ __device__ __forceinline__ void sum_entries(const FT *p, int deg, double (&f)[3]
         const FT *q = p + (int64_t)(d0 + j < deg ? d0 + j : deg - 1) * (256 * W);
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-          e[j][c] = __builtin_nontemporal_load(q + c);
+          e[j][c] = q[c];
       }
 #pragma unroll
       for (int j = 0; j < CH; ++j)
@@ -990,22 +1006,37 @@ __device__ __forceinline__ void sum_entries(const FT *p, int deg, double (&f)[3]
           for (int c = 0; c < 3; ++c)
             f[c] = f[c] + -1. * double(e[j][c]);
     }
-  } else {
+  } else if (stream) {
     for (int d = 0; d < deg; ++d, p += 256 * W)
 #pragma unroll
       for (int c = 0; c < 3; ++c)
         f[c] = f[c] + -1. * double(__builtin_nontemporal_load(p + c));
+  } else {
+    for (int d = 0; d < deg; ++d, p += 256 * W)
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+        f[c] = f[c] + -1. * double(p[c]);
   }
 }
 
+// Most bytes (element pass and gather of a step, table, nodal state and element
+// streams) up to which what a step reads once is read with plain loads: they
+// are then found in the 256 MB Infinity Cache.  Counted as read and written, so
+// the table counts twice.  Step, non-temporal -> plain, us: Tet4 FP64 73 MB 29.0
+// -> 25.9, 180 MB 46.6 -> 41.1, 302 MB 65.2 -> 59.2, 417 MB 90.6 -> 93.5, 871 MB
+// 214 -> 231; Hex8 FP64 elastic 191 MB 51 -> 49 (with the jacobian table 43),
+// 367 MB 85 -> 86 (82 -> 83), 1,236 MB 276 -> 279 (277 -> 295); FP32 within 3 %
+// either way.  Up to 65,536 nodes: Tet4 FP64 24.4 -> 21.0 us, plastic 22.4 ->
+// 20.1.
+constexpr double STREAM_BYTES = 310e6;
+
 // Up to this many nodes a gather reads its nodal state ahead of the entries
-// and the entries eight at a time (FEW).  With one wave per SIMD or less
-// (1,024 SIMDs x 64 nodes) its time is one node's chain of dependent loads;
-// above, the plain loop's other waves hide that chain, and the repeated loads
-// of the short chunks cost.  Step before -> with FEW, us: 525 nodes (1,920
-// Tet4) 14.1 -> 11.6, 1,331 (Hex8, FP64) 11.4 -> 10.3, 6,975 (plastic Tet4)
-// 19.9 -> 17.0; 158,661 nodes (FP64 Tet4) 46.0 -> 49.0.
-constexpr int64_t GATHER_FEW_NODES = 1024 * 64;
+// and the entries eight at a time (FEW).  With one or two waves per SIMD (1,024
+// SIMDs x 64 nodes) its time is one node's chain of dependent loads; above,
+// the plain loop's other waves hide that chain, and the repeated loads of the
+// short chunks cost.  Step before -> with FEW, us: 17,550 nodes (FP64 Tet4) and
+// fewer 3 less, 65,559 25.9 -> 23.4, 158,661 41.1 -> 41.2, 264,191 58.5 -> 59.8.
+constexpr int64_t GATHER_FEW_NODES = 1024 * 128;
 
 template <class FT, bool UPDATE, bool PREDICT, bool COMP, bool FEW = false>
 __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
@@ -1039,7 +1070,7 @@ __global__ void __launch_bounds__(256) k_gather_update(GatherArgs A) {
     }
   }
   double f[3];
-  sum_entries<FEW, 3>(p, deg, f);
+  sum_entries<FEW, 3>(p, deg, A.stream, f);
   if (A.fint) { // null while more steps follow in the same batch
     A.fint[n] = f[0];
     A.fint[A.nn + n] = f[1];

@@ -148,7 +148,7 @@ template <int LAW> __global__ void __launch_bounds__(STEP_HEX_EPB * 8) k_hex8_st
     }
     s_ls[el][q] = S.ls[i * 8 + q];
     HexJac pre;
-    pre.load(S.jw + (int64_t)e * 8 + q, S.nel * 8);
+    pre.load<false>(S.jw + (int64_t)e * 8 + q, S.nel * 8);
     if (base == 0) {
       step_stage<false>(S, b, s_rec);
       for (int k = t; k < 192; k += STEP_HEX_EPB * 8)
@@ -788,6 +788,7 @@ struct akx_model {
   DevBuf<int64_t> bp_off;
   DevBuf<uint8_t> bp_deg;
   int64_t bp_total = 0;
+  int64_t bp_entries = 0; // without the slices' padding
   // FP64 Tet4 partial-sum assembly: prefix partials (same bits, fewer
   // entries: each node's first-block sum, then one entry per later corner)
   // or, opted into, block partials (one entry per (block, node))
@@ -802,6 +803,7 @@ struct akx_model {
   StepArgs step{};
   DevBuf<unsigned char> step_lists;
   size_t step_lds = 0;
+  bool stream_loads = true; // more than STREAM_BYTES a step
   DevBuf<unsigned char> staging;
   Downloader download;
   DevBuf<unsigned long long> scratch_u64;
@@ -1065,8 +1067,11 @@ void build_bpa_table(akx_model *m) {
                        hipMemcpyHostToDevice));
   }
   std::vector<uint8_t> deg8(m->nn);
-  for (int64_t nd = 0; nd < m->nn; ++nd)
+  m->bp_entries = 0;
+  for (int64_t nd = 0; nd < m->nn; ++nd) {
     deg8[nd] = (uint8_t)deg[nd];
+    m->bp_entries += deg[nd];
+  }
   m->bp_off.alloc(off.size());
   m->bp_deg.alloc(std::max<int64_t>(m->nn, 1));
   HIPCHECK(hipMemcpy(m->bp_off.p, off.data(), off.size() * sizeof(int64_t),
@@ -1393,40 +1398,29 @@ void launch_elem_law(akx_model *m, Material &mat, const ElemArgs &A) {
     launch_elem_law_x<ET, CT, FT, false>(m, mat, A);
 }
 
-template <bool EXT>
-void launch_hex8_strict_x(akx_model *m, Material &mat, const ElemArgs &A) {
+template <int LAW> void launch_hex8_strict_law(akx_model *m, Material &mat, const ElemArgs &A) {
+  const dim3 grid((unsigned)A.nblocks_padded), block(64);
+  if (mat.ext())
+    hipLaunchKernelGGL((k_hex8_strict<LAW, true>), grid, block, 0, m->stream, A);
+  else if (m->stream_loads)
+    hipLaunchKernelGGL((k_hex8_strict<LAW, false, true>), grid, block, 0, m->stream, A);
+  else
+    hipLaunchKernelGGL((k_hex8_strict<LAW, false, false>), grid, block, 0, m->stream, A);
+}
+
+void launch_hex8_strict(akx_model *m, Material &mat, const ElemArgs &A) {
   require(A.jw != nullptr, "Hex8 element pass without its jacobian table");
-  dim3 grid((unsigned)A.nblocks_padded), block(64);
   switch (mat.law) {
-  case AKX_LAW_ELASTIC:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_ELASTIC, EXT>), grid, block, 0, m->stream, A);
-    break;
-  case AKX_LAW_ELASTIC_FD:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_ELASTIC_FD, EXT>), grid, block, 0, m->stream, A);
-    break;
-  case AKX_LAW_NEOHOOKEAN:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_NEOHOOKEAN, EXT>), grid, block, 0, m->stream, A);
-    break;
-  case AKX_LAW_PLASTIC_LIH:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_PLASTIC, EXT>), grid, block, 0, m->stream, A);
-    break;
-  case AKX_LAW_USER:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_USER, EXT>), grid, block, 0, m->stream, A);
-    break;
-  case AKX_LAW_USER_FD:
-    hipLaunchKernelGGL((k_hex8_strict<LAW_USER_FD, EXT>), grid, block, 0, m->stream, A);
-    break;
+  case AKX_LAW_ELASTIC: launch_hex8_strict_law<LAW_ELASTIC>(m, mat, A); break;
+  case AKX_LAW_ELASTIC_FD: launch_hex8_strict_law<LAW_ELASTIC_FD>(m, mat, A); break;
+  case AKX_LAW_NEOHOOKEAN: launch_hex8_strict_law<LAW_NEOHOOKEAN>(m, mat, A); break;
+  case AKX_LAW_PLASTIC_LIH: launch_hex8_strict_law<LAW_PLASTIC>(m, mat, A); break;
+  case AKX_LAW_USER: launch_hex8_strict_law<LAW_USER>(m, mat, A); break;
+  case AKX_LAW_USER_FD: launch_hex8_strict_law<LAW_USER_FD>(m, mat, A); break;
   default:
     throw Error(AKX_ERR_UNSUPPORTED, "unknown law");
   }
   HIPCHECK(hipGetLastError());
-}
-
-void launch_hex8_strict(akx_model *m, Material &mat, const ElemArgs &A) {
-  if (mat.ext())
-    launch_hex8_strict_x<true>(m, mat, A);
-  else
-    launch_hex8_strict_x<false>(m, mat, A);
 }
 
 template <int LAW> void launch_tet4_ppa_law(akx_model *m, Material &mat, const ElemArgs &A) {
@@ -1708,6 +1702,7 @@ GatherArgs gather_args(akx_model *m, bool per_corner = false) {
   G.cv = m->cv.p;
   G.dt = m->dt;
   G.nblocks_padded = padded_blocks(m->nn);
+  G.stream = m->stream_loads;
   return G;
 }
 
@@ -2265,6 +2260,69 @@ void solve_pipelined(akx_model *m, int64_t nb_steps) {
   HIPCHECK(hipStreamWaitEvent(m->stream, m->ev_gather[(nb_steps - 1) & 1][P - 1], 0));
 }
 
+// Bytes one launch of a kernel class cannot do without
+double kernel_bytes(const akx_model *m, int kernel_class) {
+  const double s_node = 8.0; // FP64 nodal state
+  const double s_f = (double)m->fe_elem_size();
+  int64_t nel_all = 0;
+  double extra = 0.;
+  for (auto &mp : m->mats) {
+    nel_all += mp->n;
+    if (mp->per_element) // lambda, mu per element: FP64, or the FP32 pair
+      extra += mp->n * (mp->lm_f.p ? 2.0 * 4.0 : 2.0 * 8.0);
+    if (mp->lconn.p) // staged records: 2-byte local
+      // corners instead of 4-byte node ids, plus the blocks' node lists
+      extra += -2.0 * m->nnpe * mp->n + 4.0 * (double)mp->bl_nodes.n;
+    if (mp->law == AKX_LAW_PLASTIC_LIH)
+      extra += (double)mp->n * m->nqp * (2 * (9 + 9 + 9 + 1) * 8.0); // read + write history
+    if (!mp->contiguous)
+      extra += mp->n * 4.0;
+  }
+  // table entries the element pass writes and the gather reads: one per
+  // element corner, or one per (block, distinct node) partial
+  double entries = (double)nel_all * m->nnpe;
+  if (m->bpa) {
+    const double partials = (double)m->bp_entries;
+    // corner slots (2 B) instead of table positions (4 B); per partial its
+    // slot offset (2 B) and table position (4 B)
+    extra += -2.0 * m->nnpe * nel_all + 6.0 * partials;
+    entries = partials;
+  } else if (m->ppa) {
+    // corner codes (4 B, as the positions); per summed run its slot end
+    // (2 B) and table position (4 B)
+    extra += 6.0 * (double)m->pp_runs;
+    entries = (double)m->pp_entries;
+  }
+  switch (kernel_class) {
+  case 0: // element pass: connectivity + table entries, X and u once per
+          // node, r_e write; with the Hex8 jacobian table, the table (80 B
+          // per Gauss point) instead of X
+    if (m->jw.p)
+      return nel_all * (8.0 * m->nnpe + 80.0 * m->nqp) + entries * 3.0 * s_f +
+             m->nn * 3.0 * s_node + extra;
+    return nel_all * 8.0 * m->nnpe + entries * 3.0 * s_f +
+           m->nn * (3.0 * s_node + 3.0 * s_node) + extra;
+  case 1: { // gather + update of a step followed by another: degree, r_e
+            // read, mass, blocked, a/v read+write, u read+write (fused
+            // predictor); the last step of a call also writes f_int.  The
+            // FP32 form reads and writes no a between the steps of a call
+            // (its velocity array holds the half-step velocity), and its
+            // compensation terms
+    const bool f32 = m->precision == AKX_PRECISION_FP32;
+    double per_node = 4.0 + s_node /*M*/ + 1.0 + (m->records_live() ? 3 * s_node : 0.) /*u records*/ +
+                      (f32 ? 0. : 2 * 3 * s_node) /*a*/ + 2 * 3 * s_node /*v*/ +
+                      2 * 3 * s_node /*u*/ + (m->has_fext ? 3 * s_node : 0.);
+    if (f32)
+      per_node += 2 * 2 * 3 * 4.0; // compensation terms read + write
+    return entries * (3.0 * s_f) + m->nn * (per_node - 3.0);
+  }
+  case 2:
+    return m->nn * (1.0 + 3 * s_node + 2 * 2 * 3 * s_node);
+  default:
+    throw Error(AKX_ERR_INVALID, "bad kernel class");
+  }
+}
+
 InitArgs init_args(akx_model *m, Material *mat) {
   InitArgs A{};
   A.nel = m->nel;
@@ -2784,6 +2842,7 @@ int akx_model_init_full(akx_model *m) {
       HIPCHECK(hipStreamSynchronize(m->stream));
     }
     plan_small_steps(m);
+    m->stream_loads = kernel_bytes(m, 0) + kernel_bytes(m, 1) > STREAM_BYTES;
     for (auto &mp : m->mats)
       alloc_internals(m, *mp);
     if (m->precision == AKX_PRECISION_FP32) {
@@ -3909,74 +3968,7 @@ int akx_model_get_kernel_bytes(akx_model *m, int kernel_class, double *bytes) {
   return guard([&] {
     check_ready(m);
     require(bytes != nullptr, "null output");
-    const double s_node = 8.0; // FP64 nodal state
-    const double s_f = (double)m->fe_elem_size();
-    const double s_c = m->precision == AKX_PRECISION_FP32 ? 4.0 : 8.0;
-    int64_t nel_all = 0;
-    double extra = 0.;
-    for (auto &mp : m->mats) {
-      nel_all += mp->n;
-      if (mp->per_element) // lambda, mu per element: FP64, or the FP32 pair
-        extra += mp->n * (mp->lm_f.p ? 2.0 * 4.0 : 2.0 * 8.0);
-      if (mp->lconn.p) // staged records: 2-byte local
-        // corners instead of 4-byte node ids, plus the blocks' node lists
-        extra += -2.0 * m->nnpe * mp->n + 4.0 * (double)mp->bl_nodes.n;
-      if (mp->law == AKX_LAW_PLASTIC_LIH)
-        extra += (double)mp->n * m->nqp * (2 * (9 + 9 + 9 + 1) * 8.0); // read + write history
-      if (!mp->contiguous)
-        extra += mp->n * 4.0;
-    }
-    (void)s_c;
-    // table entries the element pass writes and the gather reads: one per
-    // element corner, or one per (block, distinct node) partial
-    double entries = (double)nel_all * m->nnpe;
-    if (m->bpa) {
-      double partials = 0.;
-      for (auto &mp : m->mats)
-        for (int32_t node : mp->bl_nodes_host)
-          partials += node >= 0 ? 1. : 0.;
-      // corner slots (2 B) instead of table positions (4 B); per partial its
-      // slot offset (2 B) and table position (4 B)
-      extra += -2.0 * m->nnpe * nel_all + 6.0 * partials;
-      entries = partials;
-    } else if (m->ppa) {
-      // corner codes (4 B, as the positions); per summed run its slot end
-      // (2 B) and table position (4 B)
-      extra += 6.0 * (double)m->pp_runs;
-      entries = (double)m->pp_entries;
-    }
-    switch (kernel_class) {
-    case 0: // element pass: connectivity + table entries, X and u once per
-            // node, r_e write; with the Hex8 jacobian table, the table (80 B
-            // per Gauss point) instead of X
-      if (m->jw.p)
-        *bytes = nel_all * (8.0 * m->nnpe + 80.0 * m->nqp) + entries * 3.0 * s_f +
-                 m->nn * 3.0 * s_node + extra;
-      else
-        *bytes = nel_all * 8.0 * m->nnpe + entries * 3.0 * s_f +
-                 m->nn * (3.0 * s_node + 3.0 * s_node) + extra;
-      break;
-    case 1: { // gather + update of a step followed by another: degree, r_e
-              // read, mass, blocked, a/v read+write, u read+write (fused
-              // predictor); the last step of a call also writes f_int.  The
-              // FP32 form reads and writes no a between the steps of a call
-              // (its velocity array holds the half-step velocity), and its
-              // compensation terms
-      const bool f32 = m->precision == AKX_PRECISION_FP32;
-      double per_node = 4.0 + s_node /*M*/ + 1.0 + (m->records_live() ? 3 * s_node : 0.) /*u records*/ +
-                        (f32 ? 0. : 2 * 3 * s_node) /*a*/ + 2 * 3 * s_node /*v*/ +
-                        2 * 3 * s_node /*u*/ + (m->has_fext ? 3 * s_node : 0.);
-      if (f32)
-        per_node += 2 * 2 * 3 * 4.0; // compensation terms read + write
-      *bytes = entries * (3.0 * s_f) + m->nn * (per_node - 3.0);
-      break;
-    }
-    case 2:
-      *bytes = m->nn * (1.0 + 3 * s_node + 2 * 2 * 3 * s_node);
-      break;
-    default:
-      throw Error(AKX_ERR_INVALID, "bad kernel class");
-    }
+    *bytes = kernel_bytes(m, kernel_class);
   });
 }
 

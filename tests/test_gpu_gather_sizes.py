@@ -1,8 +1,9 @@
-"""The gather at the node count where it changes its load order (65,536 nodes:
+"""The gather at the node count where it changes its load order (131,072 nodes:
 the nodal state first and the table entries eight at a time up to there, one
-entry after another above): the FP64 path equals the oracle bit for bit on
-both sides, with nodes of 1 to 24 elements, blocked nodes, an external force
-and a partly filled last slice."""
+entry after another above) and at half of it: the FP64 path equals the oracle
+bit for bit on both sides, with nodes of 1 to 24 elements, blocked nodes, an
+external force and a partly filled last slice; and where a step's bytes no
+longer fit the cache (310 MB) and the table is read with non-temporal loads."""
 import numpy as np
 import pytest
 
@@ -12,9 +13,11 @@ from akantu2_amd import mesh as M
 
 pytestmark = pytest.mark.gpu
 
-# 65,536 and 66,560 nodes; the third Hex8 box (65,533 nodes) has a last slice of 253
-CELLS = {"_tetrahedron_4": [(63, 31, 31), (64, 31, 31)],
-         "_hexahedron_8": [(63, 31, 31), (64, 31, 31), (12, 70, 70)]}
+# 65,536 and 66,560 nodes; the third Hex8 box (65,533 nodes) has a last slice of
+# 253; 131,072 and 133,120 nodes; more than 310 MB a step
+CELLS = {"_tetrahedron_4": [(63, 31, 31), (64, 31, 31), (63, 31, 63), (64, 31, 63), (79, 66, 66)],
+         "_hexahedron_8": [(63, 31, 31), (64, 31, 31), (12, 70, 70), (63, 31, 63), (64, 31, 63),
+                           (79, 62, 62)]}
 
 
 @pytest.mark.parametrize("etype,cells", [(t, c) for t in CELLS for c in CELLS[t]])
