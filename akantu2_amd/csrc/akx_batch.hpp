@@ -24,9 +24,8 @@ struct BInst { // one per instance id
   int32_t law;
   // where the instance's displacement lives: 1 in the {X, u} node records
   // (FP64: its passes read corners from them), 0 in the [3][ncap] array u
-  // (FP32: the Tet4 block pass builds the records in LDS from X and u, the
-  // Hex8 pass reads its corners from them, and the gathers store u whole
-  // instead of half-records)
+  // (FP32: the block passes build the records in LDS from X and u, and the
+  // gathers store u whole instead of half-records)
   int32_t urec;
   int32_t pad;
 };

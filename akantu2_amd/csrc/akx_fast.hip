@@ -15,11 +15,12 @@
 // rounding per evaluation; the FP32 form uses a cancellation-free neo-Hookean
 // stress.
 //
-// Hex8: 8 lanes per element (one per Gauss point; in the last phase one per
-// node), 32 elements per 256-thread block, nodal data and Q in LDS.
+// Hex8: FP32 block passes four lanes per element, two nodes and two Gauss
+// points each; otherwise 8 lanes per element (one per Gauss point; in the last
+// phase one per node), 32 elements per 256-thread block, nodal data and Q in LDS.
 // Tet4: one thread per element (single Gauss point).
-// The same element code serves the batched FP32 form (persistent kernels
-// over the tile list of many instances, per-instance parameters).
+// The same element code serves the batched FP32 form (one tile of one instance
+// per workgroup, per-instance parameters).
 #define AKX_MATH_NS akxf
 #include "akx_args.hpp"
 #include "akx_math.hpp"

@@ -672,8 +672,7 @@ def batch_roofline(etype, law, el, nq):
     outweigh its arithmetic) is priced on HBM; the sum-factorised Hex8 neo-Hookean
     body on FP32 vector issue, with the flops per Gauss point the counters
     saw on the single-model pass that runs the same body."""
-    kernel = (f"k_batch_{'tet4_bpa' if etype == 'tet4' else 'hex8_bpa'}"
-              f"<{'plastic' if law == PL else law}>")
+    kernel = f"k_batch_bpa<{etype}, {'plastic' if law == PL else law}>"
     hbm = {"achieved": el["achieved_gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": el["achieved_gbs"] / HBM_PEAK_GBS}
     if etype == "hex8" and law == "neohookean" and os.path.exists(FLOPS_FILE):
