@@ -68,8 +68,11 @@ __global__ void __launch_bounds__(256) k_batch_tet4(BatchElemArgs A) {
   }
 }
 
+// Elastic: held to four waves per SIMD (127 instead of 130 registers), 241 -> 230
+// us a step of 737,000 elements; the neo-Hookean pass (140) would spill.
 template <int LAW, int EPB>
-__global__ void __launch_bounds__(EPB * 8) k_batch_hex8(BatchElemArgs A) {
+__global__ void __launch_bounds__(EPB * 8, LAW == LAW_ELASTIC ? 4 : 1)
+k_batch_hex8(BatchElemArgs A) {
   __shared__ double sN[EPB][8][6];
   __shared__ double sD[8][3][8];
   const int t = threadIdx.x, el = t >> 3, q = t & 7;
@@ -652,23 +655,26 @@ void upload_inst(akx_batch *b) {
 
 // Elements per tile of a group of n elements whose workgroups walk their tile
 // (groups without block tables).  A shape the caller or the autotuner chose
-// is used as it is.  Otherwise Tet4 takes one element per lane, and Hex8 up
-// to four groups of 32 elements (they run one after another; a workgroup
-// fills the dN/dxi table once), fewer while the CUs would get less than five
-// workgroups each.  Steps of FP64 batches, us, by tile:
-//   Hex8 neo-Hookean     64    128    256    512   2048 (the former tile)
-//     5,700 elements   20.4   30.2   50.2   89.9    331
-//     170,000           110    103    105    145    364
-//     2.1 M            1016   1020   1024   1044   1262
-//   Tet4 plastic, 1.06 M  207  199    187    209    243
-//                 4.5 M   840  793    728    811    868
+// is used as it is.  Otherwise Tet4 takes one element per lane, and Hex8 one
+// wave per workgroup (no barrier is waited for) with one or two rounds of eight
+// elements: two where the chip stays full, since the workgroup's dN/dxi table
+// is then filled once for both.  Steps of FP64 batches, us:
+//   Hex8 neo-Hookean, tile   8    16    32 | 256 lanes: 32   128   2048 (former)
+//     5,000 elements      11.5  15.6  23.4 |          11.7  26.3   331
+//     27,600              24.4  25.2  29.1 |          24.9
+//     73,600                47    49    55 |            48
+//     157,600             89.6  88.5  90.5 |                  94    364
+//     737,000              345   340   343 |                 349
+//   Tet4 plastic, tile     64    128   256   512   2048
+//     1.06 M              207    199   187   209    243
+//     4.5 M               840    793   728   811    868
+constexpr int64_t HEX_TILE_FEW = 100000; // elements up to which a tile is one round
 int64_t group_tile(const akx_batch *b, int etype, int64_t n) {
   if (b->launch_chosen)
     return b->tile;
   if (etype == AKX_TET4)
     return std::min(b->block, b->tile);
-  const int64_t t = n / (5 * (int64_t)b->cus) / 32 * 32;
-  return std::max<int64_t>(32, std::min<int64_t>(t, 128));
+  return n <= HEX_TILE_FEW ? 8 : 16;
 }
 
 // Bytes the element passes (class 0) or the gather (1) of one step cannot do
@@ -807,7 +813,7 @@ template <int LAW> void launch_strict(akx_batch *b, int etype, const BatchElemAr
   dim3 grid((unsigned)A.ntiles);
   if (etype == AKX_TET4)
     hipLaunchKernelGGL(k_batch_tet4<LAW>, grid, dim3(b->block), 0, b->stream, A);
-  else if (b->block == 64)
+  else if (b->block == 64 || !b->launch_chosen) // see group_tile
     hipLaunchKernelGGL((k_batch_hex8<LAW, 8>), grid, dim3(64), 0, b->stream, A);
   else if (b->block == 128)
     hipLaunchKernelGGL((k_batch_hex8<LAW, 16>), grid, dim3(128), 0, b->stream, A);

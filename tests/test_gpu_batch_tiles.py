@@ -1,6 +1,6 @@
 """FP64 batches under the default launch shape: the tile of a group follows
-its element count (32, 64, 96 or 128 Hex8 per workgroup), one tile per
-workgroup, instances whose last tile is ragged.  The arithmetic of an element
+its element count (8 or 16 Hex8 per workgroup, from 100,000 elements on), one
+tile per workgroup, instances whose last tile is ragged.  The arithmetic of an element
 does not depend on its tile, so every instance keeps the bits it has under a
 chosen shape (setLaunch), whose results the other batch tests compare with
 the oracle."""
@@ -11,8 +11,8 @@ from akantu2_amd import mesh as M
 
 pytestmark = pytest.mark.gpu
 
-# cells of the Hex8 instances: few elements (tile 32), then totals about
-# 5 x 256 x 64 and 5 x 256 x 128 elements, with ragged last tiles
+# cells of the Hex8 instances: few elements, then totals on both sides of 100,000
+# elements, with ragged last tiles
 SETS = [[(2, 1, 1)], [(33, 1, 1), (5, 3, 2)], [(43, 43, 45), (7, 3, 2)],
         [(55, 54, 56), (31, 3, 3)]]
 
