@@ -1475,6 +1475,7 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       std::memcpy(&I.dt_crit, &bits_dt, 8);
       I.dt = dt_factor * I.dt_crit;
     } catch (...) {
+      (void)hipStreamSynchronize(b->stream); // host arrays may still be read
       release_ranges(b, I);
       throw;
     }

@@ -89,3 +89,27 @@ def test_one_launch_equals_two(etype, cells, law, precision, order):
                 assert np.linalg.norm(a - b) <= bound * np.linalg.norm(b), (name, k)
     if law == PLASTIC:
         assert one.getEnergy("plastic") == two.getEnergy("plastic") > 0
+
+
+@pytest.mark.parametrize("etype,precision", [(TET, "fp64"), (TET, "fp32"), (HEX, "fp64")])
+def test_nodes_without_elements(etype, precision):
+    """Workgroups that own only nodes without elements (held: their mass is
+    zero) have empty lists."""
+    mesh = M.box_mesh(etype, 4, 3, 2, jitter=0.1, seed=2)
+    lone = np.arange(40)[:, None] * np.ones(3)
+    mesh = dataclasses.replace(mesh, nodes=np.concatenate([lone, mesh.nodes, lone]),
+                               conn=np.ascontiguousarray(mesh.conn + 40, np.int32))
+    held = np.zeros((mesh.nb_nodes, 3), bool)
+    held[:40] = held[-40:] = True
+    out = []
+    for timing in (False, True):
+        m = make(mesh, "elastic", precision, False, timing)
+        m.getBlockedDOFs()[:] = held
+        m.solveSteps(4)
+        out.append([np.array(m.getDisplacement()), np.array(m.getInternalForce())])
+    for a, b, bound in zip(*out, (1e-6, 2e-5)):
+        assert np.isfinite(a).all()
+        if precision == "fp64":
+            assert np.array_equal(a, b)
+        else:
+            assert np.linalg.norm(a - b) <= bound * np.linalg.norm(b)
