@@ -1779,18 +1779,26 @@ void launch_predictor(akx_model *m) {
 //   Tet4 FP64 neo-H.    4,032 13.6/7.5/8.2, 6,630 14.1/9.4/8.5, 10,416
 //                       14.4/12.7/10.5
 //   Tet4 FP64 plastic   525 14.8/7.4/-, 4,032 16/10.3/13.2, 6,975
-//                       16.2/16.2/13.9, 10,416 18.3/-/21.6
+//                       16.2/16.2/13.9, 10,416 18.3/-/21.6; in groups of 16 / 20
+//                       6,630 13.7/14.1, 7,168 13.9/-, 8,192 18.7/14.6 (two
+//                       launches 15.4): two of its workgroups fill a CU, and
+//                       groups of 16 become more than that
 //   Tet4 FP32 elastic   1,152 7.9/5.2/-, 4,032 8.1/5.7/6.7, 10,416 8.4/6.9/7.9,
 //                       26,691 9.5/12.0/12.1
-//   Hex8 FP64 neo-H.    1,331 10.4/7.8/-, 2,520 10.5/10.0/10.4, 4,032
-//                       10.8/12.5/10.8
+//   Hex8 FP64 neo-H.    1,331 9.5/7.8/-, 1,540 9.6/9.9/-, 2,520 9.7/10.0/10.4,
+//                       4,032 10.8/12.5/10.8 (and with the stress at finite
+//                       strain 1,540 9.4/9.4, 2,560 9.2/9.5): a second workgroup
+//                       on a CU, above 256 of them, takes what the launch saved
 //   Hex8 FP64 elastic   1,536 9.1/6.4/-, 2,520 9.2/7.7/8.0, 4,032 9.3/9.3/8.3
 // ---------------------------------------------------------------------------
 constexpr int STEP_RUN_TET4 = 8, STEP_GROUP_TET4 = 16, STEP_RUN_HEX8 = 6;
+constexpr int STEP_GROUP_PLASTIC = 20;
 constexpr int64_t STEP_RUNS_TET4 = 4096; // most nodes in runs (FP64)
-constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_PLASTIC = 8192, STEP_NODES_HEX8 = 2560;
+constexpr int64_t STEP_GROUPS_PLASTIC = 7168; // most in groups of 16 (plastic)
+constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_PLASTIC = 8192;
+constexpr int64_t STEP_NODES_HEX8 = 1536, STEP_NODES_HEX8_ELASTIC = 2560;
 static_assert(STEP_NODES_TET4 <= STEP_NODES_MAX && STEP_NODES_PLASTIC <= STEP_NODES_MAX &&
-                  STEP_NODES_HEX8 <= STEP_NODES_MAX,
+                  STEP_NODES_HEX8 <= STEP_NODES_MAX && STEP_NODES_HEX8_ELASTIC <= STEP_NODES_MAX,
               "larger meshes have no second state arrays");
 constexpr size_t STEP_LDS = 48 * 1024;
 
@@ -1879,7 +1887,10 @@ void plan_small_steps(akx_model *m) {
     return;
   const Material &mat = *m->mats[0];
   const bool f32 = m->precision == AKX_PRECISION_FP32, plastic = mat.law == AKX_LAW_PLASTIC_LIH;
-  if (m->nn > (hex ? STEP_NODES_HEX8 : plastic ? STEP_NODES_PLASTIC : STEP_NODES_TET4))
+  const int64_t most = hex       ? mat.law == AKX_LAW_ELASTIC ? STEP_NODES_HEX8_ELASTIC : STEP_NODES_HEX8
+                       : plastic ? STEP_NODES_PLASTIC
+                                 : STEP_NODES_TET4;
+  if (m->nn > most)
     return;
   if (!mat.contiguous || mat.first != 0 || mat.n != m->nel || mat.n == 0 || mat.user() ||
       (hex && (f32 || plastic)) || (plastic && f32))
@@ -1908,7 +1919,10 @@ void plan_small_steps(akx_model *m) {
   // who owns which nodes
   const int lanes = hex ? STEP_HEX_EPB : 256; // elements at a time
   const bool grouped = !hex && !f32 && nn > STEP_RUNS_TET4;
-  const int own = hex ? STEP_RUN_HEX8 : grouped ? STEP_GROUP_TET4 : STEP_RUN_TET4;
+  const int own = hex                                   ? STEP_RUN_HEX8
+                  : !grouped                            ? STEP_RUN_TET4
+                  : plastic && nn > STEP_GROUPS_PLASTIC ? STEP_GROUP_PLASTIC
+                                                        : STEP_GROUP_TET4;
   StepGroups G;
   group_nodes(m, first, around, own, lanes, grouped, G);
   const auto &[ooff, onodes, eoff, elems, noff, nodes, lcs] = G;

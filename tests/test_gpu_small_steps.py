@@ -17,12 +17,14 @@ pytestmark = pytest.mark.gpu
 TET, HEX = "_tetrahedron_4", "_hexahedron_8"
 # one cell; fewer nodes than a workgroup owns in all; a partly filled last
 # workgroup; Tet4: the largest mesh whose workgroups own runs of nodes (4,096)
-# and one above, with groups in FP64; the largest planned (Tet4 10,240 nodes,
-# plastic 8,192; Hex8 2,560) and ones above
+# and one above, with groups in FP64 (plastic: of 16 nodes to 7,168, then 20);
+# the largest planned (Tet4 10,240 nodes, plastic 8,192; Hex8 1,536, elastic
+# 2,560) and ones above
 CELLS = {TET: [(1, 1, 1), (3, 2, 2), (20, 4, 4), (15, 15, 15), (16, 15, 15)],
-         HEX: [(1, 1, 1), (4, 1, 2), (10, 10, 10), (19, 15, 7), (20, 15, 7)]}
+         HEX: [(1, 1, 1), (4, 1, 2), (10, 10, 10), (15, 11, 7), (16, 11, 7), (19, 15, 7),
+               (20, 15, 7)]}
 LARGEST = [(39, 15, 15), (40, 15, 15)]
-LARGEST_PLASTIC = [(31, 15, 15), (32, 15, 15)]
+LARGEST_PLASTIC = [(27, 15, 15), (28, 15, 15), (31, 15, 15), (32, 15, 15)]
 
 
 def shuffled(mesh, seed):
