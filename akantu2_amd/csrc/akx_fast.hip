@@ -1111,6 +1111,40 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepAr
   dof.update<true>(S, s_slot, s_run);
 }
 
+// The same for FP32 Hex8: four lanes per element (hex8_quad); a workgroup's 8
+// nodes have at most 64 elements around them.
+template <int LAW> __global__ void __launch_bounds__(256) k_hex8_step_f32(StepArgs S) {
+  extern __shared__ double2 s_rec[]; // records, then slots, then the runs' ends
+  const int64_t b = xcd_block(S.nblocks_padded);
+  if (b >= S.nblocks) // padding block
+    return;
+  const int t = threadIdx.x, q = t & 3;
+  float *s_slot = reinterpret_cast<float *>(s_rec + 3 * S.max_nodes);
+  uint8_t *s_run = reinterpret_cast<uint8_t *>(s_slot + 3 * (S.max_slots + 1));
+  const bool active = (t >> 2) < S.max_elems;
+  const int64_t i = b * S.max_elems + (active ? t >> 2 : S.max_elems - 1);
+  const uint32_t lc = reinterpret_cast<const uint32_t *>(S.lc + i * 8)[q];
+  const uint32_t ls = reinterpret_cast<const uint32_t *>(S.ls + i * 8)[q];
+  double lambda = S.lambda, mu = S.mu;
+  if (S.lm_f) {
+    const float2 lm = S.lm_f[S.lelem[i] & ~akx::STEP_GUEST];
+    lambda = lm.x;
+    mu = lm.y;
+  }
+  StepDof<true> dof;
+  dof.load(S, b);
+  for (int k = t; k < S.max_slots; k += blockDim.x)
+    s_run[k] = S.run[b * S.max_slots + k];
+  step_stage<true>(S, b, s_rec);
+  __syncthreads();
+  if (active)
+    hex8_quad<LAW>(q, lc, ls, akx::NodesLDS{reinterpret_cast<const double *>(s_rec)},
+                   lame_quad(lambda, mu, q), float(lambda), float(mu), QpViewT<double>{}, 0,
+                   s_slot);
+  __syncthreads();
+  dof.update<true>(S, s_slot, s_run);
+}
+
 // ---------------------------------------------------------------------------
 // Batched FP32 form (block-partial assembly): one tile, which is one block, of
 // one instance per workgroup; per-instance parameters, compact FP32 plastic
@@ -1342,20 +1376,23 @@ hipError_t launch_elements(int etype, int law, bool fp32, const ElemArgs &A,
               : launch_t<double, double>(etype, law, A, stream);
 }
 
-hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream) {
-  const dim3 grid((unsigned)S.nblocks_padded), block((unsigned)(S.max_elems + 63) / 64 * 64);
+template <int LAW>
+static void launch_step_law(int etype, const akx::StepArgs &S, size_t lds, hipStream_t s) {
+  const dim3 grid((unsigned)S.nblocks_padded);
+  const int lanes = (etype == 0 ? 1 : 4) * S.max_elems;
+  const dim3 block((unsigned)(lanes + 63) / 64 * 64);
+  if (etype == 0)
+    hipLaunchKernelGGL(k_tet4_step_f32<LAW>, grid, block, lds, s, S);
+  else
+    hipLaunchKernelGGL(k_hex8_step_f32<LAW>, grid, block, lds, s, S);
+}
+
+hipError_t launch_step(int etype, int law, const akx::StepArgs &S, size_t lds, hipStream_t stream) {
   switch (law) {
-  case LAW_ELASTIC:
-    hipLaunchKernelGGL(k_tet4_step_f32<LAW_ELASTIC>, grid, block, lds, stream, S);
-    break;
-  case LAW_ELASTIC_FD:
-    hipLaunchKernelGGL(k_tet4_step_f32<LAW_ELASTIC_FD>, grid, block, lds, stream, S);
-    break;
-  case LAW_NEOHOOKEAN:
-    hipLaunchKernelGGL(k_tet4_step_f32<LAW_NEOHOOKEAN>, grid, block, lds, stream, S);
-    break;
-  default:
-    return hipErrorInvalidValue;
+  case LAW_ELASTIC: launch_step_law<LAW_ELASTIC>(etype, S, lds, stream); break;
+  case LAW_ELASTIC_FD: launch_step_law<LAW_ELASTIC_FD>(etype, S, lds, stream); break;
+  case LAW_NEOHOOKEAN: launch_step_law<LAW_NEOHOOKEAN>(etype, S, lds, stream); break;
+  default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }

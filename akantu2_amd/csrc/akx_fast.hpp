@@ -15,7 +15,7 @@ int64_t elements_per_block(int etype, bool bpa = false);
 hipError_t launch_elements(int etype, int law, bool fp32, const akx::ElemArgs &A,
                            hipStream_t stream);
 // launch one step of a small FP32 Tet4 model (akx_step.hpp)
-hipError_t launch_tet4_step(int law, const akx::StepArgs &S, size_t lds, hipStream_t stream);
+hipError_t launch_step(int etype, int law, const akx::StepArgs &S, size_t lds, hipStream_t stream);
 // launch the FP32-form batched element pass (block-partial assembly) of one
 // (element type, law) group, or of all groups: the Tet4 and the Hex8 tiles
 hipError_t launch_batch_elements_f32(int etype, int law, const akx::BatchElemArgs &A,

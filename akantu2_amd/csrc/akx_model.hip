@@ -744,7 +744,7 @@ struct Material {
 };
 
 // meshes of up to this many nodes hold u, v and a twice
-constexpr int64_t STEP_NODES_MAX = 10240;
+constexpr int64_t STEP_NODES_MAX = 12288;
 // doubles or floats from one [3][nn] array of the state to the next
 inline int64_t state_stride(int64_t nn) { return (3 * nn + 31) / 32 * 32; }
 
@@ -1759,7 +1759,7 @@ void launch_predictor(akx_model *m) {
 // ---------------------------------------------------------------------------
 // One launch per step for small models (akx_step.hpp): one contiguous material
 // of a built-in law over the whole mesh; Tet4 in FP64 (with plasticity) and
-// FP32, Hex8 in FP64.
+// FP32, Hex8 in FP64 and FP32 (block partials).
 //
 // A step of two launches takes 8 to 16 us however small the mesh; in one
 // launch it takes 5 (plastic 7.5), what the host needs to queue it.  An
@@ -1767,13 +1767,14 @@ void launch_predictor(akx_model *m) {
 // nodes, so the gain ends where that fills the chip.
 //
 // A workgroup owns a run of 8 nodes (Tet4; along a row of a box they have 150
-// elements, one a lane) or 6 (Hex8; 28 elements of eight lanes).  In runs a
-// Tet4 is computed 3.1 times, a Hex8 4.6 times.  Groups of up to 16
-// neighbouring nodes (group_nodes) take that to 2.3 for Tet4, with a longer sum
-// per lane: they pay in FP64 where the runs need more than two workgroups per
-// CU.  (Hex8 in groups of 8: 4.1; no faster up to 2,560 nodes.)  The lists cost
-// initFull 0.1 ms at 1,000 nodes, 1.5 ms at 7,000.  us a step of boxes, two
-// launches / runs / groups:
+// elements, one a lane), 6 (FP64 Hex8; 28 elements of eight lanes) or up to 16
+// (FP32 Hex8; 64 elements of four lanes).  In runs a Tet4 is computed 3.1
+// times, a Hex8 4.6 times.  Groups of up to 16 neighbouring nodes (group_nodes)
+// take that to 2.3 for Tet4, with a longer sum per lane: they pay in FP64 where
+// the runs need more than two workgroups per CU.  (Hex8 in groups of 8: 4.1; no
+// faster in FP64 up to 2,560 nodes, 1 us slower in FP32.)  The lists cost
+// initFull 0.1 ms at 1,000 nodes, 1.5 ms at 7,000 (FP32 Hex8 1.1 at 11,000).
+// us a step of boxes, two launches / runs / groups:
 //   Tet4 FP64 elastic   525 nodes 12.0/5.1/-, 4,032 12.5/5.9/6.7, 10,416
 //                       13.6/9.3/8.1
 //   Tet4 FP64 neo-H.    4,032 13.6/7.5/8.2, 6,630 14.1/9.4/8.5, 10,416
@@ -1789,16 +1790,24 @@ void launch_predictor(akx_model *m) {
 //                       4,032 10.8/12.5/10.8 (and with the stress at finite
 //                       strain 1,540 9.4/9.4, 2,560 9.2/9.5): a second workgroup
 //                       on a CU, above 256 of them, takes what the launch saved
+//   Hex8 FP32 neo-H.    runs of 8 / 12 / 16 nodes: 343 8.7/5.7/-/-, 1,331
+//                       9.1/5.8/5.6/5.6, 4,096 9.1/6.6/6.7/5.6, 8,192
+//                       9.6/8.1/8.0/6.8, 11,200 9.2/-/8.9/8.0, 15,972
+//                       9.3/-/11.3/9.1 (a numbering without locality makes more
+//                       and fuller workgroups: the limit of 1,024)
+//   Hex8 FP32 elastic   4,352 8.8/-/6.3/6.1, 14,801 9.5/-/8.7/8.1
 //   Hex8 FP64 elastic   1,536 9.1/6.4/-, 2,520 9.2/7.7/8.0, 4,032 9.3/9.3/8.3
 // ---------------------------------------------------------------------------
-constexpr int STEP_RUN_TET4 = 8, STEP_GROUP_TET4 = 16, STEP_RUN_HEX8 = 6;
+constexpr int STEP_RUN_TET4 = 8, STEP_GROUP_TET4 = 16, STEP_RUN_HEX8 = 6, STEP_RUN_HEX8_F32 = 16;
 constexpr int STEP_GROUP_PLASTIC = 20;
 constexpr int64_t STEP_RUNS_TET4 = 4096; // most nodes in runs (FP64)
 constexpr int64_t STEP_GROUPS_PLASTIC = 7168; // most in groups of 16 (plastic)
 constexpr int64_t STEP_NODES_TET4 = 10240, STEP_NODES_PLASTIC = 8192;
 constexpr int64_t STEP_NODES_HEX8 = 1536, STEP_NODES_HEX8_ELASTIC = 2560;
+constexpr int64_t STEP_NODES_HEX8_F32 = 12288, STEP_GROUPS_HEX8_F32 = 1024;
 static_assert(STEP_NODES_TET4 <= STEP_NODES_MAX && STEP_NODES_PLASTIC <= STEP_NODES_MAX &&
-                  STEP_NODES_HEX8 <= STEP_NODES_MAX && STEP_NODES_HEX8_ELASTIC <= STEP_NODES_MAX,
+                  STEP_NODES_HEX8 <= STEP_NODES_MAX && STEP_NODES_HEX8_ELASTIC <= STEP_NODES_MAX &&
+                  STEP_NODES_HEX8_F32 <= STEP_NODES_MAX,
               "larger meshes have no second state arrays");
 constexpr size_t STEP_LDS = 48 * 1024;
 
@@ -1810,10 +1819,10 @@ struct StepGroups {
   std::vector<uint16_t> lcs;
 };
 
-// grow: a group starts at the lowest node left and takes, up to `own` nodes and
-// max_elems elements, the node of its elements that adds the fewest elements;
-// else the groups are runs of `own` nodes.  first, around: the elements around
-// every node.
+// Groups of up to `own` nodes with up to max_elems elements around them (one
+// node may have more).  grow: a group starts at the lowest node left and takes
+// the node of its elements that adds the fewest; else the groups are runs.
+// first, around: the elements around every node.
 void group_nodes(const akx_model *m, const std::vector<int32_t> &first,
                  const std::vector<int32_t> &around, int own, int max_elems, bool grow,
                  StepGroups &G) {
@@ -1821,7 +1830,11 @@ void group_nodes(const akx_model *m, const std::vector<int32_t> &first,
   const int32_t *conn = m->conn_host.data();
   const int32_t nn = (int32_t)m->nn;
   constexpr int16_t TAKEN = INT16_MAX / 2; // no node has that many elements
-  std::vector<int32_t> elem_in(m->nel, -1), node_in(nn, -1), node_no(nn);
+  std::vector<int32_t> elem_in(m->nel, -1);
+  struct Met {
+    int32_t in, no; // a node's latest group and its number there
+  };
+  std::vector<Met> met_in(nn, Met{-1, 0});
   std::vector<int16_t> more(256); // elements that each of the group's nodes would add
   std::vector<uint8_t> taken(nn, 0);
   G.onodes.reserve(nn);
@@ -1836,41 +1849,49 @@ void group_nodes(const akx_model *m, const std::vector<int32_t> &first,
     for (int32_t n = start;;) {
       taken[n] = 1;
       G.onodes.push_back(n);
-      if (node_in[n] == b)
-        more[node_no[n]] = TAKEN;
+      if (met_in[n].in == b)
+        more[met_in[n].no] = TAKEN;
+      const size_t most = G.lcs.size() + (size_t)(first[n + 1] - first[n]) * nnpe;
+      if (most > G.lcs.capacity())
+        G.lcs.reserve(2 * most);
+      if (more.size() < (size_t)met + (most - G.lcs.size()))
+        more.resize(2 * (met + (most - G.lcs.size())));
       for (int32_t d = first[n]; d < first[n + 1]; ++d) {
         const int32_t e = around[d];
         if (elem_in[e] == b)
           continue;
         elem_in[e] = b;
         G.elems.push_back(e);
-        const size_t at = G.lcs.size();
-        G.lcs.resize(at + nnpe);
+        uint16_t lc[8];
         for (int a = 0; a < nnpe; ++a) {
           const int32_t c = conn[(int64_t)e * nnpe + a];
-          if (node_in[c] != b) {
-            node_in[c] = b;
-            node_no[c] = met;
+          Met &at = met_in[c];
+          if (at.in != b) {
+            at = Met{b, met};
             G.nodes.push_back(c);
-            if ((size_t)met == more.size())
-              more.resize(2 * met);
-            more[met++] = taken[c] ? TAKEN : (int16_t)(first[c + 1] - first[c]);
+            if (grow)
+              more[met] = taken[c] ? TAKEN : (int16_t)(first[c + 1] - first[c]);
+            ++met;
           }
-          more[node_no[c]]--;
-          G.lcs[at + a] = (uint16_t)node_no[c];
+          if (grow)
+            more[at.no]--;
+          lc[a] = (uint16_t)at.no;
         }
+        G.lcs.insert(G.lcs.end(), lc, lc + nnpe);
       }
       if ((int)G.onodes.size() - G.ooff[b] == own)
         break;
+      const int32_t left = max_elems - ((int32_t)G.elems.size() - G.eoff[b]);
       if (!grow) {
-        if (++n == nn)
+        if (++n == nn || std::count_if(around.begin() + first[n], around.begin() + first[n + 1],
+                                       [&](int32_t e) { return elem_in[e] != b; }) > left)
           break;
         continue;
       }
       int16_t fewest = TAKEN / 2;
       for (int32_t k = 0; k < met; ++k)
         fewest = std::min(fewest, more[k]);
-      if (fewest == TAKEN / 2 || fewest > max_elems - ((int32_t)G.elems.size() - G.eoff[b]))
+      if (fewest == TAKEN / 2 || fewest > left)
         break;
       n = G.nodes[n0 + (std::find(more.begin(), more.end(), fewest) - more.begin())];
     }
@@ -1887,13 +1908,14 @@ void plan_small_steps(akx_model *m) {
     return;
   const Material &mat = *m->mats[0];
   const bool f32 = m->precision == AKX_PRECISION_FP32, plastic = mat.law == AKX_LAW_PLASTIC_LIH;
-  const int64_t most = hex       ? mat.law == AKX_LAW_ELASTIC ? STEP_NODES_HEX8_ELASTIC : STEP_NODES_HEX8
-                       : plastic ? STEP_NODES_PLASTIC
-                                 : STEP_NODES_TET4;
+  const int64_t most_hex = f32                          ? STEP_NODES_HEX8_F32
+                           : mat.law == AKX_LAW_ELASTIC ? STEP_NODES_HEX8_ELASTIC
+                                                        : STEP_NODES_HEX8;
+  const int64_t most = hex ? most_hex : plastic ? STEP_NODES_PLASTIC : STEP_NODES_TET4;
   if (m->nn > most)
     return;
   if (!mat.contiguous || mat.first != 0 || mat.n != m->nel || mat.n == 0 || mat.user() ||
-      (hex && (f32 || plastic)) || (plastic && f32))
+      (plastic && (hex || f32)) || (hex && f32 && !m->bpa))
     return;
   if (!f32 && m->ppa && m->assembly == AKX_ASSEMBLY_BLOCK_PARTIALS)
     return; // sums runs in FP64 without rounding them as the FP32 form does
@@ -1917,16 +1939,18 @@ void plan_small_steps(akx_model *m) {
       }
   }
   // who owns which nodes
-  const int lanes = hex ? STEP_HEX_EPB : 256; // elements at a time
+  const int lanes = !hex ? 256 : f32 ? 64 : STEP_HEX_EPB; // elements at a time
   const bool grouped = !hex && !f32 && nn > STEP_RUNS_TET4;
-  const int own = hex                                   ? STEP_RUN_HEX8
+  const int own = hex                                   ? f32 ? STEP_RUN_HEX8_F32 : STEP_RUN_HEX8
                   : !grouped                            ? STEP_RUN_TET4
                   : plastic && nn > STEP_GROUPS_PLASTIC ? STEP_GROUP_PLASTIC
                                                         : STEP_GROUP_TET4;
   StepGroups G;
-  group_nodes(m, first, around, own, lanes, grouped, G);
+  group_nodes(m, first, around, own, hex && !f32 ? 2 * lanes : lanes, grouped, G);
   const auto &[ooff, onodes, eoff, elems, noff, nodes, lcs] = G;
   const int64_t nb = (int64_t)ooff.size() - 1;
+  if (hex && f32 && nb > STEP_GROUPS_HEX8_F32)
+    return;
   std::vector<int32_t> owner(nn), slot0(nn);
   int32_t max_elems = 1, max_nodes = 1, max_slots = 1;
   for (int64_t b = 0; b < nb; ++b) {
@@ -1945,15 +1969,16 @@ void plan_small_steps(akx_model *m) {
                      (f32 ? max_slots : 0);
   // one lane per Tet4; at most two rounds of Hex8 (a numbering without
   // locality makes long lists)
-  if (max_elems > (hex ? 2 : 1) * lanes || lds > STEP_LDS)
+  if (max_elems > (hex && !f32 ? 2 : 1) * lanes || lds > STEP_LDS)
     return;
-  // FP32 partial sums end where the element pass's block of 256 elements does
+  // FP32 partial sums end where the element pass's block of elements does
   // (every corner is one without block assembly)
+  const int32_t block = (int32_t)akxf::elements_per_block(m->etype, true);
   std::vector<uint8_t> ends(f32 ? around.size() : 0, 1);
   if (f32 && m->bpa)
     for (int64_t n = 0; n < nn; ++n)
       for (int32_t d = first[n]; d + 1 < first[n + 1]; ++d)
-        ends[d] = around[d] / 256 != around[d + 1] / 256;
+        ends[d] = around[d] / block != around[d + 1] / block;
   // the lists, by k_step_lists from what was found here; the upload sits in the
   // force table, which nothing uses yet
   StepArgs S{};
@@ -2087,9 +2112,9 @@ void launch_small_step(akx_model *m, bool first, bool last) {
           "small-model step launched without compensation terms");
   require(!S.lam_el == !S.mu_el && (!f32 || !S.lam_el == !S.lm_f),
           "per-element parameters incomplete");
-  require(m->etype != AKX_HEX8 || S.jw, "Hex8 step launched without its jacobian table");
+  require(m->etype != AKX_HEX8 || f32 || S.jw, "Hex8 step launched without its jacobian table");
   if (f32)
-    HIPCHECK(akxf::launch_tet4_step(mat.law, S, m->step_lds, m->stream));
+    HIPCHECK(akxf::launch_step(m->etype, mat.law, S, m->step_lds, m->stream));
   else if (mat.law == AKX_LAW_ELASTIC)
     launch_step_law<LAW_ELASTIC>(m, S);
   else if (mat.law == AKX_LAW_ELASTIC_FD)

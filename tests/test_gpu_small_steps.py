@@ -19,12 +19,13 @@ TET, HEX = "_tetrahedron_4", "_hexahedron_8"
 # workgroup; Tet4: the largest mesh whose workgroups own runs of nodes (4,096)
 # and one above, with groups in FP64 (plastic: of 16 nodes to 7,168, then 20);
 # the largest planned (Tet4 10,240 nodes, plastic 8,192; Hex8 1,536, elastic
-# 2,560) and ones above
+# 2,560, FP32 12,288) and ones above
 CELLS = {TET: [(1, 1, 1), (3, 2, 2), (20, 4, 4), (15, 15, 15), (16, 15, 15)],
          HEX: [(1, 1, 1), (4, 1, 2), (10, 10, 10), (15, 11, 7), (16, 11, 7), (19, 15, 7),
                (20, 15, 7)]}
 LARGEST = [(39, 15, 15), (40, 15, 15)]
 LARGEST_PLASTIC = [(27, 15, 15), (28, 15, 15), (31, 15, 15), (32, 15, 15)]
+LARGEST_HEX32 = [(15, 15, 15), (47, 15, 15), (48, 15, 15)]
 
 
 def shuffled(mesh, seed):
@@ -58,9 +59,10 @@ LAWS = ("elastic", "neohookean")
 FORMS = [(TET, c, law, p) for c in CELLS[TET] + LARGEST for law in LAWS
          for p in ("fp64", "fp32")]
 FORMS += [(TET, c, PLASTIC, "fp64") for c in CELLS[TET] + LARGEST_PLASTIC]
-FORMS += [(HEX, c, law, "fp64") for c in CELLS[HEX] for law in LAWS]
+FORMS += [(HEX, c, law, p) for c in CELLS[HEX] + LARGEST_HEX32 for law in LAWS
+          for p in ("fp64", "fp32")]
 FORMS += [(TET, (5, 4, 4), "elastic_fd", "fp64"), (TET, (5, 4, 4), "elastic_fd", "fp32"),
-          (HEX, (5, 4, 4), "elastic_fd", "fp64")]
+          (HEX, (5, 4, 4), "elastic_fd", "fp64"), (HEX, (5, 4, 4), "elastic_fd", "fp32")]
 
 
 @pytest.mark.parametrize("order", ["grid", "random"])
