@@ -1111,8 +1111,11 @@ template <int LAW> __global__ void __launch_bounds__(256) k_tet4_step_f32(StepAr
   dof.update<true>(S, s_slot, s_run);
 }
 
-// The same for FP32 Hex8: four lanes per element (hex8_quad); a workgroup's 8
-// nodes have at most 64 elements around them.
+// The same for FP32 Hex8: four lanes per element (hex8_quad) of the up to 64
+// around a workgroup's run of nodes.  Up to some 4,000 nodes the host's queueing
+// and the load chain (lists, records, state) bound it, above the element code,
+// done 3.5 to 4.3 times.  us a step of neo-Hookean boxes against
+// two launches: 1,331 nodes 9.1 -> 5.6, 8,192 9.6 -> 6.8, 11,200 9.2 -> 8.0.
 template <int LAW> __global__ void __launch_bounds__(256) k_hex8_step_f32(StepArgs S) {
   extern __shared__ double2 s_rec[]; // records, then slots, then the runs' ends
   const int64_t b = xcd_block(S.nblocks_padded);

@@ -1769,7 +1769,7 @@ void launch_predictor(akx_model *m) {
 // A workgroup owns a run of 8 nodes (Tet4; along a row of a box they have 150
 // elements, one a lane), 6 (FP64 Hex8; 28 elements of eight lanes) or up to 16
 // (FP32 Hex8; 64 elements of four lanes).  In runs a Tet4 is computed 3.1
-// times, a Hex8 4.6 times.  Groups of up to 16 neighbouring nodes (group_nodes)
+// times, a Hex8 4.6 (FP32 4.1) times.  Groups of up to 16 neighbours (group_nodes)
 // take that to 2.3 for Tet4, with a longer sum per lane: they pay in FP64 where
 // the runs need more than two workgroups per CU.  (Hex8 in groups of 8: 4.1; no
 // faster in FP64 up to 2,560 nodes, 1 us slower in FP32.)  The lists cost
