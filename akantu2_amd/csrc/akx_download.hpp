@@ -30,7 +30,7 @@
 namespace akx {
 
 // Threads that help with copies, for the whole process: at most seven, started
-// when work is there and none is idle, gone after two idle seconds.  Waiting
+// when more work is there than threads are idle, gone after two idle seconds.  Waiting
 // threads are scheduled at once when they are woken; a new thread waits a
 // scheduler's slice (3 ms) where the CPUs are busy, as they are for a while
 // after an OpenMP loop.  Never destroyed: a thread may wait in it at exit.
@@ -70,7 +70,7 @@ public:
     std::lock_guard<std::mutex> lock(mutex);
     for (int k = 0; k < copies; ++k)
       queue.push_back(f);
-    while (threads < MOST && (int)queue.size() > threads) {
+    for (int more = (int)queue.size() - idle; more > 0 && threads < MOST; --more) {
       std::thread([this] { loop(); }).detach();
       ++threads;
     }
@@ -83,30 +83,47 @@ public:
 // that has not been scheduled yet is not waited for, and finds nothing to
 // claim when it is.
 struct ChunkJob {
-  std::atomic<int64_t> next{0}, done{0}, skipped{0};
+  std::atomic<int64_t> next{0}, done{0};
   int64_t n = 0;
   std::mutex mutex;
   std::exception_ptr error;
 
-  int64_t claim() {
-    const int64_t c = next.fetch_add(1);
-    return c < n ? c : -1;
-  }
-  void finish() { done.fetch_add(1); }
-  void fail(std::exception_ptr e) { // no further chunk is claimed
+  // the error, then what it leaves undone: the caller returns once that is
+  // counted.  No further chunk is claimed.
+  void fail(std::exception_ptr e, int64_t open) {
     {
       std::lock_guard<std::mutex> lock(mutex);
       if (!error)
         error = e;
     }
     const int64_t c = next.exchange(n);
-    if (c < n) // the caller may return once these are counted
-      skipped.fetch_add(n - c);
+    done.fetch_add(open + (c < n ? n - c : 0));
   }
 };
 
-// work(job) claims and finishes chunks until none is left; it finishes what it
-// claimed also when it throws
+// One thread's chunks: those it has claimed and not finished are its own to
+// finish, or to give up by throwing
+class Claims {
+  ChunkJob &job;
+  int64_t open = 0;
+
+public:
+  explicit Claims(ChunkJob &j) : job(j) {}
+  int64_t claim() { // -1: none left
+    const int64_t c = job.next.fetch_add(1);
+    if (c >= job.n)
+      return -1;
+    ++open;
+    return c;
+  }
+  void finish() { // the caller may return: nothing of its is touched after the last
+    --open;
+    job.done.fetch_add(1);
+  }
+  void fail(std::exception_ptr e) { job.fail(e, open); }
+};
+
+// work(claims, c) does chunk c and claims and does others until none is left
 template <class F> void run_chunks(int threads, int64_t n, const F &work) {
   auto job = std::make_shared<ChunkJob>();
   job->n = n;
@@ -114,13 +131,14 @@ template <class F> void run_chunks(int threads, int64_t n, const F &work) {
   // through it: work itself is run by a thread that has claimed a chunk
   std::shared_ptr<const F *> body = std::make_shared<const F *>(&work);
   auto loop = [job, body] {
-    const int64_t c = job->claim();
+    Claims claims(*job);
+    const int64_t c = claims.claim();
     if (c < 0)
       return; // the caller may have returned: work is not touched
     try {
-      (**body)(*job, c);
+      (**body)(claims, c);
     } catch (...) {
-      job->fail(std::current_exception());
+      claims.fail(std::current_exception());
     }
   };
   if (threads > 1)
@@ -129,7 +147,7 @@ template <class F> void run_chunks(int threads, int64_t n, const F &work) {
     } catch (...) { // no thread to be had: their share is done here
     }
   loop();
-  while (job->done.load() + job->skipped.load() < n)
+  while (job->done.load() < n)
     std::this_thread::yield();
   std::lock_guard<std::mutex> lock(job->mutex);
   if (job->error)
@@ -154,14 +172,14 @@ inline bool host_differs(const void *a, const void *b, size_t bytes) {
     return std::memcmp(a, b, bytes) != 0;
   std::atomic<bool> differ{false};
   run_chunks(T, (int64_t)((bytes + COPY_CHUNK - 1) / COPY_CHUNK),
-             [&](ChunkJob &job, int64_t c) {
-               for (; c >= 0; c = job.claim()) {
+             [&](Claims &claims, int64_t c) {
+               for (; c >= 0; c = claims.claim()) {
                  const size_t o = (size_t)c * COPY_CHUNK;
                  if (!differ.load(std::memory_order_relaxed) &&
                      std::memcmp((const char *)a + o, (const char *)b + o,
                                  std::min(COPY_CHUNK, bytes - o)) != 0)
                    differ = true;
-                 job.finish();
+                 claims.finish();
                }
              });
   return differ;
@@ -218,6 +236,16 @@ public:
   // the second copy 9.1 -> 1.6 ms (arrays used before; the comparison of two
   // such pairs at the next call 4.4 -> 1.7 ms).
   void get(int device, hipStream_t stream, std::vector<Field> &fields) {
+    try {
+      deliver(device, stream, fields);
+    } catch (...) { // kernels that were launched still write the buffers
+      (void)hipStreamSynchronize(stream);
+      throw;
+    }
+  }
+
+private:
+  void deliver(int device, hipStream_t stream, std::vector<Field> &fields) {
     size_t total = 0;
     for (auto &f : fields)
       total += (f.bytes() + 63) / 64 * 64;
@@ -275,36 +303,20 @@ public:
       events.push_back(e);
     }
     std::atomic<int> workers{0};
-    run_chunks(T, (int64_t)chunks.size(), [&](ChunkJob &job, int64_t c) {
-      // the thread's chunks in flight: claimed, the kernel launched.  After
-      // its last finish() it touches nothing of the caller's.
+    run_chunks(T, (int64_t)chunks.size(), [&](Claims &claims, int64_t c) {
+      // the thread's chunks in flight: claimed, the kernel launched
       const int w = workers.fetch_add(1);
       struct Flight {
         hipEvent_t ev;
         int64_t c;
       } fl[2] = {{events[2 * w], -1}, {events[2 * w + 1], -1}};
       unsigned char *slots = pin + (size_t)w * 2 * COPY_CHUNK;
-      struct Finish { // on every way out: what was claimed is finished
-        ChunkJob &job;
-        Flight (&fl)[2];
-        int64_t &c;
-        ~Finish() {
-          for (Flight &f : fl)
-            if (f.c >= 0) {
-              (void)hipEventSynchronize(f.ev); // its kernel writes the slot
-              job.finish();
-            }
-          if (c >= 0)
-            job.finish();
-        }
-      } finish{job, fl, c};
       HIPCHECK(hipSetDevice(device));
       for (int k = 0;; k ^= 1) {
         if (c >= 0) {
           chunks[c].f->pack(slots + k * COPY_CHUNK, chunks[c].first, chunks[c].count);
           HIPCHECK(hipEventRecord(fl[k].ev, stream));
           fl[k].c = c;
-          c = -1;
         }
         Flight &o = fl[k ^ 1]; // the one before
         if (o.c >= 0) {
@@ -316,9 +328,9 @@ public:
           if (h.f->copy)
             std::memcpy((char *)h.f->copy + at, slot, b);
           o.c = -1;
-          job.finish();
+          claims.finish();
         }
-        c = job.claim();
+        c = claims.claim();
         if (c < 0 && fl[0].c < 0 && fl[1].c < 0)
           break;
       }
