@@ -3,8 +3,11 @@
 ``build_library()`` compiles ``csrc/*.hip`` into
 ``akantu2_amd/libakantu_mi355x.so`` for gfx950.  Flags:
 - ``-ffp-contract=off``: the FP64 plain path keeps the reference's separate
-  rounding of every multiply and add (the FP32 form opts back into
-  contraction inside its own code);
+  rounding of every multiply and add.  The FP32 form and the regrouped FP64 form
+  are built with ``on``: a product is fused into a sum where the source has both
+  in one expression, and nowhere else, so an element function rounds alike in
+  every kernel that it is compiled into (``fast`` leaves that to the optimiser,
+  kernel by kernel, and an instance's bits to the launch its batch takes);
 - ``-Xclang -target-feature -Xclang -packed-fp32-ops``: no packed FP32
   instructions.
 """
@@ -19,7 +22,7 @@ LIB = os.path.join(HERE, "libakantu_mi355x.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 # source -> floating-point contraction of its translation unit
-SOURCES = {"akx_model.hip": "off", "akx_fast.hip": "fast", "akx_batch.hip": "off"}
+SOURCES = {"akx_model.hip": "off", "akx_fast.hip": "on", "akx_batch.hip": "off"}
 FLAGS = ["-O3", "-std=c++17", "--offload-arch=gfx950", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wall", "-Wno-unused-function", "-Wno-unused-variable"]

@@ -1,6 +1,9 @@
 // akx_fast.hip -- regrouped element pass of the FP32 precision form and of
-// the opt-in FP64 "fast" form.  Compiled with -ffp-contract=fast (FMA), in
-// its own translation unit and math namespace.
+// the opt-in FP64 "fast" form.  Compiled with -ffp-contract=on, in its own
+// translation unit and math namespace: a product is fused into the sum that is
+// written in the same expression, so every kernel that an element function is
+// part of gives the same bits (the launches of a batch's groups and the one of
+// all, one-launch and two-launch steps).
 //
 // Same mechanics as the reference (material.cc:98-154 + 457-584): gather u,
 // grad u at every Gauss point, constitutive law, B^T sigma (small strain) or
@@ -169,10 +172,10 @@ __device__ __forceinline__ void law_at(const VT &V, int64_t iq, CT lambda,
     for (int k = 0; k < 3; ++k)
 #pragma unroll
       for (int J = 0; J < 3; ++J) {
-        CT s = CT(0);
+        CT s = S[k][J]; // F S = S + grad u S
 #pragma unroll
         for (int m = 0; m < 3; ++m)
-          s += ((k == m ? CT(1) : CT(0)) + g[k][m]) * S[m][J];
+          s += g[k][m] * S[m][J];
         P[k][J] = s;
       }
   } else {
@@ -531,7 +534,7 @@ __device__ __forceinline__ double quad_first(double v) {
 }
 
 // One component's node values (v0 at x-, v1 at x+ of the lane's edge) ->
-// d/dxi and the parts of d/deta = e0 +- e1 and d/dzeta = z0 +- z1.
+// d/dxi and the parts of d/deta = e0 +- KD e1 and d/dzeta = z0 +- KD z1.
 __device__ __forceinline__ void quad_grad(float v0, float v1, float &dxi, float &e0, float &e1,
                                           float &z0, float &z1) {
   const float d = v1 - v0, s = HEX_KS * (v0 + v1);
@@ -541,9 +544,9 @@ __device__ __forceinline__ void quad_grad(float v0, float v1, float &dxi, float 
   const float ip = quad_x1(izd);
   dxi = izd + HEX_R * ip;
   e0 = izs - quad_x1(izs);
-  e1 = HEX_KD * (izd - ip);
+  e1 = izd - ip;
   z0 = dzs + HEX_R * quad_x1(dzs);
-  z1 = HEX_KD * (dzd + HEX_R * quad_x1(dzd));
+  z1 = dzd + HEX_R * quad_x1(dzd);
 }
 
 // The transposed steps: one force component of the lane's nodes from the
@@ -551,10 +554,11 @@ __device__ __forceinline__ void quad_grad(float v0, float v1, float &dxi, float 
 __device__ __forceinline__ void quad_force(const float (&m)[3], const float (&p)[3], float &f0,
                                            float &f1) {
   const float X = p[0] + m[0];
-  const float Se = p[1] + m[1], E = HEX_KD * (p[1] - m[1]);
+  const float Se = p[1] + m[1], de = p[1] - m[1];
   const float Sz = p[2] + m[2], Z = HEX_KD * (p[2] - m[2]);
   // I a + D b = (a + b) + partner's (r a - b)
-  const float da = (X + E) + quad_x1(HEX_R * X - E); // I_y X + D_y E
+  // I_y X + D_y E, E = KD de
+  const float da = (X + HEX_KD * de) + quad_x1(HEX_R * X - HEX_KD * de);
   const float db = Z + HEX_R * quad_x1(Z);
   const float d = (da + db) + quad_x2(HEX_R * da - db);
   const float sa = Se - quad_x1(Se);
@@ -582,6 +586,9 @@ struct LameF {
   float l, m, l_lo, m_lo;
   __device__ __forceinline__ float times_l(float x) const { return fmaf(l, x, l_lo * x); }
   __device__ __forceinline__ float times_m(float x) const { return fmaf(m, x, m_lo * x); }
+  __device__ __forceinline__ float times_m_plus(float x, float c) const {
+    return fmaf(m, x, fmaf(m_lo, x, c));
+  }
 };
 
 // b: the quad lane, s_y s_z = -1 on lanes 1 and 2
@@ -661,7 +668,8 @@ __device__ __forceinline__ void hex8_point(const float (&J)[3][3], const float (
     const float sd = 0.5f * L.times_l(e2[0] + e2[1] + e2[2]);
 #pragma unroll
     for (int v = 0; v < 6; ++v)
-      T[I6[v]][J6[v]] = T[J6[v]][I6[v]] = v < 3 ? L.times_m(e2[v]) + sd : L.times_m(e2[v]);
+      T[I6[v]][J6[v]] = T[J6[v]][I6[v]] =
+          v < 3 ? L.times_m_plus(e2[v], sd) : L.times_m(e2[v]);
     // P = sigma, or F S
 #pragma unroll
     for (int k = 0; k < 3; ++k)
@@ -711,10 +719,11 @@ __device__ __forceinline__ void hex8_quad(int b, uint32_t lc, uint32_t ls, const
     for (int c = 0; c < 3; ++c) {
       J[0][c] = Jx[c];
       H[0][c] = Hx[c];
-      J[1][c] = ix ? xe0[c] + xe1[c] : xe0[c] - xe1[c];
-      H[1][c] = ix ? ue0[c] + ue1[c] : ue0[c] - ue1[c];
-      J[2][c] = ix ? xz0[c] + xz1[c] : xz0[c] - xz1[c];
-      H[2][c] = ix ? uz0[c] + uz1[c] : uz0[c] - uz1[c];
+      const float kd = ix ? HEX_KD : -HEX_KD;
+      J[1][c] = xe0[c] + kd * xe1[c];
+      H[1][c] = ue0[c] + kd * ue1[c];
+      J[2][c] = xz0[c] + kd * xz1[c];
+      H[2][c] = uz0[c] + kd * uz1[c];
     }
     hex8_point<LAW>(J, H, L, lambda, mu, V, iq0 + (ix + 2 * b), ix ? Qp : Qm);
   }

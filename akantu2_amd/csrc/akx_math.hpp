@@ -4,8 +4,8 @@
 // The FP64 instantiation reproduces the reference's operation order so that
 // the plain path matches the CPU oracle bit for bit, apart from the last bit
 // of log() in the neo-Hookean law (device libm vs glibc).  All code here is
-// compiled with -ffp-contract=off; the FP32 precision form enables
-// contraction in its own kernels.
+// compiled with -ffp-contract=off; the FP32 precision form's own kernels with
+// on (a product and the sum it goes into in one expression are one FMA).
 //
 // Tensors are 3x3 arrays t[i][j] (row index i, column index j).
 //
@@ -143,10 +143,9 @@ template <class R> AKX_HD R jacobian_det(const R (&J)[3][3]) {
 // Matrix<Real,3,3>): used on F and C by the neo-Hookean law
 // (material_neohookean_inline_impl.hh:45-48).
 template <class R> AKX_HD R det3(const R (&m)[3][3]) {
-  R a = m[0][0] * (m[1][1] * m[2][2] - m[1][2] * m[2][1]);
-  R b = m[0][1] * (m[1][0] * m[2][2] - m[1][2] * m[2][0]);
-  R c = m[0][2] * (m[1][0] * m[2][1] - m[1][1] * m[2][0]);
-  return a - b + c;
+  return m[0][0] * (m[1][1] * m[2][2] - m[1][2] * m[2][1]) -
+         m[0][1] * (m[1][0] * m[2][2] - m[1][2] * m[2][0]) +
+         m[0][2] * (m[1][0] * m[2][1] - m[1][1] * m[2][0]);
 }
 
 template <class R> AKX_HD R cof3(const R (&m)[3][3], int i, int j) {
