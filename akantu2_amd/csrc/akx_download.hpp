@@ -9,7 +9,12 @@
 // 1 MB that one to eight threads claim in turn: each launches the next chunk's
 // kernel into one of its two pinned slots while it copies the one before out
 // (to the array and, where asked, to a second one), so the link, the copies
-// and the page faults overlap.  Times: Downloader::get.
+// and the page faults overlap.  Threads beside the caller's join once the
+// stream's earlier work is done: before, they waited for it in the runtime, which
+// spins, took CPUs from an OpenMP team of the caller's that still spun too, and
+// its next parallel region waited for a scheduler's slice or two (torch's cast of
+// a 28 MB field to FP32 after the read-back, 0.5 ms, 5 to 12 ms every other time).
+// Times: Downloader::get.
 #pragma once
 
 #include "akx_host.hpp"
@@ -123,30 +128,34 @@ public:
   void fail(std::exception_ptr e) { job.fail(e, open); }
 };
 
-// work(claims, c) does chunk c and claims and does others until none is left
-template <class F> void run_chunks(int threads, int64_t n, const F &work) {
+// work(claims, c, start) does chunk c and claims and does others until none is
+// left.  In the calling thread (*start)(k) lets up to k others help from then
+// on; in these start is null.
+using StartHelp = std::function<void(int)>;
+template <class F> void run_chunks(int64_t n, const F &work) {
   auto job = std::make_shared<ChunkJob>();
   job->n = n;
   // the threads hold the job alive and copies of what work refers to only
   // through it: work itself is run by a thread that has claimed a chunk
   std::shared_ptr<const F *> body = std::make_shared<const F *>(&work);
-  auto loop = [job, body] {
+  auto loop = [job, body](const StartHelp *start) {
     Claims claims(*job);
     const int64_t c = claims.claim();
     if (c < 0)
       return; // the caller may have returned: work is not touched
     try {
-      (**body)(claims, c);
+      (**body)(claims, c, start);
     } catch (...) {
       claims.fail(std::current_exception());
     }
   };
-  if (threads > 1)
+  const StartHelp start = [loop](int others) {
     try {
-      CopyThreads::get().submit(loop, threads - 1);
-    } catch (...) { // no thread to be had: their share is done here
+      CopyThreads::get().submit([loop] { loop(nullptr); }, others);
+    } catch (...) { // no thread to be had: their share is done by the caller
     }
-  loop();
+  };
+  loop(&start);
   while (job->done.load() < n)
     std::this_thread::yield();
   std::lock_guard<std::mutex> lock(job->mutex);
@@ -171,8 +180,10 @@ inline bool host_differs(const void *a, const void *b, size_t bytes) {
   if (T == 1)
     return std::memcmp(a, b, bytes) != 0;
   std::atomic<bool> differ{false};
-  run_chunks(T, (int64_t)((bytes + COPY_CHUNK - 1) / COPY_CHUNK),
-             [&](Claims &claims, int64_t c) {
+  run_chunks((int64_t)((bytes + COPY_CHUNK - 1) / COPY_CHUNK),
+             [&](Claims &claims, int64_t c, const StartHelp *start) {
+               if (start)
+                 (*start)(T - 1);
                for (; c >= 0; c = claims.claim()) {
                  const size_t o = (size_t)c * COPY_CHUNK;
                  if (!differ.load(std::memory_order_relaxed) &&
@@ -289,13 +300,13 @@ private:
       const Field *f;
       int64_t first, count;
     };
+    const int T = copy_threads(total);
     std::vector<Chunk> chunks;
     for (auto &f : fields) {
       const int64_t per = std::max<int64_t>(1, (int64_t)(COPY_CHUNK / f.item));
       for (int64_t i = 0; i < f.n; i += per)
         chunks.push_back({&f, i, std::min(per, f.n - i)});
     }
-    const int T = copy_threads(total);
     reserve((size_t)T * 2 * COPY_CHUNK);
     while ((int)events.size() < 2 * T) {
       hipEvent_t e;
@@ -303,7 +314,7 @@ private:
       events.push_back(e);
     }
     std::atomic<int> workers{0};
-    run_chunks(T, (int64_t)chunks.size(), [&](Claims &claims, int64_t c) {
+    run_chunks((int64_t)chunks.size(), [&](Claims &claims, int64_t c, const StartHelp *start) {
       // the thread's chunks in flight: claimed, the kernel launched
       const int w = workers.fetch_add(1);
       struct Flight {
@@ -314,13 +325,17 @@ private:
       HIPCHECK(hipSetDevice(device));
       for (int k = 0;; k ^= 1) {
         if (c >= 0) {
-          chunks[c].f->pack(slots + k * COPY_CHUNK, chunks[c].first, chunks[c].count);
+          const Chunk &h = chunks[c];
+          h.f->pack(slots + k * COPY_CHUNK, h.first, h.count);
           HIPCHECK(hipEventRecord(fl[k].ev, stream));
           fl[k].c = c;
         }
         Flight &o = fl[k ^ 1]; // the one before
         if (o.c >= 0) {
           HIPCHECK(hipEventSynchronize(o.ev));
+          if (start && T > 1) // the stream's earlier work is done
+            (*start)(T - 1);
+          start = nullptr;
           const Chunk &h = chunks[o.c];
           const size_t at = (size_t)h.first * h.f->item, b = (size_t)h.count * h.f->item;
           const unsigned char *slot = slots + (k ^ 1) * COPY_CHUNK;
