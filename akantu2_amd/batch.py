@@ -135,7 +135,9 @@ class Batch:
     # ---------------------------------------------------------- launch shape
     def setLaunch(self, block=256, tile=2048, blocks_per_cu=0, graph=True):
         """Threads per block, elements per tile and hipGraph on/off.  Every
-        workgroup does one tile; blocks_per_cu (0..32) has no effect."""
+        workgroup does one tile; blocks_per_cu (0..32) has no effect.  256
+        threads and tiles of 2048 stand for the library's own choice from the
+        instances' sizes."""
         N.check(N.lib().akx_batch_set_launch(self._h, int(block), int(tile),
                                              int(blocks_per_cu), int(bool(graph))))
 

@@ -588,9 +588,10 @@ struct akx_batch {
   int64_t nslices_live = 0;
   bool stream_loads = true; // more than STREAM_BYTES a step
   bool lists_dirty = true, inst_dirty = true;
-  // launch shape
-  int block = 256, tile = 2048, blocks_per_cu = 0, cus = 256;
-  bool launch_chosen = false; // set by set_launch or the autotuner
+  // launch shape; the default one stands for the rule (group_tile)
+  static constexpr int RULE_BLOCK = 256, RULE_TILE = 2048;
+  int block = RULE_BLOCK, tile = RULE_TILE, blocks_per_cu = 0, cus = 256;
+  bool launch_chosen() const { return block != RULE_BLOCK || tile != RULE_TILE; }
   bool use_graph = true;
   hipGraphExec_t graph = nullptr;
   int64_t plain_steps = 0; // launched one by one since the lists changed
@@ -654,8 +655,10 @@ void upload_inst(akx_batch *b) {
 }
 
 // Elements per tile of a group of n elements whose workgroups walk their tile
-// (groups without block tables).  A shape the caller or the autotuner chose
-// is used as it is.  Otherwise Tet4 takes one element per lane, and Hex8 one
+// (groups without block tables).  A shape that the caller or the autotuner chose
+// is used as it is; the default one, 256 lanes and tiles of 2,048, stands for
+// this rule (as a shape it was the slowest measured), so that switching graphs
+// on or off, or setting a shape that was read from an untouched batch, keeps it. Tet4 takes one element per lane, and Hex8 one
 // wave per workgroup (no barrier is waited for) with one or two rounds of eight
 // elements: two where the chip stays full, since the workgroup's dN/dxi table
 // is then filled once for both.  Steps of FP64 batches, us:
@@ -670,7 +673,7 @@ void upload_inst(akx_batch *b) {
 //     4.5 M               840    793   728   811    868
 constexpr int64_t HEX_TILE_FEW = 100000; // elements up to which a tile is one round
 int64_t group_tile(const akx_batch *b, int etype, int64_t n) {
-  if (b->launch_chosen)
+  if (b->launch_chosen())
     return b->tile;
   if (etype == AKX_TET4)
     return std::min(b->block, b->tile);
@@ -813,7 +816,7 @@ template <int LAW> void launch_strict(akx_batch *b, int etype, const BatchElemAr
   dim3 grid((unsigned)A.ntiles);
   if (etype == AKX_TET4)
     hipLaunchKernelGGL(k_batch_tet4<LAW>, grid, dim3(b->block), 0, b->stream, A);
-  else if (b->block == 64 || !b->launch_chosen) // see group_tile
+  else if (b->block == 64 || !b->launch_chosen()) // see group_tile
     hipLaunchKernelGGL((k_batch_hex8<LAW, 8>), grid, dim3(64), 0, b->stream, A);
   else if (b->block == 128)
     hipLaunchKernelGGL((k_batch_hex8<LAW, 16>), grid, dim3(128), 0, b->stream, A);
@@ -1606,7 +1609,6 @@ int akx_batch_set_launch(akx_batch *b, int block, int tile, int blocks_per_cu,
     b->tile = tile;
     b->blocks_per_cu = blocks_per_cu;
     b->use_graph = use_graph != 0;
-    b->launch_chosen = true;
     b->lists_dirty = true;
   });
 }
@@ -1627,8 +1629,8 @@ int akx_batch_get_launch(akx_batch *b, int *block, int *tile, int *blocks_per_cu
 }
 
 // Autotuner: times the element pass of the live instances for every
-// (threads per block, elements per tile, persistent blocks per CU) candidate
-// and keeps the fastest.  The trials leave the state untouched: the element
+// (threads per block, elements per tile, persistent blocks per CU) candidate,
+// the rule (256, 2048) among them, and keeps the fastest.  The trials leave the state untouched: the element
 // pass writes only the force table and the history buffer that the next
 // real step writes again from the same inputs.
 int akx_batch_autotune(akx_batch *b, int repeats, int *block, int *tile,
@@ -1642,9 +1644,9 @@ int akx_batch_autotune(akx_batch *b, int repeats, int *block, int *tile,
     const int blocks[3] = {64, 128, 256};
     const int tiles[5] = {256, 512, 1024, 2048, 4096};
     const int bpcs[1] = {0}; // one tile per workgroup: no persistent blocks
-    b->launch_chosen = true;
     double best = 1e300;
-    int bb = b->block, bt = b->tile, bc = b->blocks_per_cu;
+    const int block0 = b->block, tile0 = b->tile, bpc0 = b->blocks_per_cu;
+    int bb = block0, bt = tile0, bc = bpc0;
     hipEvent_t e0, e1;
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));
@@ -1674,6 +1676,10 @@ int akx_batch_autotune(akx_batch *b, int repeats, int *block, int *tile,
     } catch (...) {
       (void)hipEventDestroy(e0);
       (void)hipEventDestroy(e1);
+      b->block = block0;
+      b->tile = tile0;
+      b->blocks_per_cu = bpc0;
+      b->lists_dirty = true;
       throw;
     }
     (void)hipEventDestroy(e0);

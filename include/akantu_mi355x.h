@@ -415,13 +415,16 @@ int akx_batch_synchronize(akx_batch *b);
 int akx_batch_get_field(akx_batch *b, int instance_id, int field, double *host);
 /* Launch shape: threads per block (64, 128, 256; Hex8 uses 8 lanes per
  * element), elements per tile, hipGraph on/off.  Every workgroup does one
- * tile; blocks_per_cu (0..32) is kept for compatibility and has no effect. */
+ * tile; blocks_per_cu (0..32) is kept for compatibility and has no effect.
+ * 256 threads and tiles of 2048, the default, stand for the library's own
+ * choice from the instances' sizes. */
 int akx_batch_set_launch(akx_batch *b, int block, int tile, int blocks_per_cu,
                          int use_graph);
 int akx_batch_get_launch(akx_batch *b, int *block, int *tile,
                          int *blocks_per_cu, int *use_graph);
 /* Time the element pass of the live instances over the launch-shape
- * candidates (repeats launches each) and keep the fastest. */
+ * candidates (repeats launches each; the library's own choice, reported as
+ * 256 / 2048, is one) and keep the fastest. */
 int akx_batch_autotune(akx_batch *b, int repeats, int *block, int *tile,
                        int *blocks_per_cu, double *best_ms);
 int akx_batch_get_stats(akx_batch *b, int64_t *live, int64_t *elements,
