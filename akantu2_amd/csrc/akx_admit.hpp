@@ -5,16 +5,24 @@
 // element corner and some 40 fills and copies that took 1.3 ms for an instance
 // of some 40,000 elements (12 requests, 15.8 ms); now 0.3 ms (3.6 ms): the mesh
 // goes up once and kernels make
-//   blocks   (block-partial assembly) each block's distinct nodes, its corners'
-//            indices among them and their LDS slots, by a sort in LDS
-//   counts   the entries of every node's row of the force table, and from them
-//            the widths of its slices -- the one thing the host waits for, to
-//            find the instance's place in the arenas
+//   counts   each block's distinct nodes (block-partial assembly), by a sort in
+//            LDS, the entries of every node's row of the force table, and from
+//            them the widths of its slices -- the one thing the host waits for,
+//            to find the instance's place in the force table
+//   blocks   the sort again: the blocks' nodes, the corners' indices among them
+//            and their LDS slots
 //   rows     every row's entries, in the order they arrive
 //   ranks    each entry's place in its row: the number of smaller ones, so the
 //            order is that of the blocks or elements whatever the arrival
 //   elements, nodes   the arenas' connectivity and nodal state.
 // The tables are those of the host loops, entry by entry.
+//
+// The node and element ranges are taken before anything is uploaded, and what
+// the kernels keep between them lies in the instance's own part of the arenas
+// (connectivity, mass, force table).  The batch holds a buffer for the rest from
+// its creation: ADMIT_NODES nodes' input and the slices' and blocks' counts and
+// offsets.  So an admission allocates no device memory; sorting twice costs less
+// than reading the first sort's results back (12 requests 3.6 ms either way).
 #pragma once
 #include "akx_batch.hpp"
 #include <hip/hip_runtime.h>
@@ -22,29 +30,29 @@
 
 namespace akx {
 
+constexpr int64_t ADMIT_NODES = 128 * 1024; // uploaded at a time (a multiple of 256)
+
 struct AdmitArgs {
-  // uploaded: coordinates and velocity [nn][3] (velocity null: zero), blocked
-  // flags [nn][3] (null: none), connectivity [nel][nnpe]
+  // uploaded, of the nodes from `first` on: coordinates and velocity [][3]
+  // (velocity null: zero), blocked flags [][3] (null: none)
   const double *nodes, *velocity;
   const uint8_t *blocked3;
-  const int32_t *conn;
-  int64_t nn, nn_pad, nel;
-  int32_t nnpe, bs, pad; // elements per block; corners per block, padded
-  int64_t nblk;          // blocks (0: one table entry per element corner)
-  // scratch.  An item is a (block, distinct node) pair, at block * pad + k, or
-  // an element corner
-  int32_t *deg;    // [nn_pad] items of every node
-  int32_t *width;  // [nn_pad / 256]
-  int32_t *count;  // [nblk] distinct nodes
-  int32_t *item;   // [nblk * pad] node of an item
-  uint8_t *arrive; // place of an item in its row as it arrived
-  uint16_t *send, *lc, *ls;
+  int64_t first;
+  int64_t nn, nel;
+  int32_t nnpe, bs; // elements per block
+  int64_t nblk;     // blocks (0: one table entry per element corner)
+  // between the kernels.  x: entries of every node's row, y: those that have
+  // arrived; in the instance's part of the mass array, which is written last
+  int2 *deg;
+  int32_t *width; // [slices] longest row
+  int32_t *count; // [nblk] distinct nodes
   // the host's answer: row starts of the slices and first entry of the blocks,
   // both relative to the instance's
   const int64_t *off, *boff;
   int32_t *row; // the instance's force-table range, as one item per entry
   BBlk *blk;    // [nblk]
-  // the instance's place, and the arenas
+  // the instance's place, and the arenas.  a_conn holds the instance's own node
+  // numbers until k_admit_elements
   int64_t node0, elem0, ell0, bent0, ncap;
   int32_t *a_conn, *a_pos, *a_bnode, *a_bpos;
   uint16_t *a_lc, *a_ls, *a_bsend;
@@ -56,18 +64,40 @@ struct AdmitArgs {
   long long *first_bad;
 };
 
+// first place of a node's row
+__device__ __forceinline__ int64_t admit_row(const AdmitArgs &A, int32_t node) {
+  return A.off[node >> 8] + (node & 255);
+}
+
+// an item (block or corner) to the next place of its node's row
+__device__ __forceinline__ void admit_arrive(const AdmitArgs &A, int32_t node, int32_t item) {
+  const int d = atomicAdd(&A.deg[node].y, 1);
+  A.row[admit_row(A, node) + (int64_t)d * 256] = item;
+}
+
+// the smaller items of a node's row
+__device__ __forceinline__ int admit_rank(const AdmitArgs &A, int32_t node, int32_t item) {
+  const int64_t row = admit_row(A, node);
+  const int deg = A.deg[node].x;
+  int rank = 0;
+  for (int d = 0; d < deg; ++d)
+    rank += A.row[row + (int64_t)d * 256] < item;
+  return rank;
+}
+
 // One workgroup per block; PAD: its corners, rounded up to a power of two.
 // Corners sorted by (node, corner): a corner's position is its LDS slot, the
-// number of the distinct nodes before it its node's index.
-template <int PAD> __global__ void __launch_bounds__(256) k_admit_blocks(AdmitArgs A) {
+// number of the distinct nodes before it its node's index.  COUNT: the rows' and
+// blocks' numbers of entries only.
+template <int PAD, bool COUNT> __global__ void __launch_bounds__(256) k_admit_blocks(AdmitArgs A) {
   __shared__ unsigned long long key[PAD];
   __shared__ int wave_sum[4];
   constexpr int PER = PAD / 256;
-  const int64_t b = blockIdx.x, c0 = b * A.bs * A.nnpe;
+  const int64_t b = blockIdx.x, c0 = b * A.bs * A.nnpe, e0 = A.elem0 * A.nnpe + c0;
   const int64_t left = A.nel * A.nnpe - c0;
   const int n = (int)(left < (int64_t)A.bs * A.nnpe ? left : (int64_t)A.bs * A.nnpe);
   for (int i = threadIdx.x; i < PAD; i += 256)
-    key[i] = i < n ? (unsigned long long)A.conn[c0 + i] << 10 | i : ~0ull;
+    key[i] = i < n ? (unsigned long long)A.a_conn[e0 + i] << 10 | i : ~0ull;
   __syncthreads();
   for (int size = 2; size <= PAD; size *= 2)
     for (int step = size / 2; step > 0; step /= 2) {
@@ -104,6 +134,7 @@ template <int PAD> __global__ void __launch_bounds__(256) k_admit_blocks(AdmitAr
   int idx = upto - mine;
   for (int w = 0; w < wave; ++w)
     idx += wave_sum[w];
+  const int64_t ent = COUNT ? 0 : A.bent0 + A.boff[b];
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const int i = i0 + k;
@@ -112,33 +143,48 @@ template <int PAD> __global__ void __launch_bounds__(256) k_admit_blocks(AdmitAr
     const int32_t node = (int32_t)(key[i] >> 10);
     const int c = (int)(key[i] & 1023);
     if (is_new[k]) {
-      const int64_t at = b * A.pad + idx;
-      A.item[at] = node;
-      if (idx > 0)
-        A.send[at - 1] = (uint16_t)i; // the node before ends here
-      A.arrive[at] = (uint8_t)atomicAdd(&A.deg[node], 1); // read up to 255 items only
+      if constexpr (COUNT) {
+        atomicAdd(&A.deg[node].x, 1);
+      } else {
+        A.a_bnode[ent + idx] = (int32_t)(A.node0 + node);
+        if (idx > 0)
+          A.a_bsend[ent + idx - 1] = (uint16_t)i; // the node before ends here
+        admit_arrive(A, node, (int32_t)b);
+      }
       ++idx;
     }
-    A.ls[c0 + c] = (uint16_t)i;
-    A.lc[c0 + c] = (uint16_t)(idx - 1);
+    if constexpr (!COUNT) {
+      A.a_ls[e0 + c] = (uint16_t)i;
+      A.a_lc[e0 + c] = (uint16_t)(idx - 1);
+    }
     if (i == n - 1) {
-      A.send[b * A.pad + idx - 1] = (uint16_t)n;
-      A.count[b] = idx;
+      if constexpr (COUNT) {
+        A.count[b] = idx;
+      } else {
+        A.a_bsend[ent + idx - 1] = (uint16_t)n;
+        A.blk[b] = BBlk{ent, idx, 0};
+      }
     }
   }
 }
 
-// without block tables: the items are the element corners
-__global__ void __launch_bounds__(256) k_admit_corners(AdmitArgs A) {
+// Without block tables the items are the element corners, each in a row
+// of the table; COUNT as above.
+template <bool COUNT> __global__ void __launch_bounds__(256) k_admit_corners(AdmitArgs A) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < A.nel * A.nnpe)
-    A.arrive[i] = (uint8_t)atomicAdd(&A.deg[A.conn[i]], 1);
+  if (i >= A.nel * A.nnpe)
+    return;
+  const int32_t node = A.a_conn[A.elem0 * A.nnpe + i];
+  if constexpr (COUNT)
+    atomicAdd(&A.deg[node].x, 1);
+  else
+    admit_arrive(A, node, (int32_t)i);
 }
 
 // widest row of every slice; one workgroup per slice
 __global__ void __launch_bounds__(256) k_admit_widths(AdmitArgs A) {
   __shared__ int red[4];
-  int w = A.deg[(int64_t)blockIdx.x * 256 + threadIdx.x];
+  int w = A.deg[(int64_t)blockIdx.x * 256 + threadIdx.x].x;
 #pragma unroll
   for (int d = 32; d > 0; d /= 2)
     w = max(w, __shfl_xor(w, d));
@@ -149,80 +195,41 @@ __global__ void __launch_bounds__(256) k_admit_widths(AdmitArgs A) {
     A.width[blockIdx.x] = max(max(red[0], red[1]), max(red[2], red[3]));
 }
 
-// node of item (b, k) or of corner b * 256 + k; false past the last
-__device__ __forceinline__ bool admit_item(const AdmitArgs &A, int64_t b, int k, int64_t &at,
-                                           int32_t &node) {
-  at = A.nblk ? b * A.pad + k : b * 256 + k;
-  if (A.nblk ? k >= A.count[b] : at >= A.nel * A.nnpe)
-    return false;
-  node = A.nblk ? A.item[at] : A.conn[at];
-  return true;
-}
-__device__ __forceinline__ int64_t admit_row(const AdmitArgs &A, int32_t node) {
-  return A.off[node >> 8] + (node & 255);
-}
-
 // grid: blocks, or 256 corners each
-__global__ void __launch_bounds__(256) k_admit_rows(AdmitArgs A) {
-  const int64_t b = blockIdx.x;
-  const int most = A.nblk ? A.pad : 256;
-  for (int k = threadIdx.x; k < most; k += 256) {
-    int64_t at;
-    int32_t node;
-    if (!admit_item(A, b, k, at, node))
-      break;
-    A.row[admit_row(A, node) + (int64_t)A.arrive[at] * 256] = (int32_t)(A.nblk ? b : at);
-  }
-}
-
 __global__ void __launch_bounds__(256) k_admit_ranks(AdmitArgs A) {
   const int64_t b = blockIdx.x;
-  const int most = A.nblk ? A.pad : 256;
-  for (int k = threadIdx.x; k < most; k += 256) {
-    int64_t at;
-    int32_t node;
-    if (!admit_item(A, b, k, at, node))
-      break;
-    const int64_t row = admit_row(A, node);
-    const int32_t me = (int32_t)(A.nblk ? b : at);
-    int rank = 0;
-    for (int d = 0; d < A.deg[node]; ++d)
-      rank += A.row[row + d * 256] < me;
-    const int32_t pos = (int32_t)(A.ell0 + row + rank * 256);
-    if (A.nblk) {
-      const int64_t o = A.bent0 + A.boff[b] + k;
-      A.a_bnode[o] = (int32_t)(A.node0 + node);
-      A.a_bpos[o] = pos;
-      A.a_bsend[o] = A.send[at];
-    } else {
-      A.a_pos[A.elem0 * A.nnpe + at] = pos;
+  if (A.nblk) {
+    const int64_t ent = A.bent0 + A.boff[b];
+    for (int k = threadIdx.x; k < A.count[b]; k += 256) {
+      const int32_t node = (int32_t)(A.a_bnode[ent + k] - A.node0);
+      A.a_bpos[ent + k] =
+          (int32_t)(A.ell0 + admit_row(A, node) + admit_rank(A, node, (int32_t)b) * 256);
     }
+    return;
   }
-  if (A.nblk && threadIdx.x == 0)
-    A.blk[b] = BBlk{A.bent0 + A.boff[b], A.count[b], 0};
+  const int64_t i = b * 256 + threadIdx.x;
+  if (i >= A.nel * A.nnpe)
+    return;
+  const int64_t at = A.elem0 * A.nnpe + i;
+  const int32_t node = A.a_conn[at];
+  A.a_pos[at] = (int32_t)(A.ell0 + admit_row(A, node) + admit_rank(A, node, (int32_t)i) * 256);
 }
 
 __global__ void __launch_bounds__(256) k_admit_elements(AdmitArgs A) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= A.nel * A.nnpe)
-    return;
-  const int64_t at = A.elem0 * A.nnpe + i;
-  A.a_conn[at] = (int32_t)(A.node0 + A.conn[i]);
-  if (A.nblk) {
-    A.a_lc[at] = A.lc[i];
-    A.a_ls[at] = A.ls[i];
-  }
+  if (i < A.nel * A.nnpe)
+    A.a_conn[A.elem0 * A.nnpe + i] += (int32_t)A.node0;
 }
 
-// nodal state: X and v as given, all else zero, the padding nodes' too; these
-// are blocked
+// nodal state of the uploaded nodes' slices: X and v as given, all else zero, the
+// padding nodes' too; these are blocked
 __global__ void __launch_bounds__(256) k_admit_nodes(AdmitArgs A) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; // < nn_pad
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x, i = A.first + k; // < nn_pad
   const int64_t n = A.node0 + i;
   const bool real = i < A.nn;
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
-    const double x = real ? A.nodes[3 * i + c] : 0.;
+    const double x = real ? A.nodes[3 * k + c] : 0.;
     const int64_t o = c * A.ncap + n;
     A.a_xu[6 * n + c] = x;
     A.a_xu[6 * n + 3 + c] = 0.;
@@ -230,7 +237,7 @@ __global__ void __launch_bounds__(256) k_admit_nodes(AdmitArgs A) {
       A.a_x[o] = x;
       A.a_u[o] = 0.;
     }
-    A.a_v[o] = real && A.velocity ? A.velocity[3 * i + c] : 0.;
+    A.a_v[o] = real && A.velocity ? A.velocity[3 * k + c] : 0.;
     A.a_a[o] = 0.;
     A.a_fint[o] = 0.;
     if (A.a_cu) {
@@ -244,10 +251,10 @@ __global__ void __launch_bounds__(256) k_admit_nodes(AdmitArgs A) {
     if (A.blocked3)
 #pragma unroll
       for (int c = 0; c < 3; ++c)
-        bits |= A.blocked3[3 * i + c] ? 1 << c : 0;
+        bits |= A.blocked3[3 * k + c] ? 1 << c : 0;
   }
   A.a_blocked[n] = bits;
-  A.a_deg[n] = (uint8_t)A.deg[i];
+  A.a_deg[n] = (uint8_t)A.deg[i].x;
   if (threadIdx.x == 0)
     A.a_ell_off[n >> 8] = A.ell0 + A.off[i >> 8];
   if (i == 0) {

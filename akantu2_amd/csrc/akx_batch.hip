@@ -565,7 +565,7 @@ struct akx_batch {
   DevBuf<double> hex_tab;
   DevBuf<unsigned long long> dt_bits;
   DevBuf<long long> bad;
-  DevBuf<unsigned char> admit; // upload and scratch of an instance that joins
+  DevBuf<unsigned char> admit; // upload and counts of an instance that joins (akx_admit.hpp)
   Downloader download;
   FreeList fl_nodes, fl_tet, fl_hex, fl_ell;
   // FP32 block-partial assembly: per element its local corners and LDS
@@ -1042,6 +1042,9 @@ void do_steps(akx_batch *b, int64_t n) {
     b->inst_dirty = true; // parity bases moved
 }
 
+// bytes of a part of the admission buffer
+size_t admit_part(int64_t n, size_t size) { return ((size_t)n * size + 255) / 256 * 256; }
+
 // device bytes an instance takes in a batch (node range padded to 256,
 // force-table entries of FE_W values estimated with a 25 % slice padding)
 int64_t footprint_bytes(int precision, int etype, int law, int64_t nn, int64_t nel) {
@@ -1053,12 +1056,15 @@ int64_t footprint_bytes(int precision, int etype, int law, int64_t nn, int64_t n
   // u arrays and the two compensation terms
   double bytes = (double)nn_pad * (5 * 3 * 8 + 8 + 1 + 1 + (f32 ? 2 * 3 * 8 + 2 * 3 * 4 : 0)) +
                  (double)nn_pad / 256 * 8;
-  bytes += (double)nel * nnpe * (4 + 4 + 1.25 * FE_W * sf);
-  if (f32 && etype == AKX_TET4) // block partials: corners and slots, and at most
-                                // two distinct-node entries per element
-    bytes += (double)nel * (4 * 2 * 2 + 2 * (4 + 4 + 2));
-  else if (f32) // Hex8: slots, at most five distinct-node entries per element
-    bytes += (double)nel * (8 * 2 + 5 * (4 + 4 + 2));
+  // connectivity, force table; FP64: the corners' places in it
+  bytes += (double)nel * nnpe * (4 + (f32 ? 0 : 4) + 1.25 * FE_W * sf);
+  if (f32) { // corners and slots; per distinct-node entry (at most two per Tet4
+             // and eight per Hex8) its node, table place and slot end
+    const int bs = etype == AKX_TET4 ? BPA_TET4 : BPA_HEX8;
+    bytes += (double)nel * (nnpe * 2 * 2 + (etype == AKX_TET4 ? 2 : 8) * (4 + 4 + 2));
+    bytes += (double)((nel + bs - 1) / bs) * (4 + 8 + sizeof(BBlk)); // admission buffer
+  }
+  bytes += (double)nn_pad / 256 * (4 + 8);
   if (law == AKX_LAW_PLASTIC_LIH) // two buffers of the history
     bytes += (double)nel * nqp * 2 * (f32 ? 7 * 4 : 28 * 8);
   return (int64_t)bytes;
@@ -1175,6 +1181,13 @@ int akx_batch_create(int device, int precision, int64_t node_capacity,
                        hipMemcpyHostToDevice));
     b->dt_bits.alloc(1);
     b->bad.alloc(1);
+    const int64_t round = std::min(b->ncap, ADMIT_NODES), slices = b->ncap / 256;
+    const int64_t blocks =
+        b->bpa ? std::max((b->tcap + BPA_TET4 - 1) / BPA_TET4, (b->hexcap + BPA_HEX8 - 1) / BPA_HEX8)
+               : 0;
+    b->admit.alloc(2 * admit_part(3 * round, 8) + admit_part(3 * round, 1) +
+                   admit_part(slices + blocks, 4) + admit_part(slices + blocks, 8) +
+                   admit_part(blocks, sizeof(BBlk)));
     b->d_inst.alloc(MAX_INSTANCES);
     b->fl_nodes.reset(b->ncap);
     b->fl_tet.reset(b->tcap);
@@ -1246,86 +1259,9 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
     const int64_t bs = element_type == AKX_TET4 ? BPA_TET4 : BPA_HEX8; // per block
     const int64_t nblk = bpa ? (nb_elements + bs - 1) / bs : 0;
     const int64_t corners = nb_elements * nnpe, nsl = I.nn_pad / 256;
-    const int pad = element_type == AKX_TET4 ? 1024 : 512; // corners per block, 2^k
     static_assert(BPA_TET4 * 4 <= 1024 && BPA_HEX8 * 8 <= 512, "a block's corners fit its sort");
-    const int64_t items = bpa ? nblk * pad : corners;
-    if (I.nn_pad > b->ncap) // no scratch for what never fits
-      throw Error(AKX_ERR_MEMORY, "node arena full");
-    if (I.nel > (element_type == AKX_TET4 ? b->tcap : b->hexcap))
-      throw Error(AKX_ERR_MEMORY, "element arena full");
-    // upload and scratch
-    size_t total = 0;
-    auto take = [&](int64_t n, size_t size) {
-      const size_t at = total;
-      total += ((size_t)n * size + 255) / 256 * 256;
-      return at;
-    };
-    const size_t o_nodes = take(3 * nb_nodes, 8), o_vel = take(velocity ? 3 * nb_nodes : 0, 8),
-                 o_blocked = take(blocked_dofs ? 3 * nb_nodes : 0, 1), o_conn = take(corners, 4),
-                 o_width = take(nsl + nblk, 4), o_deg = take(I.nn_pad, 4),
-                 o_item = take(bpa ? items : 0, 4), o_arrive = take(items, 1),
-                 o_send = take(bpa ? items : 0, 2), o_lc = take(bpa ? corners : 0, 2),
-                 o_ls = take(bpa ? corners : 0, 2), o_off = take(nsl + nblk, 8),
-                 o_blk = take(nblk, sizeof(BBlk));
-    if (b->admit.n < total) {
-      sync(b); // the buffer may still be read
-      b->admit.reserve(total);
-    }
-    unsigned char *scratch = b->admit.p;
-    auto up = [&](size_t at, const void *src, size_t bytes) {
-      HIPCHECK(hipMemcpyAsync(scratch + at, src, bytes, hipMemcpyHostToDevice, b->stream));
-      return scratch + at;
-    };
-    AdmitArgs T{};
-    T.nodes = (const double *)up(o_nodes, nodes, 24 * nb_nodes);
-    if (velocity)
-      T.velocity = (const double *)up(o_vel, velocity, 24 * nb_nodes);
-    if (blocked_dofs)
-      T.blocked3 = up(o_blocked, blocked_dofs, 3 * nb_nodes);
-    T.conn = (const int32_t *)up(o_conn, conn, corners * 4);
-    T.nn = nb_nodes;
-    T.nn_pad = I.nn_pad;
-    T.nel = nb_elements;
-    T.nnpe = nnpe;
-    T.bs = (int32_t)bs;
-    T.pad = pad;
-    T.nblk = nblk;
-    T.width = (int32_t *)(scratch + o_width);
-    T.count = T.width + nsl;
-    T.deg = (int32_t *)(scratch + o_deg);
-    T.item = (int32_t *)(scratch + o_item);
-    T.arrive = scratch + o_arrive;
-    T.send = (uint16_t *)(scratch + o_send);
-    T.lc = (uint16_t *)(scratch + o_lc);
-    T.ls = (uint16_t *)(scratch + o_ls);
-    T.blk = (BBlk *)(scratch + o_blk);
-    hipLaunchKernelGGL((k_batch_fill<int32_t>), dim3(gridn(I.nn_pad)), dim3(TPB), 0, b->stream,
-                       T.deg, I.nn_pad, 0);
-    if (!bpa)
-      hipLaunchKernelGGL(k_admit_corners, dim3(gridn(corners)), dim3(256), 0, b->stream, T);
-    else if (element_type == AKX_TET4)
-      hipLaunchKernelGGL(k_admit_blocks<1024>, dim3((unsigned)nblk), dim3(256), 0, b->stream, T);
-    else
-      hipLaunchKernelGGL(k_admit_blocks<512>, dim3((unsigned)nblk), dim3(256), 0, b->stream, T);
-    hipLaunchKernelGGL(k_admit_widths, dim3((unsigned)nsl), dim3(256), 0, b->stream, T);
-    HIPCHECK(hipGetLastError());
-    // the sliced-ELL layout of this instance
-    std::vector<int32_t> found(nsl + nblk);
-    HIPCHECK(hipMemcpyAsync(found.data(), T.width, found.size() * 4, hipMemcpyDeviceToHost,
-                            b->stream));
-    sync(b);
-    std::vector<int64_t> off(nsl + nblk); // of the slices, then of the blocks
-    for (int64_t s = 0; s < nsl; ++s) {
-      require(found[s] <= 255, "a node belongs to more than 255 elements");
-      off[s] = I.nell;
-      I.nell += (int64_t)found[s] * 256;
-    }
-    I.blk_cnt.assign(found.begin() + nsl, found.end());
-    for (int64_t k = 0; k < nblk; ++k) {
-      off[nsl + k] = I.nbent;
-      I.nbent += I.blk_cnt[k];
-    }
-    // ranges in the arenas
+    // the instance's nodes and elements first: what never fits, or has to wait
+    // for its turn, uploads nothing
     if (b->inst.size() >= (size_t)MAX_INSTANCES) {
       bool slot = false;
       for (auto &J : b->inst)
@@ -1342,34 +1278,36 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
       b->fl_nodes.release(I.node0, I.nn_pad);
       throw Error(AKX_ERR_MEMORY, "element arena full");
     }
-    I.ell0 = b->fl_ell.alloc(I.nell, 256); // nell is a multiple of 256
-    if (I.ell0 < 0) {
-      b->fl_nodes.release(I.node0, I.nn_pad);
-      fl_el.release(I.elem0, I.nel);
-      throw Error(AKX_ERR_MEMORY, "force table full");
-    }
-    if (bpa) {
-      I.bent0 = b->fl_bent.alloc(I.nbent);
-      if (I.bent0 < 0) {
-        b->fl_nodes.release(I.node0, I.nn_pad);
-        fl_el.release(I.elem0, I.nel);
-        b->fl_ell.release(I.ell0, I.nell);
-        throw Error(AKX_ERR_MEMORY, "block arena full");
-      }
-    }
     try {
-      // arena connectivity, table entries, slice offsets, degrees, blocked
-      // bits, nodal state.  The rows' scratch is the instance's own (not yet
-      // used) force-table range
+      // the buffer's parts: a round of nodes, slices, blocks
+      size_t total = 0;
+      auto take = [&](int64_t n, size_t size) {
+        unsigned char *at = b->admit.p + total;
+        total += admit_part(n, size);
+        return at;
+      };
+      const int64_t round = std::min(b->ncap, ADMIT_NODES);
+      unsigned char *up_nodes = take(3 * round, 8), *up_velocity = take(3 * round, 8),
+                    *up_blocked = take(3 * round, 1), *at_found = take(nsl + nblk, 4),
+                    *at_off = take(nsl + nblk, 8), *at_blk = take(nblk, sizeof(BBlk));
+      require(total <= b->admit.n, "instance larger than the admission buffer");
+      auto up = [&](void *at, const void *src, size_t bytes) {
+        HIPCHECK(hipMemcpyAsync(at, src, bytes, hipMemcpyHostToDevice, b->stream));
+      };
       int32_t *dconn = element_type == AKX_TET4 ? b->conn_t.p : b->conn_h.p;
       int32_t *dpos = element_type == AKX_TET4 ? b->pos_t.p : b->pos_h.p;
-      T.off = (const int64_t *)up(o_off, off.data(), off.size() * 8);
-      T.boff = T.off + nsl;
-      T.row = reinterpret_cast<int32_t *>(b->fe.p + I.ell0 * FE_W * b->fe_size());
+      AdmitArgs T{};
+      T.nn = nb_nodes;
+      T.nel = nb_elements;
+      T.nnpe = nnpe;
+      T.bs = (int32_t)bs;
+      T.nblk = nblk;
+      T.deg = reinterpret_cast<int2 *>(b->mass.p + I.node0);
+      T.width = (int32_t *)at_found;
+      T.count = T.width + nsl;
+      T.blk = (BBlk *)at_blk;
       T.node0 = I.node0;
       T.elem0 = I.elem0;
-      T.ell0 = I.ell0;
-      T.bent0 = I.bent0;
       T.ncap = b->ncap;
       T.a_conn = dconn;
       T.a_pos = dpos;
@@ -1396,11 +1334,76 @@ int akx_batch_add_instance(akx_batch *b, int element_type, int law, const double
                   T.a_xu && !T.a_x == !T.a_u && !T.a_cu == !T.a_cv,
               "instance admitted without its arenas");
       const dim3 item_grid(bpa ? (unsigned)nblk : gridn(corners));
-      hipLaunchKernelGGL(k_admit_rows, item_grid, dim3(256), 0, b->stream, T);
+      auto sort_blocks = [&](auto count) {
+        constexpr bool COUNT = decltype(count)::value;
+        if (!bpa)
+          hipLaunchKernelGGL(k_admit_corners<COUNT>, item_grid, dim3(256), 0, b->stream, T);
+        else if (element_type == AKX_TET4)
+          hipLaunchKernelGGL((k_admit_blocks<1024, COUNT>), item_grid, dim3(256), 0, b->stream, T);
+        else
+          hipLaunchKernelGGL((k_admit_blocks<512, COUNT>), item_grid, dim3(256), 0, b->stream, T);
+        HIPCHECK(hipGetLastError());
+      };
+      up(dconn + I.elem0 * nnpe, conn, corners * 4);
+      hipLaunchKernelGGL((k_batch_fill<double>), dim3(gridn(I.nn_pad)), dim3(TPB), 0, b->stream,
+                         b->mass.p + I.node0, I.nn_pad, 0.); // T.deg
+      sort_blocks(std::true_type{});
+      hipLaunchKernelGGL(k_admit_widths, dim3((unsigned)nsl), dim3(256), 0, b->stream, T);
+      HIPCHECK(hipGetLastError());
+      // the sliced-ELL layout of this instance
+      std::vector<int32_t> found(nsl + nblk);
+      HIPCHECK(hipMemcpyAsync(found.data(), T.width, found.size() * 4, hipMemcpyDeviceToHost,
+                              b->stream));
+      sync(b);
+      std::vector<int64_t> off(nsl + nblk); // of the slices, then of the blocks
+      int64_t nell = 0, nbent = 0;
+      for (int64_t s = 0; s < nsl; ++s) {
+        require(found[s] <= 255, "a node belongs to more than 255 elements");
+        off[s] = nell;
+        nell += (int64_t)found[s] * 256;
+      }
+      I.blk_cnt.assign(found.begin() + nsl, found.end());
+      for (int64_t k = 0; k < nblk; ++k) {
+        off[nsl + k] = nbent;
+        nbent += I.blk_cnt[k];
+      }
+      I.ell0 = b->fl_ell.alloc(nell, 256); // nell is a multiple of 256
+      if (I.ell0 < 0)
+        throw Error(AKX_ERR_MEMORY, "force table full");
+      I.nell = nell;
+      if (bpa) {
+        I.bent0 = b->fl_bent.alloc(nbent);
+        if (I.bent0 < 0)
+          throw Error(AKX_ERR_MEMORY, "block arena full");
+        I.nbent = nbent;
+      }
+      // arena connectivity, table entries, slice offsets, degrees, blocked
+      // bits, nodal state.  The rows lie in the instance's own (not yet used)
+      // force-table range
+      up(at_off, off.data(), off.size() * 8);
+      T.off = (const int64_t *)at_off;
+      T.boff = T.off + nsl;
+      T.row = reinterpret_cast<int32_t *>(b->fe.p + I.ell0 * FE_W * b->fe_size());
+      T.ell0 = I.ell0;
+      T.bent0 = I.bent0;
+      sort_blocks(std::false_type{});
       hipLaunchKernelGGL(k_admit_ranks, item_grid, dim3(256), 0, b->stream, T);
       hipLaunchKernelGGL(k_admit_elements, dim3(gridn(corners)), dim3(256), 0, b->stream, T);
-      hipLaunchKernelGGL(k_admit_nodes, dim3((unsigned)nsl), dim3(256), 0, b->stream, T);
       HIPCHECK(hipGetLastError());
+      T.nodes = (const double *)up_nodes;
+      T.velocity = velocity ? (const double *)up_velocity : nullptr;
+      T.blocked3 = blocked_dofs ? up_blocked : nullptr;
+      for (T.first = 0; T.first < nb_nodes; T.first += round) {
+        const int64_t n = std::min(round, nb_nodes - T.first);
+        up(up_nodes, nodes + 3 * T.first, 24 * n);
+        if (velocity)
+          up(up_velocity, velocity + 3 * T.first, 24 * n);
+        if (blocked_dofs)
+          up(up_blocked, blocked_dofs + 3 * T.first, 3 * n);
+        hipLaunchKernelGGL(k_admit_nodes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                           b->stream, T);
+        HIPCHECK(hipGetLastError());
+      }
       if (law == AKX_LAW_PLASTIC_LIH) {
         AdmitHist H{};
         int comps = 0;
