@@ -736,7 +736,7 @@ constexpr int HEX_STRICT_EPB = 8;
 
 // J^-1 and w det J of one Gauss point, from the table that init fills (jw: the
 // Gauss point's column 0 of [5][stride]).  Read once per step: with STREAM,
-// non-temporal loads leave the caches to the nodal data (STREAM_BYTES; a
+// non-temporal loads leave the caches to the nodal data (STREAM_JAC_PLASTIC; a
 // template parameter, as the compiler merges the two branches of a flag into
 // plain loads).
 struct HexJac {
@@ -984,7 +984,10 @@ struct GatherArgs {
 // it the table is still in the caches the element pass wrote it to, and plain
 // loads find it there.  FEW: eight entries are loaded before the first is added
 // (the loads past the last entry repeat it and are not added), so a node waits
-// for one or two round trips instead of one per entry.
+// for one or two round trips instead of one per entry; plain loads whatever the
+// bytes, which only a plastic law's history takes above STREAM_BYTES at so few
+// nodes (step with non-temporal -> plain ones, us: plastic Tet4 325 MB 79 -> 74,
+// 454 MB 108 -> 102; plastic Hex8 340 MB 73 -> 72, 488 MB 109 -> 105).
 template <bool FEW, int W, class FT>
 __device__ __forceinline__ void sum_entries(const FT *p, int deg, bool stream, double (&f)[3]) {
   f[0] = f[1] = f[2] = 0.;
@@ -1029,6 +1032,16 @@ __device__ __forceinline__ void sum_entries(const FT *p, int deg, bool stream, d
 // either way.  Up to 65,536 nodes: Tet4 FP64 24.4 -> 21.0 us, plastic 22.4 ->
 // 20.1.
 constexpr double STREAM_BYTES = 310e6;
+
+// The same for the Hex8 jacobian table beside a plastic law's history, 3,584 of
+// the some 4,700 bytes an element moves: none of it is read again while the cache
+// holds it, where half of an elastic step's bytes are, so the table has to give
+// way earlier.  Step of plastic Hex8, non-temporal -> plain, us (plain: by where
+// the arrays came to lie): 194 MB 40.5 -> 37.2, 219 MB 44.8 -> 41.5, 234 MB 47.2 ->
+// 43..49, 253 MB 51.0 -> 46..54, 263 MB 52.0 -> 49..57, 273 MB 52.4 -> 58..59, 291
+// MB 55.6 -> 63.3, 340 MB 71.5 -> 69..77 (elastic 205 MB 48.8 -> 43.6, 307 MB 69.3
+// -> 61.6, 331 MB 74.1 -> 68.8).
+constexpr double STREAM_JAC_PLASTIC = 240e6;
 
 // Up to this many nodes a gather reads its nodal state ahead of the entries
 // and the entries eight at a time (FEW).  With one or two waves per SIMD (1,024

@@ -803,7 +803,8 @@ struct akx_model {
   StepArgs step{};
   DevBuf<unsigned char> step_lists;
   size_t step_lds = 0;
-  bool stream_loads = true; // more than STREAM_BYTES a step
+  // more than STREAM_BYTES a step; the Hex8 jacobian table (STREAM_JAC_PLASTIC)
+  bool stream_loads = true, stream_jac = true;
   DevBuf<unsigned char> staging;
   Downloader download;
   DevBuf<unsigned long long> scratch_u64;
@@ -1402,7 +1403,7 @@ template <int LAW> void launch_hex8_strict_law(akx_model *m, Material &mat, cons
   const dim3 grid((unsigned)A.nblocks_padded), block(64);
   if (mat.ext())
     hipLaunchKernelGGL((k_hex8_strict<LAW, true>), grid, block, 0, m->stream, A);
-  else if (m->stream_loads)
+  else if (m->stream_jac)
     hipLaunchKernelGGL((k_hex8_strict<LAW, false, true>), grid, block, 0, m->stream, A);
   else
     hipLaunchKernelGGL((k_hex8_strict<LAW, false, false>), grid, block, 0, m->stream, A);
@@ -2881,7 +2882,12 @@ int akx_model_init_full(akx_model *m) {
       HIPCHECK(hipStreamSynchronize(m->stream));
     }
     plan_small_steps(m);
-    m->stream_loads = kernel_bytes(m, 0) + kernel_bytes(m, 1) > STREAM_BYTES;
+    const double step_bytes = kernel_bytes(m, 0) + kernel_bytes(m, 1);
+    bool plastic = false;
+    for (auto &mp : m->mats)
+      plastic = plastic || mp->law == AKX_LAW_PLASTIC_LIH;
+    m->stream_loads = step_bytes > STREAM_BYTES;
+    m->stream_jac = step_bytes > (plastic ? STREAM_JAC_PLASTIC : STREAM_BYTES);
     for (auto &mp : m->mats)
       alloc_internals(m, *mp);
     if (m->precision == AKX_PRECISION_FP32) {
