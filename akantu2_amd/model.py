@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes as C
 import sys
+import threading
 import weakref
 
 import numpy as np
@@ -101,6 +102,43 @@ class _Mirror:
         differs = C.c_int(0)
         N.check(N.lib().akx_host_differs(_p(self.base), _p(self.snap), n, C.byref(differs)))
         return bool(differs.value)
+
+
+class _Spare:
+    """Memory of copies nothing refers to any more (a copy's and its snapshot's),
+    kept for the same field's next copy: a new array's page faults cost more than
+    the download.  At most ``LIMIT`` bytes over all models of the process, given
+    back with the model."""
+
+    LIMIT = 256 << 20  # displacement, velocity and a force of 2 million nodes
+    _lock = threading.RLock()
+    _bytes = 0
+
+    def __init__(self):
+        self._kept = {}
+
+    @staticmethod
+    def _size(arrays):
+        return sum(a.nbytes for a in arrays if a is not None)
+
+    def put(self, name, base, snap):
+        self.take(name)
+        n = self._size((base, snap))
+        with _Spare._lock:
+            if _Spare._bytes + n > self.LIMIT:
+                return
+            _Spare._bytes += n
+        self._kept[name] = (base, snap)
+
+    def take(self, name):
+        arrays = self._kept.pop(name, (None, None))
+        with _Spare._lock:
+            _Spare._bytes -= self._size(arrays)
+        return arrays
+
+    def __del__(self):
+        for name in list(self._kept):
+            self.take(name)
 
 
 class MaterialFactory:
@@ -379,7 +417,7 @@ class SolidMechanicsModel:
         self.nb_nodes = nodes.shape[0]
         self.materials = []
         self._mirrors = {}
-        self._spare = {}  # field -> arrays of its last dropped copy
+        self._spare = _Spare()
         self._initialized = False
         self._stresses_fresh = False
         self.time_step = 0.0
@@ -584,11 +622,9 @@ class SolidMechanicsModel:
                 self._drop(name)
 
     def _drop(self, name):
-        """Forget a copy nothing refers to.  Its memory (the copy's and the
-        snapshot's) is kept for the field's next copy, one per field: a new
-        array's page faults cost more than the download."""
+        """Forget a copy nothing refers to."""
         mir = self._mirrors.pop(name)
-        self._spare[name] = (mir.base, mir.snap)
+        self._spare.put(name, mir.base, mir.snap)
 
     def _download(self, mirs):
         """Fill the copies (name, mirror), all with one wait for the device."""
@@ -620,7 +656,7 @@ class SolidMechanicsModel:
     def _get(self, name):
         mir = self._mirrors.get(name)
         if mir is None:
-            base, snap = self._spare.pop(name, (None, None))
+            base, snap = self._spare.take(name)
             if base is None:
                 dtype = np.uint8 if name == "blocked_dofs" else np.float64
                 base = np.empty((self.nb_nodes, 3), dtype)
