@@ -96,6 +96,7 @@ def _declare(lib):
         "akx_model_enable_kernel_timing": (C.c_int, [_vp, C.c_int]),
         "akx_model_get_kernel_timing": (C.c_int, [_vp, C.c_int, _dp, C.POINTER(_i64)]),
         "akx_model_get_kernel_bytes": (C.c_int, [_vp, C.c_int, _dp]),
+        "akx_model_get_step_workgroups": (C.c_int, [_vp, C.POINTER(_i64)]),
         "akx_calibration_copy": (C.c_int, [C.c_int, _i64, C.c_int, _dp]),
         "akx_batch_create": (C.c_int, [C.c_int, C.c_int, _i64, _i64, _i64, C.c_int,
                                        C.POINTER(_vp)]),
@@ -124,6 +125,7 @@ def _declare(lib):
         "akx_batch_enable_kernel_timing": (C.c_int, [_vp, C.c_int]),
         "akx_batch_get_kernel_timing": (C.c_int, [_vp, C.c_int, _dp, C.POINTER(_i64)]),
         "akx_batch_get_kernel_bytes": (C.c_int, [_vp, C.c_int, _dp]),
+        "akx_batch_get_graph_steps": (C.c_int, [_vp, C.POINTER(C.c_int)]),
     }
     for name, (res, args) in sigs.items():
         fn = getattr(lib, name)

@@ -1755,6 +1755,13 @@ int akx_batch_get_kernel_bytes(akx_batch *b, int kernel_class, double *bytes) {
   });
 }
 
+int akx_batch_get_graph_steps(akx_batch *b, int *steps) {
+  return guard([&] {
+    require(b != nullptr && steps != nullptr, "null argument");
+    *steps = b->graph ? GRAPH_STEPS : 0;
+  });
+}
+
 int akx_batch_enable_kernel_timing(akx_batch *b, int enable) {
   return guard([&] {
     require(b != nullptr, "null batch");

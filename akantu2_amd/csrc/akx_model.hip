@@ -4009,6 +4009,15 @@ int akx_model_get_kernel_timing(akx_model *m, int kernel_class, double *total_ms
   });
 }
 
+int akx_model_get_step_workgroups(akx_model *m, int64_t *workgroups) {
+  return guard([&] {
+    check_ready(m);
+    require(workgroups != nullptr, "null output");
+    const bool pipelined = m->pipe_parts > 1 && m->pipe_ok;
+    *workgroups = small_steps(m) && !pipelined ? m->step.nblocks : 0;
+  });
+}
+
 int akx_model_get_kernel_bytes(akx_model *m, int kernel_class, double *bytes) {
   return guard([&] {
     check_ready(m);

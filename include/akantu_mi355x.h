@@ -352,6 +352,10 @@ int akx_model_get_kernel_timing(akx_model *m, int kernel_class,
  * array read or written once, node data once per node); for class 1 the
  * gather of a step followed by another, which does not store f_int. */
 int akx_model_get_kernel_bytes(akx_model *m, int kernel_class, double *bytes);
+/* Workgroups of the one launch that a step of the next solve call takes; 0: it
+ * takes an element pass and a gather (larger models, several or user materials,
+ * external terms, kernel timing). */
+int akx_model_get_step_workgroups(akx_model *m, int64_t *workgroups);
 /* Streaming device copy of `bytes` (read + write), repeated; average time
  * per copy in ms.  No counterpart in the reference: it calibrates the HBM
  * byte counters and reports the measured copy bandwidth. */
@@ -439,6 +443,9 @@ int akx_batch_get_kernel_timing(akx_batch *b, int kernel_class,
                                 double *total_ms, int64_t *launches);
 /* Unique bytes one launch of the class moves over the live instances. */
 int akx_batch_get_kernel_bytes(akx_batch *b, int kernel_class, double *bytes);
+/* Steps one replay of the batch's graph does; 0: none is captured (steps are
+ * launched one by one until the instances have stayed the same for a while). */
+int akx_batch_get_graph_steps(akx_batch *b, int *steps);
 
 #ifdef __cplusplus
 }
