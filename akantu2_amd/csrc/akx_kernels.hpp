@@ -633,10 +633,12 @@ __global__ void __launch_bounds__(256) k_tet4_strict_lds(ElemArgs A) {
 // registers it holds the summed runs' slots.
 constexpr int PPA_TB = 256;
 
-// MAT: grad u and the stress are stored (computeAllStresses); a variant of its
-// own, whose addresses kept 10 to 18 registers more alive in every step's pass:
-// 106 -> 88 to 96, five waves per SIMD instead of four.  4.4 M elements, us:
-// elastic 130 -> 122, finite strain 141 -> 138, neo-Hookean 145 -> 145.
+// MAT: grad u and the stress are stored where A asks for them (computeAllStresses).
+// The elastic and neo-Hookean steps have a variant without: the addresses kept 10
+// to 18 registers more alive, 106 -> 88 to 96, five waves per SIMD instead of
+// four; 4.4 M elements, us: elastic 130 -> 122, finite strain 141 -> 138,
+// neo-Hookean 145 -> 145.  The plastic law (198 registers) and external terms (106
+// -> 98 to 100, four waves) gain no wave and have the one variant.
 template <int LAW, bool EXT, bool MAT>
 __global__ void __launch_bounds__(PPA_TB) k_tet4_ppa(ElemArgs A) {
   extern __shared__ double2 s_rec[]; // [bl_maxu][3] records, later [t_slots][3] slots

@@ -1427,14 +1427,13 @@ void launch_hex8_strict(akx_model *m, Material &mat, const ElemArgs &A) {
 template <int LAW> void launch_tet4_ppa_law(akx_model *m, Material &mat, const ElemArgs &A) {
   const dim3 grid((unsigned)A.nblocks_padded), block(PPA_TB);
   const size_t lds = std::max((size_t)A.bl_maxu * 48, (size_t)A.t_slots * 24);
-  if (mat.ext() && A.grad_u)
+  if (mat.ext())
     hipLaunchKernelGGL((k_tet4_ppa<LAW, true, true>), grid, block, lds, m->stream, A);
-  else if (mat.ext())
-    hipLaunchKernelGGL((k_tet4_ppa<LAW, true, false>), grid, block, lds, m->stream, A);
-  else if (A.grad_u)
+  else if (LAW == LAW_PLASTIC || A.grad_u)
     hipLaunchKernelGGL((k_tet4_ppa<LAW, false, true>), grid, block, lds, m->stream, A);
   else
-    hipLaunchKernelGGL((k_tet4_ppa<LAW, false, false>), grid, block, lds, m->stream, A);
+    hipLaunchKernelGGL((k_tet4_ppa<LAW, false, LAW == LAW_PLASTIC>), grid, block, lds, m->stream,
+                       A);
 }
 
 void launch_tet4_ppa(akx_model *m, Material &mat, const ElemArgs &A) {
