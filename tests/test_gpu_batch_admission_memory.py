@@ -90,3 +90,32 @@ def test_too_many_elements_around_a_node_is_refused_and_gives_back():
     assert b.capacityLeft() == left
     b.add(M.box_mesh(TET, 3, 3, 3), "elastic")
     b.solveStep(2)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_more_nodes_than_one_round(precision):
+    """140,608 nodes: their input goes up in two rounds of up to 131,072."""
+    import numpy as np
+
+    import oracle
+
+    mesh = M.box_mesh(HEX, 51, 51, 51, jitter=0.1, seed=2)
+    rng = np.random.default_rng(4)
+    blocked = rng.random((mesh.nb_nodes, 3)) < 0.1
+    v0 = 0.05 * rng.standard_normal((mesh.nb_nodes, 3))
+    b = Batch(precision, nodes=mesh.nb_nodes + 512, hexes=mesh.nb_elements + 4096)
+    i = b.add(mesh, "elastic", E=1.2, nu=0.28, blocked=blocked, velocity=v0)
+    b.solveStep(2)
+    o = oracle.OracleModel(mesh.etype, mesh.nodes, mesh.conn, "elastic", E=1.2, nu=0.28)
+    o.init_full()
+    o.blocked[:] = blocked
+    o.v[:] = v0
+    o.set_time_step(b.timeStep(i)[0])
+    o.solve_steps(2)
+    for f, w in (("nodes", mesh.nodes), ("displacement", o.u), ("velocity", o.v),
+                 ("internal_force", o.f_int)):
+        g = b.get(i, f)
+        if precision == "fp64" or f == "nodes":
+            assert np.array_equal(g, w), f
+        else:
+            assert np.abs(g - w).max() <= 1e-5 * np.abs(w).max(), f
