@@ -4,10 +4,10 @@ device (the C ABI's ``akx_batch``).
 Each instance is what the reference runs as its own ``SolidMechanicsModel``
 with one material, ``_explicit_lumped_mass`` and zero external force
 (solid_mechanics_model.cc:186-232, model_solver.cc:267-280).  All live
-instances step together: one persistent element launch per (element type,
-law) group and one persistent nodal gather launch per step, replayed from a
-hipGraph of two steps.  An instance's results do not depend on which other
-instances share the batch.
+instances step together: an element launch for each (element type, law) group,
+in FP32 usually one for all, and a nodal gather launch per step, replayed from a
+hipGraph of 16 steps once the instances have stayed the same for 512.  An
+instance's results do not depend on which other instances share the batch.
 """
 from __future__ import annotations
 

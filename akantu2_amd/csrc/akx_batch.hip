@@ -535,7 +535,7 @@ struct HostInst {
   int64_t ell0 = 0, nell = 0;            // force-table entries
   int64_t steps = 0;                     // steps done
   bool urec = true;                      // u in the node records (BInst::urec)
-  // block-partial assembly (Tet4, FP32): the instance's block-entry range
+  // block-partial assembly (FP32): the instance's block-entry range
   // and the distinct-node count of each of its blocks
   int64_t bent0 = 0, nbent = 0;
   std::vector<int32_t> blk_cnt;

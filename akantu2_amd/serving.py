@@ -9,11 +9,10 @@ a number of steps.  The server keeps one ``Batch`` (device arenas) and loops:
    (``akx_batch_footprint``) fits the server's budget, a slot is free and the
    arenas have room; admission uploads the mesh and computes the lumped mass
    and the stable time step on the device, and the state then stays resident;
-3. one chunk of steps advances every live request together (one persistent
-   element launch per group and one gather launch per step, replayed from a
-   hipGraph); the chunk ends when the nearest request finishes or after about
-   ``chunk_ms`` of device time, so newly arrived requests wait at most one
-   chunk;
+3. one chunk of steps advances every live request together (an element launch
+   per group or one for all, and a gather launch per step); the chunk ends when
+   the nearest request finishes or after about ``chunk_ms`` of device time, so
+   newly arrived requests wait at most one chunk;
 4. finished requests are read back and retired, which frees their memory for
    the queue.
 
