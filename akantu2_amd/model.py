@@ -124,16 +124,18 @@ class _Spare:
     def put(self, name, base, snap):
         self.take(name)
         n = self._size((base, snap))
-        with _Spare._lock:
-            if _Spare._bytes + n > self.LIMIT:
+        cls = type(self)
+        with cls._lock:
+            if cls._bytes + n > cls.LIMIT:
                 return
-            _Spare._bytes += n
+            cls._bytes += n
         self._kept[name] = (base, snap)
 
     def take(self, name):
         arrays = self._kept.pop(name, (None, None))
-        with _Spare._lock:
-            _Spare._bytes -= self._size(arrays)
+        cls = type(self)  # (also while the interpreter takes its modules down)
+        with cls._lock:
+            cls._bytes -= self._size(arrays)
         return arrays
 
     def __del__(self):
