@@ -46,7 +46,7 @@ def test_admission_allocates_nothing(etype, cells, law, precision):
           f"{(after - first) / MB:.1f} MB, footprint {want / MB:.1f} MB", flush=True)
     assert after - before <= 4 * MB
     # the 4,096 elements more, the small instance, a fixed part (a round of nodes'
-    # input 6.4 MB, tables) and the driver's granularity
+    # input 6.4 MB, tables) and the allocator's granularity
     assert after - first <= 1.01 * want + 32 * MB
 
 
